@@ -1,12 +1,10 @@
 // Kernels of hybrid decoder designs: an fp32 residual stream with scalar-gain RMS norms on the
 // sublayer outputs, gated recurrences whose state lives in per-sequence fp32 slots (minGRU,
-// gated linear attention), attention with separate key / value widths under a chunk or window
-// mask over a paged cache, and a shape-agnostic GEMM for the projections that the MFMA kernels
-// (gemm*.hip: bf16, K a multiple of 64) do not take, including every product of the true-fp32
-// mode. Everything a recurrence or a softmax touches is fp32; only tensors that feed the next
+// gated linear attention), and attention with separate key / value widths under a chunk or window
+// mask over a paged cache. Everything a recurrence or a softmax touches is fp32; only tensors that feed the next
 // matrix product are written in the activation type (bf16 or fp32, a launch-time flag).
 // Pre-norm designs add: a residual step fused with a per-coordinate RMS norm or with a Dynamic Tanh
-// norm, latent attention's cached row, matrix memories, per-head products, gated units (plain and
+// norm, latent attention's cached row, matrix memories, gated units (plain and
 // clamped), and attention whose values are its keys before they rotate in neighbouring pairs.
 // The two attention kernels take options that further designs combine: row strides of the planes (values that are a
 // column block of the key rows), a cap on the scores, a bias per unit of distance, a sink in the softmax (of score zero or
@@ -1243,149 +1241,6 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(
   }
 }
 
-// ---------------------------------------------------------------- shape-agnostic GEMM
-// C[M, N] = A[M, K] W[N, K]^T (+ bias) with fp32 accumulation on the vector ALUs: 64 x 64 tiles,
-// 16-deep slabs in LDS, 4 x 4 outputs per thread. Any M, N, K; A, W and C each fp32 or bf16; A may be
-// a column slice (row stride lda).
-// epi 1: square of relu.
-template <bool AF32, bool WF32, bool CF32>
-__global__ __launch_bounds__(256) void gemm_any_kernel(const void* __restrict__ A, int lda, const void* __restrict__ W,
-                                                       const void* __restrict__ bias, void* __restrict__ C, int M, int N,
-                                                       int K, int epi) {
-  __shared__ float As[16][64 + 4];
-  __shared__ float Ws[16][64 + 4];
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const typename Act<AF32>::type* a = static_cast<const typename Act<AF32>::type*>(A);
-  const typename Act<WF32>::type* w = static_cast<const typename Act<WF32>::type*>(W);
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    for (int i = threadIdx.x; i < 64 * 16; i += 256) {
-      const int r = i >> 4, k = i & 15;
-      As[k][r] = (m0 + r < M && k0 + k < K) ? Act<AF32>::load(a, static_cast<size_t>(m0 + r) * lda + k0 + k) : 0.f;
-      Ws[k][r] = (n0 + r < N && k0 + k < K) ? Act<WF32>::load(w, static_cast<size_t>(n0 + r) * K + k0 + k) : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      float av[4], wv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        av[i] = As[k][ty * 4 + i];
-        wv[i] = Ws[k][tx * 4 + i];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += av[i] * wv[j];
-    }
-    __syncthreads();
-  }
-  typename Act<CF32>::type* c = static_cast<typename Act<CF32>::type*>(C);
-  const typename Act<WF32>::type* bs = static_cast<const typename Act<WF32>::type*>(bias);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = m0 + ty * 4 + i;
-    if (r >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int col = n0 + tx * 4 + j;
-      if (col >= N) continue;
-      float v = acc[i][j] + (bs != nullptr ? Act<WF32>::load(bs, col) : 0.f);
-      if (epi == 1) {
-        v = fmaxf(v, 0.f);
-        v *= v;
-      }
-      Act<CF32>::store(c, static_cast<size_t>(r) * N + col, v);
-    }
-  }
-}
-
-// ---------------------------------------------------------------- per-head products
-// C[m, h, :] = W[h] A[m, h, :] for H heads side by side: A [M, H*K] (row stride lda), W [H, N, K],
-// C [M, H*N]. The tiling of gemm_any_kernel with the head as the third grid dimension. With
-// ``gate`` [M, H] (row stride ld_gate) the head's outputs are scaled by sigmoid(gate[m, h]); ``gate_full``: the gate
-// is [M, H*N], one logit per output. Head h's inputs start at column h * a_hs of A, its outputs at column h * c_hs
-// of C (row stride c_ld): heads may be column blocks of wider per-head rows on either side.
-// RPT rows per thread: a block covers 16 * RPT rows x 64 columns. Few rows (decode steps) take RPT = 1, which
-// spreads the same products over four times as many waves.
-template <bool AF32, bool WF32, bool CF32, int RPT>
-__global__ __launch_bounds__(256) void head_linear_kernel(const void* __restrict__ A, int lda, const void* __restrict__ W,
-                                                          void* __restrict__ C, const float* __restrict__ gate,
-                                                          int ld_gate, int M, int H, int N, int K, int a_hs, int c_ld,
-                                                          int c_hs, int gate_full) {
-  constexpr int KS = 32;                            // slab depth: per-head depths are short, so few, deep slabs
-  constexpr int TM = 16 * RPT;
-  constexpr int NA = TM * KS / 256, NW = 64 * KS / 256;
-  __shared__ float As[KS][TM + 4];
-  __shared__ float Ws[KS][64 + 4];
-  const int h = blockIdx.z;
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * 64;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const typename Act<AF32>::type* a = static_cast<const typename Act<AF32>::type*>(A) + static_cast<size_t>(h) * a_hs;
-  const typename Act<WF32>::type* w = static_cast<const typename Act<WF32>::type*>(W) + static_cast<size_t>(h) * N * K;
-  float acc[RPT][4] = {};
-  // the next slab's elements are loaded into registers before the current one is multiplied, so the
-  // loads' latency hides behind the products
-  float ra[NA], rw[NW];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int j = 0; j < NA; ++j) {
-      const int i = threadIdx.x + 256 * j;
-      const int r = i / KS, k = i % KS;
-      ra[j] = (m0 + r < M && k0 + k < K) ? Act<AF32>::load(a, static_cast<size_t>(m0 + r) * lda + k0 + k) : 0.f;
-    }
-#pragma unroll
-    for (int j = 0; j < NW; ++j) {
-      const int i = threadIdx.x + 256 * j;
-      const int r = i / KS, k = i % KS;
-      rw[j] = (n0 + r < N && k0 + k < K) ? Act<WF32>::load(w, static_cast<size_t>(n0 + r) * K + k0 + k) : 0.f;
-    }
-  };
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += KS) {
-#pragma unroll
-    for (int j = 0; j < NA; ++j) {
-      const int i = threadIdx.x + 256 * j;
-      As[i % KS][i / KS] = ra[j];
-    }
-#pragma unroll
-    for (int j = 0; j < NW; ++j) {
-      const int i = threadIdx.x + 256 * j;
-      Ws[i % KS][i / KS] = rw[j];
-    }
-    __syncthreads();
-    if (k0 + KS < K) fetch(k0 + KS);
-#pragma unroll
-    for (int k = 0; k < KS; ++k) {
-      float av[RPT], wv[4];
-#pragma unroll
-      for (int i = 0; i < RPT; ++i) av[i] = As[k][ty * RPT + i];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) wv[i] = Ws[k][tx * 4 + i];
-#pragma unroll
-      for (int i = 0; i < RPT; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += av[i] * wv[j];
-    }
-    __syncthreads();
-  }
-  typename Act<CF32>::type* c = static_cast<typename Act<CF32>::type*>(C);
-#pragma unroll
-  for (int i = 0; i < RPT; ++i) {
-    const int r = m0 + ty * RPT + i;
-    if (r >= M) continue;
-    const float g = gate != nullptr && !gate_full ? sigmoidf_(gate[static_cast<size_t>(r) * ld_gate + h]) : 1.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int col = n0 + tx * 4 + j;
-      if (col >= N) continue;
-      const float ge = gate_full ? sigmoidf_(gate[static_cast<size_t>(r) * ld_gate + h * N + col]) : g;
-      Act<CF32>::store(c, static_cast<size_t>(r) * c_ld + static_cast<size_t>(h) * c_hs + col, acc[i][j] * ge);
-    }
-  }
-}
-
 }  // namespace
 
 // ================================================================= launchers
@@ -1682,37 +1537,6 @@ LC_EXPORT int lc_latent_write(const void* proj, int ld, int col0, int R, const v
   LC_RETURN_LAST_ERROR();
 }
 
-LC_EXPORT int lc_head_linear(const void* A, int a_f32, int lda, const void* W, int w_f32, void* C, int c_f32,
-                             const void* gate, int ld_gate, int M, int H, int N, int K, int a_hs, int c_ld, int c_hs,
-                             int gate_full, hipStream_t st) {
-  if (M <= 0 || N <= 0 || H <= 0) return 0;
-  if (K <= 0 || a_hs < K || lda < (H - 1) * a_hs + K || H > 65535 || c_hs < N || c_ld < (H - 1) * c_hs + N) return -1;
-  if (gate != nullptr && ld_gate < (gate_full ? H * N : H)) return -1;
-  if (gate == nullptr && gate_full) return -1;
-  const bool few = M <= 64;                          // decode steps: one row per thread, four times the blocks
-  const dim3 grid((N + 63) / 64, few ? (M + 15) / 16 : (M + 63) / 64, H), block(256);
-#define LC_HL(A32, W32, C32)                                                                                       \
-  if (few)                                                                                                         \
-    head_linear_kernel<A32, W32, C32, 1><<<grid, block, 0, st>>>(A, lda, W, C, static_cast<const float*>(gate), ld_gate, \
-                                                                 M, H, N, K, a_hs, c_ld, c_hs, gate_full);         \
-  else                                                                                                             \
-    head_linear_kernel<A32, W32, C32, 4><<<grid, block, 0, st>>>(A, lda, W, C, static_cast<const float*>(gate), ld_gate, \
-                                                                 M, H, N, K, a_hs, c_ld, c_hs, gate_full)
-  const int sel = (a_f32 ? 4 : 0) | (w_f32 ? 2 : 0) | (c_f32 ? 1 : 0);
-  switch (sel) {
-    case 0: LC_HL(false, false, false); break;
-    case 1: LC_HL(false, false, true); break;
-    case 2: LC_HL(false, true, false); break;
-    case 3: LC_HL(false, true, true); break;
-    case 4: LC_HL(true, false, false); break;
-    case 5: LC_HL(true, false, true); break;
-    case 6: LC_HL(true, true, false); break;
-    default: LC_HL(true, true, true); break;
-  }
-#undef LC_HL
-  LC_RETURN_LAST_ERROR();
-}
-
 LC_EXPORT int lc_headnorm_gate(const void* o, const void* w, const void* gate, int ld_gate, void* out, int act_f32,
                                int T, int H, int Dv, float eps, int ld_head, int w_stride, int gate_kind, const void* m,
                                int ld_out, hipStream_t st) {
@@ -1846,27 +1670,5 @@ LC_EXPORT int lc_attn_tile(const void* q, const void* kc, const void* vc, int ca
   else LC_TILE(false, false);
 #undef LC_TILE
 #undef LC_TILE_K
-  LC_RETURN_LAST_ERROR();
-}
-
-// A may be a column slice of a wider matrix: ``lda`` is its row stride in elements.
-LC_EXPORT int lc_gemm_any(const void* A, int a_f32, int lda, const void* W, int w_f32, const void* bias, void* C,
-                          int c_f32, int M, int N, int K, int epi, hipStream_t st) {
-  if (M <= 0 || N <= 0) return 0;
-  if (K <= 0 || lda < K) return -1;
-  const dim3 grid((N + 63) / 64, (M + 63) / 64), block(256);
-#define LC_GA(A32, W32, C32) gemm_any_kernel<A32, W32, C32><<<grid, block, 0, st>>>(A, lda, W, bias, C, M, N, K, epi)
-  const int sel = (a_f32 ? 4 : 0) | (w_f32 ? 2 : 0) | (c_f32 ? 1 : 0);
-  switch (sel) {
-    case 0: LC_GA(false, false, false); break;
-    case 1: LC_GA(false, false, true); break;
-    case 2: LC_GA(false, true, false); break;
-    case 3: LC_GA(false, true, true); break;
-    case 4: LC_GA(true, false, false); break;
-    case 5: LC_GA(true, false, true); break;
-    case 6: LC_GA(true, true, false); break;
-    default: LC_GA(true, true, true); break;
-  }
-#undef LC_GA
   LC_RETURN_LAST_ERROR();
 }

@@ -1,7 +1,6 @@
 // Routed feed-forwards of hybrid decoder designs: a softmax or sigmoid router (or a softmax over the chosen logits) with a bias-corrected,
 // group-limited top-k choice, a counting sort of the (token, choice) pairs by expert for any number
-// of experts, per-expert products of any shape and type over the sorted rows (fp32 accumulation on
-// the vector ALUs, like the shape-agnostic GEMM), and the fp32 mix of the chosen experts' outputs,
+// of experts, and the fp32 mix of the chosen experts' outputs,
 // in which experts without tensors ("identity experts") return their input.
 #include "hybrid_common.h"
 
@@ -163,79 +162,6 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t* __restric
   }
 }
 
-// ---------------------------------------------------------------- per-expert products over sorted rows
-// Sorted position p in [offsets[e], offsets[e + 1]) gives C[p] = W[e] A[row_index[p]] (A[p] without
-// an index); W [E, N, K]. Tiles of 64 positions x 64 columns as in the shape-agnostic GEMM; tile
-// blockIdx.y belongs to the expert whose run of tiles it falls into (experts are walked in order;
-// at most ceil(rows / 64) + E tiles exist). epi 1: square of relu.
-template <bool AF32, bool WF32, bool CF32>
-__global__ __launch_bounds__(256) void gemm_any_grouped_kernel(const void* __restrict__ A, int lda,
-                                                               const int32_t* __restrict__ row_index,
-                                                               const int32_t* __restrict__ offsets,
-                                                               const void* __restrict__ W, void* __restrict__ C, int E,
-                                                               int N, int K, int epi) {
-  __shared__ float As[16][64 + 4];
-  __shared__ float Ws[16][64 + 4];
-  __shared__ int rows[64];
-  int e = 0, tile = blockIdx.y, lo = 0, hi = 0;
-  for (; e < E; ++e) {
-    lo = offsets[e];
-    hi = offsets[e + 1];
-    const int nt = (hi - lo + 63) >> 6;
-    if (tile < nt) break;
-    tile -= nt;
-  }
-  if (e >= E) return;                                // the same for the whole block
-  const int p0 = lo + tile * 64;
-  const int M = min(64, hi - p0);
-  const int n0 = blockIdx.x * 64;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  if (threadIdx.x < 64) rows[threadIdx.x] = threadIdx.x < M ? (row_index != nullptr ? row_index[p0 + threadIdx.x] : p0 + threadIdx.x) : 0;
-  __syncthreads();
-  const typename Act<AF32>::type* a = static_cast<const typename Act<AF32>::type*>(A);
-  const typename Act<WF32>::type* w = static_cast<const typename Act<WF32>::type*>(W) + static_cast<size_t>(e) * N * K;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    for (int i = threadIdx.x; i < 64 * 16; i += 256) {
-      const int r = i >> 4, k = i & 15;
-      As[k][r] = (r < M && k0 + k < K) ? Act<AF32>::load(a, static_cast<size_t>(rows[r]) * lda + k0 + k) : 0.f;
-      Ws[k][r] = (n0 + r < N && k0 + k < K) ? Act<WF32>::load(w, static_cast<size_t>(n0 + r) * K + k0 + k) : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      float av[4], wv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        av[i] = As[k][ty * 4 + i];
-        wv[i] = Ws[k][tx * 4 + i];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += av[i] * wv[j];
-    }
-    __syncthreads();
-  }
-  typename Act<CF32>::type* c = static_cast<typename Act<CF32>::type*>(C);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = ty * 4 + i;
-    if (r >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int col = n0 + tx * 4 + j;
-      if (col >= N) continue;
-      float v = acc[i][j];
-      if (epi == 1) {
-        v = fmaxf(v, 0.f);
-        v *= v;
-      }
-      Act<CF32>::store(c, static_cast<size_t>(p0 + r) * N + col, v);
-    }
-  }
-}
-
 // ---------------------------------------------------------------- mix of the chosen experts
 // out[t] = sum_k wts[t, k] * (ye[slot_of[t, k]] if ids[t, k] < E else h[t]) (+ shared[t]), fp32. One block per token.
 // No weights given: 1 (designs whose weight went into the expert's input). ``shared_gate`` (one logit per token,
@@ -291,33 +217,6 @@ LC_EXPORT int lc_moe_sort(const void* ids, int T, int top, int n, void* offsets,
   moe_sort_kernel<<<dim3(1), dim3(1024), 2 * static_cast<size_t>(n) * sizeof(int), st>>>(
       static_cast<const int32_t*>(ids), T * top, top, n, static_cast<int32_t*>(offsets), static_cast<int32_t*>(sorted_src),
       static_cast<int32_t*>(slot_of), static_cast<const float*>(wts), static_cast<float*>(sorted_wts));
-  LC_RETURN_LAST_ERROR();
-}
-
-// ``rows``: an upper bound of offsets[E] known to the host (tokens x choices).
-LC_EXPORT int lc_gemm_any_grouped(const void* A, int a_f32, int lda, const void* row_index, const void* offsets,
-                                  const void* W, int w_f32, void* C, int c_f32, int rows, int E, int N, int K, int epi,
-                                  hipStream_t st) {
-  if (rows <= 0 || N <= 0 || E <= 0) return 0;
-  if (K <= 0 || lda < K) return -1;
-  const int tiles = (rows + 63) / 64 + E;
-  if (tiles > 65535) return -1;
-  const dim3 grid((N + 63) / 64, tiles), block(256);
-#define LC_GG(A32, W32, C32)                                                                                     \
-  gemm_any_grouped_kernel<A32, W32, C32><<<grid, block, 0, st>>>(A, lda, static_cast<const int32_t*>(row_index), \
-                                                                 static_cast<const int32_t*>(offsets), W, C, E, N, K, epi)
-  const int sel = (a_f32 ? 4 : 0) | (w_f32 ? 2 : 0) | (c_f32 ? 1 : 0);
-  switch (sel) {
-    case 0: LC_GG(false, false, false); break;
-    case 1: LC_GG(false, false, true); break;
-    case 2: LC_GG(false, true, false); break;
-    case 3: LC_GG(false, true, true); break;
-    case 4: LC_GG(true, false, false); break;
-    case 5: LC_GG(true, false, true); break;
-    case 6: LC_GG(true, true, false); break;
-    default: LC_GG(true, true, true); break;
-  }
-#undef LC_GG
   LC_RETURN_LAST_ERROR();
 }
 

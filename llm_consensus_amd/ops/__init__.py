@@ -126,7 +126,7 @@ class LinearWeight:
         """W row-major [N, K] in final row order (already interleaved when swiglu). With
         ``any_shape`` a weight the MFMA kernels do not take (fp32, or a reduction depth that is
         no multiple of 64) stays row-major on the GPU too and goes through the shape-agnostic
-        kernel (hybrid.hip); without it such a weight is an error at the first product."""
+        kernels (hybrid_gemm.hip); without it such a weight is an error at the first product."""
         device = torch.device(device) if device is not None else W.device
         N, K = W.shape
         W = W.to(device=device, dtype=dtype)
@@ -884,8 +884,7 @@ def _f32flag(dtype: torch.dtype) -> int:
 
 
 def linear_any(x: torch.Tensor, w: LinearWeight, out_f32: bool = True, epi_relu2: bool = False) -> torch.Tensor:
-    """y = x W^T (+ bias) for a row-major weight of any shape and type (fp32 accumulation on the
-    vector ALUs). ``epi_relu2``: the square of relu in the epilogue."""
+    """y = x W^T (+ bias) for a row-major weight of any shape and type (fp32 matrix instructions). ``epi_relu2``: the square of relu in the epilogue."""
     M = x.shape[0]
     odt = torch.float32 if out_f32 else torch.bfloat16
     if x.shape[1] != w.k:
@@ -1425,7 +1424,7 @@ def grouped_linear(x: torch.Tensor, row_index: Optional[torch.Tensor], offsets: 
                    out_dtype: torch.dtype, rows: int, relu2_epi: bool = False, glu_clamp=None) -> torch.Tensor:
     """Per-expert products over expert-sorted rows: position p in [offsets[e], offsets[e+1]) gives
     W[e] x[row_index[p]] (x[p] without an index); ``relu2_epi``: square of relu. W is either a
-    row-major tensor [E, N, K] of any shape and type (fp32 accumulation on the vector ALUs) or
+    row-major tensor [E, N, K] of any shape and type (fp32 matrix instructions) or
     packed ``ExpertWeights`` (bf16 activations, the grouped MFMA kernels: one panel per expert for a
     few hundred rows, 128 x 128 tiles beyond). Positions of experts >= E are left unwritten.
     ``glu_clamp`` = (row_scale fp32 [rows] or None, limit, slope, shift), packed weights marked ``swiglu``

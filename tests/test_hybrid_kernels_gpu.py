@@ -46,6 +46,24 @@ def test_gemm_any(a_dt, w_dt, out_f32, M, N, K):
         torch.testing.assert_close(y, want, **tol)
 
 
+# rows kernel: 1, 2 and 4 row tiles, 4 and 16 waves, a last chunk of the depth that is short; tile kernel: 1, 2 and 4 depth
+# groups, groups whose last slabs lie behind the depth; widths and depths off every border; a column slice off the 16-byte border
+@pytest.mark.parametrize("M,N,K,first", [(1, 33, 1024, 0), (16, 1024, 500, 4), (17, 48, 129, 0), (33, 17000, 64, 0), (64, 96, 1000, 1),
+                                         (65, 65, 260, 0), (130, 31, 4096, 3), (300, 4000, 132, 8), (600, 6100, 127, 0), (67, 9000, 20, 4)])
+@pytest.mark.parametrize("a_dt,w_dt", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16), (torch.bfloat16, torch.bfloat16)])
+def test_gemm_any_edges(a_dt, w_dt, M, N, K, first):
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    wide = torch.randn(M, first + K + 4, generator=g, device=DEV).to(a_dt)
+    wide[:, :first] = float("nan")                    # what stands beside the slice is not read as an operand
+    wide[:, first + K:] = float("nan")
+    W = (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).to(w_dt)
+    w = ops.LinearWeight.from_dense(W, torch.randn(N, generator=g, device=DEV), DEV, dtype=w_dt, plain=True)
+    got = ops.linear_any(wide[:, first:first + K], w)
+    want = wide[:, first:first + K].double() @ W.double().T + w.bias.double()
+    # fp32 sums of K products of about unit variance over sqrt(K): well inside K eps / 2 of the largest sums
+    torch.testing.assert_close(got.double(), want, atol=2e-5, rtol=2e-5)
+
+
 @pytest.mark.parametrize("dt", ACTS)
 def test_embed_rows_and_scalar_norm(dt):
     g = torch.Generator().manual_seed(1)
