@@ -1032,3 +1032,25 @@ def test_portions_in_tiles_of_32_keys(D, Dv, BSZ, chunk, window):
                                       n_portions=3, portion_rows=235, max_len=longest, out=wide[:, 8:8 + H * Dv], value_share=share, **dopt)
                 torch.testing.assert_close(got.float().cpu(), want, **(_tol(dt) if dt == torch.bfloat16 else dict(atol=3e-5, rtol=3e-5)))
                 assert not wide[:, :8].any() and not wide[:, 8 + H * Dv:].any()
+
+
+# widths with value heads side by side (one launch, two launches, four heads in one) and the widest keys; scores whose cap is
+# far (series) and near (library tanh); a silent entry of score zero; one and two groups of waves
+@pytest.mark.parametrize("D,Dv,G,every", [(128, 128, 2, True), (128, 128, 4, True), (64, 32, 4, True), (192, 128, 1, False), (192, 256, 1, False),
+                                          (128, 256, 2, False)])
+@pytest.mark.parametrize("cap,gain,sink,window", [(50.0, 1.0, True, 0), (4.0, 6.0, True, 33), (0.0, 1.0, True, 90), (20.0, 3.0, False, 0)])
+def test_caps_sinks_and_value_heads_in_tiles_of_32_keys(D, Dv, G, every, cap, gain, sink, window):
+    g = torch.Generator().manual_seed(D + Dv + window + G)
+    H, BSZ, MB = 4, 32, 11
+    lens, starts = [65, 16, 150], [0, 301, 77]
+    cu, pos, rs = _seqs(lens, starts)
+    T = int(cu[-1])
+    tables = torch.randperm(3 * MB, generator=g).to(torch.int32).view(3, MB)
+    q = gain * torch.randn(T, H * D, generator=g)
+    kc, vc = torch.randn(3 * MB, G, BSZ, D, generator=g).bfloat16(), torch.randn(3 * MB, G, BSZ, Dv, generator=g).bfloat16()
+    want = ref.attn_masked(q, kc, vc, tables, cu, pos, H, G, D, Dv, D ** -0.5, 0, window, torch.float32, cap, sink, every)
+    c = lambda t: t.to(DEV)   # noqa: E731
+    for dt, longest in ((torch.float32, 150), (torch.float32, 20000), (torch.bfloat16, 150)):
+        got = ops.attn_masked(c(q), c(kc), c(vc), c(tables), c(cu), c(rs), c(pos), H, G, D, Dv, D ** -0.5, 0, window, dt, n_portions=3,
+                              portion_rows=T, max_len=longest, softcap=cap, sink=sink, all_value_heads=every)
+        torch.testing.assert_close(got.float().cpu(), want, **(_tol(dt) if dt == torch.bfloat16 else dict(atol=3e-5, rtol=3e-5)))
