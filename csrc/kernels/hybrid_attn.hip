@@ -71,6 +71,34 @@ LC_DEVICE void split3_any(float a, float b, uint32_t& w0, uint32_t& w1, uint32_t
   w0 = ua | (ub << 16);
 }
 
+// Eight neighbouring numbers of a row times s, and the eight weights of a lane, as operands.
+LC_DEVICE void split_row8(const float* src, float s, bf16x8& a0, bf16x8& a1, bf16x8& a2) {
+  const float4 x = *reinterpret_cast<const float4*>(src), y = *reinterpret_cast<const float4*>(src + 4);
+  uint32_t c[3][4];
+  split3_any(x.x * s, x.y * s, c[0][0], c[1][0], c[2][0]);
+  split3_any(x.z * s, x.w * s, c[0][1], c[1][1], c[2][1]);
+  split3_any(y.x * s, y.y * s, c[0][2], c[1][2], c[2][2]);
+  split3_any(y.z * s, y.w * s, c[0][3], c[1][3], c[2][3]);
+  a0 = __builtin_bit_cast(bf16x8, u32x4{c[0][0], c[0][1], c[0][2], c[0][3]});
+  a1 = __builtin_bit_cast(bf16x8, u32x4{c[1][0], c[1][1], c[1][2], c[1][3]});
+  a2 = __builtin_bit_cast(bf16x8, u32x4{c[2][0], c[2][1], c[2][2], c[2][3]});
+}
+LC_DEVICE void split_weights(const float (&p)[2][4], bf16x8& a0, bf16x8& a1, bf16x8& a2) {
+  uint32_t c[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) split3(p[i >> 1][2 * (i & 1)], p[i >> 1][2 * (i & 1) + 1], c[0][i], c[1][i], c[2][i]);
+  a0 = __builtin_bit_cast(bf16x8, u32x4{c[0][0], c[0][1], c[0][2], c[0][3]});
+  a1 = __builtin_bit_cast(bf16x8, u32x4{c[1][0], c[1][1], c[1][2], c[1][3]});
+  a2 = __builtin_bit_cast(bf16x8, u32x4{c[2][0], c[2][1], c[2][2], c[2][3]});
+}
+// Values as the operand's transpose: lane lr of a group of 16 addresses four columns of row lr >> 2 and receives column lr of the
+// four rows; the second four rows stand ``skip`` numbers on.
+LC_DEVICE bf16x8 transposed8(bf16_t* p, int skip) {
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + skip));
+  return bf16x8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+}
+
 // tanh to fp32 accuracy: small arguments (capped scores mostly are) by the odd series, whose next term is 2e-10 of the result
 // at 1/4; a wave with any larger one takes the library function.
 LC_DEVICE float tanh_series(float x) {
@@ -154,22 +182,7 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void attn_keys32_kernel(TileArgs a
     const float* src = a.q + (static_cast<size_t>(row0 + 16 * wave + (on ? lr : 0)) * a.H + h) * D + 8 * lk;
     const float s = on ? a.scale * (CAP ? 1.f : kLog2e) : 0.f;
 #pragma unroll
-    for (int kk = 0; kk < DK; ++kk) {
-      const float4 x = *reinterpret_cast<const float4*>(src + 32 * kk), y = *reinterpret_cast<const float4*>(src + 32 * kk + 4);
-      u32x4 w0, w1, w2;
-      uint32_t c0, c1, c2;
-      split3_any(x.x * s, x.y * s, c0, c1, c2);
-      w0.x = c0, w1.x = c1, w2.x = c2;
-      split3_any(x.z * s, x.w * s, c0, c1, c2);
-      w0.y = c0, w1.y = c1, w2.y = c2;
-      split3_any(y.x * s, y.y * s, c0, c1, c2);
-      w0.z = c0, w1.z = c1, w2.z = c2;
-      split3_any(y.z * s, y.w * s, c0, c1, c2);
-      w0.w = c0, w1.w = c1, w2.w = c2;
-      q[0][kk] = __builtin_bit_cast(bf16x8, w0);
-      q[1][kk] = __builtin_bit_cast(bf16x8, w1);
-      q[2][kk] = __builtin_bit_cast(bf16x8, w2);
-    }
+    for (int kk = 0; kk < DK; ++kk) split_row8(src + 32 * kk, s, q[0][kk], q[1][kk], q[2][kk]);
   }
   // staging: a tile's keys lie in one block of the cache (its size is a multiple of 32)
   u32x4 kr[KU], vr[VU];
@@ -295,32 +308,13 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void attn_keys32_kernel(TileArgs a
           for (int r = 0; r < 4; ++r) o[t][r] *= corr;
       }
       bf16x8 w[3];
-      {
-        u32x4 w0, w1, w2;
-        uint32_t c0, c1, c2;
-        split3(p[0][0], p[0][1], c0, c1, c2);
-        w0.x = c0, w1.x = c1, w2.x = c2;
-        split3(p[0][2], p[0][3], c0, c1, c2);
-        w0.y = c0, w1.y = c1, w2.y = c2;
-        split3(p[1][0], p[1][1], c0, c1, c2);
-        w0.z = c0, w1.z = c1, w2.z = c2;
-        split3(p[1][2], p[1][3], c0, c1, c2);
-        w0.w = c0, w1.w = c1, w2.w = c2;
-        w[0] = __builtin_bit_cast(bf16x8, w0);
-        w[1] = __builtin_bit_cast(bf16x8, w1);
-        w[2] = __builtin_bit_cast(bf16x8, w2);
-      }
-      // lane lr of a group of 16 addresses row 4 lk + (lr >> 2), columns 4 (lr & 3) .. + 3, and receives column lr of the four rows
+      split_weights(p, w[0], w[1], w[2]);
       bf16_t* vs = Vs + buf * kKeys * VS + (4 * lk + (lr >> 2)) * VS + 4 * (lr & 3);
 #pragma unroll
       for (int t = 0; t < VT; t += 4) {
         bf16x8 v[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vs + 16 * (t + i)));
-          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vs + 16 * VS + 16 * (t + i)));
-          v[i] = bf16x8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        }
+        for (int i = 0; i < 4; ++i) v[i] = transposed8(vs + 16 * (t + i), 16 * VS);
 #pragma unroll
         for (int c = 2; c >= 0; --c)                 // the small parts first; four independent chains
 #pragma unroll
@@ -360,6 +354,252 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void attn_keys32_kernel(TileArgs a
   typename Act<AF32>::type* dst = static_cast<typename Act<AF32>::type*>(a.out) + tok * a.o_row + static_cast<size_t>(h) * a.o_ld + a.o_col0 + 4 * lk;
 #pragma unroll
   for (int t = 0; t < VT; ++t) store_act4<AF32>(dst, 16 * t, make_float4(o[t][0] * fin, o[t][1] * fin, o[t][2] * fin, o[t][3] * fin));
+}
+
+// ---------------------------------------------------------------- single rows (decoded tokens, short portions)
+// The same products for ONE row: the operand's 16 "rows" are the query heads that share a key head, so that a key is read once
+// for all of them. Bound by the latency of a chain of key tiles: a block is eight waves that take the row's tiles of 32 keys in
+// turn and join their sums in LDS. Blocks along z take 64 or 128 value columns each (of one wide head, or of the value heads side
+// by side; scores are formed again there). A wave reads its keys straight into operands; bf16 values pass through a patch of LDS
+// of the wave's own to be read transposed. Over fp32 planes both products run on v_mfma_f32_16x16x4_f32, whose operands come
+// from memory as they lie (depth 16 kk + 4 (lane >> 4) + i of a key, four neighbouring value columns of a lane).
+// Against a wave per (row, head) that walked its keys alone (attn_masked_kernel, hybrid.hip, which still serves the other widths and
+// block sizes): 4 rows over 700 keys, 16 heads on the values of 4: 110 -> 16 us; over latent rows of 192: 65 -> 18 us; 32 rows over
+// 60-100 keys, two maps of 128 over values of 256: 15.3 -> 7.7 us; 3 fp32 rows over 330 keys: 51 -> 21 us.
+constexpr int kRowWaves = 8;
+
+struct RowArgs {
+  const float* q;                // [T, H * D]
+  const void* kc;
+  const void* vc;
+  const int32_t* block_tables;
+  int MB;
+  const int32_t* row_seq;
+  const int32_t* positions;
+  void* out;
+  int H, G, BS;
+  float scale;
+  int chunk, window, k_ld, v_ld, v_share;
+  float softcap;
+  int sink;
+  const float* sinks;
+  const float* slopes;           // score taken off per unit of distance, per head (null: none)
+  int keep;                      // first keys visible whatever the window or chunk
+  const float* gate;
+  int ld_gate;
+  float out_scale;
+  int o_row, o_ld, vh0, head_cols;
+};
+
+template <bool CF32, bool AF32, int DK, int VT>
+__global__ __launch_bounds__(64 * kRowWaves, 2) void attn_rows_kernel(RowArgs a) {
+  constexpr int D = 32 * DK, NC = 16 * VT, VS = NC + 16;
+  constexpr int kPatch = kKeys * VS;                 // bf16 numbers; at least the NC * 16 sums of a wave
+  static_assert(kPatch * 2 >= NC * 16 * 4, "a wave's sums fit its patch");
+  __shared__ __attribute__((aligned(16))) bf16_t patch[kRowWaves][kPatch];
+  __shared__ float ms[kRowWaves][16], ls[kRowWaves][16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+  const int t = blockIdx.x;
+  const int seq = a.row_seq[t], p = a.positions[t];
+  if (seq < 0 || p < 0) return;                      // the same for the whole block
+  const int per = a.H / a.G, parts = (per + 15) / 16;
+  const int g = blockIdx.y / parts, h0 = g * per + 16 * (blockIdx.y % parts), nh = min(16, (g + 1) * per - h0);
+  const int h = h0 + min(lr, nh - 1);
+  int lo = 0;
+  if (a.chunk > 0) lo = (p / a.chunk) * a.chunk;
+  if (a.window > 0) lo = max(lo, p - a.window + 1);
+  const int32_t* table = a.block_tables + static_cast<size_t>(seq) * a.MB;
+  // tiles of 32 keys that lie in one block of the cache: those of the kept first keys, then those from lo on
+  const int kept = min((min(a.keep, lo) + kKeys - 1) / kKeys, lo / kKeys), tiles = kept + p / kKeys - lo / kKeys + 1;
+  const int c0 = blockIdx.z * NC;                    // this block's first column
+  const int vhead = a.vh0 >= 0 ? a.vh0 + c0 / a.head_cols : g / a.v_share, GV = a.G / a.v_share;
+  const int vcol = a.vh0 >= 0 ? c0 % a.head_cols : c0;
+  const float slope = a.slopes != nullptr ? a.slopes[h] : 0.f;
+  constexpr int QF = CF32 ? 2 * DK : 1, QS = CF32 ? 1 : DK;
+  float4 qf[QF];
+  bf16x8 qs[3][QS];
+  {
+    const float* src = a.q + (static_cast<size_t>(t) * a.H + h) * D;
+    if constexpr (CF32) {
+#pragma unroll
+      for (int kk = 0; kk < 2 * DK; ++kk) {
+        const float4 v = *reinterpret_cast<const float4*>(src + 16 * kk + 4 * lk);
+        qf[kk] = make_float4(v.x * a.scale, v.y * a.scale, v.z * a.scale, v.w * a.scale);
+      }
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < DK; ++kk) split_row8(src + 32 * kk + 8 * lk, a.scale, qs[0][kk], qs[1][kk], qs[2][kk]);
+    }
+  }
+  float m = -INFINITY, l = 0.f;
+  f32x4 o[VT];
+#pragma unroll
+  for (int i = 0; i < VT; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16_t* own = patch[wave];
+  for (int i = wave; i < tiles; i += kRowWaves) {
+    const int j0 = (i < kept ? i : lo / kKeys + i - kept) * kKeys;
+    const size_t block = table[j0 / a.BS];
+    const int off = j0 % a.BS;
+    const size_t k_at = ((block * a.G + g) * a.BS + off) * a.k_ld, v_at = ((block * GV + vhead) * a.BS + off) * a.v_ld + vcol;
+    f32x4 s[2][2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) s[e][0] = s[e][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int VU = CF32 ? 1 : NC / 16;           // 16-byte units of the values per lane
+    u32x4 vr[VU];
+    if constexpr (CF32) {
+      const float* kb = static_cast<const float*>(a.kc) + k_at + 4 * lk;
+#pragma unroll
+      for (int kk = 0; kk < 2 * DK; ++kk)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float4 k = *reinterpret_cast<const float4*>(kb + (16 * e + lr) * a.k_ld + 16 * kk);
+          s[e][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.x, qf[kk].x, s[e][0], 0, 0, 0);
+          s[e][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.y, qf[kk].y, s[e][1], 0, 0, 0);
+          s[e][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.z, qf[kk].z, s[e][0], 0, 0, 0);
+          s[e][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.w, qf[kk].w, s[e][1], 0, 0, 0);
+        }
+    } else {
+      const bf16_t* kb = static_cast<const bf16_t*>(a.kc) + k_at + 8 * lk;
+      const bf16_t* vb = static_cast<const bf16_t*>(a.vc) + v_at;
+      bf16x8 k[DK][2];
+#pragma unroll
+      for (int kk = 0; kk < DK; ++kk)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) k[kk][e] = *reinterpret_cast<const bf16x8*>(kb + (16 * e + lr) * a.k_ld + 32 * kk);
+#pragma unroll
+      for (int u = 0; u < VU; ++u) {                 // (in flight while the scores are formed)
+        const int x = lane + 64 * u;
+        vr[u] = *reinterpret_cast<const u32x4*>(vb + (x / (NC / 8)) * a.v_ld + (x % (NC / 8)) * 8);
+      }
+#pragma unroll
+      for (int kk = 0; kk < DK; ++kk) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) s[e][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[kk][e], qs[2][kk], s[e][1], 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) s[e][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[kk][e], qs[0][kk], s[e][0], 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) s[e][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[kk][e], qs[1][kk], s[e][1], 0, 0, 0);
+      }
+    }
+    float w[2][4];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int j = j0 + 16 * e + 4 * lk + r;
+        float x = s[e][0][r] + s[e][1][r] - slope * static_cast<float>(p - j);
+        if (a.softcap > 0.f) x = a.softcap * tanhf(x / a.softcap);
+        w[e][r] = j <= p && (j >= lo || j < a.keep) ? x * kLog2e : -INFINITY;
+      }
+    const float top = fmaxf(fmaxf(fmaxf(w[0][0], w[0][1]), fmaxf(w[0][2], w[0][3])), fmaxf(fmaxf(w[1][0], w[1][1]), fmaxf(w[1][2], w[1][3])));
+    const float mn = fmaxf(m, swap_max(top));
+    const float base = mn == -INFINITY ? 0.f : mn;
+    const float corr = fast_exp2(m - base);
+    m = mn;
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) w[e][r] = fast_exp2(w[e][r] - base);
+    l = l * corr + (((w[0][0] + w[0][1]) + (w[0][2] + w[0][3])) + ((w[1][0] + w[1][1]) + (w[1][2] + w[1][3])));
+#pragma unroll
+    for (int i2 = 0; i2 < VT; ++i2)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[i2][r] *= corr;
+    if constexpr (CF32) {
+      const float* vb = static_cast<const float*>(a.vc) + v_at;
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = 16 * e + 4 * lk + r;
+          const bool on = j0 + key <= p;             // (cells nobody wrote may hold no numbers)
+#pragma unroll
+          for (int c = 0; c < VT; c += 4) {
+            float4 v = *reinterpret_cast<const float4*>(vb + key * a.v_ld + 16 * c + 4 * lr);
+            if (!on) v = make_float4(0.f, 0.f, 0.f, 0.f);
+            o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.x, w[e][r], o[c], 0, 0, 0);
+            o[c + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.y, w[e][r], o[c + 1], 0, 0, 0);
+            o[c + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.z, w[e][r], o[c + 2], 0, 0, 0);
+            o[c + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.w, w[e][r], o[c + 3], 0, 0, 0);
+          }
+        }
+    } else {
+#pragma unroll
+      for (int u = 0; u < VU; ++u) {
+        const int x = lane + 64 * u, key = x / (NC / 8);
+        if (j0 + key > p) vr[u] = u32x4{0u, 0u, 0u, 0u};
+        *reinterpret_cast<u32x4*>(own + key * VS + (x % (NC / 8)) * 8) = vr[u];
+      }
+      bf16x8 ws[3];
+      split_weights(w, ws[0], ws[1], ws[2]);
+      // the patch is this wave's own: its LDS accesses execute in order, the fences keep the compiler from moving them
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      bf16_t* vs = own + (4 * lk + (lr >> 2)) * VS + 4 * (lr & 3);
+#pragma unroll
+      for (int c = 0; c < VT; c += 4) {
+        bf16x8 v[4];
+#pragma unroll
+        for (int i2 = 0; i2 < 4; ++i2) v[i2] = transposed8(vs + 16 * (c + i2), 16 * VS);
+#pragma unroll
+        for (int x = 2; x >= 0; --x)
+#pragma unroll
+          for (int i2 = 0; i2 < 4; ++i2) o[c + i2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[i2], ws[x], o[c + i2], 0, 0, 0);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");       // read before the next tile overwrites it
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  l = swap_sum(l);
+  if (lk == 0) {
+    ms[wave][lr] = m;
+    ls[wave][lr] = l;
+  }
+  const int used = min(tiles, kRowWaves);            // waves that took a tile
+  if (wave < used) {
+    float* mine = reinterpret_cast<float*>(own);
+#pragma unroll
+    for (int c = 0; c < VT; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mine[(4 * c + r) * 64 + lane] = o[c][r];
+  }
+  __syncthreads();
+  const float sink0 = a.sinks != nullptr ? a.sinks[h] * kLog2e : 0.f;
+  float top = a.sink ? sink0 : -INFINITY;
+  for (int i = 0; i < used; ++i) top = fmaxf(top, ms[i][lr]);
+  const float base = top == -INFINITY ? 0.f : top;
+  float sum = a.sink ? fast_exp2(sink0 - base) : 0.f;
+  f32x4 x[(VT + kRowWaves - 1) / kRowWaves];
+#pragma unroll
+  for (int c = 0; c < (VT + kRowWaves - 1) / kRowWaves; ++c) x[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < used; ++i) {
+    const float f = fast_exp2(ms[i][lr] - base);
+    sum += f * ls[i][lr];
+    const float* theirs = reinterpret_cast<const float*>(patch[i]);
+#pragma unroll
+    for (int c = 0; c < (VT + kRowWaves - 1) / kRowWaves; ++c) {
+      const int tile = wave + kRowWaves * c;
+      if (tile < VT) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[c][r] += f * theirs[(4 * tile + r) * 64 + lane];
+      }
+    }
+  }
+  if (lr >= nh) return;
+  const float fin = a.out_scale * (a.gate != nullptr ? sigmoidf_(a.gate[static_cast<size_t>(t) * a.ld_gate + h]) : 1.f) / sum;
+  typename Act<AF32>::type* dst = static_cast<typename Act<AF32>::type*>(a.out) + static_cast<size_t>(t) * a.o_row + static_cast<size_t>(h) * a.o_ld + c0;
+#pragma unroll
+  for (int c = 0; c < (VT + kRowWaves - 1) / kRowWaves; ++c) {
+    const int tile = wave + kRowWaves * c;
+    if (tile >= VT) continue;
+    if constexpr (CF32) {                            // (accumulator c's columns are 64 (c / 4) + 4 (4 lk + r) + c % 4)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) Act<AF32>::store(dst, 64 * (tile / 4) + 4 * (4 * lk + r) + tile % 4, x[c][r] * fin);
+    } else {
+      store_act4<AF32>(dst, 16 * tile + 4 * lk, make_float4(x[c][0] * fin, x[c][1] * fin, x[c][2] * fin, x[c][3] * fin));
+    }
+  }
 }
 
 }  // namespace
@@ -424,5 +664,50 @@ LC_EXPORT int lc_attn_keys32(const void* q, const void* kc, const void* vc, cons
   else LC_K32(12, 16);
 #undef LC_K32
 #undef LC_K32_G
+  LC_RETURN_LAST_ERROR();
+}
+
+// Columns per block of attn_rows_kernel for these widths (0: it does not take them).
+static int rows_cols(int D, int Dv, int BS) {
+  if (BS % kKeys || (D != 64 && D != 128 && D != 192)) return 0;
+  return Dv % 128 == 0 ? 128 : Dv % 64 == 0 ? 64 : 0;
+}
+
+// Whether lc_attn_rows takes the shape (1) or not (0).
+LC_EXPORT int lc_attn_rows_ok(int D, int Dv, int BS) { return rows_cols(D, Dv, BS) > 0; }
+
+// T rows of any sequences, one at a time; planes and options as for lc_attn_masked (all_heads: every value head's columns side by
+// side whatever the query head, else its own).
+LC_EXPORT int lc_attn_rows(const void* q, const void* kc, const void* vc, int cache_f32, const void* block_tables, int MB,
+                           const void* row_seq, const void* positions, void* out, int act_f32, int T, int H, int G, int D, int Dv,
+                           int BS, float scale, int chunk, int window, int k_ld, int v_ld, float softcap, int sink, const void* sinks,
+                           const void* slopes, int keep, const void* gate, int ld_gate, float out_scale, int o_row, int v_share,
+                           int all_heads, int o_ld, hipStream_t st) {
+  if (T <= 0) return 0;
+  const int cols = rows_cols(D, Dv, BS), total = all_heads ? G * Dv : Dv, line = cache_f32 ? 4 : 8;
+  if (cols == 0 || H <= 0 || G <= 0 || H % G || MB <= 0 || v_share <= 0 || G % v_share || (all_heads && v_share != 1)) return -1;
+  if (k_ld < D || v_ld < Dv || k_ld % line || v_ld % line || !aligned16(q) || !aligned16(kc) || !aligned16(vc)) return -1;
+  if (o_ld < total || o_row < H * o_ld || o_ld % 4 || o_row % 4 || reinterpret_cast<uintptr_t>(out) % (act_f32 ? 16 : 8)) return -1;
+  if (softcap < 0.f || keep < 0 || (gate != nullptr && ld_gate < H) || (sinks != nullptr && !sink)) return -1;
+  const RowArgs a{static_cast<const float*>(q), kc, vc, static_cast<const int32_t*>(block_tables), MB,
+                  static_cast<const int32_t*>(row_seq), static_cast<const int32_t*>(positions), out, H, G, BS, scale, chunk, window,
+                  k_ld, v_ld, v_share, softcap, sink, static_cast<const float*>(sinks), static_cast<const float*>(slopes), keep,
+                  static_cast<const float*>(gate), ld_gate, out_scale, o_row, o_ld, all_heads ? 0 : -1, Dv};
+  const dim3 grid(T, G * ((H / G + 15) / 16), total / cols), block(64 * kRowWaves);
+  if (grid.y > 65535 || grid.z > 65535) return -1;
+#define LC_ROWS(C32, A32)                                                                 \
+  do {                                                                                    \
+    if (D == 64 && cols == 64) attn_rows_kernel<C32, A32, 2, 4><<<grid, block, 0, st>>>(a);      \
+    else if (D == 64) attn_rows_kernel<C32, A32, 2, 8><<<grid, block, 0, st>>>(a);        \
+    else if (D == 128 && cols == 64) attn_rows_kernel<C32, A32, 4, 4><<<grid, block, 0, st>>>(a); \
+    else if (D == 128) attn_rows_kernel<C32, A32, 4, 8><<<grid, block, 0, st>>>(a);       \
+    else if (cols == 64) attn_rows_kernel<C32, A32, 6, 4><<<grid, block, 0, st>>>(a);     \
+    else attn_rows_kernel<C32, A32, 6, 8><<<grid, block, 0, st>>>(a);                     \
+  } while (0)
+  if (cache_f32 && act_f32) LC_ROWS(true, true);
+  else if (cache_f32) LC_ROWS(true, false);
+  else if (act_f32) LC_ROWS(false, true);
+  else LC_ROWS(false, false);
+#undef LC_ROWS
   LC_RETURN_LAST_ERROR();
 }

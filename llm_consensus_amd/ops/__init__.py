@@ -1145,8 +1145,9 @@ def attn_masked(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, b
 
     The first ``n_portions`` sequences (rows [0, portion_rows), the longest of
     ``max_len`` rows) are prompt portions and go, 64 rows of a head per block, through fp32 MFMA
-    tiles (of 32 keys for common widths and plain masks over bf16 planes, of 16 otherwise); the rows behind them (single decoded tokens) and shapes the tiles do not take go
-    through the row kernel, one wave per (row, head)."""
+    tiles (of 32 keys for common widths and masks that are an interval per row over bf16 planes, of 16 otherwise); the rows behind
+    them (single decoded tokens) and shapes the tiles do not take go through the row kernels: eight waves per row and key head
+    at common widths, else one wave per (row, head)."""
     T = q.shape[0]
     if value_share < 1 or G % value_share or (value_share > 1 and all_value_heads):
         raise ValueError("attn_masked: the key heads that share a value head divide the key heads")
@@ -1210,6 +1211,13 @@ def attn_masked(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, b
     if first < T:
         if Dv > 512:
             raise ValueError("attn_masked: the row kernel takes value widths up to 512")
+        line = 4 if cf else 8
+        if k_ld % line == 0 and v_ld % line == 0 and o_row % 4 == 0 and _hip().lib().lc_attn_rows_ok(D, Dv, BS) and \
+                all(t.data_ptr() % 16 == 0 for t in (q[first:], k_cache, v_cache, out[first:])):
+            _hip().call("lc_attn_rows", q[first:].data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), cf, block_tables.data_ptr(), MB,
+                        row_seq[first:].data_ptr(), positions[first:].data_ptr(), out[first:].data_ptr(), af, T - first, H, G, D, Dv,
+                        BS, float(scale), int(chunk), int(window), k_ld, v_ld, *opts(first), 1 if all_value_heads else 0, o_ld)
+            return out
         # (value heads side by side: a block along z per value head; the short rows' scores are formed again there)
         _hip().call("lc_attn_masked", q[first:].data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), cf,
                     block_tables.data_ptr(), MB, row_seq[first:].data_ptr(), positions[first:].data_ptr(),

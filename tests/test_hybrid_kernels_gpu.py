@@ -1054,3 +1054,35 @@ def test_caps_sinks_and_value_heads_in_tiles_of_32_keys(D, Dv, G, every, cap, ga
         got = ops.attn_masked(c(q), c(kc), c(vc), c(tables), c(cu), c(rs), c(pos), H, G, D, Dv, D ** -0.5, 0, window, dt, n_portions=3,
                               portion_rows=T, max_len=longest, softcap=cap, sink=sink, all_value_heads=every)
         torch.testing.assert_close(got.float().cpu(), want, **(_tol(dt) if dt == torch.bfloat16 else dict(atol=3e-5, rtol=3e-5)))
+
+
+# one row at a time: contexts of one key, of one tile, of as many tiles as there are waves and more, window and chunk borders inside
+# tiles, kept first keys beside and inside them; more heads than an operand has rows; columns of 64 and 128, one wide head, value
+# heads side by side; cells behind the row's position hold no numbers
+@pytest.mark.parametrize("cache", ACTS)
+@pytest.mark.parametrize("H,G,D,Dv,every,share", [(4, 2, 64, 64, False, 1), (20, 1, 128, 128, False, 1), (8, 4, 128, 256, False, 2), (4, 2, 64, 192, True, 1),
+                                                  (6, 2, 192, 128, True, 1), (5, 5, 128, 64, False, 1)])
+@pytest.mark.parametrize("chunk,window,keep,cap", [(0, 0, 0, 0.0), (0, 90, 5, 8.0), (100, 0, 70, 0.0), (0, 33, 0, 0.0)])
+def test_single_rows_split_over_waves(cache, H, G, D, Dv, every, share, chunk, window, keep, cap):
+    g = torch.Generator().manual_seed(H + D + Dv + window)
+    BSZ, MB = 64, 10
+    starts = [0, 31, 32, 255, 256, 600, 333, 99]
+    T = len(starts)
+    cu, pos, rs = _seqs([1] * T, starts)
+    tables = torch.randperm(T * MB, generator=g).to(torch.int32).view(T, MB)
+    q, gates = torch.randn(T, H * D, generator=g), torch.randn(T, H, generator=g)
+    kc, vc = torch.randn(T * MB, G, BSZ, D, generator=g).to(cache), torch.randn(T * MB, G // share, BSZ, Dv, generator=g).to(cache)
+    for b, s in enumerate(starts):
+        for j in range(s + 1, MB * BSZ):
+            kc[tables[b, j // BSZ], :, j % BSZ] = float("nan")
+            vc[tables[b, j // BSZ], :, j % BSZ] = float("nan")
+    sinks, slopes = torch.randn(H, generator=g), torch.rand(H, generator=g) * 0.05
+    c = lambda t: t.to(DEV)   # noqa: E731
+    for opt in ({}, dict(sinks=sinks, slopes=slopes, gate=gates, out_scale=0.7)):
+        want = ref.attn_masked(q, kc, vc, tables, cu, pos, H, G, D, Dv, D ** -0.5, chunk, window, torch.float32, cap, False, every, keep=keep,
+                               value_share=share, **opt)
+        dopt = {k: c(v) if torch.is_tensor(v) else v for k, v in opt.items()}
+        for dt in ACTS:
+            got = ops.attn_masked(c(q), c(kc), c(vc), c(tables), c(cu), c(rs), c(pos), H, G, D, Dv, D ** -0.5, chunk, window, dt, softcap=cap,
+                                  all_value_heads=every, keep=keep, value_share=share, **dopt)
+            torch.testing.assert_close(got.float().cpu(), want, **(_tol(dt) if dt == torch.bfloat16 else dict(atol=3e-5, rtol=3e-5)))
