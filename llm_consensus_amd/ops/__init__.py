@@ -61,10 +61,17 @@ KGEMM_LONG_K_MAX_M = 4
 KGEMM_FORCE_NTW = int(os.environ.get("LC_KGEMM_NTW", "-1"))
 
 
-def _hip():
-    from . import hip
+_bindings = None
 
-    return hip
+
+def _hip():
+    """The kernel bindings, imported at the first launch (hosts without the library use the rest of this module)."""
+    global _bindings
+    if _bindings is None:
+        from . import hip
+
+        _bindings = hip
+    return _bindings
 
 
 # ---------------------------------------------------------------------------- weights
