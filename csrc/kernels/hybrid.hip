@@ -109,40 +109,6 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const int32_t* __restri
   }
 }
 
-// ---------------------------------------------------------------- scalar-gain RMS norm of a sublayer output
-// With y: x += y * rsqrt(mean(y^2) + eps) * gain, xa = x. Without: xa = x * rsqrt(mean(x^2) + eps) * gain.
-// WAVES = 1: one wave per row, four rows per block (many rows: bandwidth-bound). WAVES = 4: one
-// block per row (decode steps: few rows, latency-bound, so a row is spread over 256 lanes).
-template <bool AF32, int WAVES>
-__global__ __launch_bounds__(256) void scalar_norm_add_kernel(float* __restrict__ x, const float* __restrict__ y,
-                                                              const float* __restrict__ gain, float eps,
-                                                              void* __restrict__ xa, int T, int d) {
-  __shared__ float red[16];
-  constexpr int LANES = 64 * WAVES;
-  const int row = WAVES == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
-  const int lane = WAVES == 1 ? (threadIdx.x & 63) : threadIdx.x;
-  if (WAVES == 1 && row >= T) return;
-  float* xr = x + static_cast<size_t>(row) * d;
-  const float* src = y != nullptr ? y + static_cast<size_t>(row) * d : xr;
-  const float g = gain[0];
-  float ss = 0.f;
-  for (int c = lane; c < d; c += LANES) {
-    const float v = src[c];
-    ss += v * v;
-  }
-  ss = WAVES == 1 ? wave_sum(ss) : block_sum(ss, red);
-  const float r = g / sqrtf(ss / static_cast<float>(d) + eps);
-  typename Act<AF32>::type* a = static_cast<typename Act<AF32>::type*>(xa);
-  for (int c = lane; c < d; c += LANES) {
-    float v = src[c] * r;
-    if (y != nullptr) {
-      v += xr[c];
-      xr[c] = v;
-    }
-    if (a != nullptr) Act<AF32>::store(a, static_cast<size_t>(row) * d + c, v);
-  }
-}
-
 // out [T, cols] = relu(y[:, :cols])^2 for y of row stride ld.
 template <bool AF32>
 __global__ void relu2_kernel(const float* __restrict__ y, void* __restrict__ out, long long n, int cols, int ld) {
@@ -501,36 +467,6 @@ __global__ void mlstm_prepare_kernel(const float* __restrict__ proj, int ld, con
   const float* row = proj + t * ld;
   const float2 g = gates[t * H + c / D];
   prep[i] = make_float4(row[c] * qscale, row[HD + c] * g.y, g.x, 0.f);
-}
-
-// ---------------------------------------------------------------- pre-norm residual step
-// x += y (when y is given), xa = x * rsqrt(mean(x^2) + eps) * w (when w is given). WAVES as in the
-// scalar-gain kernel above.
-template <bool AF32, int WAVES>
-__global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ x, const float* __restrict__ y,
-                                                          const float* __restrict__ w, float eps,
-                                                          void* __restrict__ xa, int T, int d) {
-  __shared__ float red[16];
-  constexpr int LANES = 64 * WAVES;
-  const int row = WAVES == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
-  const int lane = WAVES == 1 ? (threadIdx.x & 63) : threadIdx.x;
-  if (WAVES == 1 && row >= T) return;
-  float* xr = x + static_cast<size_t>(row) * d;
-  const float* yr = y != nullptr ? y + static_cast<size_t>(row) * d : nullptr;
-  float ss = 0.f;
-  for (int c = lane; c < d; c += LANES) {
-    float v = xr[c];
-    if (yr != nullptr) {
-      v += yr[c];
-      xr[c] = v;
-    }
-    ss += v * v;
-  }
-  if (w == nullptr) return;                         // the same for every thread
-  ss = WAVES == 1 ? wave_sum(ss) : block_sum(ss, red);
-  const float r = 1.f / sqrtf(ss / static_cast<float>(d) + eps);
-  typename Act<AF32>::type* a = static_cast<typename Act<AF32>::type*>(xa);
-  for (int c = lane; c < d; c += LANES) Act<AF32>::store(a, static_cast<size_t>(row) * d + c, xr[c] * r * w[c]);
 }
 
 // act(gate) * up of y [T, 2n] = (gate | up); act: relu (kind 0), silu (1) or the tanh form of gelu (2). ``ldo``: row stride of
@@ -1272,23 +1208,6 @@ LC_EXPORT int lc_embed_rows(const void* ids, const void* E, int e_f32, void* x, 
   LC_RETURN_LAST_ERROR();
 }
 
-LC_EXPORT int lc_scalar_norm_add(void* x, const void* y, const void* gain, float eps, void* xa, int act_f32, int T,
-                                 int d, hipStream_t st) {
-  if (T <= 0) return 0;
-  if (d <= 0) return -1;
-  const bool few = T <= 512;
-  const dim3 grid(few ? T : (T + 3) / 4), block(256);
-#define LC_SN(A32, WAVES)                                                                                       \
-  scalar_norm_add_kernel<A32, WAVES><<<grid, block, 0, st>>>(static_cast<float*>(x), static_cast<const float*>(y), \
-                                                             static_cast<const float*>(gain), eps, xa, T, d)
-  if (act_f32 && few) LC_SN(true, 4);
-  else if (act_f32) LC_SN(true, 1);
-  else if (few) LC_SN(false, 4);
-  else LC_SN(false, 1);
-#undef LC_SN
-  LC_RETURN_LAST_ERROR();
-}
-
 // y [T, >= cols] with row stride ld -> out [T, cols].
 LC_EXPORT int lc_relu2(const void* y, void* out, int act_f32, int T, int cols, int ld, hipStream_t st) {
   if (T <= 0 || cols <= 0) return 0;
@@ -1430,23 +1349,6 @@ LC_EXPORT int lc_mlstm_scan(const void* proj, int ld, void* state, long long sta
       static_cast<const float*>(proj), ld, gates, static_cast<float4*>(prep), n, H, D, 1.f / sqrtf(static_cast<float>(D)));
   return launch_linear_scan(proj, ld, prep, state, state_stride, cu_q, positions, slots, out, B, H, D, Dv + 1, 1, max_len,
                             scratch, st);
-}
-
-LC_EXPORT int lc_add_rmsnorm(void* x, const void* y, const void* w, float eps, void* xa, int act_f32, int T, int d,
-                             hipStream_t st) {
-  if (T <= 0) return 0;
-  if (d <= 0 || (w != nullptr && xa == nullptr)) return -1;
-  const bool few = T <= 512;
-  const dim3 grid(few ? T : (T + 3) / 4), block(256);
-#define LC_AN(A32, WAVES)                                                                                          \
-  add_rmsnorm_kernel<A32, WAVES><<<grid, block, 0, st>>>(static_cast<float*>(x), static_cast<const float*>(y),    \
-                                                         static_cast<const float*>(w), eps, xa, T, d)
-  if (act_f32 && few) LC_AN(true, 4);
-  else if (act_f32) LC_AN(true, 1);
-  else if (few) LC_AN(false, 4);
-  else LC_AN(false, 1);
-#undef LC_AN
-  LC_RETURN_LAST_ERROR();
 }
 
 LC_EXPORT int lc_glu(const void* y, int parts, int tiled, void* out, int act_f32, int T, int n, int kind, int ldo, hipStream_t st) {

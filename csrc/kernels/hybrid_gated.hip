@@ -13,13 +13,16 @@
 namespace {
 
 // ---------------------------------------------------------------- residual step with a gate and two norms
-// With y [T, d] (a product whose depth was split comes as the slabs of its partial sums): v = y * sigmoid(gate) (gate given: logits, row stride ld_gate), then rms-normed times w_out (w_out
-// given), x += v. With w_in: h = x / sqrt(mean(x^2) + eps) * w_in, written to ``ha`` in the activation type and, when
+// With y [T, d] (a product whose depth was split comes as the slabs of its partial sums, its bias apart): v = y * sigmoid(gate)
+// (gate given: logits, row stride ld_gate), then rms-normed times w_out (w_out given), x += v. ``one_gain``: w_out and w_in are
+// ONE number each. ``copy``: instead of a norm (no w_in) ``ha`` is x itself in the activation type. With w_in: h = x / sqrt(mean(x^2) + eps) * w_in, written to ``ha`` in the activation type and, when
 // given, to ``h32``. With ``mu`` (steps whose sequences all have ONE row): ``hs`` = h + (h' - h) * mu in the
 // activation type, h' the sequence's stored row (zeros at position 0), and h becomes the stored row. With ``w_in2``: ``ha2`` =
 // x / sqrt(mean(x^2) + eps) * w_in2 beside it (two sublayers that read the same stream through norms of their own).
-// A block per row. Rows of up to 4 * 256 * kStepVec coordinates whose pieces are 16-byte aligned (VEC) stay in registers
-// between the sums; others are read again.
+// A block per row, bound by memory. Rows of up to 4 * 256 * kStepVec coordinates whose pieces are 16-byte aligned (VEC) stay in
+// registers between the sums; others are read again. Every residual step of the designs with one stream is this launch: kernels
+// of their own with a wave per row, 4-byte accesses and rows read twice took 27 us (1500 rows of 2048, a norm) and 37 us (2048
+// rows, one gain on the result) behind a launch of 10-13 us that summed four slabs; with the slabs read here 13 and 20 us
 constexpr int kStepVec = 4;
 
 LC_DEVICE float4 shift4(const float4& h, const float4& p, const float4& m) {
@@ -31,6 +34,7 @@ struct StepArgs {
   const float* y;                // ``parts`` slabs of [T, d], ``slab`` elements apart, whose sum is the sublayer's result
   int parts;
   size_t slab;
+  const bf16_t* bias;            // [d] of y (null: none)
   const float* gate;
   int ld_gate;
   const float* w_out;
@@ -40,6 +44,7 @@ struct StepArgs {
   float* h32;
   const float* w_in2;            // a second norm of the same row (null: none)
   void* ha2;
+  int one_gain, copy;
   // the shift of single-row sequences
   const float* mu;
   float* state;
@@ -84,6 +89,10 @@ __global__ __launch_bounds__(256) void gated_step_kernel(StepArgs a) {
             const float4 w = reinterpret_cast<const float4*>(a.y + s * a.slab + row)[c];
             v = make_float4(v.x + w.x, v.y + w.y, v.z + w.z, v.w + w.w);
           }
+          if (a.bias != nullptr) {
+            const float4 b = load_act4<false>(a.bias + 4 * c);
+            v = make_float4(v.x + b.x, v.y + b.y, v.z + b.z, v.w + b.w);
+          }
           if (grow != nullptr) {
             const float4 g = reinterpret_cast<const float4*>(grow)[c];
             v = make_float4(v.x * sigmoidf_(g.x), v.y * sigmoidf_(g.y), v.z * sigmoidf_(g.z), v.w * sigmoidf_(g.w));
@@ -94,19 +103,28 @@ __global__ __launch_bounds__(256) void gated_step_kernel(StepArgs a) {
       }
     }
     if (a.y != nullptr) {
-      const float r = a.w_out != nullptr ? 1.f / sqrtf(block_sum(ss, red) / static_cast<float>(d) + a.eps) : 1.f;
+      float r = a.w_out != nullptr ? 1.f / sqrtf(block_sum(ss, red) / static_cast<float>(d) + a.eps) : 1.f;
+      const bool each = a.w_out != nullptr && !a.one_gain;
+      if (a.w_out != nullptr && a.one_gain) r *= a.w_out[0];
 #pragma unroll
       for (int i = 0; i < kStepVec; ++i) {
         const int c = threadIdx.x + 256 * i;
         if (c < n4) {
           float4 w = make_float4(1.f, 1.f, 1.f, 1.f);
-          if (a.w_out != nullptr) w = reinterpret_cast<const float4*>(a.w_out)[c];
+          if (each) w = reinterpret_cast<const float4*>(a.w_out)[c];
           xv[i].x += yv[i].x * r * w.x;
           xv[i].y += yv[i].y * r * w.y;
           xv[i].z += yv[i].z * r * w.z;
           xv[i].w += yv[i].w * r * w.w;
           reinterpret_cast<float4*>(a.x + row)[c] = xv[i];
         }
+      }
+    }
+    if (a.copy) {                                     // the same for every thread
+#pragma unroll
+      for (int i = 0; i < kStepVec; ++i) {
+        const int c = threadIdx.x + 256 * i;
+        if (c < n4) store_act4<AF32>(a.ha, row + 4 * c, xv[i]);
       }
     }
     if (a.w_in == nullptr) return;                    // the same for every thread
@@ -118,7 +136,7 @@ __global__ __launch_bounds__(256) void gated_step_kernel(StepArgs a) {
     for (int i = 0; i < kStepVec; ++i) {
       const int c = threadIdx.x + 256 * i;
       if (c < n4) {
-        const float4 w = reinterpret_cast<const float4*>(a.w_in)[c];
+        const float4 w = a.one_gain ? make_float4(a.w_in[0], a.w_in[0], a.w_in[0], a.w_in[0]) : reinterpret_cast<const float4*>(a.w_in)[c];
         const float4 h = make_float4(xv[i].x * r2 * w.x, xv[i].y * r2 * w.y, xv[i].z * r2 * w.z, xv[i].w * r2 * w.w);
         store_act4<AF32>(a.ha, row + 4 * c, h);
         if (a.w_in2 != nullptr) {
@@ -140,6 +158,7 @@ __global__ __launch_bounds__(256) void gated_step_kernel(StepArgs a) {
     auto result = [&](int c) {
       float v = a.y[row + c];
       for (int s = 1; s < a.parts; ++s) v += a.y[s * a.slab + row + c];
+      if (a.bias != nullptr) v += bf16_to_f32(a.bias[c]);
       return grow != nullptr ? v * sigmoidf_(grow[c]) : v;
     };
     if (a.y != nullptr && a.w_out != nullptr) {
@@ -154,15 +173,16 @@ __global__ __launch_bounds__(256) void gated_step_kernel(StepArgs a) {
     for (int c = threadIdx.x; c < d; c += 256) {
       float v = a.x[row + c];
       if (a.y != nullptr) {
-        v += result(c) * r * (a.w_out != nullptr ? a.w_out[c] : 1.f);
+        v += result(c) * r * (a.w_out != nullptr ? a.w_out[a.one_gain ? 0 : c] : 1.f);
         a.x[row + c] = v;
       }
+      if (a.copy) Act<AF32>::store(static_cast<act_t*>(a.ha), row + c, v);
       s2 += v * v;
     }
     if (a.w_in == nullptr) return;
     const float r2 = 1.f / sqrtf(block_sum(s2, red) / static_cast<float>(d) + a.eps);
     for (int c = threadIdx.x; c < d; c += 256) {      // (a thread reads what it wrote itself)
-      const float h = a.x[row + c] * r2 * a.w_in[c];
+      const float h = a.x[row + c] * r2 * a.w_in[a.one_gain ? 0 : c];
       Act<AF32>::store(static_cast<act_t*>(a.ha), row + c, h);
       if (a.w_in2 != nullptr) Act<AF32>::store(static_cast<act_t*>(a.ha2), row + c, a.x[row + c] * r2 * a.w_in2[c]);
       if (a.h32 != nullptr) a.h32[row + c] = h;
@@ -360,25 +380,27 @@ __global__ void softcap_kernel(float* __restrict__ x, long long n, float cap) {
 }  // namespace
 
 // ================================================================= launchers
-LC_EXPORT int lc_gated_step(void* x, const void* y, int parts, const void* gate, int ld_gate, const void* w_out, const void* w_in,
-                            float eps, void* ha, void* h32, const void* w_in2, void* ha2, int act_f32, const void* mu, void* state,
+LC_EXPORT int lc_gated_step(void* x, const void* y, int parts, const void* bias, const void* gate, int ld_gate, const void* w_out, const void* w_in,
+                            float eps, void* ha, void* h32, const void* w_in2, void* ha2, int one_gain, int copy, int act_f32, const void* mu, void* state,
                             long long state_stride, const void* row_seq, const void* positions, const void* slots, void* hs,
                             int T, int d, hipStream_t st) {
   if (T <= 0) return 0;
   if (d <= 0 || parts < 1 || (y == nullptr && w_in == nullptr) || (w_in != nullptr && ha == nullptr)) return -1;
+  if ((bias != nullptr && y == nullptr) || (copy && (y == nullptr || w_in != nullptr || ha == nullptr)) || (one_gain && w_in2 != nullptr)) return -1;
   if (gate != nullptr && (y == nullptr || ld_gate < d)) return -1;
   if (w_in2 != nullptr && (w_in == nullptr || ha2 == nullptr)) return -1;
   if (mu != nullptr && (w_in == nullptr || hs == nullptr || state == nullptr || row_seq == nullptr || positions == nullptr ||
                         slots == nullptr || state_stride < d))
     return -1;
   const StepArgs a{static_cast<float*>(x), static_cast<const float*>(y), parts, static_cast<size_t>(T) * d,
-                   static_cast<const float*>(gate), ld_gate, static_cast<const float*>(w_out), static_cast<const float*>(w_in), eps, ha, static_cast<float*>(h32),
-                   static_cast<const float*>(w_in2), ha2,
+                   static_cast<const bf16_t*>(bias), static_cast<const float*>(gate), ld_gate, static_cast<const float*>(w_out), static_cast<const float*>(w_in), eps, ha, static_cast<float*>(h32),
+                   static_cast<const float*>(w_in2), ha2, one_gain, copy,
                    static_cast<const float*>(mu), static_cast<float*>(state), state_stride,
                    static_cast<const int32_t*>(row_seq), static_cast<const int32_t*>(positions),
                    static_cast<const int32_t*>(slots), hs, d};
   const bool vec = d % 4 == 0 && d <= 4 * 256 * kStepVec && ld_gate % 4 == 0 && state_stride % 4 == 0 && aligned16(x) &&
-                   aligned16(y) && aligned16(gate) && aligned16(w_out) && aligned16(w_in) && aligned16(ha) &&
+                   aligned16(y) && aligned16(gate) && (one_gain || (aligned16(w_out) && aligned16(w_in))) && aligned16(ha) &&
+                   reinterpret_cast<uintptr_t>(bias) % 8 == 0 &&
                    aligned16(h32) && aligned16(w_in2) && aligned16(ha2) && aligned16(mu) && aligned16(state) && aligned16(hs);
 #define LC_GS(A32, V) gated_step_kernel<A32, V><<<dim3(T), dim3(256), 0, st>>>(a)
   if (act_f32 && vec) LC_GS(true, true);

@@ -171,6 +171,75 @@ __global__ __launch_bounds__(256) void hc_step_kernel(float* __restrict__ xs, co
   }
 }
 
+// The same for rows of whole 16-byte pieces of up to 4 * 256 * kHcVec coordinates: a block per row, four neighbouring coordinates
+// per access, the old streams in registers; y may be the slabs of a product whose depth was split, its bias apart. 2361 rows of
+// 2 x 2048 with four slabs: 24 us (a wave per row with 4-byte accesses 54 us, behind a launch of 11 us for the slabs).
+constexpr int kHcVec = 4;
+
+LC_DEVICE float4 axpy4(float a, const float4& x, const float4& y) {
+  return make_float4(a * x.x + y.x, a * x.y + y.y, a * x.z + y.z, a * x.w + y.w);
+}
+
+template <bool AF32, int SMAX>
+__global__ __launch_bounds__(256) void hc_step4_kernel(float* __restrict__ xs, const float* __restrict__ y, int parts, size_t slab,
+                                                       const bf16_t* __restrict__ bias, const float* __restrict__ mix,
+                                                       const float* __restrict__ outw, const float* __restrict__ inw,
+                                                       const float* __restrict__ normw, float eps, float* __restrict__ u_out,
+                                                       void* __restrict__ xa, int S, int d) {
+  __shared__ float red[16];
+  const size_t row = static_cast<size_t>(blockIdx.x) * d;
+  float* xr = xs + row * S;
+  const int n4 = d / 4;
+  float4 u[kHcVec];
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < kHcVec; ++e) {
+    const int c = threadIdx.x + 256 * e;
+    u[e] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (c >= n4) continue;
+    float4 v[SMAX];
+#pragma unroll
+    for (int s = 0; s < SMAX; ++s)
+      if (s < S) v[s] = *reinterpret_cast<const float4*>(xr + static_cast<size_t>(s) * d + 4 * c);
+    if (y != nullptr) {
+      float4 r = *reinterpret_cast<const float4*>(y + row + 4 * c);
+#pragma unroll 8
+      for (int s = 1; s < parts; ++s) r = axpy4(1.f, *reinterpret_cast<const float4*>(y + s * slab + row + 4 * c), r);
+      if (bias != nullptr) r = axpy4(1.f, load_act4<false>(bias + 4 * c), r);
+      float4 n[SMAX];
+#pragma unroll
+      for (int j = 0; j < SMAX; ++j) {
+        if (j >= S) continue;
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int s = 0; s < SMAX; ++s)
+          if (s < S) a = axpy4(mix[s * S + j], v[s], a);
+        n[j] = axpy4(outw[j], r, a);
+        *reinterpret_cast<float4*>(xr + static_cast<size_t>(j) * d + 4 * c) = n[j];
+      }
+#pragma unroll
+      for (int j = 0; j < SMAX; ++j)
+        if (j < S) v[j] = n[j];
+    }
+    if (inw != nullptr) {
+#pragma unroll
+      for (int s = 0; s < SMAX; ++s)
+        if (s < S) u[e] = axpy4(inw[s], v[s], u[e]);
+      if (u_out != nullptr) *reinterpret_cast<float4*>(u_out + row + 4 * c) = u[e];
+      ss += u[e].x * u[e].x + u[e].y * u[e].y + u[e].z * u[e].z + u[e].w * u[e].w;
+    }
+  }
+  if (normw == nullptr || inw == nullptr) return;    // the same for every thread
+  const float r = 1.f / sqrtf(block_sum(ss, red) / static_cast<float>(d) + eps);
+#pragma unroll
+  for (int e = 0; e < kHcVec; ++e) {
+    const int c = threadIdx.x + 256 * e;
+    if (c >= n4) continue;
+    const float4 w = *reinterpret_cast<const float4*>(normw + 4 * c);
+    store_act4<AF32>(xa, row + 4 * c, make_float4(u[e].x * r * w.x, u[e].y * r * w.y, u[e].z * r * w.z, u[e].w * r * w.w));
+  }
+}
+
 // ---------------------------------------------------------------- rotary positions on q, k and v; cache write
 // One block per token. qkv [T, ld] fp32: q [H*D] | k [G*D] | v [G*Dv] (biases already added by the product). The
 // first rot_dims coordinates of every query and key head turn by position * inv_freq[i] in the pair layout
@@ -312,13 +381,31 @@ LC_EXPORT int lc_hc_init(const void* x0, const void* w, float eps, void* xs, int
   LC_RETURN_LAST_ERROR();
 }
 
-LC_EXPORT int lc_hc_step(void* xs, const void* y, const void* mix, const void* outw, const void* inw, const void* normw,
+LC_EXPORT int lc_hc_step(void* xs, const void* y, int parts, const void* bias, const void* mix, const void* outw, const void* inw, const void* normw,
                          float eps, void* u_out, void* xa, int act_f32, int T, int S, int d, hipStream_t st) {
   if (T <= 0) return 0;
   if (d <= 0 || S <= 0 || S > kMaxStreams || xs == nullptr) return -1;
   if (y != nullptr && (mix == nullptr || outw == nullptr)) return -1;
   if (normw != nullptr && (inw == nullptr || xa == nullptr)) return -1;
   if (u_out != nullptr && inw == nullptr) return -1;
+  if (parts < 1 || (y == nullptr && (parts != 1 || bias != nullptr))) return -1;
+  if (d % 4 == 0 && d <= 4 * 256 * kHcVec && aligned16(xs) && aligned16(y) && aligned16(normw) && aligned16(u_out) && aligned16(xa) &&
+      reinterpret_cast<uintptr_t>(bias) % 8 == 0) {
+#define LC_HC4(A32, SMAX)                                                                                                     \
+  hc_step4_kernel<A32, SMAX><<<dim3(T), dim3(256), 0, st>>>(                                                                  \
+      static_cast<float*>(xs), static_cast<const float*>(y), parts, static_cast<size_t>(T) * d, static_cast<const bf16_t*>(bias), \
+      static_cast<const float*>(mix), static_cast<const float*>(outw), static_cast<const float*>(inw),                        \
+      static_cast<const float*>(normw), eps, static_cast<float*>(u_out), xa, S, d)
+    if (act_f32 && S <= 2) LC_HC4(true, 2);
+    else if (act_f32 && S <= 4) LC_HC4(true, 4);
+    else if (act_f32) LC_HC4(true, kMaxStreams);
+    else if (S <= 2) LC_HC4(false, 2);
+    else if (S <= 4) LC_HC4(false, 4);
+    else LC_HC4(false, kMaxStreams);
+#undef LC_HC4
+    LC_RETURN_LAST_ERROR();
+  }
+  if (parts != 1 || bias != nullptr) return -1;      // (such rows come summed)
   const bool few = T <= 512;
   const dim3 grid(few ? T : (T + 3) / 4), block(256);
 #define LC_HC(A32, WAVES, SMAX)                                                                                    \

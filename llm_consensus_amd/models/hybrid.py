@@ -1502,15 +1502,20 @@ class HybridModel:
             elif l.type == "mingru":
                 zxg = ops.linear(xa, L.proj, out_f32=True)
                 y = ops.mingru_scan(zxg, cache.state(i), lay.cu_q, positions, lay.state_slots, dt, self._max_len)
-                y = ops.linear(y, L.out, out_f32=True)
+                y = self._result(y, L.out)
             else:
                 y = self._gla(i, L, xa, positions, lay, cache)
             xa = ops.scalar_norm_add(x, y, L.norm1, eps, dt)
             if L.up is not None:
-                xa = ops.scalar_norm_add(x, ops.linear(self._relu2_up(xa, L.up), L.down, out_f32=True), L.norm2, eps, dt)
+                xa = ops.scalar_norm_add(x, self._result(self._relu2_up(xa, L.up), L.down), L.norm2, eps, dt)
             if taps is not None:
                 taps.append(x.clone())
         return x
+
+    def _result(self, a: torch.Tensor, w: ops.LinearWeight):
+        """A sublayer's last product: fp32, and where its depth was split the slabs as they are (the residual step sums
+        them). (The Dynamic Tanh step takes whole results.)"""
+        return ops.linear(a, w, out_f32=True, defer_reduce=self.cfg.design.norm != "dyt")
 
     def _relu2_up(self, xa: torch.Tensor, up: ops.LinearWeight) -> torch.Tensor:
         """relu(up x)^2 in the activation type: an epilogue of the shape-agnostic product, one more
@@ -1662,7 +1667,7 @@ class HybridModel:
                 self._attention_diff(r, L, h1, positions, slot_mapping, lay, cache, both[:, :n])
             if l.ff:
                 ops.glu_linear(h2, L.gate_up, "gelu_tanh", dt, out=both[:, n:])
-            y = ops.linear(both, L.out, out_f32=True, defer_reduce=True)
+            y = self._result(both, L.out)
             nxt = self.layers[runs[r + 1][0]] if r + 1 < len(runs) else None
             h1, h2 = ops.dual_norm_step(x, y, nxt.norm1 if nxt else None, nxt.norm2 if nxt else None, eps, dt)
             if taps is not None:
@@ -1698,7 +1703,7 @@ class HybridModel:
     def _clamped_dense(self, L: HybridLayer, fi: torch.Tensor) -> torch.Tensor:
         d, n, des = self.cfg.hidden_size, L.spec.ff, self.cfg.design
         act = ops.glu_clamped(fi, d, d + n, n, L.spec.ff_limit, self.dtype, slope=des.glu_slope, shift=des.glu_shift)
-        return ops.linear(act, L.down, out_f32=True)
+        return self._result(act, L.down)
 
     def _gated_experts(self, L: HybridLayer, xa: torch.Tensor, z: torch.Tensor) -> torch.Tensor:
         """Routed feed-forward of silu-gated experts; z: router logits in the first columns. silu(g) u is the clamped gated
@@ -1740,13 +1745,13 @@ class HybridModel:
                             gate=proj[:, C:C + H] if l.head_gate else None, out_scale=l.out_scale,
                             out=both[:, :H * Dv] if both is not None else None)
         if both is None:
-            return ops.linear(a, L.out, out_f32=True)
+            return self._result(a, L.out)
         hd, hv = g.heads * g.dim, g.heads * g.vdim
         o = ops.lightning_scan(proj[:, C:], L.decay, cache.state_part(r, "memory"), lay.cu_q, positions, lay.state_slots,
                                g.heads, g.dim, g.vdim, self._max_len)
         g0 = C + 2 * hd + hv
         ops.rownorm_gate(o, L.head_norm, proj[:, g0:g0 + hv], self.cfg.rms_eps, self.dtype, out=both[:, H * Dv:])
-        return ops.linear(both, L.out, out_f32=True)
+        return self._result(both, L.out)
 
     def _residual_norm(self, x: torch.Tensor, y: Optional[torch.Tensor], norm, out: Optional[torch.Tensor] = None):
         """x += m * y (when y is given) and the design's norm of the new x in the activation type (when a
@@ -1763,10 +1768,10 @@ class HybridModel:
 
     def _dense_ff(self, L: HybridLayer, xa: torch.Tensor) -> torch.Tensor:
         if L.act is not None:               # (biases ride in the products)
-            return ops.linear(ops.xielu(ops.linear(xa, L.up, out_f32=True), L.act[0], L.act[1], self.dtype), L.down, out_f32=True)
+            return self._result(ops.xielu(ops.linear(xa, L.up, out_f32=True), L.act[0], L.act[1], self.dtype), L.down)
         if L.gate_up is not None:
-            return ops.linear(ops.glu(ops.linear(xa, L.gate_up, out_f32=True), self.dtype, "relu"), L.down, out_f32=True)
-        return ops.linear(self._relu2_up(xa, L.up), L.down, out_f32=True)
+            return self._result(ops.glu(ops.linear(xa, L.gate_up, out_f32=True), self.dtype, "relu"), L.down)
+        return self._result(self._relu2_up(xa, L.up), L.down)
 
     def _routed_ff(self, L: HybridLayer, xa: torch.Tensor) -> torch.Tensor:
         e = L.spec.moe
@@ -1821,7 +1826,7 @@ class HybridModel:
         a = ops.attn_masked(q, kc, cache.v(r), lay.block_tables, lay.cu_q, lay.row_seq, positions, l.heads, l.kv_heads, l.dim,
                             l.vdim, l.scale, 0, l.window, self.dtype, n_portions=self._portions[0],
                             portion_rows=self._portions[1], max_len=self._max_len)
-        return ops.linear(a, L.out, out_f32=True)
+        return self._result(a, L.out)
 
     def _attention_talk(self, r: int, L: HybridLayer, xa, positions, slot_mapping, lay: StepLayout, cache: HybridCache):
         """Attention whose heads' softmax weights are mixed before they meet the values. The mix is linear in the
@@ -1837,7 +1842,7 @@ class HybridModel:
                             l.scale, 0, l.window, torch.float32, n_portions=self._portions[0], portion_rows=self._portions[1],
                             max_len=self._max_len, softcap=l.softcap, sink=l.sink, all_value_heads=True)
         a = ops.talk_mix(o, L.talk, positions, L.inv_freq_v, l.heads, l.kv_heads, l.vdim, self.dtype)
-        return ops.linear(a, L.out, out_f32=True)
+        return self._result(a, L.out)
 
     def _latent_attention_rot(self, r: int, L: HybridLayer, xa, positions, slot_mapping, lay: StepLayout, cache: HybridCache):
         """Latent attention with a turned key part shared by all heads. The cached row is [compressed row | key part];
@@ -1858,7 +1863,7 @@ class HybridModel:
                             max_len=self._max_len)
         g0 = nq + (W if own else 0)
         o = ops.head_linear(a, L.value_up, self.dtype, gate=proj[:, g0:g0 + H * Dv], gate_full=True)
-        return ops.linear(o, L.out, out_f32=True)
+        return self._result(o, L.out)
 
     def _latent_attention(self, i: int, L: HybridLayer, xa, positions, slot_mapping, lay: StepLayout, cache: HybridCache):
         l = L.spec
@@ -1871,7 +1876,7 @@ class HybridModel:
                             0, 0, self.dtype, n_portions=self._portions[0], portion_rows=self._portions[1],
                             max_len=self._max_len)
         o = ops.head_linear(a, L.value_up, self.dtype, gate=proj[:, hd + R:hd + R + l.heads])
-        return ops.linear(o, L.out, out_f32=True)
+        return self._result(o, L.out)
 
     def _mlstm(self, i: int, L: HybridLayer, xa, positions, lay: StepLayout, cache: HybridCache):
         l = L.spec
@@ -1881,7 +1886,7 @@ class HybridModel:
                               l.gate_cap, self._max_len)
         y = ops.mlstm_out(o, m, L.head_norm, proj[:, 2 * hd + hv:2 * hd + 2 * hv], l.heads, l.vdim, self.cfg.rms_eps,
                           self.dtype)
-        return ops.linear(y, L.out, out_f32=True)
+        return self._result(y, L.out)
 
     def _attention(self, i: int, L: HybridLayer, xa, positions, slot_mapping, lay: StepLayout, cache: HybridCache):
         l = L.spec
@@ -1894,7 +1899,7 @@ class HybridModel:
         a = ops.attn_masked(q, kc, vc, lay.block_tables, lay.cu_q, lay.row_seq, positions, l.heads, l.kv_heads, l.dim,
                             l.vdim, l.scale, l.chunk, l.window, self.dtype, n_portions=self._portions[0],
                             portion_rows=self._portions[1], max_len=self._max_len)
-        return ops.linear(a, L.out, out_f32=True)
+        return self._result(a, L.out)
 
     def _gla(self, i: int, L: HybridLayer, xa, positions, lay: StepLayout, cache: HybridCache):
         l = L.spec
@@ -1904,7 +1909,7 @@ class HybridModel:
         o = ops.gla_scan(proj, logits, cache.state(i), lay.cu_q, positions, lay.state_slots, l.heads, l.dim, l.vdim,
                          l.tau, self._max_len)
         y = ops.headnorm_gate(o, L.head_norm, proj[:, 2 * hd + hv:2 * hd + 2 * hv], l.vdim, self.cfg.rms_eps, self.dtype)
-        return ops.linear(y, L.out, out_f32=True)
+        return self._result(y, L.out)
 
     def logits(self, hidden_rows: torch.Tensor) -> torch.Tensor:
         """fp32 logits [R, V] of the given rows of the residual stream (final norm, then the head)."""

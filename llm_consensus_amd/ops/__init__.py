@@ -973,20 +973,21 @@ def embed_rows(ids: torch.Tensor, E: torch.Tensor, act_dtype: Optional[torch.dty
 
 def scalar_norm_add(x: torch.Tensor, y: Optional[torch.Tensor], gain: torch.Tensor, eps: float,
                     act_dtype: torch.dtype) -> torch.Tensor:
-    """x (fp32 residual stream, in place) += y / sqrt(mean(y^2) + eps) * gain and the new x in
+    """x (fp32 residual stream, in place) += y / sqrt(mean(y^2) + eps) * gain (y may be a ``PartialSum``) and the new x in
     ``act_dtype``; without ``y``: the normed x in ``act_dtype`` (x untouched). ``gain`` is an
     fp32 tensor of one element."""
     if not x.is_cuda:
         return ref.scalar_norm_add(x, y, gain, eps, act_dtype)
     T, d = x.shape
-    if y is not None and (y.shape != x.shape or y.dtype != torch.float32):
+    if y is not None and not _is_result(y, x):
         raise ValueError("scalar_norm_add: the sublayer output must be fp32 of the stream's shape")
     if x.dtype != torch.float32 or not x.is_contiguous():
         raise ValueError("scalar_norm_add: the residual stream is a contiguous fp32 tensor")
     alias = y is not None and act_dtype == torch.float32       # the fp32 'copy' is the stream itself
     xa = None if alias else torch.empty(T, d, dtype=act_dtype, device=x.device)
-    _hip().call("lc_scalar_norm_add", x.data_ptr(), _hip().ptr(y.contiguous() if y is not None else None),
-                gain.data_ptr(), float(eps), _hip().ptr(xa), _f32flag(act_dtype), T, d)
+    if T:
+        _residual_step(x, y, w_out=gain if y is not None else None, w_in=gain if y is None else None, eps=eps, act_dtype=act_dtype, ha=xa,
+                       one_gain=True, copy=xa is not None and y is not None)
     return x if alias else xa
 
 
@@ -1236,7 +1237,7 @@ def attn_masked(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, b
 # ---- pre-norm designs, latent attention, mLSTM, routed feed-forwards (hybrid.hip, hybrid_moe.hip) ----
 def add_rmsnorm(x: torch.Tensor, y: Optional[torch.Tensor], w: Optional[torch.Tensor], eps: float,
                 act_dtype: torch.dtype) -> Optional[torch.Tensor]:
-    """The residual step of a pre-norm layer in one launch: x (fp32 stream, in place) += y, and the
+    """The residual step of a pre-norm layer in one launch: x (fp32 stream, in place) += y (it may be a ``PartialSum``), and the
     input of the next sublayer x / sqrt(mean(x^2) + eps) * w in ``act_dtype`` (``w``: fp32 [d], any
     offset already folded in). Without ``y`` only the norm; without ``w`` only the sum (returns None)."""
     if not x.is_cuda:
@@ -1244,13 +1245,12 @@ def add_rmsnorm(x: torch.Tensor, y: Optional[torch.Tensor], w: Optional[torch.Te
     T, d = x.shape
     if x.dtype != torch.float32 or not x.is_contiguous():
         raise ValueError("add_rmsnorm: the residual stream is a contiguous fp32 tensor")
-    if y is not None and (y.shape != x.shape or y.dtype != torch.float32):
+    if y is not None and not _is_result(y, x):
         raise ValueError("add_rmsnorm: the sublayer output must be fp32 of the stream's shape")
     if y is None and w is None:
         return None
     xa = torch.empty(T, d, dtype=act_dtype, device=x.device) if w is not None else None
-    _hip().call("lc_add_rmsnorm", x.data_ptr(), _hip().ptr(y.contiguous() if y is not None else None), _hip().ptr(w),
-                float(eps), _hip().ptr(xa), _f32flag(act_dtype), T, d)
+    _residual_step(x, y, w_in=w, eps=eps, act_dtype=act_dtype, ha=xa)
     return xa
 
 
@@ -1341,13 +1341,27 @@ def mlstm_out(o: torch.Tensor, m: torch.Tensor, w: torch.Tensor, gate: torch.Ten
     return out
 
 
-def _slabs(y, what: str) -> Tuple[torch.Tensor, int]:
-    """(storage, number of fp32 slabs whose sum is y) of a matrix or of a ``PartialSum``."""
+def _slabs(y, what: str, bias: bool = False):
+    """(storage, number of fp32 slabs whose sum is y, bias) of a matrix or of a ``PartialSum``."""
     if isinstance(y, PartialSum):
-        if y.bias is not None:
+        if y.bias is not None and not bias:
             raise ValueError(f"{what}: partial sums of a product without a bias")
-        return y.part, y.part.shape[0]
-    return y.contiguous(), 1
+        return y.part, y.part.shape[0], y.bias
+    return y.contiguous(), 1, None
+
+
+def _is_result(y, x: torch.Tensor) -> bool:
+    """Whether y is an fp32 sublayer result of the stream's shape (a matrix or a ``PartialSum``)."""
+    return tuple(y.shape) == tuple(x.shape) and (isinstance(y, PartialSum) or y.dtype == torch.float32)
+
+
+def _residual_step(x: torch.Tensor, y, w_out=None, w_in=None, w_in2=None, eps: float = 0.0, act_dtype=torch.float32, ha=None, ha2=None,
+                   one_gain: bool = False, copy: bool = False) -> None:
+    """The residual step's launch (lc_gated_step) without gates and shifts."""
+    p = _hip().ptr
+    part, parts, bias = _slabs(y, "residual step", bias=True) if y is not None else (None, 1, None)
+    _hip().call("lc_gated_step", x.data_ptr(), p(part), parts, p(bias), None, 0, p(w_out), p(w_in), float(eps), p(ha), None, p(w_in2),
+                p(ha2), 1 if one_gain else 0, 1 if copy else 0, _f32flag(act_dtype), None, None, 0, None, None, None, None, *x.shape)
 
 
 def glu_linear(x: torch.Tensor, w: LinearWeight, kind: str, act_dtype: torch.dtype, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -1379,7 +1393,7 @@ def glu(y, act_dtype: torch.dtype, kind: str = "relu", out: Optional[torch.Tenso
     T, n = y.shape[0], y.shape[1] // 2
     if tiled and n % 16:
         raise ValueError("glu: tiles of 16 columns")
-    y, parts = _slabs(y, "glu")
+    y, parts, _ = _slabs(y, "glu")
     if not y.is_cuda:
         r = ref.glu(y.view(T, n // 16, 2, 16).transpose(1, 2).reshape(T, 2 * n) if tiled else y, act_dtype, kind)
         return r if out is None else out.copy_(r)
@@ -1603,14 +1617,14 @@ def hc_step(xs: torch.Tensor, y: Optional[torch.Tensor], mix: Optional[torch.Ten
             in_w: Optional[torch.Tensor], norm_w: Optional[torch.Tensor], eps: float,
             act_dtype: Optional[torch.dtype]) -> Optional[torch.Tensor]:
     """One launch between two sublayers of a residual of S parallel streams xs (fp32 [T, S, d], in place). With
-    ``y`` (fp32 [T, d], the sublayer's result): every new stream is a mixture of the old ones plus its share of
+    ``y`` (fp32 [T, d], the sublayer's result; it may be a ``PartialSum``): every new stream is a mixture of the old ones plus its share of
     y, xs[:, j] <- sum_s mix[s, j] xs[:, s] + out_w[j] y. With ``in_w``: the next sublayer's input
     u = sum_s in_w[s] xs[:, s]; returned RMS-normed times ``norm_w`` in ``act_dtype``, or, without a norm weight,
     as it is in fp32. Without ``in_w`` nothing is returned."""
     T, S, d = xs.shape
     if xs.dtype != torch.float32 or not xs.is_contiguous() or S > MAX_STREAMS:
         raise ValueError(f"hc_step: the streams are a contiguous fp32 [T, S, d] tensor, S <= {MAX_STREAMS}")
-    if y is not None and (y.shape != (T, d) or y.dtype != torch.float32 or mix is None or out_w is None
+    if y is not None and (not _is_result(y, xs[:, 0]) or mix is None or out_w is None
                           or mix.numel() != S * S or out_w.numel() != S):
         raise ValueError("hc_step: an fp32 [T, d] result with mix [S, S] and out [S]")
     if (in_w is not None and in_w.numel() != S) or (norm_w is not None and (in_w is None or norm_w.numel() != d)):
@@ -1624,7 +1638,10 @@ def hc_step(xs: torch.Tensor, y: Optional[torch.Tensor], mix: Optional[torch.Ten
         return None
     u = torch.empty(T, d, dtype=torch.float32, device=xs.device) if in_w is not None and norm_w is None else None
     xa = torch.empty(T, d, dtype=act_dtype, device=xs.device) if norm_w is not None else None
-    _hip().call("lc_hc_step", xs.data_ptr(), _hip().ptr(y.contiguous() if y is not None else None), _hip().ptr(mix),
+    if isinstance(y, PartialSum) and (d % 4 or d > 4096):        # (rows that the launch reads coordinate by coordinate)
+        y = y.reduce(out_f32=True)
+    part, parts, bias = _slabs(y, "hc_step", bias=True) if y is not None else (None, 1, None)
+    _hip().call("lc_hc_step", xs.data_ptr(), _hip().ptr(part), parts, _hip().ptr(bias), _hip().ptr(mix),
                 _hip().ptr(out_w), _hip().ptr(in_w), _hip().ptr(norm_w), float(eps), _hip().ptr(u), _hip().ptr(xa),
                 _f32flag(act_dtype) if xa is not None else 0, T, S, d)
     return xa if xa is not None else u
@@ -1748,7 +1765,7 @@ def gated_step(x: torch.Tensor, y: Optional[torch.Tensor], gate: Optional[torch.
     T, d = x.shape
     if x.dtype != torch.float32 or not x.is_contiguous():
         raise ValueError("gated_step: the residual stream is a contiguous fp32 tensor")
-    if y is not None and (y.shape != x.shape or y.dtype != torch.float32):
+    if y is not None and not _is_result(y, x):
         raise ValueError("gated_step: the sublayer output must be fp32 of the stream's shape")
     if gate is not None and (y is None or gate.shape != x.shape or gate.dtype != torch.float32 or gate.stride(1) != 1):
         raise ValueError("gated_step: gate logits are fp32 [T, d] and need a sublayer output")
@@ -1766,9 +1783,10 @@ def gated_step(x: torch.Tensor, y: Optional[torch.Tensor], gate: Optional[torch.
     h32 = torch.empty(T, d, dtype=torch.float32, device=dev) if (w_in is not None and want_f32 and not f32) else None
     hs = torch.empty(T, d, dtype=act_dtype, device=dev) if shift is not None else None
     p = _hip().ptr
-    _hip().call("lc_gated_step", x.data_ptr(), p(y.contiguous() if y is not None else None), 1, p(gate),
+    part, parts, bias = _slabs(y, "gated_step", bias=True) if y is not None else (None, 1, None)
+    _hip().call("lc_gated_step", x.data_ptr(), p(part), parts, p(bias), p(gate),
                 max(gate.stride(0), d) if gate is not None else 0, p(w_out), p(w_in), float(eps), p(ha), p(h32),
-                None, None, _f32flag(act_dtype), p(shift.mu) if shift else None, p(shift.state) if shift else None,
+                None, None, 0, 0, _f32flag(act_dtype), p(shift.mu) if shift else None, p(shift.state) if shift else None,
                 max(shift.state.stride(0), d) if shift else 0, p(lay.row_seq) if shift else None,
                 p(positions) if shift else None, p(lay.state_slots) if shift else None, p(hs), T, d)
     return ha, (ha if f32 else h32), hs
@@ -1782,7 +1800,7 @@ def dual_norm_step(x: torch.Tensor, y, w1: Optional[torch.Tensor], w2: Optional[
     T, d = x.shape
     if x.dtype != torch.float32 or not x.is_contiguous():
         raise ValueError("dual_norm_step: the residual stream is a contiguous fp32 tensor")
-    if y is not None and (y.shape != x.shape or (torch.is_tensor(y) and y.dtype != torch.float32)):
+    if y is not None and not _is_result(y, x):
         raise ValueError("dual_norm_step: the sublayers' output must be fp32 of the stream's shape")
     if w1 is None and w2 is not None:
         raise ValueError("dual_norm_step: the second norm stands beside the first")
@@ -1792,10 +1810,7 @@ def dual_norm_step(x: torch.Tensor, y, w1: Optional[torch.Tensor], w2: Optional[
         return None, None
     h1 = torch.empty(T, d, dtype=act_dtype, device=x.device) if w1 is not None else None
     h2 = torch.empty(T, d, dtype=act_dtype, device=x.device) if w2 is not None else None
-    p = _hip().ptr
-    part, parts = _slabs(y, "dual_norm_step") if y is not None else (None, 1)
-    _hip().call("lc_gated_step", x.data_ptr(), p(part), parts, None, 0, None, p(w1), float(eps),
-                p(h1), None, p(w2), p(h2), _f32flag(act_dtype), None, None, 0, None, None, None, None, T, d)
+    _residual_step(x, y, w_in=w1, w_in2=w2, eps=eps, act_dtype=act_dtype, ha=h1, ha2=h2)
     return h1, h2
 
 

@@ -61,7 +61,6 @@ _SIGNATURES = {
     "lc_scatter_rows": [_P, _P, _P, _I, _I, _P, _P],
     # hybrid decoders (hybrid.hip)
     "lc_embed_rows": [_P, _P, _I, _P, _P, _I, _I, _I, _I, _P, _P, _F, _P, _P, _P, _L, _L, _L, _P, _L, _P, _P, _P, _P],
-    "lc_scalar_norm_add": [_P, _P, _P, _F, _P, _I, _I, _I, _P],
     "lc_relu2": [_P, _P, _I, _I, _I, _I, _P],
     "lc_mingru_scan": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P, _P],
     "lc_gla_scan": [_P, _I, _P, _P, _L, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _P, _P, _P],
@@ -78,7 +77,6 @@ _SIGNATURES = {
     "lc_attn_keys32": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _I, _F, _I, _P, _P, _I, _F, _I, _I,
                        _I, _I, _I, _I, _P],
     "lc_gemm_any": [_P, _I, _I, _P, _I, _P, _P, _I, _I, _I, _I, _I, _P],
-    "lc_add_rmsnorm": [_P, _P, _P, _F, _P, _I, _I, _I, _P],
     "lc_latent_write": [_P, _I, _I, _I, _P, _F, _P, _P, _I, _I, _I, _P],
     "lc_head_linear": [_P, _I, _I, _P, _I, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P],
     "lc_mlstm_scan": [_P, _I, _P, _L, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _P, _P, _P],
@@ -88,13 +86,13 @@ _SIGNATURES = {
     "lc_rope_pairs_write": [_P, _I, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P],
     # parallel residual streams, rotary values, mixed heads' weights, rotated latent keys, xIELU (hybrid_streams.hip)
     "lc_hc_init": [_P, _P, _F, _P, _I, _I, _I, _P],
-    "lc_hc_step": [_P, _P, _P, _P, _P, _P, _F, _P, _P, _I, _I, _I, _I, _P],
+    "lc_hc_step": [_P, _P, _I, _P, _P, _P, _P, _P, _F, _P, _P, _I, _I, _I, _I, _P],
     "lc_rope_qkv_write": [_P, _I, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P],
     "lc_talk_mix": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "lc_latent_rope_write": [_P, _I, _I, _P, _F, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "lc_xielu": [_P, _I, _P, _I, _I, _I, _F, _F, _P],
     # gated residual steps, token shifts, attention pre-processing with convolutions and mixed values (hybrid_gated.hip)
-    "lc_gated_step": [_P, _P, _I, _P, _I, _P, _P, _F, _P, _P, _P, _P, _I, _P, _P, _L, _P, _P, _P, _P, _I, _I, _P],
+    "lc_gated_step": [_P, _P, _I, _P, _P, _I, _P, _P, _F, _P, _P, _P, _P, _I, _I, _I, _P, _P, _L, _P, _P, _P, _P, _I, _I, _P],
     "lc_token_shift": [_P, _P, _P, _L, _P, _P, _P, _P, _P, _I, _I, _I, _P],
     "lc_attn_prep": [_P, _I, _P, _I, _P, _L, _I, _P, _P, _F, _P, _I, _I, _F, _I, _F, _F, _P, _I, _F, _P, _P, _P, _P, _P, _P, _P, _P,
                      _I, _P, _I, _I, _I, _I, _I, _I, _P],

@@ -1086,3 +1086,30 @@ def test_single_rows_split_over_waves(cache, H, G, D, Dv, every, share, chunk, w
             got = ops.attn_masked(c(q), c(kc), c(vc), c(tables), c(cu), c(rs), c(pos), H, G, D, Dv, D ** -0.5, chunk, window, dt, softcap=cap,
                                   all_value_heads=every, keep=keep, value_share=share, **dopt)
             torch.testing.assert_close(got.float().cpu(), want, **(_tol(dt) if dt == torch.bfloat16 else dict(atol=3e-5, rtol=3e-5)))
+
+
+# rows in registers (whole 16-byte pieces up to 4096), rows read again (odd widths, wider ones); few and many slabs; a bias beside them
+@pytest.mark.parametrize("dt", ACTS)
+@pytest.mark.parametrize("T,d,parts", [(3, 2048, 4), (5, 4096, 16), (2, 4100, 2), (4, 70, 3), (600, 64, 1)])
+def test_residual_steps_sum_slabs_and_bias(dt, T, d, parts):
+    g = torch.Generator().manual_seed(T + d)
+    x, part, bias = torch.randn(T, d, generator=g), torch.randn(parts, T, d, generator=g), torch.randn(d, generator=g).bfloat16()
+    y, w, gain = part.sum(0) + bias.float(), torch.rand(d, generator=g) + 0.5, torch.tensor([1.3])
+    slabs = lambda: ops.PartialSum(part.to(DEV), bias.to(DEV))   # noqa: E731
+    tol = _tol(dt) if dt == torch.bfloat16 else dict(atol=5e-5, rtol=5e-5)
+    xr, xd = x.clone(), x.to(DEV)
+    for fn, arg in (("scalar_norm_add", gain), ("add_rmsnorm", w)):
+        want, got = getattr(ref, fn)(xr, y, arg, 1e-5, dt), getattr(ops, fn)(xd, slabs(), arg.to(DEV), 1e-5, dt)
+        torch.testing.assert_close(got.float().cpu(), want.float(), **tol)
+        torch.testing.assert_close(xd.cpu(), xr, atol=5e-5, rtol=5e-5)
+    if d % 32 and (d % 4 or d > 4096):
+        return                                        # (a sum of slabs on their own takes whole groups of 32 columns)
+    for S in (1, 2, 3):
+        xs = torch.randn(T, S, d, generator=g)
+        mix, ow, iw = torch.randn(S, S, generator=g), torch.randn(S, generator=g), torch.randn(S, generator=g)
+        xr, xd = xs.clone(), xs.to(DEV)
+        for norm in (w, None):
+            want = ref.hc_step(xr, y, mix, ow, iw, norm, 1e-5, dt)
+            got = ops.hc_step(xd, slabs(), mix.to(DEV), ow.to(DEV), iw.to(DEV), norm.to(DEV) if norm is not None else None, 1e-5, dt)
+            torch.testing.assert_close(got.float().cpu(), want.float(), **(tol if norm is not None else dict(atol=2e-4, rtol=2e-4)))
+            torch.testing.assert_close(xd.cpu(), xr, atol=2e-4, rtol=2e-4)
