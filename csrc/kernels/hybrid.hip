@@ -170,18 +170,9 @@ __global__ void mingru_scan_kernel(const float* __restrict__ zxg, float* __restr
 
 // ---------------------------------------------------------------- gated linear attention
 // proj [T, ld]: q | k | v at columns 0, H*D, 2*H*D; decay [T, H*D] logits. One block per
-// (value-column tile of 64, head, sequence x segment); thread dv keeps column dv of the head's
+// (value-column tile of 64, head, sequence); thread dv keeps column dv of the head's
 // state S [D, Dv] in registers (DMAX >= D). q, k and the decay come prepared (gla_prepare_kernel);
-// per token S = a * S + k v^T, o = S^T q.
-// Long portions run as segments of seg_len rows side by side, in three passes:
-//   scan_segment_state_kernel: what each segment's rows alone add to the state (from zero) goes to
-//           ``cs`` [B, nseg, H, D, Dv] and the product of its decays to ``ca`` [B, nseg, H, D]. No
-//           outputs are needed here, so every state ELEMENT is its own short recurrence and a
-//           thread owns a few of them: thousands of independent chains instead of one per column;
-//   gla_carry_kernel turns the local states into each segment's incoming state, in place;
-//   mode 2  each segment starts from its incoming state, writes its outputs; the last one stores
-//           the sequence's state.
-// mode 0: the whole sequence in one block (decoded tokens, short portions).
+// per token S = a * S + k v^T, o = S^T q. Decoded tokens and short portions; longer ones: hybrid_linear.hip.
 // Everything the recurrence reads per (token, head, key channel), computed once and in parallel:
 // (q / sqrt(D), k, decay, -) with decay = sigmoid(logit)^(1/tau) = exp(log_sigmoid(logit) / tau).
 __global__ void gla_prepare_kernel(const float* __restrict__ proj, int ld, const float* __restrict__ decay,
@@ -202,26 +193,19 @@ __global__ __launch_bounds__(64) void gla_scan_kernel(const float* __restrict__ 
                                                       const int32_t* __restrict__ cu_q,
                                                       const int32_t* __restrict__ positions,
                                                       const int32_t* __restrict__ slots, float* __restrict__ out, int H,
-                                                      int D, int Dv, int mode, int nseg, int seg_len,
-                                                      const float* __restrict__ cs, long long state_stride, int ones,
-                                                      int v_silu) {
-  const int b = blockIdx.z / nseg, seg = blockIdx.z % nseg, h = blockIdx.y;
+                                                      int D, int Dv, long long state_stride, int ones, int v_silu) {
+  const int b = blockIdx.z, h = blockIdx.y;
   const int dv = blockIdx.x * 64 + threadIdx.x;
   const int slot = slots[b];
   const int q0 = cu_q[b], q1 = cu_q[b + 1];
   if (slot < 0 || q1 <= q0) return;
-  const int r0 = mode == 0 ? q0 : q0 + seg * seg_len;
-  const int r1 = mode == 0 ? q1 : min(q1, r0 + seg_len);
-  if (r0 >= q1) return;
   const bool live = dv < Dv;
   float S[DMAX];
   float* st = state + static_cast<size_t>(slot) * state_stride + static_cast<size_t>(h) * D * Dv;
   const int Dvr = Dv - ones;                      // value columns that come from the projection
-  const float* seg_s = cs != nullptr ? cs + ((static_cast<size_t>(b) * nseg + seg) * H + h) * D * Dv : nullptr;
-  const float* from = mode == 2 ? seg_s : st;
-  const bool zero = mode == 0 && positions[q0] == 0;
+  const bool zero = positions[q0] == 0;
 #pragma unroll
-  for (int d = 0; d < DMAX; ++d) S[d] = (!zero && live && d < D) ? from[static_cast<size_t>(d) * Dv + dv] : 0.f;
+  for (int d = 0; d < DMAX; ++d) S[d] = (!zero && live && d < D) ? st[static_cast<size_t>(d) * Dv + dv] : 0.f;
   // Lane j of the wave loads the prepared operands of key channels j, j + 64, ... of the token (one
   // coalesced 16-byte load per lane, the next token's in flight during the current one); the
   // channel loop then broadcasts them lane by lane (v_readlane) to meet every lane's state column.
@@ -238,12 +222,12 @@ __global__ __launch_bounds__(64) void gla_scan_kernel(const float* __restrict__ 
     }
     vv = !live ? 0.f : (dv < Dvr ? proj[static_cast<size_t>(t) * ld + 2 * H * D + h * Dvr + dv] : 1.f);
   };
-  fetch(r0, nxt, vnxt);
-  for (int t = r0; t < r1; ++t) {
+  fetch(q0, nxt, vnxt);
+  for (int t = q0; t < q1; ++t) {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) cur[i] = nxt[i];
     vcur = v_silu ? siluf_(vnxt) : vnxt;
-    if (t + 1 < r1) fetch(t + 1, nxt, vnxt);
+    if (t + 1 < q1) fetch(t + 1, nxt, vnxt);
     float o = 0.f;
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
@@ -261,100 +245,10 @@ __global__ __launch_bounds__(64) void gla_scan_kernel(const float* __restrict__ 
     }
     if (live) out[static_cast<size_t>(t) * H * Dv + h * Dv + dv] = o;
   }
-  if (live && r1 == q1) {
+  if (live) {
 #pragma unroll
     for (int d = 0; d < DMAX; ++d)
       if (d < D) st[static_cast<size_t>(d) * Dv + dv] = S[d];
-  }
-}
-
-// A segment's own contribution to the state, from zero: cs[d, dv] = sum_t (prod_{r > t} a_r[d]) k_t[d] v_t[dv] over
-// its rows, and ca[d] = prod_t a_t[d]. One block per (tile of 32 key channels x 128 value columns, head,
-// sequence x segment); the segment's operands are staged in LDS once (seg_len <= kSegRows), a thread
-// owns 4 x 4 state elements and walks the rows: acc <- a acc + k v.
-constexpr int kSegRows = 64, kSegD = 32, kSegV = 128;
-
-__global__ __launch_bounds__(256) void scan_segment_state_kernel(
-    const float* __restrict__ proj, int ld, const float4* __restrict__ prep, const int32_t* __restrict__ cu_q,
-    const int32_t* __restrict__ slots, int H, int D, int Dv, int nseg, int seg_len, float* __restrict__ cs,
-    float* __restrict__ ca, int ones, int v_silu) {
-  __shared__ float2 ka[kSegRows][kSegD];            // (k, a) of the tile's key channels
-  __shared__ float vs[kSegRows][kSegV];
-  const int b = blockIdx.z / nseg, seg = blockIdx.z % nseg, h = blockIdx.y;
-  const int ndt = (D + kSegD - 1) / kSegD;
-  const int d0 = (blockIdx.x % ndt) * kSegD, v0 = (blockIdx.x / ndt) * kSegV;
-  const int q0 = cu_q[b], q1 = cu_q[b + 1];
-  if (slots[b] < 0 || q1 <= q0) return;
-  const int r0 = q0 + seg * seg_len;
-  if (r0 >= q1) return;                               // the same for the whole block
-  const int n = min(seg_len, q1 - r0);
-  const int Dvr = Dv - ones;
-  for (int i = threadIdx.x; i < kSegRows * kSegD; i += 256) {
-    const int t = i / kSegD, d = d0 + i % kSegD;
-    float2 e = make_float2(0.f, 1.f);                 // rows and channels past the end change nothing
-    if (t < n && d < D) {
-      const float4 x = prep[(static_cast<size_t>(r0 + t) * H + h) * D + d];
-      e = make_float2(x.y, x.z);
-    }
-    ka[t][i % kSegD] = e;
-  }
-  for (int i = threadIdx.x; i < kSegRows * kSegV; i += 256) {
-    const int t = i / kSegV, dv = v0 + i % kSegV;
-    float v = 0.f;
-    if (t < n && dv < Dv) v = dv < Dvr ? proj[static_cast<size_t>(r0 + t) * ld + 2 * H * D + h * Dvr + dv] : 1.f;
-    if (v_silu) v = siluf_(v);
-    vs[t][i % kSegV] = v;
-  }
-  __syncthreads();
-  const int td = (threadIdx.x >> 5) * 4, tv = threadIdx.x & 31;   // channels td .. td + 3, columns tv + 32 j
-  float acc[4][4] = {};
-  float ap[4] = {1.f, 1.f, 1.f, 1.f};
-  for (int t = 0; t < n; ++t) {
-    float vv[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) vv[j] = vs[t][tv + 32 * j];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float2 e = ka[t][td + i];
-      ap[i] *= e.y;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = e.y * acc[i][j] + e.x * vv[j];
-    }
-  }
-  float* out = cs + ((static_cast<size_t>(b) * nseg + seg) * H + h) * D * Dv;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d = d0 + td + i;
-    if (d >= D) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int dv = v0 + tv + 32 * j;
-      if (dv < Dv) out[static_cast<size_t>(d) * Dv + dv] = acc[i][j];
-    }
-    if (v0 == 0 && tv == 0) ca[((static_cast<size_t>(b) * nseg + seg) * H + h) * D + d] = ap[i];
-  }
-}
-
-// Between the two segment passes: cs[b, s] holds segment s's local state on entry and the state the
-// segment STARTS from on exit (the sequence's own state for s = 0). One thread per state element.
-__global__ void gla_carry_kernel(float* __restrict__ cs, const float* __restrict__ ca, const float* __restrict__ state,
-                                 const int32_t* __restrict__ cu_q, const int32_t* __restrict__ positions,
-                                 const int32_t* __restrict__ slots, int H, int D, int Dv, int nseg, int seg_len,
-                                 long long state_stride) {
-  const int b = blockIdx.y;
-  const size_t n = static_cast<size_t>(H) * D * Dv;
-  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int slot = slots[b];
-  const int q0 = cu_q[b], q1 = cu_q[b + 1];
-  if (i >= n || slot < 0 || q1 <= q0) return;
-  const size_t hd = i / Dv;                         // (head, key channel)
-  float carry = positions[q0] == 0 ? 0.f : state[static_cast<size_t>(slot) * state_stride + i];
-  const int used = (q1 - q0 + seg_len - 1) / seg_len;
-  for (int s = 0; s < used; ++s) {
-    float* p = cs + (static_cast<size_t>(b) * nseg + s) * n + i;
-    const float local = *p;
-    *p = carry;
-    carry = ca[(static_cast<size_t>(b) * nseg + s) * H * D + hd] * carry + local;
   }
 }
 
@@ -413,25 +307,28 @@ __global__ void lightning_prepare_kernel(const float* __restrict__ proj, int ld,
 // i = cap tanh(. / cap) and f = log sigmoid(cap tanh(. / cap)) (cap 0: no cap), the running maximum
 // m_t = max(f_t + m_(t-1), i_t) (0 before the first token) stabilises
 //   S_t = a_t S_(t-1) + b_t k_t v_t^T,  a_t = exp(f_t + m_(t-1) - m_t),  b_t = exp(i_t - m_t).
-// One wave per (head, sequence): 64 tokens at a time, the lanes compute the gates of their tokens and
-// the maxima come from a wave scan (m -> max(m + F, I) composes as (F1 + F2, max(I1 + F2, I2))).
+// One block per (head, sequence), up to 1024 tokens at a time: the lanes compute the gates of their tokens and
+// the maxima come from a scan of the wave and then over the waves (m -> max(m + F, I) composes as (F1 + F2, max(I1 + F2, I2))).
+// Latency-bound, so the launch takes as many waves as the longest portion has groups of 64 tokens (1500 tokens, 16 heads: 8 us;
+// one wave that walked them took 31).
 // Writes (a, b) per (token, head), m per (token, head), and the sequence's last m behind its state.
 LC_DEVICE float soft_cap(float x, float cap) { return cap > 0.f ? cap * tanhf(x / cap) : x; }
 
-__global__ __launch_bounds__(64) void mlstm_gates_kernel(const float* __restrict__ proj, int ld, int col_i,
+__global__ __launch_bounds__(1024) void mlstm_gates_kernel(const float* __restrict__ proj, int ld, int col_i,
                                                          float* __restrict__ state, long long state_stride,
                                                          long long m_offset, const int32_t* __restrict__ cu_q,
                                                          const int32_t* __restrict__ positions,
                                                          const int32_t* __restrict__ slots, float2* __restrict__ gates,
                                                          float* __restrict__ m_out, int H, float cap) {
-  const int h = blockIdx.x, b = blockIdx.y, lane = threadIdx.x;
+  __shared__ float wf[16], wi[16];                  // (F, I) of whole waves
+  const int h = blockIdx.x, b = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   const int slot = slots[b];
   const int q0 = cu_q[b], q1 = cu_q[b + 1];
-  if (slot < 0 || q1 <= q0) return;
+  if (slot < 0 || q1 <= q0) return;                  // the same for the whole block
   float* ms = state + static_cast<size_t>(slot) * state_stride + m_offset + h;
   float m = positions[q0] == 0 ? 0.f : *ms;
-  for (int r0 = q0; r0 < q1; r0 += 64) {
-    const int t = r0 + lane;
+  for (int r0 = q0; r0 < q1; r0 += blockDim.x) {
+    const int t = r0 + threadIdx.x;
     const bool valid = t < q1;
     const float iv = valid ? soft_cap(proj[static_cast<size_t>(t) * ld + col_i + h], cap) : -INFINITY;
     const float fv = valid ? logsigmoidf_(soft_cap(proj[static_cast<size_t>(t) * ld + col_i + H + h], cap)) : 0.f;
@@ -444,16 +341,25 @@ __global__ __launch_bounds__(64) void mlstm_gates_kernel(const float* __restrict
         F = Fp + F;
       }
     }
-    const float mt = fmaxf(m + F, I);
+    if (lane == 63) {
+      wf[wave] = F;
+      wi[wave] = I;
+    }
+    __syncthreads();
+    float from = m;                                  // the maximum in front of this wave's tokens, then behind the last wave's
+    for (int w = 0; w < wave; ++w) from = fmaxf(from + wf[w], wi[w]);
+    const float mt = fmaxf(from + F, I);
     float mp = __shfl_up(mt, 1, 64);
-    if (lane == 0) mp = m;
+    if (lane == 0) mp = from;
     if (valid) {
       gates[static_cast<size_t>(t) * H + h] = make_float2(expf(fv + mp - mt), expf(iv - mt));
       m_out[static_cast<size_t>(t) * H + h] = mt;
     }
-    m = __shfl(mt, min(63, q1 - 1 - r0), 64);
+    for (int w = wave; w < waves; ++w) from = fmaxf(from + wf[w], wi[w]);
+    m = from;
+    __syncthreads();                                 // read before the next tokens' sums overwrite them
   }
-  if (lane == 0) *ms = m;
+  if (threadIdx.x == 0) *ms = m;
 }
 
 // (q / sqrt(D), b k, a, -) per (token, head, key channel): the operands of the scan below.
@@ -1262,48 +1168,32 @@ LC_EXPORT int lc_mingru_scan(const void* zxg, void* state, const void* cu_q, con
 // S <- a S + k v^T over Dv value columns, the last ``ones`` of which read v = 1; ``v_silu``: v is silu of the projection.
 static int launch_linear_scan(const void* proj, int ld, const void* prep, void* state, long long state_stride,
                               const void* cu_q, const void* positions, const void* slots, void* out, int B, int H, int D,
-                              int Dv, int ones, int max_len, void* scratch, hipStream_t st, int v_silu = 0) {
-  const bool segmented = max_len > 2 * kScanSegment;
-  if (segmented && scratch == nullptr) return -1;
-  const int nseg = segmented ? (max_len + kScanSegment - 1) / kScanSegment : 1;
-  const dim3 grid((Dv + 63) / 64, H, B * nseg), block(64);
-  float* cs = static_cast<float*>(scratch);
-  float* ca = segmented ? cs + static_cast<size_t>(B) * nseg * H * D * Dv : nullptr;
-#define LC_GLA(DMAX, MODE)                                                                                             \
+                              int Dv, int ones, hipStream_t st, int v_silu = 0) {
+  const dim3 grid((Dv + 63) / 64, H, B), block(64);
+#define LC_GLA(DMAX)                                                                                                   \
   gla_scan_kernel<DMAX><<<grid, block, 0, st>>>(static_cast<const float*>(proj), ld, static_cast<const float4*>(prep), \
                                                 static_cast<float*>(state), static_cast<const int32_t*>(cu_q),      \
                                                 static_cast<const int32_t*>(positions),                             \
                                                 static_cast<const int32_t*>(slots), static_cast<float*>(out), H, D, \
-                                                Dv, MODE, nseg, kScanSegment, cs, state_stride, ones, v_silu)
-#define LC_GLA_D(MODE)          \
-  if (D <= 32) LC_GLA(32, MODE);  \
-  else if (D <= 64) LC_GLA(64, MODE); \
-  else if (D <= 128) LC_GLA(128, MODE); \
-  else LC_GLA(256, MODE)
-  if (segmented) {
-    static_assert(kScanSegment <= kSegRows, "a segment's rows are staged in LDS at once");
-    const dim3 sgrid(((D + kSegD - 1) / kSegD) * ((Dv + kSegV - 1) / kSegV), H, B * nseg);
-    scan_segment_state_kernel<<<sgrid, dim3(256), 0, st>>>(
-        static_cast<const float*>(proj), ld, static_cast<const float4*>(prep), static_cast<const int32_t*>(cu_q),
-        static_cast<const int32_t*>(slots), H, D, Dv, nseg, kScanSegment, cs, ca, ones, v_silu);
-    const size_t n = static_cast<size_t>(H) * D * Dv;
-    gla_carry_kernel<<<dim3(static_cast<unsigned>((n + 255) / 256), B), dim3(256), 0, st>>>(
-        cs, ca, static_cast<const float*>(state), static_cast<const int32_t*>(cu_q),
-        static_cast<const int32_t*>(positions), static_cast<const int32_t*>(slots), H, D, Dv, nseg, kScanSegment,
-        state_stride);
-    LC_GLA_D(2);
-  } else {
-    LC_GLA_D(0);
-  }
-#undef LC_GLA_D
+                                                Dv, state_stride, ones, v_silu)
+  if (D <= 32) LC_GLA(32);
+  else if (D <= 64) LC_GLA(64);
+  else if (D <= 128) LC_GLA(128);
+  else LC_GLA(256);
 #undef LC_GLA
   LC_RETURN_LAST_ERROR();
 }
 
-// ``prep``: T * H * D float4 of scratch for the per-token operands (gla_prepare_kernel).
+// Portions from this many rows on are taken in chunks (hybrid_linear.hip): the scan is a chain of 2 D dependent instructions per
+// row, the chunks' three launches take the same time for any length up to 64. 16 heads of 128, one portion: 16 rows 41 us in chunks
+// and 102 row by row, 8 rows 41 and 56, 4 rows 41 and 34; eight portions of 16 rows 76 and 106.
+constexpr int kChunkFrom = 16;
+
+LC_EXPORT int lc_linear_in_chunks(int max_len) { return max_len >= kChunkFrom; }
+
 LC_EXPORT int lc_gla_scan(const void* proj, int ld, const void* decay, void* state, long long state_stride,
                           const void* cu_q, const void* positions, const void* slots, void* out, int T, int B, int H,
-                          int D, int Dv, float tau, int max_len, void* scratch, void* prep, hipStream_t st) {
+                          int D, int Dv, float tau, void* prep, hipStream_t st) {
   if (B <= 0) return 0;
   if (H <= 0 || D <= 0 || Dv <= 0 || D > 256 || ld < 2 * H * D + H * Dv || !(tau > 0.f)) return -1;
   if (prep == nullptr || T <= 0 || state_stride < static_cast<long long>(H) * D * Dv) return -1;
@@ -1311,44 +1201,52 @@ LC_EXPORT int lc_gla_scan(const void* proj, int ld, const void* decay, void* sta
   gla_prepare_kernel<<<dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st>>>(
       static_cast<const float*>(proj), ld, static_cast<const float*>(decay), static_cast<float4*>(prep), n, H * D,
       1.f / tau, 1.f / sqrtf(static_cast<float>(D)));
-  return launch_linear_scan(proj, ld, prep, state, state_stride, cu_q, positions, slots, out, B, H, D, Dv, 0, max_len,
-                            scratch, st);
+  return launch_linear_scan(proj, ld, prep, state, state_stride, cu_q, positions, slots, out, B, H, D, Dv, 0, st);
 }
 
 // One constant decay per head (``decay`` [H]); q, k and v are silu of the projection; no scale on q.
 LC_EXPORT int lc_lightning_scan(const void* proj, int ld, const void* decay, void* state, long long state_stride,
                                 const void* cu_q, const void* positions, const void* slots, void* out, int T, int B, int H,
-                                int D, int Dv, int max_len, void* scratch, void* prep, hipStream_t st) {
+                                int D, int Dv, void* prep, hipStream_t st) {
   if (B <= 0 || T <= 0) return 0;
   if (H <= 0 || D <= 0 || Dv <= 0 || D > 256 || ld < 2 * H * D + H * Dv || decay == nullptr) return -1;
   if (prep == nullptr || state_stride < static_cast<long long>(H) * D * Dv) return -1;
   const long long n = static_cast<long long>(T) * H * D;
   lightning_prepare_kernel<<<dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st>>>(
       static_cast<const float*>(proj), ld, static_cast<const float*>(decay), static_cast<float4*>(prep), n, H, D);
-  return launch_linear_scan(proj, ld, prep, state, state_stride, cu_q, positions, slots, out, B, H, D, Dv, 0, max_len,
-                            scratch, st, 1);
+  return launch_linear_scan(proj, ld, prep, state, state_stride, cu_q, positions, slots, out, B, H, D, Dv, 0, st, 1);
 }
 
-// mLSTM: gates and running maxima, prepared operands, then the scan over Dv + 1 value columns (the
-// extra column, v = 1, is the normaliser). ``prep``: T * H * (4 D + 2) floats; ``out`` [T, H * (Dv + 1)];
-// ``m_out`` [T, H]; a slot of ``state`` holds H * D * (Dv + 1) floats and then the H maxima.
-LC_EXPORT int lc_mlstm_scan(const void* proj, int ld, void* state, long long state_stride, const void* cu_q,
-                            const void* positions, const void* slots, void* out, void* m_out, int T, int B, int H, int D,
-                            int Dv, float cap, int max_len, void* scratch, void* prep, hipStream_t st) {
+// mLSTM gates and running maxima: ``gates`` [T, H] pairs, ``m_out`` [T, H]; a slot of ``state`` holds H * D * (Dv + 1) floats and
+// then the H maxima.
+LC_EXPORT int lc_mlstm_gates(const void* proj, int ld, void* state, long long state_stride, const void* cu_q, const void* positions,
+                             const void* slots, void* gates, void* m_out, int T, int B, int H, int D, int Dv, float cap, int max_len,
+                             hipStream_t st) {
   if (B <= 0 || T <= 0) return 0;
-  if (H <= 0 || D <= 0 || Dv <= 0 || D > 256 || ld < 2 * H * D + 2 * H * Dv + 2 * H || cap < 0.f) return -1;
+  if (H <= 0 || D <= 0 || Dv <= 0 || ld < 2 * H * D + 2 * H * Dv + 2 * H || cap < 0.f) return -1;
   const long long n_s = static_cast<long long>(H) * D * (Dv + 1);
-  if (prep == nullptr || m_out == nullptr || state_stride < n_s + H) return -1;
-  const long long n = static_cast<long long>(T) * H * D;
-  float2* gates = reinterpret_cast<float2*>(static_cast<float4*>(prep) + n);
-  mlstm_gates_kernel<<<dim3(H, B), dim3(64), 0, st>>>(
+  if (gates == nullptr || m_out == nullptr || state_stride < n_s + H) return -1;
+  const int waves = std::max(1, std::min(16, (max_len + 63) / 64));
+  mlstm_gates_kernel<<<dim3(H, B), dim3(64 * waves), 0, st>>>(
       static_cast<const float*>(proj), ld, 2 * H * D + 2 * H * Dv, static_cast<float*>(state), state_stride, n_s,
-      static_cast<const int32_t*>(cu_q), static_cast<const int32_t*>(positions), static_cast<const int32_t*>(slots), gates,
-      static_cast<float*>(m_out), H, cap);
+      static_cast<const int32_t*>(cu_q), static_cast<const int32_t*>(positions), static_cast<const int32_t*>(slots),
+      static_cast<float2*>(gates), static_cast<float*>(m_out), H, cap);
+  LC_RETURN_LAST_ERROR();
+}
+
+// mLSTM behind its gates: prepared operands (``prep``: T * H * D float4), then the scan over Dv + 1 value columns (the extra
+// column, v = 1, is the normaliser); ``out`` [T, H * (Dv + 1)].
+LC_EXPORT int lc_mlstm_scan(const void* proj, int ld, const void* gates, void* state, long long state_stride, const void* cu_q,
+                            const void* positions, const void* slots, void* out, int T, int B, int H, int D,
+                            int Dv, void* prep, hipStream_t st) {
+  if (B <= 0 || T <= 0) return 0;
+  if (H <= 0 || D <= 0 || Dv <= 0 || D > 256 || ld < 2 * H * D + H * Dv || gates == nullptr) return -1;
+  if (prep == nullptr || state_stride < static_cast<long long>(H) * D * (Dv + 1)) return -1;
+  const long long n = static_cast<long long>(T) * H * D;
   mlstm_prepare_kernel<<<dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st>>>(
-      static_cast<const float*>(proj), ld, gates, static_cast<float4*>(prep), n, H, D, 1.f / sqrtf(static_cast<float>(D)));
-  return launch_linear_scan(proj, ld, prep, state, state_stride, cu_q, positions, slots, out, B, H, D, Dv + 1, 1, max_len,
-                            scratch, st);
+      static_cast<const float*>(proj), ld, static_cast<const float2*>(gates), static_cast<float4*>(prep), n, H, D,
+      1.f / sqrtf(static_cast<float>(D)));
+  return launch_linear_scan(proj, ld, prep, state, state_stride, cu_q, positions, slots, out, B, H, D, Dv + 1, 1, st);
 }
 
 LC_EXPORT int lc_glu(const void* y, int parts, int tiled, void* out, int act_f32, int T, int n, int kind, int ldo, hipStream_t st) {

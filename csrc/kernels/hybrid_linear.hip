@@ -1,0 +1,414 @@
+// Linear attention of prompt portions in chunks of 64 rows on the matrix cores (fp32): gated linear attention (a decay per key
+// channel), matrix memories with exponential gates and linear attention with one constant decay per head. Per head, with state
+// S [D, Dv] and per row t a decay a_t [D]:  S <- a_t S + k_t v_t^T,  o_t = S^T q_t.
+//
+// Unrolled over a chunk with incoming state S_0, and with A_(r,t] the product of the decays of rows r + 1 .. t:
+//   o_t = (q_t A_(0,t])^T S_0 + sum_(r <= t) s_tr v_r,   s_tr = sum_d q_t[d] k_r[d] A_(r,t][d],
+//   S_64 = A_(0,64] S_0 + sum_r (k_r A_(r,64]) v_r^T.
+// A chunk is four blocks of 16 rows. Only PRODUCTS of decays are formed, never quotients or logarithms, so that
+// strong decays underflow to zero instead of cancelling: prefix products to a block's rows (onto q), suffix products from a
+// block's rows to its end (onto k), whole blocks' products between them. Pairs of rows of one block go channel by channel in
+// registers.
+//   linear_chunk:  per (chunk, head), side by side: what the chunk's rows add to the state, and its decays' product.
+//   linear_carry:  chunk after chunk, a thread per state element: the state each chunk starts from; the sequence's new state.
+//   linear_out:    per (chunk, head), side by side: scores, S_0's share, values.
+// 2048 rows, 16 heads of 128 x 128: 41 + 18 + 56 us (35 + 18 + 54 with one decay per row). Before, segments of 32 rows were
+// scanned row by row, a state column per thread, over operands that a launch of their own had written out (16 bytes per row and
+// channel): 354 us in all. Error against 64 bits, 2048 rows: 3.6e-7 before, 3.5e-7 now, with strong decays 2.1e-7 and 1.1e-7.
+//
+// Chunks of all portions are numbered cu_q[b] / 64 + b + c, so that scratch grows with rows.
+#include "hybrid_common.h"
+
+namespace {
+
+constexpr int kRows = 64;
+
+struct LinearArgs {
+  const float* proj;             // [T, ld]: q | k | v at columns 0, H D, 2 H D
+  int ld;
+  // kinds: 0 decays sigmoid(logit)^(1 / tau); 1 (a, b) per row and head, b onto k; 2 one decay per head, silu on q, k and v
+  const float* decay;            // kind 0: logits [T, H D]; kind 2: [H]
+  const float2* gates;           // kind 1: [T, H]
+  float inv_tau, qscale;
+  float* state;
+  long long state_stride;
+  const int32_t* cu_q;
+  const int32_t* positions;
+  const int32_t* slots;
+  float* out;                    // [T, H Dv]
+  float* cs;                     // [chunks, H, D, Dv]: the chunk's own share, then the state it starts from
+  float* ca;                     // [chunks, H, D]: products of the chunk's decays
+  int H, D, Dv, ones;            // the last ``ones`` of the Dv value columns read 1
+};
+
+struct ChunkRows {
+  int row0, n;                   // rows of the step; n <= 0: no such chunk
+  size_t at;                     // the chunk's number
+};
+
+LC_DEVICE ChunkRows chunk_rows(const LinearArgs& a, int b, int c) {
+  const int q0 = a.cu_q[b], q1 = a.cu_q[b + 1];
+  ChunkRows r{q0 + c * kRows, 0, static_cast<size_t>(q0 / kRows + b + c)};
+  if (a.slots[b] >= 0) r.n = min(kRows, q1 - r.row0);
+  return r;
+}
+
+// A wave's sixteen rows of one key channel: q (QUERY), k and the decays; rows and channels past the end change nothing.
+template <int KIND, bool QUERY>
+LC_DEVICE void load_rows(const LinearArgs& a, const ChunkRows& c, int h, int first, int d, float (&q)[16], float (&k)[16], float (&x)[16]) {
+  const int ch = min(d, a.D - 1), HD = a.H * a.D;
+  const size_t row = static_cast<size_t>(c.row0) + first;
+  const float* src = a.proj + row * a.ld + h * a.D + ch;
+  const float* dec = KIND == 0 ? a.decay + row * HD + h * a.D + ch : nullptr;
+  const float2* gates = KIND == 1 ? a.gates + row * a.H + h : nullptr;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int at = max(0, min(r, c.n - 1 - first));  // (the last row again, or, in a block of rows behind it, the block's first: masked)
+    const int safe = first < c.n ? at : -first;
+    if (QUERY) q[r] = src[safe * a.ld];
+    k[r] = src[safe * a.ld + HD];
+    if (KIND == 0) x[r] = dec[safe * HD];
+    if (KIND == 1) {
+      const float2 g = gates[safe * a.H];
+      x[r] = g.x;
+      k[r] *= g.y;
+    }
+    if (KIND == 2) x[r] = a.decay[h];
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const bool on = first + r < c.n && d < a.D;
+    if (KIND == 0) x[r] = expf(logsigmoidf_(x[r]) * a.inv_tau);
+    if (KIND == 2) {
+      k[r] = siluf_(k[r]);
+      if (QUERY) q[r] = siluf_(q[r]);
+    } else if (QUERY) {
+      q[r] *= a.qscale;
+    }
+    if (!on) {
+      x[r] = 1.f;
+      k[r] = 0.f;
+      if (QUERY) q[r] = 0.f;
+    }
+  }
+}
+
+// Four rows r0 .. r0 + 3 of a chunk's value column (zeros past its rows and columns): the second operand of four matrix instructions.
+template <int KIND>
+LC_DEVICE void value_rows(const LinearArgs& a, const ChunkRows& c, int h, int r0, int col, float (&v)[4]) {
+  const int from = a.Dv - a.ones;                    // value columns that come from the projection
+  const float* src = a.proj + static_cast<size_t>(c.row0) * a.ld + 2 * a.H * a.D + h * from + min(col, from - 1);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float x = src[min(r0 + j, c.n - 1) * a.ld];
+    if (KIND == 2) x = siluf_(x);
+    if (col >= from) x = 1.f;
+    v[j] = r0 + j < c.n && col < a.Dv ? x : 0.f;
+  }
+}
+
+// ---------------------------------------------------------------- a chunk's share of the state
+// Waves: 4 blocks of rows x NL slices of 64 key channels.
+template <int KIND, int DP>
+__global__ __launch_bounds__(4 * DP) void linear_chunk_kernel(LinearArgs a, int tiles_per_block) {
+  constexpr int KS = DP + 4, NL = DP / 64, WAVES = 4 * NL;
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* ks = lds;                                   // [64][KS]: k times the decays behind it in its block
+  float* tot = ks + kRows * KS;                      // [4][DP]: products of whole blocks
+  const int h = blockIdx.y, ncb = (a.Dv + 16 * tiles_per_block - 1) / (16 * tiles_per_block);
+  const int b = blockIdx.z / ncb, cb = blockIdx.z % ncb;
+  const ChunkRows c = chunk_rows(a, b, blockIdx.x);
+  if (c.n <= 0) return;                              // the same for the whole block
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  {
+    const int rb = wave & 3, d = lane + 64 * (wave >> 2);
+    float k[16], x[16];
+    load_rows<KIND, false>(a, c, h, 16 * rb, d, k, k, x);
+    float suf = 1.f;
+#pragma unroll
+    for (int r = 15; r >= 0; --r) {
+      ks[(16 * rb + r) * KS + d] = k[r] * suf;
+      suf *= x[r];
+    }
+    tot[rb * DP + d] = suf;
+  }
+  __syncthreads();
+  if (cb == 0)
+    for (int d = threadIdx.x; d < a.D; d += 64 * WAVES)
+      a.ca[(c.at * a.H + h) * a.D + d] = tot[d] * tot[DP + d] * tot[2 * DP + d] * tot[3 * DP + d];
+  float* cs = a.cs + (c.at * a.H + h) * a.D * a.Dv;
+  // a wave takes every WAVES-th tile of 16 columns over all channels: values are read once
+  for (int ct = cb * tiles_per_block + wave; ct < min((cb + 1) * tiles_per_block, (a.Dv + 15) / 16); ct += WAVES) {
+    const int col = 16 * ct + lr;
+    float v[4][4];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) value_rows<KIND>(a, c, h, 16 * kk + 4 * lk, col, v[kk]);
+    for (int dt = 0; 16 * dt < a.D; ++dt) {
+      const int d = 16 * dt + lr;
+      f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+      float later = 1.f;
+#pragma unroll
+      for (int kk = 3; kk >= 0; --kk) {              // (block kk's rows; the blocks behind it decay them)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[j & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ks[(16 * kk + 4 * lk + j) * KS + d] * later, v[kk][j], acc[j & 1], 0, 0, 0);
+        later *= tot[kk * DP + d];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * dt + 4 * lk + r;
+        if (row < a.D && col < a.Dv) cs[row * a.Dv + col] = acc[0][r] + acc[1][r];
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------- the state each chunk starts from
+// One thread per state element; eight chunks' loads in flight at a time.
+__global__ __launch_bounds__(256) void linear_carry_kernel(LinearArgs a) {
+  const int b = blockIdx.y, slot = a.slots[b];
+  const size_t n = static_cast<size_t>(a.H) * a.D * a.Dv, i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int q0 = a.cu_q[b], q1 = a.cu_q[b + 1];
+  if (i >= n || slot < 0 || q1 <= q0) return;
+  const size_t hd = i / a.Dv, hdn = static_cast<size_t>(a.H) * a.D, first = q0 / kRows + b;
+  float* st = a.state + static_cast<size_t>(slot) * a.state_stride + i;
+  float s = a.positions[q0] == 0 ? 0.f : *st;
+  const int used = (q1 - q0 + kRows - 1) / kRows;
+  for (int c0 = 0; c0 < used; c0 += 8) {
+    float own[8], dec[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const size_t at = first + min(c0 + j, used - 1);
+      own[j] = a.cs[at * n + i];
+      dec[j] = a.ca[at * hdn + hd];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (c0 + j < used) {
+        a.cs[(first + c0 + j) * n + i] = s;
+        s = dec[j] * s + own[j];
+      }
+  }
+  *st = s;
+}
+
+// ---------------------------------------------------------------- a chunk's results
+template <int N>
+LC_DEVICE float rotate_add(float v) {                // inside the 16 lanes of a DPP row
+  const int b = __builtin_bit_cast(int, v);
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(b, b, 0x120 + N, 0xf, 0xf, false));
+}
+
+// Sixteen values of 64 lanes each: the sum of value i + 4 (lane >> 4 & 1) + 8 (lane >> 5) comes back in x[i], i < 4.
+LC_DEVICE void sum_over_lanes(float (&x)[16]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(__float_as_uint(x[i]), __float_as_uint(x[i + 8]), false, false));
+    x[i] = __uint_as_float(r.x) + __uint_as_float(r.y);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(__float_as_uint(x[i]), __float_as_uint(x[i + 4]), false, false));
+    x[i] = rotate_add<1>(rotate_add<2>(rotate_add<4>(rotate_add<8>(__uint_as_float(r.x) + __uint_as_float(r.y)))));
+  }
+}
+
+template <int DP>
+constexpr int out_lds() {
+  return (kRows * (DP + 4) + 48 * (DP + 4) + kRows * (kRows + 4) + 4 * DP) * 4;
+}
+
+// Waves as above. (Four waves to a SIMD: the state's rows are loaded behind the scores, not ahead of them.)
+template <int KIND, int DP>
+__global__ __launch_bounds__(4 * DP, 4) void linear_out_kernel(LinearArgs a, int tiles_per_block) {
+  constexpr int KS = DP + 4, SS = kRows + 4, NL = DP / 64, KK = DP / 16, WAVES = 4 * NL;
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* qs = lds;                                   // [64][KS]: q times the decays of its block up to it
+  float* ks = qs + kRows * KS;                       // [48][KS]: k times the decays behind it in its block (the last block's: not needed)
+  float* ss = ks + 48 * KS;                          // [64][SS]: scores
+  float* tot = ss + kRows * SS;                      // [4][DP]
+  const int h = blockIdx.y, ncb = (a.Dv + 16 * tiles_per_block - 1) / (16 * tiles_per_block);
+  const int b = blockIdx.z / ncb, cb = blockIdx.z % ncb;
+  const ChunkRows c = chunk_rows(a, b, blockIdx.x);
+  if (c.n <= 0) return;                              // the same for the whole block
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  {
+    const int rb = wave & 3, slice = wave >> 2, d = lane + 64 * slice;
+    float q[16], k[16], x[16], own[16];
+    load_rows<KIND, true>(a, c, h, 16 * rb, d, q, k, x);
+    float pre = 1.f, suf = 1.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      pre *= x[r];
+      qs[(16 * rb + r) * KS + d] = q[r] * pre;
+    }
+    tot[rb * DP + d] = pre;
+    if (rb < 3) {
+#pragma unroll
+      for (int r = 15; r >= 0; --r) {
+        ks[(16 * rb + r) * KS + d] = k[r] * suf;
+        suf *= x[r];
+      }
+    }
+    // pairs of rows of this block: k_r decays row by row and meets every later query
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      float w = k[r], s[16];
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        if (t > r) w *= x[t];
+        s[t] = t < r ? 0.f : q[t] * w;
+      }
+      sum_over_lanes(s);
+      own[r] = lr == 0 ? s[0] : lr == 1 ? s[1] : lr == 2 ? s[2] : s[3];
+      __builtin_amdgcn_sched_barrier(0);             // (rows side by side would not fit the registers)
+    }
+    // the slices' sums in turn
+    float* dst = ss + (16 * rb + lr + 4 * (lk & 1) + 8 * (lk >> 1)) * SS + 16 * rb;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      if (slice == i && lr < 4) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dst[r] = i == 0 ? own[r] : dst[r] + own[r];
+      }
+      __syncthreads();
+    }
+  }
+  // pairs of rows of different blocks i > j; the blocks between them decay every channel
+  auto cross = [&](int i, int j) {
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+      const int d = 16 * kk + 4 * lk;
+      float4 q = *reinterpret_cast<const float4*>(qs + (16 * i + lr) * KS + d);
+      const float4 k = *reinterpret_cast<const float4*>(ks + (16 * j + lr) * KS + d);
+      for (int m = j + 1; m < i; ++m) {
+        const float4 f = *reinterpret_cast<const float4*>(tot + m * DP + d);
+        q = make_float4(q.x * f.x, q.y * f.y, q.z * f.z, q.w * f.w);
+      }
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q.x, k.x, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q.y, k.y, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q.z, k.z, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q.w, k.w, acc, 0, 0, 0);
+      if (kk & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ss[(16 * i + 4 * lk + r) * SS + 16 * j + lr] = acc[r];
+  };
+  // six tiles over the waves, the deepest first
+  for (int p = wave; p < 6; p += WAVES) {
+    if (p == 0) cross(3, 0);
+    else if (p == 1) cross(2, 0);
+    else if (p == 2) cross(3, 1);
+    else if (p == 3) cross(1, 0);
+    else if (p == 4) cross(2, 1);
+    else cross(3, 2);
+  }
+  __syncthreads();
+  const float* s0 = a.cs + (c.at * a.H + h) * a.D * a.Dv;
+  const int row_tiles = (c.n + 15) / 16, ct1 = min((cb + 1) * tiles_per_block, (a.Dv + 15) / 16);
+  for (int ct = cb * tiles_per_block + wave; ct < ct1; ct += WAVES) {
+    const int col = 16 * ct + lr, sc = min(col, a.Dv - 1);
+    f32x4 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float v[4][4];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) value_rows<KIND>(a, c, h, 16 * kk + 4 * lk, col, v[kk]);
+    constexpr int KB = 4;                            // depths of the state whose loads are in flight together
+#pragma unroll
+    for (int k0 = 0; k0 < KK; k0 += KB) {
+      float s[KB][4];
+#pragma unroll
+      for (int kk = 0; kk < KB; ++kk)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[kk][j] = s0[min(16 * (k0 + kk) + 4 * lk + j, a.D - 1) * a.Dv + sc];
+#pragma unroll
+      for (int kk = 0; kk < KB; ++kk) {
+        const int d = 16 * (k0 + kk) + 4 * lk;       // (past D the queries are zeros)
+        float4 f = make_float4(1.f, 1.f, 1.f, 1.f);  // decays of the blocks before row tile i
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float4 q = *reinterpret_cast<const float4*>(qs + (16 * i + lr) * KS + d);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.x * f.x, s[kk][0], acc[i], 0, 0, 0);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.y * f.y, s[kk][1], acc[i], 0, 0, 0);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.z * f.z, s[kk][2], acc[i], 0, 0, 0);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.w * f.w, s[kk][3], acc[i], 0, 0, 0);
+          if (i < 3) {
+            const float4 g = *reinterpret_cast<const float4*>(tot + i * DP + d);
+            f = make_float4(f.x * g.x, f.y * g.y, f.z * g.z, f.w * g.w);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);           // (one depth's operands at a time: all of them would spill)
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int kk = 0; kk <= i; ++kk) {
+        const float4 w = *reinterpret_cast<const float4*>(ss + (16 * i + lr) * SS + 16 * kk + 4 * lk);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, v[kk][0], acc[i], 0, 0, 0);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, v[kk][1], acc[i], 0, 0, 0);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.z, v[kk][2], acc[i], 0, 0, 0);
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.w, v[kk][3], acc[i], 0, 0, 0);
+      }
+    if (col >= a.Dv) continue;
+    for (int i = 0; i < row_tiles; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = 16 * i + 4 * lk + r;
+        const float o = i == 0 ? acc[0][r] : i == 1 ? acc[1][r] : i == 2 ? acc[2][r] : acc[3][r];
+        if (t < c.n) a.out[static_cast<size_t>(c.row0 + t) * a.H * a.Dv + h * a.Dv + col] = o;
+      }
+  }
+}
+
+template <int KIND, int DP>
+int launch_linear(const LinearArgs& a, int B, int max_len, hipStream_t st) {
+  constexpr int chunk_bytes = (kRows * (DP + 4) + 4 * DP) * 4;
+  static LcDeviceOnce once;
+  once.run([] {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(linear_chunk_kernel<KIND, DP>), hipFuncAttributeMaxDynamicSharedMemorySize, chunk_bytes);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(linear_out_kernel<KIND, DP>), hipFuncAttributeMaxDynamicSharedMemorySize, out_lds<DP>());
+  });
+  const int chunks = (max_len + kRows - 1) / kRows, tiles = (a.Dv + 15) / 16;
+  // few chunks and heads: their columns go to several blocks (the keys' part is formed again in each)
+  const int blocks = std::max(1, std::min(tiles, static_cast<int>(256 / std::max(1LL, static_cast<long long>(chunks) * a.H * B))));
+  const int per = (tiles + blocks - 1) / blocks, nc = (tiles + per - 1) / per;
+  if (a.H > 65535 || static_cast<long long>(B) * nc > 65535) return -1;
+  linear_chunk_kernel<KIND, DP><<<dim3(chunks, a.H, B * nc), dim3(4 * DP), chunk_bytes, st>>>(a, per);
+  const long long n = static_cast<long long>(a.H) * a.D * a.Dv;
+  linear_carry_kernel<<<dim3(static_cast<unsigned>((n + 255) / 256), B), dim3(256), 0, st>>>(a);
+  linear_out_kernel<KIND, DP><<<dim3(chunks, a.H, B * nc), dim3(4 * DP), out_lds<DP>(), st>>>(a, per);
+  LC_RETURN_LAST_ERROR();
+}
+
+template <int DP>
+int launch_linear_kind(const LinearArgs& a, int kind, int B, int max_len, hipStream_t st) {
+  if (kind == 0) return launch_linear<0, DP>(a, B, max_len, st);
+  return kind == 1 ? launch_linear<1, DP>(a, B, max_len, st) : launch_linear<2, DP>(a, B, max_len, st);
+}
+
+}  // namespace
+
+// fp32 numbers of scratch for a step of T rows in B sequences (``lc_linear_chunks``).
+LC_EXPORT long long lc_linear_scratch_floats(int T, int B, int H, int D, int Dv) {
+  return static_cast<long long>(T / kRows + B) * H * D * (static_cast<long long>(Dv) + 1);
+}
+
+// Prompt portions of up to max_len rows. kind, decay and gates as in LinearArgs; Dv value columns, the last ``ones`` of them 1.
+LC_EXPORT int lc_linear_chunks(const void* proj, int ld, int kind, const void* decay, const void* gates, float inv_tau, float qscale,
+                               void* state, long long state_stride, const void* cu_q, const void* positions, const void* slots,
+                               void* out, int T, int B, int H, int D, int Dv, int ones, int max_len, void* scratch, hipStream_t st) {
+  if (B <= 0 || T <= 0 || max_len <= 0) return 0;
+  if (H <= 0 || D <= 0 || D > 256 || Dv <= ones || ones < 0 || kind < 0 || kind > 2 || (kind == 1 ? gates : decay) == nullptr) return -1;
+  if (ld < 2 * H * D + H * (Dv - ones) || state_stride < static_cast<long long>(H) * D * Dv || scratch == nullptr) return -1;
+  float* cs = static_cast<float*>(scratch);
+  const LinearArgs a{static_cast<const float*>(proj), ld, static_cast<const float*>(decay), static_cast<const float2*>(gates),
+                     inv_tau, qscale, static_cast<float*>(state), state_stride, static_cast<const int32_t*>(cu_q),
+                     static_cast<const int32_t*>(positions), static_cast<const int32_t*>(slots), static_cast<float*>(out), cs,
+                     cs + static_cast<size_t>(T / kRows + B) * H * D * Dv, H, D, Dv, ones};
+  if (D <= 64) return launch_linear_kind<64>(a, kind, B, max_len, st);
+  if (D <= 128) return launch_linear_kind<128>(a, kind, B, max_len, st);
+  return launch_linear_kind<256>(a, kind, B, max_len, st);
+}

@@ -1113,3 +1113,40 @@ def test_residual_steps_sum_slabs_and_bias(dt, T, d, parts):
             got = ops.hc_step(xd, slabs(), mix.to(DEV), ow.to(DEV), iw.to(DEV), norm.to(DEV) if norm is not None else None, 1e-5, dt)
             torch.testing.assert_close(got.float().cpu(), want.float(), **(tol if norm is not None else dict(atol=2e-4, rtol=2e-4)))
             torch.testing.assert_close(xd.cpu(), xr, atol=2e-4, rtol=2e-4)
+
+
+# chunks of 64 rows in blocks of 16: portions around both, several sequences with and without a state, decays that vanish within a
+# row beside rows that hardly decay, key widths in one, two and four slices of channels (partly filled), one column and many
+@pytest.mark.parametrize("kind", ["gla", "mlstm", "lightning"])
+@pytest.mark.parametrize("H,D,Dv", [(2, 64, 16), (3, 128, 128), (1, 200, 33), (2, 12, 7), (1, 96, 300)])
+def test_linear_attention_in_chunks(kind, H, D, Dv):
+    g = torch.Generator().manual_seed(H + D + Dv)
+    lens, starts = [17, 64, 1, 130, 65, 5], [0, 7, 50, 0, 3, 0]
+    cu, pos, rs = _seqs(lens, starts)
+    T, slots = int(cu[-1]), torch.tensor([3, 1, 0, 5, 2, 4], dtype=torch.int32)
+    width = 2 * H * D + 2 * H * Dv + 2 * H
+    proj = torch.randn(T, width + 3, generator=g) * 0.5
+    c = lambda t: t.to(DEV)   # noqa: E731
+    step = (cu, pos, slots)
+    if kind == "gla":
+        dec = torch.randn(T, H * D, generator=g) * 4.0
+        dec[::5] = -60.0                                 # (sigmoid^(1/2) of -60: 1e-13)
+        dec[:, ::3] += 8.0
+        state = torch.randn(6, H * D * Dv, generator=g)
+        sd = c(state)
+        want = ref.gla_scan(proj, dec, state, *step, H, D, Dv, 2.0)
+        got = ops.gla_scan(c(proj), c(dec), sd, *map(c, step), H, D, Dv, 2.0, max_len=130)
+    elif kind == "mlstm":
+        proj[:, 2 * H * D + 2 * H * Dv + H:width] += 2.0
+        state = torch.randn(6, H * D * (Dv + 1) + H, generator=g)
+        sd = c(state)
+        (want, m), (got, md) = ref.mlstm_scan(proj, state, *step, H, D, Dv, 15.0), ops.mlstm_scan(c(proj), sd, *map(c, step), H, D, Dv, 15.0, max_len=130)
+        torch.testing.assert_close(md.cpu(), m, atol=2e-5, rtol=2e-5)
+    else:
+        dec = torch.rand(H, generator=g)
+        state = torch.randn(6, H * D * Dv, generator=g)
+        sd = c(state)
+        want = ref.lightning_scan(proj, dec, state, *step, H, D, Dv)
+        got = ops.lightning_scan(c(proj), c(dec), sd, *map(c, step), H, D, Dv, max_len=130)
+    torch.testing.assert_close(got.cpu(), want, atol=2e-4, rtol=2e-4)      # sums over 130 rows and D channels of numbers up to 1e2
+    torch.testing.assert_close(sd.cpu(), state, atol=2e-4, rtol=2e-4)
