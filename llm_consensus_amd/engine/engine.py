@@ -1438,7 +1438,8 @@ class Engine:
             if st.kind == core.RequestKind.Score:
                 out.scores = st.scores
             if st.kind == core.RequestKind.Embed and st.embed_sum is not None:
-                out.embedding = ops.l2_normalize(st.embed_sum.view(1, -1))[0].cpu().numpy()
+                with self._on_stream():      # behind the step that summed the rows: nothing else waits for it
+                    out.embedding = ops.l2_normalize(st.embed_sum.view(1, -1))[0].cpu().numpy()
             self._done[f.request_id] = out
             self.metrics.inc("requests.finished")
             self.metrics.observe("request.latency_ms", (out.finished_at - out.submitted_at) * 1e3)

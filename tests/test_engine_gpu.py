@@ -307,6 +307,22 @@ def test_back_to_back_steps_that_sample_nothing_do_not_mix_their_inputs():
         assert np.allclose(g, want, atol=2e-2), float(np.abs(g - want).max())
 
 
+def test_embeddings_are_read_on_the_stream_that_computed_them(monkeypatch):
+    """A step of embedding requests alone leaves the host nothing to wait for, so the kernel that
+    normalises an embedding has to queue behind the step on the engine's own stream."""
+    from llm_consensus_amd import ops
+
+    _, gpu = models("small-llama", seed=5, std=0.1)
+    eng = Engine(gpu, num_kv_blocks=64, block_size=64)
+    on, real = [], ops.l2_normalize
+    monkeypatch.setattr(ops, "l2_normalize",
+                        lambda x: (on.append(torch.cuda.current_stream().cuda_stream), real(x))[1])
+    rids = [eng.submit([5, 6, 7 + i], core.RequestKind.Embed) for i in range(3)]
+    eng.run_until_done()
+    assert all(np.isfinite(eng.pop_result(r).embedding).all() for r in rids)
+    assert eng.stream is not None and on == [eng.stream.cuda_stream] * 3
+
+
 def test_warm_up_records_every_configured_decode_graph_before_the_first_request():
     """After Engine.warm_up() no request of a warmed-up shape records anything: the first request
     costs what a later one costs (/root/reference/src/main.rs:428-445 answers its first question
