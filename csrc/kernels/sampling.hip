@@ -5,7 +5,7 @@
 //                     temperature == 0 selects the arg-max (log-prob under softmax(logits)).
 //                     Top-k / top-p never sort the vocabulary: the kept set is {z >= thr}
 //                     and thr is found by a 12-way threshold search (per-thread LDS
-//                     histograms), each sweep one coalesced 16-byte-per-lane pass over the row.
+//                     histograms), each sweep one pass over the row.
 //                     The top-p cut is DEFINED by that search: the largest threshold of the
 //                     grid refined kSearchPassesP times inside [max - 30, max] whose kept mass
 //                     still reaches top_p (at most 1.4e-3 below the exact sort-based cut; the
@@ -73,6 +73,33 @@ LC_DEVICE void for_each_strided(const float* __restrict__ row, int V, bool vec, 
   }
 }
 
+constexpr int kQuads = 8;                          // 16-byte loads a thread has in flight per step of a sweep
+constexpr int kStep = kThreads * 4;                // elements one load of the block covers
+constexpr int kHeldV = kQuads * kStep;             // vocabularies up to here stay in registers between the sweeps
+
+// Four elements from i on; what lies past the end reads as -inf, which carries no mass.
+LC_DEVICE f32x4 load_quad(const float* __restrict__ row, int i, int V, bool vec) {
+  f32x4 v = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  if (vec) {
+    if (i < V) v = *reinterpret_cast<const f32x4*>(row + i);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (i + q < V) v[q] = row[i + q];
+  }
+  return v;
+}
+
+// One block per row, so a row's time is what one CU needs for its sweeps: arg-max and mass, four
+// (top-p) or up to six (top-k) histogram sweeps, the draw. What bounds them is not the 64 bytes a
+// clock that a CU takes from the L2 (128 K entries: 3.5 us a sweep) but what waits on something:
+// loads are issued eight at a time, tails included; sums over the block read the LDS once, twelve
+// waves a bin each, and the group that holds the draw is found by a scan over one wave. Then it is the
+// ~18 vector instructions a histogram entry takes (a float add in the LDS itself is no way around:
+// 40 clocks a wave, 227 us for 128 256 entries). Up to 32768 entries the row is read once and HELD
+// in 32 registers per thread. Measured with top-p, 32 rows: 32 000 entries 51.6 -> 26 us, 128 256 entries 92 -> 72 us
+// (arg-max alone 8.7 -> 7.5 and 21 -> 16 us).
+template <bool HELD>
 __global__ __launch_bounds__(kThreads) void sample_kernel(
     const float* __restrict__ logits, int V, int ld, const int32_t* __restrict__ row_index,
     const float* __restrict__ temperature, const float* __restrict__ top_p, const int32_t* __restrict__ top_k,
@@ -81,7 +108,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(
   __shared__ float red[16];
   __shared__ float sv[kWaves];
   __shared__ int si[kWaves];
-  __shared__ float multi[kWaves][kBins];
+  __shared__ float bin_sum[kBins];
   extern __shared__ float hist[];  // [kBins][kThreads]
   __shared__ float seg_sum[kWaves * kGroups];
   __shared__ float bc[2];
@@ -94,21 +121,66 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(
   const bool greedy = !(T > 0.f);
   const float inv_t = greedy ? 1.f : 1.f / T;
 
-  // ---- pass 1: arg-max of z = logit / T and, in the same sweep, the partition function ----
+  f32x4 held[kQuads];
+  if constexpr (HELD) {
+#pragma unroll
+    for (int u = 0; u < kQuads; ++u) held[u] = load_quad(row, threadIdx.x * 4 + u * kStep, V, vec);
+  }
+  // f(v, i): eight quads of the row, quad u at element i + u * kStep, for every thread of the block
+  auto sweep = [&](auto&& f) {
+    if constexpr (HELD) {
+      f(held, static_cast<int>(threadIdx.x) * 4);
+    } else {
+      f32x4 v[kQuads];
+      int i = threadIdx.x * 4;
+      if (vec) {
+        for (int base = kHeldV; base <= V; base += kHeldV, i += kHeldV) {
+#pragma unroll
+          for (int u = 0; u < kQuads; ++u) v[u] = *reinterpret_cast<const f32x4*>(row + i + u * kStep);
+          f(v, i);
+        }
+      }
+      for (; i - static_cast<int>(threadIdx.x) * 4 < V; i += kHeldV) {
+#pragma unroll
+        for (int u = 0; u < kQuads; ++u) v[u] = load_quad(row, i + u * kStep, V, vec);
+        f(v, i);
+      }
+    }
+  };
+
+  // ---- sweep 1: arg-max of z = logit / T and, in the same sweep, the partition function ----
   // Every thread keeps a running maximum m and the sum of exp(z - m) over what it has seen
-  // (rescaled whenever m grows); the block then rebases the per-thread sums on the global max.
+  // (rescaled when a step's 32 entries raise m); the block then rebases the per-thread sums on the
+  // global max. NaN entries compare false everywhere and -inf ones (ragged vocabulary shards) are 0.
   ArgMax am{-INFINITY, 0x7fffffff};
-  float run_m = -INFINITY, run_s = 0.f;
-  for_each_strided(row, V, vec, [&](float x, int i) {
-    const float z = x * inv_t;
-    am = argmax_combine(am, ArgMax{z, i});
-    if (z > run_m) {
-      run_s = run_s * __expf(run_m - z) + 1.f;     // exp(-inf) = 0 on the first element
-      run_m = z;
-    } else if (z > -INFINITY) {                    // -inf pads (ragged vocabulary shards) carry no mass
-      run_s += __expf(z - run_m);
+  float run_s = 0.f;
+  sweep([&](const f32x4 (&v)[kQuads], int i) {
+    float m = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < kQuads; ++u)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) m = fmaxf(m, v[u][q] * inv_t);
+    if (m > am.v) {
+      run_s = am.v > -INFINITY ? run_s * __expf(am.v - m) : 0.f;
+      int at = 0x7fffffff;
+#pragma unroll
+      for (int u = kQuads - 1; u >= 0; --u)
+#pragma unroll
+        for (int q = 3; q >= 0; --q)
+          if (v[u][q] * inv_t == m) at = i + u * kStep + q;
+      am = ArgMax{m, at};
+    }
+    if (am.v > -INFINITY) {
+#pragma unroll
+      for (int u = 0; u < kQuads; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float z = v[u][q] * inv_t;
+          run_s += z == am.v ? 1.f : z < am.v ? __expf(z - am.v) : 0.f;
+        }
     }
   });
+  const float run_m = am.v;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1)
     am = argmax_combine(am, ArgMax{__shfl_xor(am.v, off, 64), __shfl_xor(am.i, off, 64)});
@@ -118,9 +190,10 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(
   }
   __syncthreads();
   am = ArgMax{sv[0], si[0]};
+#pragma unroll
   for (int i = 1; i < kWaves; ++i) am = argmax_combine(am, ArgMax{sv[i], si[i]});
   const float zmax = am.v;
-  const float total = block_sum(run_m > -INFINITY ? run_s * __expf(run_m - zmax) : 0.f, red);
+  const float total = block_sum(run_m == zmax ? run_s : run_m > -INFINITY ? run_s * __expf(run_m - zmax) : 0.f, red);
   // A row without a single finite comparable entry (all NaN: a poisoned forward pass) leaves the
   // arg-max index at its sentinel. It must never be used as an index or handed to the caller.
   if (am.i < 0 || am.i >= V) am.i = 0;
@@ -153,36 +226,45 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(
     const int passes = phase == 0 ? kSearchPasses : kSearchPassesP;
     for (int it = 0; it < passes; ++it) {
       // Per-thread histogram over kBins equal sub-intervals of [lo, hi): thread t owns column t
-      // of hist[kBins][kThreads] (conflict-free, no atomics), so suffix sums give the mass (or
-      // count) above each threshold t_j = lo + w*j.
+      // of hist[kBins][kThreads] (conflict-free, nothing shared, so the order of the sums is fixed)
+      // and suffix sums give the mass (or count) above each threshold t_j = lo + w*j.
       const float w = (hi - lo) * (1.f / kBins);
       const float inv_w = w > 0.f ? 1.f / w : 0.f;
 #pragma unroll
       for (int j = 0; j < kBins; ++j) hist[j * kThreads + threadIdx.x] = 0.f;
-      for_each_strided(row, V, vec, [&](float x, int) {
-        const float z = x * inv_t;
-        if (z >= lo && (hi_is_max || z < hi)) {
-          int b = static_cast<int>((z - lo) * inv_w);
-          b = b < kBins - 1 ? b : kBins - 1;
-          hist[b * kThreads + threadIdx.x] += phase == 0 ? 1.f : __expf(z - zmax);
-        }
+      sweep([&](const f32x4 (&v)[kQuads], int) {
+#pragma unroll
+        for (int u = 0; u < kQuads; ++u)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const float z = v[u][q] * inv_t;
+            if (z >= lo && (hi_is_max || z < hi)) {
+              int b = static_cast<int>((z - lo) * inv_w);
+              b = b < kBins - 1 ? b : kBins - 1;
+              hist[b * kThreads + threadIdx.x] += phase == 0 ? 1.f : __expf(z - zmax);
+            }
+          }
       });
-      float bins[kBins];
-#pragma unroll
-      for (int j = 0; j < kBins; ++j) bins[j] = wave_sum(hist[j * kThreads + threadIdx.x]);
       __syncthreads();
-      if (lane == 0) {
+      if (wid < kBins) {
+        float t = 0.f;
 #pragma unroll
-        for (int j = 0; j < kBins; ++j) multi[wid][j] = bins[j];
+        for (int c = 0; c < kWaves; ++c) t += hist[wid * kThreads + c * 64 + lane];
+        t = wave_sum(t);
+        if (lane == 0) bin_sum[wid] = t;
       }
       __syncthreads();
       // every thread walks the thresholds from the top; the result is block-uniform
+      float bins[kBins];
+#pragma unroll
+      for (int j = 0; j < kBins; ++j) bins[j] = bin_sum[j];
       int best = -1;
       float cum = above, best_v = 0.f, above_best = above;
-      for (int j = kBins - 1; j >= 0 && best < 0; --j) {
+#pragma unroll
+      for (int j = kBins - 1; j >= 0; --j) {
         const float before = cum;
-        for (int wv = 0; wv < kWaves; ++wv) cum += multi[wv][j];
-        if (cum >= target) {
+        cum += bins[j];
+        if (best < 0 && cum >= target) {
           best = j;
           best_v = cum;
           above_best = before;
@@ -203,78 +285,107 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(
     if (found && phase == 0 && use_p) {
       // top-p is relative to the mass that survived top-k
       float m = 0.f;
-      for_each_strided(row, V, vec, [&](float x, int) {
-        const float z = x * inv_t;
-        m += z >= thr ? __expf(z - zmax) : 0.f;
+      sweep([&](const f32x4 (&v)[kQuads], int) {
+#pragma unroll
+        for (int u = 0; u < kQuads; ++u)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const float z = v[u][q] * inv_t;
+            m += z >= thr ? __expf(z - zmax) : 0.f;
+          }
       });
       kept_mass = block_sum(m, red);
     }
   }
 
   // ---- draw: locate u * kept_mass in the index-ordered CDF of the kept set ----
-  const float u = rng_uniform(seeds[r], static_cast<uint32_t>(steps ? steps[r] : 0), 0);
-  // Each wave owns a contiguous segment of the vocabulary, cut into kGroups groups; the sweep below
-  // leaves one mass per (wave, group), thread 0 picks the group that holds the target and only
-  // that group (1/128 of the row) is walked again, by its wave, with prefix scans.
-  const int gsz = (((V + kWaves - 1) / kWaves + kGroups - 1) / kGroups + 255) & ~255;   // multiple of 256
-  const int seg = gsz * kGroups;
-  const int s0 = wid * seg, s1 = min(V, s0 + seg);
-  auto kept_w = [&](int i) -> float {
-    if (i >= s1) return 0.f;
-    const float z = row[i] * inv_t;
-    return z >= thr ? __expf(z - zmax) : 0.f;
-  };
-  // weights of elements i .. i+3 (i is a multiple of 4): one 16-byte load when the row allows it
-  auto kept_w4 = [&](int i) -> f32x4 {
-    if (vec && i < s1) {   // V % 4 == 0 and segment bounds are multiples of 4: the quad is whole
-      const f32x4 x = *reinterpret_cast<const f32x4*>(row + i);
-      f32x4 w;
+  const float u01 = rng_uniform(seeds[r], static_cast<uint32_t>(steps ? steps[r] : 0), 0);
+  // The row is cut into 128 groups of a multiple of 256 elements; the sweep below leaves one mass per
+  // group, the first wave picks the group that holds the target and only that group is walked again,
+  // by one wave, with prefix scans. Up to kHeldV entries group g is [256 g, 256 g + 256): quad u of
+  // wave w holds group u * kWaves + w. Longer rows give every wave kGroups groups of its own.
+  const int gsz = (((V + kWaves - 1) / kWaves + kGroups - 1) / kGroups + 255) & ~255;
+  auto weights = [&](f32x4 x) -> f32x4 {
+    f32x4 w;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float z = x[q] * inv_t;
-        w[q] = z >= thr ? __expf(z - zmax) : 0.f;
-      }
-      return w;
+    for (int q = 0; q < 4; ++q) {
+      const float z = x[q] * inv_t;
+      w[q] = z >= thr ? __expf(z - zmax) : 0.f;
     }
-    return f32x4{kept_w(i), kept_w(i + 1), kept_w(i + 2), kept_w(i + 3)};
+    return w;
   };
+  // weights of the elements i .. i+3 of a group that ends before `end` (thr can be -inf: what lies
+  // past the end must weigh nothing then either)
+  auto kept_w4 = [&](int i) -> f32x4 {
+    f32x4 w = weights(load_quad(row, i, V, vec));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w[q] = i + q < V ? w[q] : 0.f;
+    return w;
+  };
+  static_assert(kQuads == kGroups, "a thread's quads are its wave's groups");
+  float mass[kGroups];
+#pragma unroll
+  for (int g = 0; g < kGroups; ++g) mass[g] = 0.f;
+  if constexpr (HELD) {
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) {
+      const f32x4 w4 = weights(held[g]);
+      const int i = threadIdx.x * 4 + g * kStep;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) mass[g] += i + q < V ? w4[q] : 0.f;
+    }
+  } else {
+    for (int s = 0; s < gsz; s += 256) {
+      f32x4 v[kGroups];
+      const int i = wid * kGroups * gsz + s + lane * 4;
+#pragma unroll
+      for (int g = 0; g < kGroups; ++g) v[g] = load_quad(row, i + g * gsz, V, vec);
+#pragma unroll
+      for (int g = 0; g < kGroups; ++g) {
+        const f32x4 w4 = weights(v[g]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) mass[g] += i + g * gsz + q < V ? w4[q] : 0.f;
+      }
+    }
+  }
 #pragma unroll
   for (int g = 0; g < kGroups; ++g) {
-    float mine = 0.f;
-    const int g1 = min(s1, s0 + (g + 1) * gsz);
-    for (int i = s0 + g * gsz + lane * 4; i < g1; i += 256) {
-      const f32x4 w4 = kept_w4(i);
-      mine += w4[0] + w4[1] + w4[2] + w4[3];
-    }
-    mine = wave_sum(mine);
-    if (lane == 0) seg_sum[wid * kGroups + g] = mine;
+    const float m = wave_sum(mass[g]);
+    if (lane == 0) seg_sum[HELD ? g * kWaves + wid : wid * kGroups + g] = m;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float grand = 0.f;
-    for (int w2 = 0; w2 < kWaves * kGroups; ++w2) grand += seg_sum[w2];
-    const float target = u * grand;
-    float run = 0.f;
-    int owner = 0;
-    for (int w2 = 0; w2 < kWaves * kGroups; ++w2) {
-      if (seg_sum[w2] > 0.f) {
-        owner = w2;  // last non-empty group so far: fallback when target == grand
-        if (target < run + seg_sum[w2]) break;
-      }
-      run += seg_sum[w2];
+  if (wid == 0) {
+    // two groups per lane; the owner is the first non-empty group whose end lies beyond the target,
+    // or the last non-empty one where rounding leaves the target at the very end
+    static_assert(kWaves * kGroups == 128, "two groups per lane");
+    const float a = seg_sum[2 * lane], b = seg_sum[2 * lane + 1];
+    float incl = a + b;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const float o = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += o;
     }
-    run = 0.f;
-    for (int w2 = 0; w2 < owner; ++w2) run += seg_sum[w2];
-    bc[0] = fmaxf(target - run, 0.f);
-    bc[1] = grand;
-    bci[0] = owner;
+    float before = __shfl_up(incl, 1, 64);
+    if (lane == 0) before = 0.f;
+    const float grand = __shfl(incl, 63, 64), target = u01 * grand;
+    const bool hit_a = a > 0.f && target < before + a, hit_b = b > 0.f && target < incl;
+    const unsigned long long hits = __ballot(hit_a || hit_b), full = __ballot(a > 0.f || b > 0.f);
+    const int at = hits ? __ffsll(static_cast<long long>(hits)) - 1
+                        : full ? 63 - __clzll(static_cast<long long>(full)) : 0;
+    if (lane == at) {
+      const bool second = hits ? !hit_a : b > 0.f;
+      bc[0] = fmaxf(target - (second ? before + a : before), 0.f);
+      bc[1] = grand;
+      bci[0] = 2 * lane + (second ? 1 : 0);
+    }
   }
   __syncthreads();
-  if (wid == bci[0] / kGroups) {
+  const int owner = bci[0];
+  if (wid == (HELD ? owner & (kWaves - 1) : owner / kGroups)) {
     const float resid = bc[0], grand = bc[1];
     float run = 0.f;
     int tok = -1, last_kept = -1;
-    const int gb = s0 + (bci[0] % kGroups) * gsz, ge = min(s1, gb + gsz);
+    const int gb = owner * gsz, ge = min(V, gb + gsz);
     for (int base = gb; base < ge && tok < 0; base += 256) {
       const int i = base + lane * 4;
       const f32x4 w4 = kept_w4(i);
@@ -434,7 +545,8 @@ LC_EXPORT int lc_sample(const void* logits, int V, int ld, const void* row_index
                         const void* top_p, const void* top_k, const void* seeds, const void* steps,
                         void* out_token, void* out_logprob, int R, hipStream_t stream) {
   if (R <= 0) return 0;
-  sample_kernel<<<dim3(R), dim3(kThreads), kBins * kThreads * sizeof(float), stream>>>(
+  auto kernel = V <= kHeldV ? sample_kernel<true> : sample_kernel<false>;
+  kernel<<<dim3(R), dim3(kThreads), kBins * kThreads * sizeof(float), stream>>>(
       static_cast<const float*>(logits), V, ld, static_cast<const int32_t*>(row_index),
       static_cast<const float*>(temperature), static_cast<const float*>(top_p),
       static_cast<const int32_t*>(top_k), static_cast<const uint64_t*>(seeds),

@@ -537,6 +537,32 @@ def test_sampler_never_returns_an_out_of_range_token_for_poisoned_rows():
     assert 0 <= int(g[0]) < V
 
 
+@pytest.mark.parametrize("V,off", [(1, 0), (3, 0), (255, 0), (257, 1), (4096, 0), (4100, 1), (32768, 0), (32772, 0), (32769, 0),
+                                   (65536, 2), (151936, 0)])
+def test_sampler_at_the_edges_of_its_sweeps(V, off):
+    """Vocabularies around one wave, one load of the block, the largest row held in registers and one
+    entry more, aligned rows and not: draws agree with the oracle except where fp32 rounding (1e-6 of
+    the mass) lies between the two, arg-max rows agree exactly; one infinite entry is the arg-max."""
+    R = 16
+    logits = torch.empty(R * (V + off) + off, dtype=torch.float32, device=DEV)[off:].view(R, V + off)[:, :V]
+    src = rand(R, V, scale=2.0, seed=V)
+    src[3, V // 2] = float("inf")
+    logits.copy_(src.to(DEV))
+    temp = torch.tensor([0.0, 0.8, 1.0, 0.0] * 4)
+    top_p = torch.tensor([1.0, 0.3, 0.9, 1.0, 1.0, 1.0, 0.5, 1.0] * 2)
+    top_k = torch.tensor([0, 0, 0, 0, 0, 7, 40, 0] * 2, dtype=torch.int32)
+    seeds = torch.arange(R, dtype=torch.int64) * 31 + V
+    tok, lp = ops.sample(logits, temp.to(DEV), top_p.to(DEV), top_k.to(DEV), seeds.to(DEV), None)
+    want, wlp = ref.sample(src, temp, top_p, top_k, seeds, torch.zeros(R, dtype=torch.int32))
+    tok, lp, g = tok.cpu(), lp.cpu(), temp == 0
+    assert torch.equal(tok[g], src[g].argmax(-1).int())
+    assert float(lp[3]) == 0.0
+    same = tok == want
+    assert int((~same).sum()) <= 1, (tok, want)
+    same[3] = False
+    assert torch.allclose(lp[same], wlp[same], atol=2e-3)
+
+
 def test_sampler_statistics_and_reproducibility():
     V, R = 64, 4096
     base = torch.tensor([2.0, 1.0, 0.5, 0.0] + [-4.0] * (V - 4))
