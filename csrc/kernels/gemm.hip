@@ -218,7 +218,8 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ part, const bf16_
     const size_t m = i / (N / 4);
     const int n = static_cast<int>(i % (N / 4)) * 4;
     f32x4 v = *reinterpret_cast<const f32x4*>(part + m * N + n);
-    for (int s = 1; s < S; ++s) {
+#pragma unroll 8
+    for (int s = 1; s < S; ++s) {                    // (several slabs in flight)
       const f32x4 p = *reinterpret_cast<const f32x4*>(part + s * slab + m * N + n);
       v += p;
     }

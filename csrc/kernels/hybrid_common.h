@@ -108,7 +108,7 @@ LC_DEVICE void conv_rows4(const ConvIn& a, const RowSeq& s, const float* st, int
     src[j] = k >= 0 ? a.x + static_cast<size_t>(s.first + k) * a.ld
                     : (s.fresh ? nullptr : st + static_cast<size_t>(k + TAPS - 1) * a.C);
   }
-  for (int c = threadIdx.x * 4; c < a.C; c += 1024) {
+  for (int c = threadIdx.x * 4; c < a.C; c += 4 * blockDim.x) {
     float4 x[TAPS], w[TAPS];
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) {
@@ -139,9 +139,9 @@ LC_DEVICE void conv_token(const ConvIn& a, const RowSeq& s, const float* st, int
   } else if (a.vec && a.taps == 4) {
     conv_rows4<4, SILU>(a, s, st, r, u);
   } else if (a.vec && a.taps == 0 && !SILU) {
-    for (int c = threadIdx.x * 4; c < a.C; c += 1024) *reinterpret_cast<float4*>(u + c) = *reinterpret_cast<const float4*>(row + c);
+    for (int c = threadIdx.x * 4; c < a.C; c += 4 * blockDim.x) *reinterpret_cast<float4*>(u + c) = *reinterpret_cast<const float4*>(row + c);
   } else if (a.taps > 0) {
-    for (int c = threadIdx.x; c < a.C; c += 256) {
+    for (int c = threadIdx.x; c < a.C; c += blockDim.x) {
       float y = 0.f;
       for (int j = 0; j < a.taps; ++j) {
         const int k = r - hist + j;                  // input row inside the portion, < 0: before it
@@ -153,7 +153,7 @@ LC_DEVICE void conv_token(const ConvIn& a, const RowSeq& s, const float* st, int
       u[c] = conv_act<SILU>(y);
     }
   } else {
-    for (int c = threadIdx.x; c < a.C; c += 256) u[c] = conv_act<SILU>(row[c]);
+    for (int c = threadIdx.x; c < a.C; c += blockDim.x) u[c] = conv_act<SILU>(row[c]);
   }
 }
 
@@ -161,7 +161,7 @@ LC_DEVICE void conv_token(const ConvIn& a, const RowSeq& s, const float* st, int
 // has read the old ones). A thread owns a channel (four of them): all its inputs are read before one is written.
 template <int HIST>
 LC_DEVICE void conv_keep4(const ConvIn& a, const RowSeq& s, float* st) {
-  for (int c = threadIdx.x * 4; c < a.C; c += 1024) {
+  for (int c = threadIdx.x * 4; c < a.C; c += 4 * blockDim.x) {
     float4 in[HIST];
 #pragma unroll
     for (int j = 0; j < HIST; ++j) {
@@ -180,7 +180,7 @@ LC_DEVICE void conv_keep(const ConvIn& a, const RowSeq& s, float* st) {
   if (a.vec && hist == 1) return conv_keep4<1>(a, s, st);
   if (a.vec && hist == 2) return conv_keep4<2>(a, s, st);
   if (a.vec && hist == 3) return conv_keep4<3>(a, s, st);
-  for (int c = threadIdx.x; c < a.C; c += 256)
+  for (int c = threadIdx.x; c < a.C; c += blockDim.x)
     for (int j = 0; j < hist; ++j) {                 // (row j + rows is read before row j + 1 is written)
       const int k = s.rows - hist + j;
       float in = 0.f;
@@ -189,5 +189,12 @@ LC_DEVICE void conv_keep(const ConvIn& a, const RowSeq& s, float* st) {
       st[static_cast<size_t>(j) * a.C + c] = in;
     }
 }
+
+// Threads of a kernel that gives every row of ``width`` fp32 coordinates a block. With few rows nothing
+// but the block's own loads hides what they wait for, so a thread takes one piece of four coordinates: the residual step over 16
+// slabs of 32 rows of 2048 took 8.6 us with 256 threads and takes 4.2 us. With more rows than two per CU other blocks do, and
+// four waves a row leave the sums over the block short: a norm of 2048 rows of 2048 10.9 us, with 512 threads 11.9 us (of 512 rows
+// of 4096 6.3 and 5.9 us).
+inline int row_block_threads(int T, int width) { return T > 512 || width <= 1024 ? 256 : width <= 2048 ? 512 : 1024; }
 
 }  // namespace

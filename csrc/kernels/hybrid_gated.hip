@@ -56,8 +56,8 @@ struct StepArgs {
   int d;
 };
 
-template <bool AF32, bool VEC>
-__global__ __launch_bounds__(256) void gated_step_kernel(StepArgs a) {
+template <bool AF32, bool VEC, int THREADS>
+__global__ __launch_bounds__(THREADS) void gated_step_kernel(StepArgs a) {
   __shared__ float red[16];
   const int t = blockIdx.x, d = a.d;
   const size_t row = static_cast<size_t>(t) * d;
@@ -73,12 +73,26 @@ __global__ __launch_bounds__(256) void gated_step_kernel(StepArgs a) {
     }
   }
   if constexpr (VEC) {
+    constexpr int kPer = 256 * kStepVec / THREADS;    // pieces of four coordinates per thread
+    constexpr bool kAhead = THREADS > 256;            // one block per CU: gains and the stored row ahead of the sums they follow
     const int n4 = d / 4;
-    float4 xv[kStepVec], yv[kStepVec];
+    const bool each = a.w_out != nullptr && !a.one_gain;
+    float4 xv[kPer], yv[kPer], wo[kPer], wi[kPer], pv[kPer];
     float ss = 0.f;
+    if constexpr (kAhead) {
 #pragma unroll
-    for (int i = 0; i < kStepVec; ++i) {
-      const int c = threadIdx.x + 256 * i;
+      for (int i = 0; i < kPer; ++i) {
+        const int c = threadIdx.x + THREADS * i;
+        if (c < n4) {
+          if (each) wo[i] = reinterpret_cast<const float4*>(a.w_out)[c];
+          if (a.w_in != nullptr && !a.one_gain) wi[i] = reinterpret_cast<const float4*>(a.w_in)[c];
+          if (!fresh) pv[i] = reinterpret_cast<const float4*>(prev)[c];
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int c = threadIdx.x + THREADS * i;
       xv[i] = yv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (c < n4) {
         xv[i] = reinterpret_cast<const float4*>(a.x + row)[c];
@@ -104,14 +118,13 @@ __global__ __launch_bounds__(256) void gated_step_kernel(StepArgs a) {
     }
     if (a.y != nullptr) {
       float r = a.w_out != nullptr ? 1.f / sqrtf(block_sum(ss, red) / static_cast<float>(d) + a.eps) : 1.f;
-      const bool each = a.w_out != nullptr && !a.one_gain;
       if (a.w_out != nullptr && a.one_gain) r *= a.w_out[0];
 #pragma unroll
-      for (int i = 0; i < kStepVec; ++i) {
-        const int c = threadIdx.x + 256 * i;
+      for (int i = 0; i < kPer; ++i) {
+        const int c = threadIdx.x + THREADS * i;
         if (c < n4) {
           float4 w = make_float4(1.f, 1.f, 1.f, 1.f);
-          if (each) w = reinterpret_cast<const float4*>(a.w_out)[c];
+          if (each) w = kAhead ? wo[i] : reinterpret_cast<const float4*>(a.w_out)[c];
           xv[i].x += yv[i].x * r * w.x;
           xv[i].y += yv[i].y * r * w.y;
           xv[i].z += yv[i].z * r * w.z;
@@ -122,21 +135,21 @@ __global__ __launch_bounds__(256) void gated_step_kernel(StepArgs a) {
     }
     if (a.copy) {                                     // the same for every thread
 #pragma unroll
-      for (int i = 0; i < kStepVec; ++i) {
-        const int c = threadIdx.x + 256 * i;
+      for (int i = 0; i < kPer; ++i) {
+        const int c = threadIdx.x + THREADS * i;
         if (c < n4) store_act4<AF32>(a.ha, row + 4 * c, xv[i]);
       }
     }
     if (a.w_in == nullptr) return;                    // the same for every thread
     float s2 = 0.f;
 #pragma unroll
-    for (int i = 0; i < kStepVec; ++i) s2 += xv[i].x * xv[i].x + xv[i].y * xv[i].y + xv[i].z * xv[i].z + xv[i].w * xv[i].w;
+    for (int i = 0; i < kPer; ++i) s2 += xv[i].x * xv[i].x + xv[i].y * xv[i].y + xv[i].z * xv[i].z + xv[i].w * xv[i].w;
     const float r2 = 1.f / sqrtf(block_sum(s2, red) / static_cast<float>(d) + a.eps);
 #pragma unroll
-    for (int i = 0; i < kStepVec; ++i) {
-      const int c = threadIdx.x + 256 * i;
+    for (int i = 0; i < kPer; ++i) {
+      const int c = threadIdx.x + THREADS * i;
       if (c < n4) {
-        const float4 w = a.one_gain ? make_float4(a.w_in[0], a.w_in[0], a.w_in[0], a.w_in[0]) : reinterpret_cast<const float4*>(a.w_in)[c];
+        const float4 w = a.one_gain ? make_float4(a.w_in[0], a.w_in[0], a.w_in[0], a.w_in[0]) : kAhead ? wi[i] : reinterpret_cast<const float4*>(a.w_in)[c];
         const float4 h = make_float4(xv[i].x * r2 * w.x, xv[i].y * r2 * w.y, xv[i].z * r2 * w.z, xv[i].w * r2 * w.w);
         store_act4<AF32>(a.ha, row + 4 * c, h);
         if (a.w_in2 != nullptr) {
@@ -146,7 +159,7 @@ __global__ __launch_bounds__(256) void gated_step_kernel(StepArgs a) {
         if (a.h32 != nullptr) reinterpret_cast<float4*>(a.h32 + row)[c] = h;
         if (a.mu != nullptr) {
           float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
-          if (!fresh) p = reinterpret_cast<const float4*>(prev)[c];
+          if (!fresh) p = kAhead ? pv[i] : reinterpret_cast<const float4*>(prev)[c];
           store_act4<AF32>(a.hs, row + 4 * c, shift4(h, p, reinterpret_cast<const float4*>(a.mu)[c]));
           if (prev != nullptr) reinterpret_cast<float4*>(prev)[c] = h;
         }
@@ -273,7 +286,7 @@ struct PrepArgs {
 };
 
 template <bool CF32>
-__global__ __launch_bounds__(256) void attn_prep_kernel(PrepArgs a) {
+__global__ __launch_bounds__(1024) void attn_prep_kernel(PrepArgs a) {
   extern __shared__ float lds[];
   __shared__ float red[16];
   const int H = a.H, G = a.G, GV = a.GV, D = a.D, Dv = a.Dv;
@@ -291,13 +304,13 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(PrepArgs a) {
     if (count == 0) return;                          // served by the portion's first row
   }
   float* st = s.slot >= 0 ? a.in.state + static_cast<size_t>(s.slot) * a.in.state_stride : nullptr;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, waves = blockDim.x >> 6;
   const int half = a.rot_dims >> 1;
   for (int rr = 0; rr < count; ++rr) {
     const int t = t0 + rr;
     const int pos = a.positions[t];
     conv_token<false>(a.in, s, st, t - s.first, u);
-    for (int j = threadIdx.x; j < half; j += 256) {
+    for (int j = threadIdx.x; j < half; j += blockDim.x) {
       constexpr double kTwoPi = 6.283185307179586476925286766559;
       double ang = static_cast<double>(pos) * a.inv_freq[j];
       ang -= kTwoPi * rint(ang / kTwoPi);
@@ -311,15 +324,15 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(PrepArgs a) {
     if (a.t_coef != 0.f) temp += a.t_coef * logf(static_cast<float>(floor((pos + 1.0) / a.t_every) + 1.0));
     if (a.norm == 1) {
       float sq = 0.f, sk = 0.f;
-      for (int i = threadIdx.x; i < nq; i += 256) sq += u[i] * u[i];
-      for (int i = threadIdx.x; i < nk; i += 256) sk += u[nq + i] * u[nq + i];
+      for (int i = threadIdx.x; i < nq; i += blockDim.x) sq += u[i] * u[i];
+      for (int i = threadIdx.x; i < nk; i += blockDim.x) sk += u[nq + i] * u[nq + i];
       const float rq = 1.f / sqrtf(block_sum(sq, red) / static_cast<float>(nq) + a.eps);
       const float rk = 1.f / sqrtf(block_sum(sk, red) / static_cast<float>(nk) + a.eps);
-      for (int i = threadIdx.x; i < nq; i += 256) u[i] *= rq * a.qn[i];
-      for (int i = threadIdx.x; i < nk; i += 256) u[nq + i] *= rk * a.kn[i];
+      for (int i = threadIdx.x; i < nq; i += blockDim.x) u[i] *= rq * a.qn[i];
+      for (int i = threadIdx.x; i < nk; i += blockDim.x) u[nq + i] *= rk * a.kn[i];
       __syncthreads();
     } else if (a.norm == 2) {
-      for (int g = wave; g < H + G; g += 4) {        // q heads, then key heads: a wave owns a head
+      for (int g = wave; g < H + G; g += waves) {        // q heads, then key heads: a wave owns a head
         float* head = u + g * D;
         const float* w = g < H ? a.qn : a.kn;
         float ss = 0.f;
@@ -341,7 +354,7 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(PrepArgs a) {
       return i < half ? v * c - head[i + half] * sn : v * c + head[i - half] * sn;
     };
     const int rep = H / G;
-    for (int g = wave; g < H; g += 4) {
+    for (int g = wave; g < H; g += waves) {
       // (several maps per head: the queries of one key head lie side by side)
       const int m = g % a.maps, qh = g / a.maps;
       const int at = ((qh / rep) * a.maps + m) * rep + qh % rep;
@@ -351,10 +364,10 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(PrepArgs a) {
     const size_t blk = slot >= 0 ? slot / a.BS : 0, off = slot >= 0 ? slot % a.BS : 0;
     typedef typename Act<CF32>::type cache_t;
     if (slot >= 0)
-      for (int g = wave; g < G; g += 4)
+      for (int g = wave; g < G; g += waves)
         for (int i = lane; i < D; i += 64)
           Act<CF32>::store(static_cast<cache_t*>(a.kc), ((blk * G + g) * a.BS + off) * D + i, turned(u + nq + g * D, i));
-    for (int g = wave; g < GV; g += 4)
+    for (int g = wave; g < GV; g += waves)
       for (int i = lane; i < Dv; i += 64) {
         const int at = g * Dv + i;
         float v = u[nq + nk + at];
@@ -402,11 +415,18 @@ LC_EXPORT int lc_gated_step(void* x, const void* y, int parts, const void* bias,
                    aligned16(y) && aligned16(gate) && (one_gain || (aligned16(w_out) && aligned16(w_in))) && aligned16(ha) &&
                    reinterpret_cast<uintptr_t>(bias) % 8 == 0 &&
                    aligned16(h32) && aligned16(w_in2) && aligned16(ha2) && aligned16(mu) && aligned16(state) && aligned16(hs);
-#define LC_GS(A32, V) gated_step_kernel<A32, V><<<dim3(T), dim3(256), 0, st>>>(a)
-  if (act_f32 && vec) LC_GS(true, true);
-  else if (act_f32) LC_GS(true, false);
-  else if (vec) LC_GS(false, true);
-  else LC_GS(false, false);
+  const int threads = vec ? row_block_threads(T, d) : 256;
+#define LC_GS(A32, V, N) gated_step_kernel<A32, V, N><<<dim3(T), dim3(N), 0, st>>>(a)
+#define LC_GSA(V, N)              \
+  do {                            \
+    if (act_f32) LC_GS(true, V, N); \
+    else LC_GS(false, V, N);      \
+  } while (0)
+  if (threads == 1024) LC_GSA(true, 1024);
+  else if (threads == 512) LC_GSA(true, 512);
+  else if (vec) LC_GSA(true, 256);
+  else LC_GSA(false, 256);
+#undef LC_GSA
 #undef LC_GS
   LC_RETURN_LAST_ERROR();
 }
@@ -466,8 +486,9 @@ LC_EXPORT int lc_attn_prep(const void* qkv, int ld, const void* conv_w, int taps
                    static_cast<const int32_t*>(positions), static_cast<const int32_t*>(slots),
                    static_cast<const int32_t*>(slot_mapping), kc, vc, static_cast<float*>(q_out), H, G, GV, D, Dv, BS, maps, T,
                    (T + 7) / 8};
-  if (cache_f32) attn_prep_kernel<true><<<dim3(8 * ((T + 7) / 8)), dim3(256), lds, st>>>(a);
-  else attn_prep_kernel<false><<<dim3(8 * ((T + 7) / 8)), dim3(256), lds, st>>>(a);
+  const int threads = row_block_threads(T, C);
+  if (cache_f32) attn_prep_kernel<true><<<dim3(8 * ((T + 7) / 8)), dim3(threads), lds, st>>>(a);
+  else attn_prep_kernel<false><<<dim3(8 * ((T + 7) / 8)), dim3(threads), lds, st>>>(a);
   LC_RETURN_LAST_ERROR();
 }
 

@@ -1150,3 +1150,16 @@ def test_linear_attention_in_chunks(kind, H, D, Dv):
         got = ops.lightning_scan(c(proj), c(dec), sd, *map(c, step), H, D, Dv, max_len=130)
     torch.testing.assert_close(got.cpu(), want, atol=2e-4, rtol=2e-4)      # sums over 130 rows and D channels of numbers up to 1e2
     torch.testing.assert_close(sd.cpu(), state, atol=2e-4, rtol=2e-4)
+
+
+@pytest.mark.parametrize("T", [1, 512, 513])
+@pytest.mark.parametrize("d", [1024, 1028, 2048, 2052, 4096])
+def test_residual_step_at_the_edges_of_its_block_sizes(T, d):
+    """Blocks of 256, 512 and 1024 threads per row, whole and with idle threads, slabs summed on the way."""
+    g = torch.Generator().manual_seed(T + d)
+    x, part, w = torch.randn(T, d, generator=g), torch.randn(3, T, d, generator=g), torch.randn(d, generator=g)
+    xg = x.to(DEV)
+    h = ops.add_rmsnorm(xg, ops.PartialSum(part.to(DEV)), w.to(DEV), 1e-5, torch.float32)
+    want = ops.add_rmsnorm(x, part.sum(0), w, 1e-5, torch.float32)
+    assert torch.allclose(xg.cpu(), x, atol=2e-6)          # (four fp32 numbers of a few units, summed)
+    assert torch.allclose(h.cpu(), want, rtol=1e-5, atol=1e-5)
