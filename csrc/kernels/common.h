@@ -42,6 +42,14 @@ LC_DEVICE bf16_t f32_to_bf16(float f) { return static_cast<bf16_t>(pack_bf16x2(f
 // which is what a softmax weight that small should do anyway).
 LC_DEVICE float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+LC_DEVICE float relu2(float x) {
+  x = fmaxf(x, 0.f);
+  return x * x;
+}
+
+// x > 0: ap x^2 + x / 2; x <= 0: an (exp(x) - 1 - x) + x / 2 (ap = softplus(p), an = 1/2 + softplus(q), made by the host)
+LC_DEVICE float xielu(float x, float ap, float an) { return (x > 0.f ? ap * x * x : an * (expm1f(x) - x)) + 0.5f * x; }
+
 LC_DEVICE float wave_sum(float v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);

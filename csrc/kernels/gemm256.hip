@@ -121,7 +121,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const bf16_t* __restrict__
                                                       int ldy, int tiles_m, int tiles_n,
                                                       long long expert_stride = 0,
                                                       const int32_t* __restrict__ offsets = nullptr, int E = 0,
-                                                      int nk_per_split = 0) {
+                                                      int nk_per_split = 0, float ap = 0.f, float an = 0.f) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -375,7 +375,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const bf16_t* __restrict__
             const int nb = nbase + i * 16 + 4 * g;
             float v[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r] + (bias ? bf16_to_f32(bias[nb + r]) : 0.f);
+            for (int r = 0; r < 4; ++r) v[r] = column_act<EPI>(acc[i][j][r] + (bias ? bf16_to_f32(bias[nb + r]) : 0.f), ap, an);
             o[0] = pack_bf16x2(v[0], v[1]);
             o[1] = pack_bf16x2(v[2], v[3]);
             chunk = i * 2 + (g >> 1);
@@ -411,7 +411,7 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const bf16_t* __restrict__
       } else {
         const size_t slab = (EPI == EPI_F32) ? static_cast<size_t>(blockIdx.y) * M * ldy : 0;
         store_tile<EPI>(acc[i][j], nullptr, Y, gridDim.y > 1 ? nullptr : bias, mbase + j * 16, nbase + i * 16, M, N,
-                        ldy, lane, slab);
+                        ldy, lane, slab, ap, an);
       }
     }
 }
@@ -431,7 +431,7 @@ LC_EXPORT int lc_gemm256_splitk(const void* Wp, const void* X, void* Y, int M, i
                                 int splits, hipStream_t stream);
 
 LC_EXPORT int lc_gemm256(const void* Wp, const void* X, void* Y, const void* bias, int M, int N, int K,
-                         int n_pad, int ldy, int epi, hipStream_t stream) {
+                         int n_pad, int ldy, int epi, float ap, float an, hipStream_t stream) {
   if (M <= 0) return 0;
   if (K % 64 || n_pad % 256 || N > n_pad) return -1;
   const int tiles_m = (M + G2_BM - 1) / G2_BM, tiles_n = n_pad / G2_BN;
@@ -449,6 +449,28 @@ LC_EXPORT int lc_gemm256(const void* Wp, const void* X, void* Y, const void* bia
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm256_kernel<EPI_SWIGLU>),
                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
   });
+  if (epi == EPI_GEGLU || epi == EPI_REGLU || epi_acts(epi)) {          // (one form of the main loop)
+    static LcDeviceOnce act_once;
+    act_once.run([&] {
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm256_kernel<EPI_GEGLU, false, 2>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, G2B_LDS);
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm256_kernel<EPI_REGLU, false, 2>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, G2B_LDS);
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm256_kernel<EPI_RELU2, false, 2>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, G2B_LDS);
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm256_kernel<EPI_XIELU, false, 2>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, G2B_LDS);
+    });
+#define G2_ACT(E)                                                                                                     \
+  gemm256_kernel<E, false, 2><<<grid, block, G2B_LDS, stream>>>(w, x, Y, b, M, N, K, ldy, tiles_m, tiles_n, 0, nullptr, 0, 0, \
+                                                                ap, an)
+    if (epi == EPI_GEGLU) G2_ACT(EPI_GEGLU);
+    else if (epi == EPI_REGLU) G2_ACT(EPI_REGLU);
+    else if (epi == EPI_RELU2) G2_ACT(EPI_RELU2);
+    else G2_ACT(EPI_XIELU);
+#undef G2_ACT
+    LC_RETURN_LAST_ERROR();
+  }
   if (g2_sched() == 2) {
     static LcDeviceOnce s2_once;
     s2_once.run([&] {
@@ -456,8 +478,6 @@ LC_EXPORT int lc_gemm256(const void* Wp, const void* X, void* Y, const void* bia
                           hipFuncAttributeMaxDynamicSharedMemorySize, G2B_LDS);
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm256_kernel<EPI_F32, false, 2>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, G2B_LDS);
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm256_kernel<EPI_GEGLU, false, 2>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, G2B_LDS);
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm256_kernel<EPI_SWIGLU, false, 2>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, G2B_LDS);
     });
@@ -467,8 +487,6 @@ LC_EXPORT int lc_gemm256(const void* Wp, const void* X, void* Y, const void* bia
       gemm256_kernel<EPI_F32, false, 2><<<grid, block, G2B_LDS, stream>>>(w, x, Y, b, M, N, K, ldy, tiles_m, tiles_n);
     else if (epi == EPI_SWIGLU)
       gemm256_kernel<EPI_SWIGLU, false, 2><<<grid, block, G2B_LDS, stream>>>(w, x, Y, b, M, N, K, ldy, tiles_m, tiles_n);
-    else if (epi == EPI_GEGLU)
-      gemm256_kernel<EPI_GEGLU, false, 2><<<grid, block, G2B_LDS, stream>>>(w, x, Y, b, M, N, K, ldy, tiles_m, tiles_n);
     else
       return -2;
     LC_RETURN_LAST_ERROR();

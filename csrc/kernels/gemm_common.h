@@ -9,13 +9,17 @@ enum Epilogue : int {
   EPI_BF16 = 0,    // Y bf16 [M, ldy]  (+bias)
   EPI_F32 = 1,     // Y f32  [M, ldy]  (+bias); with split-K: slab blockIdx.y of [S, M, ldy], no bias
   EPI_SWIGLU = 2,  // n-tiles alternate gate/up; Y bf16 [M, N/2] = silu(gate)*up (+bias before act)
-  EPI_RELU2 = 3,   // Y bf16 [M, ldy] = relu(. + bias)^2 (the grouped kernels)
+  EPI_RELU2 = 3,   // Y bf16 [M, ldy] = relu(. + bias)^2 (the grouped kernels, gemm256, kgemm)
   EPI_GLU_CLAMPED = 4,  // n-tiles alternate gate/up; Y bf16 [M, N/2] = clamped gated unit with a scale per row (the grouped kernels)
   EPI_GEGLU = 5,   // as EPI_SWIGLU with the tanh form of gelu instead of silu (gemm256)
+  EPI_REGLU = 6,   // ... with relu (gemm256)
+  EPI_XIELU = 7,   // Y bf16 [M, ldy] = xielu(. + bias) (gemm256, kgemm)
 };
 
 // Epilogues that store act(gate) * up.
-constexpr bool epi_gated(int epi) { return epi == EPI_SWIGLU || epi == EPI_GEGLU; }
+constexpr bool epi_gated(int epi) { return epi == EPI_SWIGLU || epi == EPI_GEGLU || epi == EPI_REGLU; }
+// Epilogues that store act(.) of single columns.
+constexpr bool epi_acts(int epi) { return epi == EPI_RELU2 || epi == EPI_XIELU; }
 
 // Constants of the clamped gated unit: with s = row_scale[row] (1 without the array), g = min(s * gate, limit),
 // u = clamp(s * up, -limit, limit), the output is g * sigmoid(slope * g) * (u + shift).
@@ -30,7 +34,15 @@ LC_DEVICE float silu(float x) { return x / (1.f + __expf(-x)); }
 LC_DEVICE float gelu_tanh(float x) { return x / (1.f + __expf(-1.5957691216057308f * (x + 0.044715f * x * x * x))); }
 
 template <int EPI>
-LC_DEVICE float gate_act(float x) { return EPI == EPI_GEGLU ? gelu_tanh(x) : silu(x); }
+LC_DEVICE float gate_act(float x) { return EPI == EPI_GEGLU ? gelu_tanh(x) : EPI == EPI_REGLU ? fmaxf(x, 0.f) : silu(x); }
+
+// The activation of an EPI_RELU2 or EPI_XIELU epilogue (ap, an: the two numbers of xIELU), v itself in the others.
+template <int EPI>
+LC_DEVICE float column_act(float v, float ap, float an) {
+  if constexpr (EPI == EPI_RELU2) return relu2(v);
+  if constexpr (EPI == EPI_XIELU) return xielu(v, ap, an);
+  return v;
+}
 
 // The clamped gated unit over a gate tile and the up tile next to it (same layout as the SwiGLU store below).
 // ``row_scale`` is indexed like the output rows.
@@ -58,7 +70,7 @@ LC_DEVICE void store_tile_glu_clamped(const f32x4& acc, const f32x4& acc_up, voi
 template <int EPI>
 LC_DEVICE void store_tile(const f32x4& acc, const f32x4* acc_up, void* __restrict__ Y,
                           const bf16_t* __restrict__ bias, int m0, int n0, int M, int N, int ldy,
-                          int lane, size_t slab_off) {
+                          int lane, size_t slab_off, float ap = 0.f, float an = 0.f) {
   const int m = m0 + (lane & 15);
   const int nb = n0 + 4 * (lane >> 4);
   if (m >= M) return;
@@ -85,14 +97,11 @@ LC_DEVICE void store_tile(const f32x4& acc, const f32x4* acc_up, void* __restric
     float v[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r] = acc[r] + ((bias && nb + r < N) ? bf16_to_f32(bias[nb + r]) : 0.f);
-    if constexpr (EPI == EPI_RELU2) {
+    if constexpr (epi_acts(EPI)) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        v[r] = fmaxf(v[r], 0.f);
-        v[r] *= v[r];
-      }
+      for (int r = 0; r < 4; ++r) v[r] = column_act<EPI>(v[r], ap, an);
     }
-    if constexpr (EPI == EPI_BF16 || EPI == EPI_RELU2) {
+    if constexpr (EPI == EPI_BF16 || epi_acts(EPI)) {
       bf16_t* dst = static_cast<bf16_t*>(Y) + static_cast<size_t>(m) * ldy + nb;
       if (nb + 3 < N) {
         u32x2 o;

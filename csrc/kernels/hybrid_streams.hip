@@ -350,20 +350,6 @@ __global__ __launch_bounds__(256) void latent_rope_write_kernel(
     Act<CF32>::store(dst, static_cast<size_t>(slot) * W + R + c, turned(c0 + R, c, rd, cs_lat, pairs, 1.f));
 }
 
-// ---------------------------------------------------------------- xIELU
-// z > 0: ap z^2 + z / 2; z <= 0: an (exp(z) - 1 - z) + z / 2 (ap = softplus(p), an = 1/2 + softplus(q), made by the
-// host). y fp32 [T, n] with row stride ld (a column block of a wider matrix); out [T, n] in the activation type.
-template <bool AF32>
-__global__ void xielu_kernel(const float* __restrict__ y, int ld, void* __restrict__ out, long long total, int n, float ap,
-                             float an) {
-  const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  const long long t = i / n;
-  const float z = y[t * ld + (i - t * n)];
-  const float r = z > 0.f ? ap * z * z + 0.5f * z : an * (expm1f(z) - z) + 0.5f * z;
-  Act<AF32>::store(static_cast<typename Act<AF32>::type*>(out), i, r);
-}
-
 }  // namespace
 
 // ================================================================= launchers
@@ -482,17 +468,5 @@ LC_EXPORT int lc_latent_rope_write(const void* proj, int ld, int col_c, const vo
   if (cache_f32) LC_LR(true);
   else LC_LR(false);
 #undef LC_LR
-  LC_RETURN_LAST_ERROR();
-}
-
-LC_EXPORT int lc_xielu(const void* y, int ld, void* out, int act_f32, int T, int n, float ap, float an, hipStream_t st) {
-  if (T <= 0 || n <= 0) return 0;
-  if (ld < n) return -1;
-  const long long total = static_cast<long long>(T) * n;
-  const dim3 grid(static_cast<unsigned>((total + 255) / 256)), block(256);
-  if (act_f32)
-    xielu_kernel<true><<<grid, block, 0, st>>>(static_cast<const float*>(y), ld, out, total, n, ap, an);
-  else
-    xielu_kernel<false><<<grid, block, 0, st>>>(static_cast<const float*>(y), ld, out, total, n, ap, an);
   LC_RETURN_LAST_ERROR();
 }

@@ -21,7 +21,7 @@ template <int MT, int NTW, int EPI>
 __global__ __launch_bounds__(512) void kgemm_kernel(const bf16_t* __restrict__ Wp,
                                                     const bf16_t* __restrict__ X, void* __restrict__ Y,
                                                     const bf16_t* __restrict__ bias, int M, int N, int K,
-                                                    int ldy) {
+                                                    int ldy, float ap, float an) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int NF = NTW * MT;  // accumulator fragments per wave
   const int lane = threadIdx.x & 63;
@@ -104,22 +104,28 @@ __global__ __launch_bounds__(512) void kgemm_kernel(const bf16_t* __restrict__ W
         if (n & 1) continue;
         store_tile<EPI>(acc[n][m], &acc[(n + 1) % NTW][m], Y, bias, m * 16, (nt0 + n) * 16, M, N, ldy, lane, 0);
       } else {
-        store_tile<EPI>(acc[n][m], nullptr, Y, bias, m * 16, (nt0 + n) * 16, M, N, ldy, lane, 0);
+        store_tile<EPI>(acc[n][m], nullptr, Y, bias, m * 16, (nt0 + n) * 16, M, N, ldy, lane, 0, ap, an);
       }
     }
 }
 
 template <int MT, int NTW>
 int launch_k(int epi, const bf16_t* Wp, const bf16_t* X, void* Y, const bf16_t* bias, int M, int N, int K,
-             int ldy, int n_pad, hipStream_t stream) {
+             int ldy, int n_pad, float ap, float an, hipStream_t stream) {
   const dim3 grid(n_pad / (16 * NTW)), block(512);
   const size_t lds = 4 * NTW * MT * 64 * sizeof(f32x4);
   if (epi == EPI_BF16)
-    kgemm_kernel<MT, NTW, EPI_BF16><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy);
+    kgemm_kernel<MT, NTW, EPI_BF16><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy, ap, an);
   else if (epi == EPI_F32)
-    kgemm_kernel<MT, NTW, EPI_F32><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy);
+    kgemm_kernel<MT, NTW, EPI_F32><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy, ap, an);
+  else if (epi == EPI_RELU2)
+    kgemm_kernel<MT, NTW, EPI_RELU2><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy, ap, an);
+  else if (epi == EPI_XIELU)
+    kgemm_kernel<MT, NTW, EPI_XIELU><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy, ap, an);
+  else if (epi != EPI_SWIGLU)
+    return -3;
   else if constexpr (NTW >= 2)
-    kgemm_kernel<MT, NTW, EPI_SWIGLU><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy);
+    kgemm_kernel<MT, NTW, EPI_SWIGLU><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy, ap, an);
   else
     return -3;
   return static_cast<int>(hipGetLastError());
@@ -129,7 +135,7 @@ int launch_k(int epi, const bf16_t* Wp, const bf16_t* X, void* Y, const bf16_t* 
 
 // M <= 64, K % 32 == 0, n_pad % 128 == 0. ntw = n-tiles (16 columns) per workgroup: 1, 2 or 4.
 LC_EXPORT int lc_kgemm(const void* Wp, const void* X, void* Y, const void* bias, int M, int N, int K,
-                       int n_pad, int ldy, int epi, int ntw, hipStream_t stream) {
+                       int n_pad, int ldy, int epi, int ntw, float ap, float an, hipStream_t stream) {
   if (M <= 0) return 0;
   if (M > 64 || K % 32 || n_pad % 128 || N > n_pad) return -1;
   auto w = static_cast<const bf16_t*>(Wp);
@@ -137,9 +143,9 @@ LC_EXPORT int lc_kgemm(const void* Wp, const void* X, void* Y, const void* bias,
   auto b = static_cast<const bf16_t*>(bias);
   const int mt = (M + 15) / 16;
 #define LC_K(MT_)                                                                          \
-  if (ntw == 1) return launch_k<MT_, 1>(epi, w, x, Y, b, M, N, K, ldy, n_pad, stream);     \
-  if (ntw == 2) return launch_k<MT_, 2>(epi, w, x, Y, b, M, N, K, ldy, n_pad, stream);     \
-  if (ntw == 4) return launch_k<MT_, 4>(epi, w, x, Y, b, M, N, K, ldy, n_pad, stream);     \
+  if (ntw == 1) return launch_k<MT_, 1>(epi, w, x, Y, b, M, N, K, ldy, n_pad, ap, an, stream);     \
+  if (ntw == 2) return launch_k<MT_, 2>(epi, w, x, Y, b, M, N, K, ldy, n_pad, ap, an, stream);     \
+  if (ntw == 4) return launch_k<MT_, 4>(epi, w, x, Y, b, M, N, K, ldy, n_pad, ap, an, stream);     \
   return -1;
   if (mt <= 1) { LC_K(1) }
   if (mt <= 2) { LC_K(2) }

@@ -1171,6 +1171,14 @@ class HybridModel:
                 b = torch.cat([b, b.new_zeros(extra)], 0) if b is not None else None
             return ops.LinearWeight.from_dense(W, b, dev, dtype=dt, any_shape=True)
 
+        def gate_up(f: str) -> ops.LinearWeight:
+            gate, up = load(f + "gate"), load(f + "up")
+            if gate.shape[0] % 16:
+                return lin(torch.cat([gate, up], 0))
+            w = lin(ops.interleave_gate_up(gate, up))      # (tiles of gate and up: the gated unit can be the product's epilogue)
+            w.tiled = True
+            return w
+
         def f32(t: torch.Tensor) -> torch.Tensor:
             return t.to(torch.float32).reshape(-1).contiguous()
 
@@ -1314,11 +1322,7 @@ class HybridModel:
                 else:
                     kw["experts_up"], kw["experts_down"] = ups.to(dt).contiguous(), downs.to(dt).contiguous()
             elif l.ff and c.design.parallel_ff:
-                if l.ff % 16 == 0:                  # (tiles of gate and up: the gated unit can be the product's epilogue)
-                    kw["gate_up"] = lin(ops.interleave_gate_up(load(f + "gate"), load(f + "up")))
-                    kw["gate_up"].tiled = True
-                else:
-                    kw["gate_up"] = lin(torch.cat([load(f + "gate"), load(f + "up")], 0))
+                kw["gate_up"] = gate_up(f)
             elif l.ff and c.design.sandwich:
                 kw["down"] = lin(load(f + "down"))
             elif l.ff and c.design.dense_ff == "xielu":
@@ -1328,7 +1332,7 @@ class HybridModel:
                           act=(float(sp[0]), 0.5 + float(sp[1])))
             elif l.ff:
                 if c.design.dense_ff == "glu_relu":
-                    kw["gate_up"] = lin(torch.cat([load(f + "gate"), load(f + "up")], 0))
+                    kw["gate_up"] = gate_up(f)
                 else:
                     kw["up"] = lin(load(f + "up"))
                 kw["down"] = lin(load(f + "down"))
@@ -1507,7 +1511,7 @@ class HybridModel:
                 y = self._gla(i, L, xa, positions, lay, cache)
             xa = ops.scalar_norm_add(x, y, L.norm1, eps, dt)
             if L.up is not None:
-                xa = ops.scalar_norm_add(x, self._result(self._relu2_up(xa, L.up), L.down), L.norm2, eps, dt)
+                xa = ops.scalar_norm_add(x, self._result(ops.act_linear(xa, L.up, "relu2", self.dtype), L.down), L.norm2, eps, dt)
             if taps is not None:
                 taps.append(x.clone())
         return x
@@ -1516,13 +1520,6 @@ class HybridModel:
         """A sublayer's last product: fp32, and where its depth was split the slabs as they are (the residual step sums
         them). (The Dynamic Tanh step takes whole results.)"""
         return ops.linear(a, w, out_f32=True, defer_reduce=self.cfg.design.norm != "dyt")
-
-    def _relu2_up(self, xa: torch.Tensor, up: ops.LinearWeight) -> torch.Tensor:
-        """relu(up x)^2 in the activation type: an epilogue of the shape-agnostic product, one more
-        launch behind the packed MFMA product."""
-        if up.is_packed or not xa.is_cuda:
-            return ops.relu2(ops.linear(xa, up, out_f32=True), self.dtype)
-        return ops.linear_any(xa, up, out_f32=self.dtype == torch.float32, epi_relu2=True)
 
     def _forward_pre_norm(self, token_ids, positions, slot_mapping, meta, lay: StepLayout, cache: HybridCache,
                           taps: Optional[list]) -> torch.Tensor:
@@ -1768,10 +1765,10 @@ class HybridModel:
 
     def _dense_ff(self, L: HybridLayer, xa: torch.Tensor) -> torch.Tensor:
         if L.act is not None:               # (biases ride in the products)
-            return self._result(ops.xielu(ops.linear(xa, L.up, out_f32=True), L.act[0], L.act[1], self.dtype), L.down)
+            return self._result(ops.act_linear(xa, L.up, "xielu", self.dtype, *L.act), L.down)
         if L.gate_up is not None:
-            return self._result(ops.glu(ops.linear(xa, L.gate_up, out_f32=True), self.dtype, "relu"), L.down)
-        return self._result(self._relu2_up(xa, L.up), L.down)
+            return self._result(ops.glu_linear(xa, L.gate_up, "relu", self.dtype), L.down)
+        return self._result(ops.act_linear(xa, L.up, "relu2", self.dtype), L.down)
 
     def _routed_ff(self, L: HybridLayer, xa: torch.Tensor) -> torch.Tensor:
         e = L.spec.moe

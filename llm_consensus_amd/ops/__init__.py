@@ -15,7 +15,7 @@ import torch
 
 from . import reference as ref
 
-EPI_BF16, EPI_F32, EPI_SWIGLU, EPI_GEGLU = 0, 1, 2, 5
+EPI_BF16, EPI_F32, EPI_SWIGLU, EPI_RELU2, EPI_GEGLU, EPI_REGLU, EPI_XIELU = 0, 1, 2, 3, 5, 6, 7
 
 # M at or below which the decode kernels (one activation panel) are used instead of the tile kernels.
 WS_MAX_M = int(os.environ.get("LC_WS_MAX_M", "256"))
@@ -278,9 +278,12 @@ def linear(x: torch.Tensor, w: LinearWeight, out_f32: bool = False, defer_reduce
             return y
         if GEMM256_MIN_TILES >= 0 and w.n_pad % 256 == 0 and tiles256 >= GEMM256_MIN_TILES:
             # long K (down projections): four waves of 128 x 128 with the accumulators in AGPRs
-            kern = "lc_gemm256w" if use_four_wave_gemm(w.k, epi == EPI_F32) else "lc_gemm256"
-            h.call(kern, w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad,
-                   out_n, epi)
+            if use_four_wave_gemm(w.k, epi == EPI_F32):
+                h.call("lc_gemm256w", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad,
+                       out_n, epi)
+            else:
+                h.call("lc_gemm256", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad,
+                       out_n, epi, 0.0, 0.0)
             return y
         h.call("lc_gemm_tile", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad,
                out_n, epi)
@@ -289,7 +292,7 @@ def linear(x: torch.Tensor, w: LinearWeight, out_f32: bool = False, defer_reduce
     ntw = _kgemm_ntw(w.n_pad, M, w.swiglu, w.k)
     if ntw:   # a handful of rows, narrow output: K split over the waves of one workgroup
         h.call("lc_kgemm", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad,
-               out_n, epi, ntw)
+               out_n, epi, ntw, 0.0, 0.0)
         return y
     # 257..320 column tiles of 128 (Qwen2.5-7B gate/up: 296): a second round would keep 40 CUs busy
     # as long as the first kept 256; workgroups of 160 columns cover the matrix in one round
@@ -299,7 +302,7 @@ def linear(x: torch.Tensor, w: LinearWeight, out_f32: bool = False, defer_reduce
     # a second round of 128-column tiles would start; 256x256 tiles (half as many) do better.
     if M > 128 and not wide and w.n_pad // 128 > 256 and w.n_pad % 256 == 0 and GEMM256_MIN_TILES >= 0:
         h.call("lc_gemm256", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad,
-               out_n, epi)
+               out_n, epi, 0.0, 0.0)
         return y
     kernel, splits, extra = "lc_gemm_panel", _choose_panel_splits(w.n_pad, w.k) if w.n % 32 == 0 else 1, (1 if PANEL_DEEP else 0,)
     if wide:
@@ -992,15 +995,58 @@ def scalar_norm_add(x: torch.Tensor, y: Optional[torch.Tensor], gain: torch.Tens
 
 
 def relu2(y: torch.Tensor, act_dtype: torch.dtype) -> torch.Tensor:
-    """relu(y)^2 of an fp32 matrix (may be a column slice of a wider one) in ``act_dtype``."""
-    if not y.is_cuda:
-        return ref.relu2(y, act_dtype)
-    if y.dim() != 2 or y.stride(1) != 1 or y.dtype != torch.float32:
-        raise ValueError("relu2: an fp32 matrix with unit column stride")
-    T, cols = y.shape
-    out = torch.empty(T, cols, dtype=act_dtype, device=y.device)
-    _hip().call("lc_relu2", y.data_ptr(), out.data_ptr(), _f32flag(act_dtype), T, cols, max(y.stride(0), cols))
+    """relu(y)^2 of an fp32 matrix (may be a column slice of a wider one, or a ``PartialSum``) in ``act_dtype``."""
+    return _column_act(y, "relu2", 0.0, 0.0, act_dtype)
+
+
+def _column_act(y, kind: str, ap: float, an: float, act_dtype: torch.dtype) -> torch.Tensor:
+    if not isinstance(y, PartialSum):
+        if not y.is_cuda:
+            return ref.relu2(y, act_dtype) if kind == "relu2" else ref.xielu(y, ap, an, act_dtype)
+        if y.dim() != 2 or y.stride(1) != 1 or y.dtype != torch.float32:
+            raise ValueError(f"{kind}: an fp32 matrix with unit column stride")
+    T, n = y.shape
+    part, parts, bias, ld = (y.part, y.part.shape[0], y.bias, n) if isinstance(y, PartialSum) else (y, 1, None, max(y.stride(0), n))
+    out = torch.empty(T, n, dtype=act_dtype, device=part.device)
+    _hip().call("lc_act", part.data_ptr(), parts, ld, _hip().ptr(bias), out.data_ptr(), _f32flag(act_dtype), T, n, COLUMN_ACTS.index(kind),
+                float(ap), float(an))
     return out
+
+
+COLUMN_ACTS = ("relu2", "xielu")
+
+
+def act_linear(x: torch.Tensor, w: LinearWeight, kind: str, act_dtype: torch.dtype, ap: float = 0.0, an: float = 0.0) -> torch.Tensor:
+    """act(x @ W^T + bias) in ``act_dtype`` (kind: "relu2", or "xielu" with its two numbers). Packed products of bf16 activations
+    that are one launch of 256 x 256 tiles or of the split-in-the-workgroup kernel apply it to their accumulators; otherwise it
+    is a launch behind the fp32 product, which also sums the slabs of a split one."""
+    if not x.is_cuda:
+        return _column_act(linear(x, w, out_f32=True), kind, ap, an, act_dtype)
+    if not w.is_packed:
+        if kind == "relu2":
+            return linear_any(x, w, out_f32=act_dtype == torch.float32, epi_relu2=True)
+        return _column_act(linear(x, w, out_f32=True), kind, ap, an, act_dtype)
+    M = x.shape[0]
+    if x.dtype == torch.bfloat16 and act_dtype == torch.bfloat16 and not w.swiglu and M > 0:
+        h, epi = _hip(), EPI_RELU2 if kind == "relu2" else EPI_XIELU
+        ntw = _kgemm_ntw(w.n_pad, M, False, w.k) if M <= WS_MAX_M else 0
+        if ntw or _whole_tiles256(M, w):
+            x, y = x.contiguous(), torch.empty(M, w.n, dtype=act_dtype, device=x.device)
+            args = (w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, w.n, epi)
+            if ntw:
+                h.call("lc_kgemm", *args, ntw, float(ap), float(an))
+            else:
+                h.call("lc_gemm256", *args, float(ap), float(an))
+            return y
+    return _column_act(linear(x, w, out_f32=True, defer_reduce=True), kind, ap, an, act_dtype)
+
+
+def _whole_tiles256(M: int, w: LinearWeight) -> bool:
+    """Whether a product of M rows is one launch of 256 x 256 tiles whose depth is not split."""
+    if M <= WS_MAX_M or w.n_pad % 256 or GEMM256_MIN_TILES < 0:
+        return False
+    tiles = ((M + 255) // 256) * (w.n_pad // 256)
+    return tiles >= max(GEMM256_MIN_TILES, 1) and _choose_gemm256_splits(tiles, w.k) == 1
 
 
 def _scan_scratch(B: int, max_len: int, state_floats: int, decay_floats: int, device) -> Optional[torch.Tensor]:
@@ -1384,21 +1430,22 @@ def _residual_step(x: torch.Tensor, y, w_out=None, w_in=None, w_in2=None, eps: f
 def glu_linear(x: torch.Tensor, w: LinearWeight, kind: str, act_dtype: torch.dtype, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """act(gate) * up of x's product with ``w`` (rows gate | up, or in alternate tiles of 16 when ``w.tiled``), [T, n] in
     ``act_dtype``, into ``out`` (a block of a wider matrix) when given. Large bf16 products of tiled weights store the gated unit
-    from their accumulators (gelu_tanh); otherwise the fp32 product is gated in a launch of its own, which also sums the slabs
+    from their accumulators (gelu_tanh, relu); otherwise the fp32 product is gated in a launch of its own, which also sums the slabs
     of a split one."""
     M, n = x.shape[0], w.n // 2
-    if x.is_cuda and w.is_packed and w.tiled and w.bias is None and kind == "gelu_tanh" and act_dtype == torch.bfloat16 \
-            and M > WS_MAX_M and w.n_pad % 256 == 0 and GEMM256_MIN_TILES >= 0:
-        tiles = ((M + 255) // 256) * (w.n_pad // 256)
+    if x.is_cuda and w.is_packed and w.tiled and w.bias is None and kind in GLU_EPILOGUES and act_dtype == torch.bfloat16 \
+            and _whole_tiles256(M, w):
         y = _out_block(out, M, n, act_dtype, x.device, "glu_linear")
         ldy = max(y.stride(0), n)
-        if tiles >= max(GEMM256_MIN_TILES, 1) and _choose_gemm256_splits(tiles, w.k) == 1 and ldy % 8 == 0 and y.data_ptr() % 16 == 0:
-            _hip().call("lc_gemm256", w.data.data_ptr(), x.contiguous().data_ptr(), y.data_ptr(), None, M, w.n, w.k, w.n_pad, ldy, EPI_GEGLU)
+        if ldy % 8 == 0 and y.data_ptr() % 16 == 0:
+            _hip().call("lc_gemm256", w.data.data_ptr(), x.contiguous().data_ptr(), y.data_ptr(), None, M, w.n, w.k, w.n_pad, ldy,
+                        GLU_EPILOGUES[kind], 0.0, 0.0)
             return y
     return glu(linear(x, w, out_f32=True, defer_reduce=True), act_dtype, kind, out=out, tiled=w.tiled)
 
 
 GLU_KINDS = ("relu", "silu", "gelu_tanh")
+GLU_EPILOGUES = {"gelu_tanh": EPI_GEGLU, "relu": EPI_REGLU}
 
 
 def glu(y, act_dtype: torch.dtype, kind: str = "relu", out: Optional[torch.Tensor] = None, tiled: bool = False) -> torch.Tensor:
@@ -1743,16 +1790,9 @@ def latent_rope_write(proj: torch.Tensor, col_c: int, w: Optional[torch.Tensor],
 
 
 def xielu(y: torch.Tensor, ap: float, an: float, act_dtype: torch.dtype) -> torch.Tensor:
-    """xIELU of an fp32 matrix (may be a column slice): ap z^2 + z / 2 above zero, an (exp(z) - 1 - z) + z / 2 at
-    and below it, in ``act_dtype``."""
-    if not y.is_cuda:
-        return ref.xielu(y, ap, an, act_dtype)
-    if y.dim() != 2 or y.stride(1) != 1 or y.dtype != torch.float32:
-        raise ValueError("xielu: an fp32 matrix with unit column stride")
-    T, n = y.shape
-    out = torch.empty(T, n, dtype=act_dtype, device=y.device)
-    _hip().call("lc_xielu", y.data_ptr(), max(y.stride(0), n), out.data_ptr(), _f32flag(act_dtype), T, n, float(ap), float(an))
-    return out
+    """xIELU of an fp32 matrix (may be a column slice, or a ``PartialSum``): ap z^2 + z / 2 above zero, an (exp(z) - 1 - z) + z / 2
+    at and below it, in ``act_dtype``."""
+    return _column_act(y, "xielu", ap, an, act_dtype)
 
 
 # ---- gated residual steps between two norms, token shift, convolved / normed / mixed attention inputs, linear attention

@@ -25,10 +25,10 @@ _SIGNATURES = {
     "lc_embed_pool": [_P, _P, _P, _P, _I, _I, _I, _P],
     "lc_l2_normalize": [_P, _P, _I, _I, _P],
     "lc_gemm_tile": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
-    "lc_gemm256": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
+    "lc_gemm256": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _P],
     "lc_gemm256w": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "lc_gemm_panel": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P],
-    "lc_kgemm": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
+    "lc_kgemm": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _P],
     "lc_splitk_reduce": [_P, _P, _P, _I, _I, _I, _I, _I, _P],
     "lc_gemm_grouped": [_P, _L, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P],
     "lc_gemm256_splitk": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
@@ -61,7 +61,7 @@ _SIGNATURES = {
     "lc_scatter_rows": [_P, _P, _P, _I, _I, _P, _P],
     # hybrid decoders (hybrid.hip)
     "lc_embed_rows": [_P, _P, _I, _P, _P, _I, _I, _I, _I, _P, _P, _F, _P, _P, _P, _L, _L, _L, _P, _L, _P, _P, _P, _P],
-    "lc_relu2": [_P, _P, _I, _I, _I, _I, _P],
+    "lc_act": [_P, _I, _I, _P, _P, _I, _I, _I, _I, _F, _F, _P],
     "lc_mingru_scan": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P, _P],
     "lc_gla_scan": [_P, _I, _P, _P, _L, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _P],
     "lc_linear_chunks": [_P, _I, _I, _P, _P, _F, _F, _P, _L, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P],
@@ -93,7 +93,6 @@ _SIGNATURES = {
     "lc_rope_qkv_write": [_P, _I, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P],
     "lc_talk_mix": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "lc_latent_rope_write": [_P, _I, _I, _P, _F, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P],
-    "lc_xielu": [_P, _I, _P, _I, _I, _I, _F, _F, _P],
     # gated residual steps, token shifts, attention pre-processing with convolutions and mixed values (hybrid_gated.hip)
     "lc_gated_step": [_P, _P, _I, _P, _P, _I, _P, _P, _F, _P, _P, _P, _P, _I, _I, _I, _P, _P, _L, _P, _P, _P, _P, _I, _I, _P],
     "lc_token_shift": [_P, _P, _P, _L, _P, _P, _P, _P, _P, _I, _I, _I, _P],

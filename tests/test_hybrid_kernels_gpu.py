@@ -1163,3 +1163,30 @@ def test_residual_step_at_the_edges_of_its_block_sizes(T, d):
     want = ops.add_rmsnorm(x, part.sum(0), w, 1e-5, torch.float32)
     assert torch.allclose(xg.cpu(), x, atol=2e-6)          # (four fp32 numbers of a few units, summed)
     assert torch.allclose(h.cpu(), want, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 256, 128), (8, 100, 64), (9, 512, 2048), (257, 256, 64), (300, 512, 2048), (2048, 4096, 256), (2100, 4090, 64)])
+@pytest.mark.parametrize("kind", ["relu2", "xielu"])
+def test_activation_of_a_product(M, N, K, kind):
+    """Products whose epilogue is the activation (few rows, whole tiles of 256, ragged edges) and split ones whose slabs the
+    activation's launch sums, with and without a bias."""
+    g = torch.Generator().manual_seed(M + N)
+    x, W, b = torch.randn(M, K, generator=g).bfloat16(), torch.randn(N, K, generator=g) / K ** 0.5, torch.randn(N, generator=g)
+    act = (lambda y: ref.relu2(y, torch.float32)) if kind == "relu2" else (lambda y: ref.xielu(y, 0.7, 0.9, torch.float32))
+    for bias in (None, b):
+        w = ops.LinearWeight.from_dense(W, bias, DEV)
+        y = x.float() @ W.bfloat16().float().T
+        want = act(y + bias.bfloat16().float() if bias is not None else y)
+        got = ops.act_linear(x.to(DEV), w, kind, torch.bfloat16, 0.7, 0.9)
+        assert got.shape == (M, N)
+        torch.testing.assert_close(got.float().cpu(), want, **_tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 512, 2048), (300, 512, 2048), (2048, 4096, 256), (2100, 2048, 64)])
+def test_relu_gated_unit_of_a_product_with_tiled_weights(M, N, K):
+    g = torch.Generator().manual_seed(M)
+    x, Wg, Wu = torch.randn(M, K, generator=g).bfloat16(), *(torch.randn(N // 2, K, generator=g) * 2 / K ** 0.5 for _ in range(2))
+    w = ops.LinearWeight.from_dense(ops.interleave_gate_up(Wg, Wu), None, DEV)
+    w.tiled = True
+    want = ref.glu(torch.cat([x.float() @ Wg.bfloat16().float().T, x.float() @ Wu.bfloat16().float().T], 1), torch.float32, "relu")
+    torch.testing.assert_close(ops.glu_linear(x.to(DEV), w, "relu", torch.bfloat16).float().cpu(), want, **_tol(torch.bfloat16))
