@@ -49,13 +49,19 @@ def set_concurrent_engines(n: int) -> None:
         PANEL_DEEP = n <= 1
 # In-workgroup K-split decode kernel (kgemm.hip): widest output it is used for, and a test override
 # (-1 = automatic, 0 = never, 1/2/4 = force that many n-tiles per workgroup).
-KGEMM_MAX_N = int(os.environ.get("LC_KGEMM_MAX_N", "8192"))
+KGEMM_MAX_N = int(os.environ.get("LC_KGEMM_MAX_N", str(1 << 30)))
+KGEMM_MAX_N_GATED = int(os.environ.get("LC_KGEMM_MAX_N", "8192"))
 # Most rows the in-workgroup K-split kernel is used for. Measured against the panel kernel (with
 # non-temporal weight loads) on HBM-resident weights: at 1 row it wins on the narrow projections
-# (6144x4096 10.9 vs 13.0 us, 4096x4096 7.9 vs 9.3) and ties on the wide ones; at 8 rows it still wins
-# those (11.9 vs 13.5, 8.4 vs 9.4) but loses where K is long (3584x18944: 26.5 vs 23.9); at 16 rows it
-# loses everywhere (4096x14336: 28.3 vs 21.4, 3584x18944: 36.3 vs 24.2).
+# (6144x4096 10.9 vs 13.0 us, 4096x4096 7.9 vs 9.3) and on wide ones that are not gated with one
+# n-tile per workgroup (128256x4096 153 vs 179, 32000x2048 21 vs 27, 16384x4096 22 vs 31; the gated
+# 28672x4096 ties); at 8 rows it still wins there, wide ones with two n-tiles (11.9 vs 13.5, 8.4 vs
+# 9.4, 167 vs 181, 22 vs 27), but loses where K is long (3584x18944: 26.5 vs 23.9); at 16 rows it
+# loses (4096x14336: 28.3 vs 21.4, 3584x18944: 36.3 vs 24.2, 152064x3584: 184 vs 182) except on
+# wide outputs over a short K (128256x2048 85 vs 102, 16384x2048 13.7 vs 19.3).
 KGEMM_MAX_M = int(os.environ.get("LC_KGEMM_MAX_M", "8"))
+KGEMM_SHORT_K = 2048         # up to this K outputs of more than 8192 columns use it up to KGEMM_SHORT_K_MAX_M rows
+KGEMM_SHORT_K_MAX_M = 2 * KGEMM_MAX_M
 KGEMM_LONG_K = 8192          # beyond this K the kernel is only used up to KGEMM_LONG_K_MAX_M rows
 KGEMM_LONG_K_MAX_M = 4
 KGEMM_FORCE_NTW = int(os.environ.get("LC_KGEMM_NTW", "-1"))
@@ -154,18 +160,17 @@ class LinearWeight:
 
 def _kgemm_ntw(n_pad: int, M: int, swiglu: bool, K: int = 0) -> int:
     """n-tiles per workgroup for the in-workgroup K-split kernel, or 0 to use another kernel.
-    It re-reads the activations once per workgroup from L2, so it is limited to M <= 64 and
-    to outputs narrow enough that this stays below the weight traffic."""
+    It re-reads the activations once per workgroup from L2, so it is limited to a few rows."""
     if KGEMM_FORCE_NTW >= 0:
         return KGEMM_FORCE_NTW if M <= 64 else 0
-    if M > KGEMM_MAX_M or n_pad > KGEMM_MAX_N or (K > KGEMM_LONG_K and M > KGEMM_LONG_K_MAX_M):
+    wide = n_pad > 8192
+    if n_pad > (KGEMM_MAX_N_GATED if swiglu else KGEMM_MAX_N) or (K > KGEMM_LONG_K and M > KGEMM_LONG_K_MAX_M):
         return 0
-    for ntw in (4, 2, 1):
-        if swiglu and ntw < 2:
-            break
-        if n_pad // (16 * ntw) >= 256:
-            return ntw
-    return 2 if swiglu else 1
+    if M > KGEMM_MAX_M and not (wide and K <= KGEMM_SHORT_K and M <= KGEMM_SHORT_K_MAX_M):
+        return 0
+    if not swiglu and (M <= 4 or n_pad < 8192):
+        return 1
+    return 4 if swiglu and n_pad >= 16384 else 2
 
 
 def _choose_panel_splits(n_pad: int, K: int) -> int:

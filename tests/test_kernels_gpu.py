@@ -154,6 +154,16 @@ def test_kgemm_in_workgroup_ksplit(M, N, K, ntw):
         ops.KGEMM_FORCE_NTW = old
 
 
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16, 17])
+@pytest.mark.parametrize("N,K", [(8192, 64), (8200, 2048), (8320, 2112)])
+def test_few_rows_against_outputs_around_the_rule_for_wide_ones(M, N, K):
+    X, W = bf(rand(M, K, scale=0.5)), bf(rand(N, K, scale=0.5, seed=1))
+    lw = ops.LinearWeight.from_dense(W, None, DEV)
+    want = ref.linear(X, W, None, torch.float32)
+    assert rel_err(ops.linear(X.to(DEV), lw), want) < 6e-3
+    assert rel_err(ops.linear(X.to(DEV), lw, out_f32=True), want) < 1e-4
+
+
 @pytest.mark.parametrize("M", [1, 7, 16, 33, 64, 100, 128, 200, 256])
 @pytest.mark.parametrize("N,K", [(256, 1024), (1152, 896), (128, 4096)])
 def test_panel_gemm_with_and_without_splitk(M, N, K):
