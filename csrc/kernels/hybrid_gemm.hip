@@ -22,6 +22,7 @@ struct AnyGemm {
   int epi;                       // 1: square of relu
   int a_hs, c_hs;                // first column of head h in A and in C
   int ld_gate, gate_full;
+  int splits;                    // > 1: part s of the depth leaves its sums in slab s of C (fp32, [M, ldc] each; no bias, epi or gate)
 };
 
 // Elements i .. i + 3 of p as floats, zeros from the n-th on (n may be negative).
@@ -37,8 +38,12 @@ LC_DEVICE float4 load4_any(const void* p, int f32, int vec, size_t i, int n) {
   return make_float4(v[0], v[1], v[2], v[3]);
 }
 
-LC_DEVICE void finish_any(const AnyGemm& g, int h, int row, int col, float v) {
+LC_DEVICE void finish_any(const AnyGemm& g, int h, int row, int col, float v, int split) {
   if (row >= g.M || col >= g.N) return;
+  if (g.splits > 1) {
+    static_cast<float*>(g.C)[(static_cast<size_t>(split) * g.M + row) * g.ldc + col] = v;
+    return;
+  }
   if (g.bias != nullptr) v += g.w_f32 ? static_cast<const float*>(g.bias)[col] : bf16_to_f32(static_cast<const bf16_t*>(g.bias)[col]);
   if (g.epi == 1) {
     v = fmaxf(v, 0.f);
@@ -82,10 +87,11 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_any_rows_kernel(AnyGemm g) {
       for (int m = 0; m < MT; ++m) ad[m][s] = load4_any(g.A, g.a_f32, g.a_vec, a_row[m] + k, g.K - k);
     }
   };
-  const int chunks = (g.K + 31) / 32;
-  if (wave < chunks) fetch(w, a, wave);
-  for (int c = wave; c < chunks; c += WAVES) {
-    if (c + WAVES < chunks) fetch(wn, an, c + WAVES);
+  const int chunks = (g.K + 31) / 32, per = (chunks + g.splits - 1) / g.splits;
+  const int first = blockIdx.y * per + wave, last = min(static_cast<int>(blockIdx.y + 1) * per, chunks);
+  if (first < last) fetch(w, a, first);
+  for (int c = first; c < last; c += WAVES) {
+    if (c + WAVES < last) fetch(wn, an, c + WAVES);
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -108,7 +114,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_any_rows_kernel(AnyGemm g) {
 #pragma unroll
   for (int i = 1; i < WAVES; ++i) sum += red[i][wave][lane];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) finish_any(g, h, 16 * wave + lr, n0 + 4 * lq + r, sum[r]);
+  for (int r = 0; r < 4; ++r) finish_any(g, h, 16 * wave + lr, n0 + 4 * lq + r, sum[r], blockIdx.y);
 }
 
 // ---------------------------------------------------------------- more rows
@@ -128,7 +134,8 @@ __global__ __launch_bounds__(256 * KG) void gemm_any_tile_kernel(AnyGemm g, cons
   const int tid = threadIdx.x & 255, kg = threadIdx.x >> 8, lane = tid & 63, wave = tid >> 6;
   const int lr = lane & 15, lq = lane >> 4, wm = wave >> 1, wn = wave & 1;
   const int n0 = blockIdx.x * 64;
-  int m0 = blockIdx.y * 64, h = blockIdx.z;
+  const int split = g.splits > 1 ? blockIdx.z : 0;     // (products per head are not split)
+  int m0 = blockIdx.y * 64, h = g.splits > 1 ? 0 : blockIdx.z;
   size_t w_first = static_cast<size_t>(h) * g.N * g.K;
   if constexpr (GROUPED) {
     int e = 0, tile = blockIdx.y, lo = 0, hi = 0;
@@ -149,10 +156,11 @@ __global__ __launch_bounds__(256 * KG) void gemm_any_tile_kernel(AnyGemm g, cons
   if (GROUPED && row_index != nullptr) a_at = row_index[a_at];
   const size_t a_row = static_cast<size_t>(a_at) * g.lda + static_cast<size_t>(h) * g.a_hs;
   const size_t w_row = w_first + static_cast<size_t>(min(n0 + sr, g.N - 1)) * g.K;
-  const int slabs = ((g.K + 15) / 16 + KG - 1) / KG;   // per group; behind the last depth slabs are zeros
+  const int groups = KG * g.splits;
+  const int slabs = ((g.K + 15) / 16 + groups - 1) / groups;   // per group; behind the last depth slabs are zeros
   float4 ra, rw;
   auto fetch = [&](int s) {
-    const int k = 16 * (kg * slabs + s) + sk;
+    const int k = 16 * ((split * KG + kg) * slabs + s) + sk;
     ra = load4_any(g.A, g.a_f32, g.a_vec, a_row + k, g.K - k);
     rw = load4_any(g.W, g.w_f32, g.w_vec, w_row + k, g.K - k);
   };
@@ -203,7 +211,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_any_tile_kernel(AnyGemm g, cons
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        finish_any(g, h, m0 + 32 * wm + 16 * i + 4 * lq + r, n0 + 32 * wn + 16 * j + lr, acc[i][j][r]);
+        finish_any(g, h, m0 + 32 * wm + 16 * i + 4 * lq + r, n0 + 32 * wn + 16 * j + lr, acc[i][j][r], split);
 }
 
 template <int KG, bool GROUPED>
@@ -223,7 +231,7 @@ int launch_tiles(const AnyGemm& g, const dim3& grid, const int32_t* row_index, c
 // Depth groups: enough waves for four on each of the 1024 SIMDs, none shorter than four slabs.
 template <bool GROUPED>
 int tiles_any(const AnyGemm& g, int m_tiles, int heads, const int32_t* row_index, const int32_t* offsets, int E, hipStream_t st) {
-  const dim3 grid((g.N + 63) / 64, m_tiles, heads);
+  const dim3 grid((g.N + 63) / 64, m_tiles, g.splits > 1 ? g.splits : heads);
   const long long blocks = static_cast<long long>(grid.x) * grid.y * grid.z;
   if (blocks <= 512 && g.K >= 256) return launch_tiles<4, GROUPED>(g, grid, row_index, offsets, E, st);
   if (blocks <= 1024 && g.K >= 128) return launch_tiles<2, GROUPED>(g, grid, row_index, offsets, E, st);
@@ -232,7 +240,7 @@ int tiles_any(const AnyGemm& g, int m_tiles, int heads, const int32_t* row_index
 
 template <int WAVES>
 int rows_any(const AnyGemm& g, int heads, hipStream_t st) {
-  const dim3 grid((g.N + 15) / 16, 1, heads), block(64 * WAVES);
+  const dim3 grid((g.N + 15) / 16, g.splits, heads), block(64 * WAVES);
   if (g.M <= 16)
     gemm_any_rows_kernel<WAVES, 1><<<grid, block, 0, st>>>(g);
   else if (g.M <= 32)
@@ -250,7 +258,7 @@ int any_product(const AnyGemm& g, int heads, hipStream_t st) {
   }
   // sixteen waves give 64 blocks (1024 outputs) the loads in flight of 256 CUs; from 1024 blocks on, or where the depth is four
   // turns at most, four waves hold as many and a block ends sooner
-  const bool wide = static_cast<long long>((g.N + 15) / 16) * heads >= 1024 || g.K <= 128;
+  const bool wide = static_cast<long long>((g.N + 15) / 16) * heads >= 1024 || g.K / g.splits <= 128;
   return wide ? rows_any<4>(g, heads, st) : rows_any<16>(g, heads, st);
 }
 
@@ -259,13 +267,14 @@ int four_border(const void* p, int f32) { return reinterpret_cast<uintptr_t>(p) 
 }  // namespace
 
 // ================================================================= launchers
-// A may be a column slice of a wider matrix: ``lda`` is its row stride in elements.
+// A may be a column slice of a wider matrix: ``lda`` is its row stride in elements. ``splits`` > 1: C is [splits, M, N] fp32, the
+// sums of as many parts of the depth.
 LC_EXPORT int lc_gemm_any(const void* A, int a_f32, int lda, const void* W, int w_f32, const void* bias, void* C,
-                          int c_f32, int M, int N, int K, int epi, hipStream_t st) {
+                          int c_f32, int M, int N, int K, int epi, int splits, hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
-  if (K <= 0 || lda < K) return -1;
+  if (K <= 0 || lda < K || splits < 1 || splits > 64 || (splits > 1 && (bias != nullptr || epi != 0 || !c_f32))) return -1;
   const AnyGemm g{A, W, bias, C, nullptr, a_f32, w_f32, c_f32, K % 4 == 0 && lda % 4 == 0 && four_border(A, a_f32),
-                  K % 4 == 0 && four_border(W, w_f32), lda, N, M, N, K, epi, 0, 0, 0, 0};
+                  K % 4 == 0 && four_border(W, w_f32), lda, N, M, N, K, epi, 0, 0, 0, 0, splits};
   return any_product(g, 1, st);
 }
 
@@ -281,7 +290,7 @@ LC_EXPORT int lc_head_linear(const void* A, int a_f32, int lda, const void* W, i
   if (gate == nullptr && gate_full) return -1;
   const AnyGemm g{A, W, nullptr, C, static_cast<const float*>(gate), a_f32, w_f32, c_f32,
                   K % 4 == 0 && lda % 4 == 0 && a_hs % 4 == 0 && four_border(A, a_f32), K % 4 == 0 && four_border(W, w_f32),
-                  lda, c_ld, M, N, K, 0, a_hs, c_hs, ld_gate, gate_full};
+                  lda, c_ld, M, N, K, 0, a_hs, c_hs, ld_gate, gate_full, 1};
   return any_product(g, H, st);
 }
 
@@ -294,6 +303,6 @@ LC_EXPORT int lc_gemm_any_grouped(const void* A, int a_f32, int lda, const void*
   const int tiles = (rows + 63) / 64 + E;
   if (tiles > 65535) return -1;
   const AnyGemm g{A, W, nullptr, C, nullptr, a_f32, w_f32, c_f32, K % 4 == 0 && lda % 4 == 0 && four_border(A, a_f32),
-                  K % 4 == 0 && four_border(W, w_f32), lda, N, rows, N, K, epi, 0, 0, 0, 0};
+                  K % 4 == 0 && four_border(W, w_f32), lda, N, rows, N, K, epi, 0, 0, 0, 0, 1};
   return tiles_any<true>(g, tiles, 1, static_cast<const int32_t*>(row_index), static_cast<const int32_t*>(offsets), E, st);
 }

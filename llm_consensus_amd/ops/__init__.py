@@ -259,7 +259,7 @@ def linear(x: torch.Tensor, w: LinearWeight, out_f32: bool = False, defer_reduce
     if not w.is_packed:
         if w.swiglu or w.data.dim() != 2:
             raise RuntimeError("GPU linear needs packed weights (LinearWeight.from_dense on a cuda device)")
-        return linear_any(x, w, out_f32)
+        return linear_any(x, w, out_f32, defer_reduce=defer_reduce)
     if x.dtype != torch.bfloat16:
         raise TypeError(f"the MFMA products take bf16 activations, got {x.dtype}")
     x = x.contiguous()
@@ -898,8 +898,23 @@ def _f32flag(dtype: torch.dtype) -> int:
     raise TypeError(f"activation type {dtype}: bf16 or fp32")
 
 
-def linear_any(x: torch.Tensor, w: LinearWeight, out_f32: bool = True, epi_relu2: bool = False) -> torch.Tensor:
-    """y = x W^T (+ bias) for a row-major weight of any shape and type (fp32 matrix instructions). ``epi_relu2``: the square of relu in the epilogue."""
+def _choose_any_splits(M: int, N: int, K: int) -> int:
+    """Parts of the depth of a shape-agnostic product whose consumer sums slabs. Up to 64 rows a block owns 16 outputs: parts of
+    at least 256 depths until every CU has a block (3 rows in fp32, 1024 outputs: K = 1024 5.9 -> 3.9 us, K = 4096 15.3 -> 7.4 us;
+    a second block per CU no longer pays, 2048 x 2048 at 32 rows 10.7 and 11.4 us). With more rows tiles of 64 x 64: up to 128 of
+    them leave CUs idle (128 rows, 1024 outputs: K = 1024 25 -> 7.4 us, K = 4096 88 -> 16 us), more of them gain from shorter
+    blocks (804 rows, K = 4096: 89 -> 78 us) while the depth pays for reading the slabs (K = 1024: 27 -> 26 us, does not)."""
+    if M <= 64:
+        return max(1, min(256 // ((N + 15) // 16), K // 256))
+    tiles = ((M + 63) // 64) * ((N + 63) // 64)
+    if tiles <= 128:
+        return max(1, min(8, K // 128))
+    return 1 if K < 2048 else min(8 if tiles <= 256 else 4, K // 512)
+
+
+def linear_any(x: torch.Tensor, w: LinearWeight, out_f32: bool = True, epi_relu2: bool = False, defer_reduce: bool = False):
+    """y = x W^T (+ bias) for a row-major weight of any shape and type (fp32 matrix instructions). ``epi_relu2``: the square of relu
+    in the epilogue. With ``defer_reduce`` an fp32 product without a bias may come back as a ``PartialSum``."""
     M = x.shape[0]
     odt = torch.float32 if out_f32 else torch.bfloat16
     if x.shape[1] != w.k:
@@ -911,11 +926,12 @@ def linear_any(x: torch.Tensor, w: LinearWeight, out_f32: bool = True, epi_relu2
         raise ValueError("linear_any takes row-major weights")
     if x.stride(1) != 1:
         x = x.contiguous()              # (a column slice of a wider matrix is taken as it is)
-    y = torch.empty(M, w.n, dtype=odt, device=x.device)
+    splits = _choose_any_splits(M, w.n, w.k) if defer_reduce and out_f32 and not epi_relu2 and w.bias is None and M > 0 else 1
+    y = torch.empty((splits, M, w.n) if splits > 1 else (M, w.n), dtype=odt, device=x.device)
     _hip().call("lc_gemm_any", x.data_ptr(), _f32flag(x.dtype), x.stride(0) if M > 1 else max(x.stride(0), w.k),
                 w.data.data_ptr(), _f32flag(w.data.dtype),
-                _hip().ptr(w.bias), y.data_ptr(), 1 if out_f32 else 0, M, w.n, w.k, 1 if epi_relu2 else 0)
-    return y
+                _hip().ptr(w.bias), y.data_ptr(), 1 if out_f32 else 0, M, w.n, w.k, 1 if epi_relu2 else 0, splits)
+    return PartialSum(y) if splits > 1 else y
 
 
 @dataclass

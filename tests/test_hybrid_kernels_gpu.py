@@ -1190,3 +1190,16 @@ def test_relu_gated_unit_of_a_product_with_tiled_weights(M, N, K):
     w.tiled = True
     want = ref.glu(torch.cat([x.float() @ Wg.bfloat16().float().T, x.float() @ Wu.bfloat16().float().T], 1), torch.float32, "relu")
     torch.testing.assert_close(ops.glu_linear(x.to(DEV), w, "relu", torch.bfloat16).float().cpu(), want, **_tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1024, 4096), (3, 100, 3000), (64, 48, 2050), (65, 64, 512), (65, 70, 1030), (130, 1024, 4096), (800, 1000, 2050)])
+@pytest.mark.parametrize("adt", [torch.float32, torch.bfloat16])
+def test_split_products_of_any_shape(M, N, K, adt):
+    """Slabs of a depth that is no multiple of a part, of a turn or of four; their sum against the whole product."""
+    g = torch.Generator().manual_seed(M + K)
+    x, W = torch.randn(M, K, generator=g).to(adt), torch.randn(N, K, generator=g) / K ** 0.5
+    w = ops.LinearWeight.from_dense(W, None, DEV, dtype=torch.float32, plain=True)
+    y = ops.linear_any(x.to(DEV), w, defer_reduce=True)
+    assert isinstance(y, ops.PartialSum) and tuple(y.shape) == (M, N)
+    want = (x.double() @ W.double().T).float()
+    torch.testing.assert_close(y.part.sum(0).cpu(), want, atol=2e-5, rtol=1e-5)      # (fp32 sums of a few thousand terms around 1/64)
