@@ -157,6 +157,9 @@ __global__ __launch_bounds__(256) void act_kernel(const float* __restrict__ y, i
 //           (S <- a S + b is associative), scans its rows again from there and writes the outputs;
 //           the last segment stores the state.
 // mode 0 is the whole sequence in one go (decoded tokens, short portions): nseg = 1, no carry.
+// Bound by the sigmoids (about 20 us of vector instructions for 2048 rows of 2048 channels in the two passes, which also move
+// 90 MB) once loads are out: a thread asks for eight rows, or sixteen carries, before it uses the first; one at a time waited
+// for each (2048 rows of 2048 channels 65 us, now 29 us).
 template <bool AF32>
 __global__ void mingru_scan_kernel(const float* __restrict__ zxg, float* __restrict__ state,
                                    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ positions,
@@ -172,21 +175,42 @@ __global__ void mingru_scan_kernel(const float* __restrict__ zxg, float* __restr
   const int r1 = mode == 0 ? q1 : min(q1, r0 + seg_len);
   if (r0 >= q1) return;
   float* cb = carry != nullptr ? carry + static_cast<size_t>(b) * nseg * 2 * w : nullptr;
+  constexpr int U = 8, UC = 16;                        // rows and carries in flight per thread
   float S = 0.f, A = 1.f;
   if (mode != 1) {
     S = positions[q0] == 0 ? 0.f : state[static_cast<size_t>(slot) * w + c];
-    for (int k = 0; k < seg && mode == 2; ++k)
-      S = cb[(static_cast<size_t>(k) * 2) * w + c] * S + cb[(static_cast<size_t>(k) * 2 + 1) * w + c];
+    for (int k0 = 0; k0 < seg && mode == 2; k0 += UC) {
+      float ca[UC], cs[UC];
+#pragma unroll
+      for (int u = 0; u < UC; ++u) {
+        const size_t k = 2 * static_cast<size_t>(min(k0 + u, seg - 1));
+        ca[u] = cb[k * w + c];
+        cs[u] = cb[(k + 1) * w + c];
+      }
+#pragma unroll
+      for (int u = 0; u < UC; ++u)
+        if (k0 + u < seg) S = ca[u] * S + cs[u];
+    }
   }
   typename Act<AF32>::type* o = static_cast<typename Act<AF32>::type*>(out);
-  for (int t = r0; t < r1; ++t) {
-    const float* row = zxg + static_cast<size_t>(t) * 3 * w;
-    const float z = sigmoidf_(row[c]);
-    const float u = row[w + c];
-    const float cand = u >= 0.f ? u + 0.5f : sigmoidf_(u);
-    S = (1.f - z) * S + z * cand;
-    if (mode == 1) A *= 1.f - z;
-    else Act<AF32>::store(o, static_cast<size_t>(t) * w + c, S * siluf_(row[2 * w + c]));
+  for (int t0 = r0; t0 < r1; t0 += U) {
+    float zl[U], ul[U], gl[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float* row = zxg + static_cast<size_t>(min(t0 + u, r1 - 1)) * 3 * w;
+      zl[u] = row[c];
+      ul[u] = row[w + c];
+      if (mode != 1) gl[u] = row[2 * w + c];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (t0 + u >= r1) break;
+      const float z = sigmoidf_(zl[u]);
+      const float cand = ul[u] >= 0.f ? ul[u] + 0.5f : sigmoidf_(ul[u]);
+      S = (1.f - z) * S + z * cand;
+      if (mode == 1) A *= 1.f - z;
+      else Act<AF32>::store(o, static_cast<size_t>(t0 + u) * w + c, S * siluf_(gl[u]));
+    }
   }
   if (mode == 1) {
     cb[(static_cast<size_t>(seg) * 2) * w + c] = A;
@@ -1169,9 +1193,9 @@ LC_EXPORT int lc_act(const void* y, int parts, int ld, const void* bias, void* o
 
 // ``max_len``: the longest portion of the step (host-known). Portions longer than two segments take
 // the segmented passes; ``scratch`` then holds B * nseg * 2 * w floats (see lc_scan_scratch_floats).
-// 32 rows: the pass that writes the outputs is a dependent chain per state column, so twice the waves of
-// half the length finish sooner (2048-row prompt, 16 heads: 301 us with 64-row segments, 212 us with 32).
-constexpr int kScanSegment = 32;
+// 16 rows: a row is ~110 instructions of its wave (three sigmoids), so short segments give few rows the waves they lack
+// (64 rows 22 us with segments of 32 and 12.6 us with 16; 333 rows of 2048 channels 22 and 15 us; 2048 rows 31 and 29 us).
+constexpr int kScanSegment = 16;
 
 LC_EXPORT long long lc_scan_scratch_floats(int B, int max_len, long long state_floats, long long decay_floats) {
   if (max_len <= 2 * kScanSegment) return 0;
