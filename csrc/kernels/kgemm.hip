@@ -12,6 +12,9 @@
 //     counted vmcnt keeps loads in flight continuously;
 //   * the 8 partial accumulator sets are summed through LDS (tree, 3 barriers) and wave 0..
 //     apply the epilogue (bias / bf16 / fp32 / fused SwiGLU).
+// Gated products with one n-tile per workgroup take half a gate tile and half of the up tile beside it as their
+// 16 operand rows. Two whole tiles give 28672 columns 896 workgroups, three and a half per CU, so that CUs with
+// four finish last (43.7 us at one row of 4096); 1792 of half the size are seven each: 37.0 us (6.3 TB/s).
 // Same packed-weight layout and MFMA orientation as gemm.hip (weights = A operand).
 #include "gemm_common.h"
 
@@ -45,7 +48,11 @@ __global__ __launch_bounds__(512) void kgemm_kernel(const bf16_t* __restrict__ W
     row = row < M ? row : M - 1;
     xrow[m] = X + static_cast<size_t>(row) * K + 8 * (lane >> 4);
   }
-  const bf16_t* wbase = Wp + static_cast<size_t>(nt0) * KT * 512 + lane * 8;
+  // HALF: 8 gate and the 8 up columns that belong to them, half a tile of each, as one operand of 16 rows
+  constexpr bool HALF = EPI == EPI_SWIGLU && NTW == 1;
+  const int pair = blockIdx.x >> 1, hf = blockIdx.x & 1;
+  const bf16_t* wbase = HALF ? Wp + static_cast<size_t>(2 * pair + ((lane >> 3) & 1)) * KT * 512 + (8 * hf + (lane & 7) + 16 * (lane >> 4)) * 8
+                             : Wp + static_cast<size_t>(nt0) * KT * 512 + lane * 8;
 
   auto load = [&](bf16x8 (&wf)[NTW], bf16x8 (&xf)[MT], int kt) {
 #pragma unroll
@@ -63,21 +70,26 @@ __global__ __launch_bounds__(512) void kgemm_kernel(const bf16_t* __restrict__ W
         acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[n], xf[m], acc[n][m], 0, 0, 0);
   };
 
-  // 4-deep register ring, statically indexed (unrolled by 4)
-  bf16x8 w0[NTW], w1[NTW], w2[NTW], w3[NTW], x0[MT], x1[MT], x2[MT], x3[MT];
+  // register ring of four k-tiles, statically indexed (eight or twelve gain nothing: 4096 x 14336 20.5, 20.6, 20.7 us at one row)
+  constexpr int R = 4;
+  bf16x8 wr[R][NTW], xr[R][MT];
+#pragma unroll
+  for (int u = 0; u < R; ++u)
+    if (kt_lo + u < kt_hi) load(wr[u], xr[u], kt_lo + u);
   int kt = kt_lo;
-  if (kt + 0 < kt_hi) load(w0, x0, kt + 0);
-  if (kt + 1 < kt_hi) load(w1, x1, kt + 1);
-  if (kt + 2 < kt_hi) load(w2, x2, kt + 2);
-  for (; kt < kt_hi; kt += 4) {
-    if (kt + 3 < kt_hi) load(w3, x3, kt + 3);
-    fma(w0, x0);
-    if (kt + 4 < kt_hi) load(w0, x0, kt + 4);
-    if (kt + 1 < kt_hi) fma(w1, x1);
-    if (kt + 5 < kt_hi) load(w1, x1, kt + 5);
-    if (kt + 2 < kt_hi) fma(w2, x2);
-    if (kt + 6 < kt_hi) load(w2, x2, kt + 6);
-    if (kt + 3 < kt_hi) fma(w3, x3);
+  for (; kt + 2 * R <= kt_hi; kt += R) {
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      fma(wr[u], xr[u]);
+      load(wr[u], xr[u], kt + R + u);
+    }
+  }
+  for (; kt < kt_hi; kt += R) {
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      if (kt + u < kt_hi) fma(wr[u], xr[u]);
+      if (kt + R + u < kt_hi) load(wr[u], xr[u], kt + R + u);
+    }
   }
 
   // ---- cross-wave reduction through LDS: 8 -> 4 -> 2 -> 1 ----
@@ -96,6 +108,28 @@ __global__ __launch_bounds__(512) void kgemm_kernel(const bf16_t* __restrict__ W
     __syncthreads();
   }
   if (wave != 0) return;
+  if constexpr (HALF) {
+    const int col = 16 * pair + 8 * hf + 4 * (lane >> 4);          // (lanes 0 .. 31: gate rows of the operand)
+    const int gb = 32 * pair + 8 * hf + 4 * (lane >> 4);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float g = acc[0][m][r], u = __shfl(g, lane + 32, 64);
+        const bool in = bias != nullptr && lane < 32 && gb < N;
+        v[r] = silu(g + (in ? bf16_to_f32(bias[gb + r]) : 0.f)) * (u + (in ? bf16_to_f32(bias[gb + 16 + r]) : 0.f));
+      }
+      const int row = 16 * m + (lane & 15);
+      if (lane < 32 && row < M && gb < N) {
+        u32x2 o;
+        o[0] = pack_bf16x2(v[0], v[1]);
+        o[1] = pack_bf16x2(v[2], v[3]);
+        *reinterpret_cast<u32x2*>(static_cast<bf16_t*>(Y) + static_cast<size_t>(row) * ldy + col) = o;
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int n = 0; n < NTW; ++n)
 #pragma unroll
@@ -114,26 +148,20 @@ int launch_k(int epi, const bf16_t* Wp, const bf16_t* X, void* Y, const bf16_t* 
              int ldy, int n_pad, float ap, float an, hipStream_t stream) {
   const dim3 grid(n_pad / (16 * NTW)), block(512);
   const size_t lds = 4 * NTW * MT * 64 * sizeof(f32x4);
-  if (epi == EPI_BF16)
-    kgemm_kernel<MT, NTW, EPI_BF16><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy, ap, an);
-  else if (epi == EPI_F32)
-    kgemm_kernel<MT, NTW, EPI_F32><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy, ap, an);
-  else if (epi == EPI_RELU2)
-    kgemm_kernel<MT, NTW, EPI_RELU2><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy, ap, an);
-  else if (epi == EPI_XIELU)
-    kgemm_kernel<MT, NTW, EPI_XIELU><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy, ap, an);
-  else if (epi != EPI_SWIGLU)
-    return -3;
-  else if constexpr (NTW >= 2)
-    kgemm_kernel<MT, NTW, EPI_SWIGLU><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy, ap, an);
-  else
-    return -3;
+#define LC_KG(E) kgemm_kernel<MT, NTW, E><<<grid, block, lds, stream>>>(Wp, X, Y, bias, M, N, K, ldy, ap, an)
+  if (epi == EPI_BF16) LC_KG(EPI_BF16);
+  else if (epi == EPI_F32) LC_KG(EPI_F32);
+  else if (epi == EPI_RELU2) LC_KG(EPI_RELU2);
+  else if (epi == EPI_XIELU) LC_KG(EPI_XIELU);
+  else if (epi == EPI_SWIGLU) LC_KG(EPI_SWIGLU);
+  else return -3;
+#undef LC_KG
   return static_cast<int>(hipGetLastError());
 }
 
 }  // namespace
 
-// M <= 64, K % 32 == 0, n_pad % 128 == 0. ntw = n-tiles (16 columns) per workgroup: 1, 2 or 4.
+// M <= 64, K % 32 == 0, n_pad % 128 == 0. ntw = n-tiles (16 columns) per workgroup: 1, 2 or 4 (gated, 1: two halves).
 LC_EXPORT int lc_kgemm(const void* Wp, const void* X, void* Y, const void* bias, int M, int N, int K,
                        int n_pad, int ldy, int epi, int ntw, float ap, float an, hipStream_t stream) {
   if (M <= 0) return 0;

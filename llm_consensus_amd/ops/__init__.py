@@ -50,13 +50,12 @@ def set_concurrent_engines(n: int) -> None:
 # In-workgroup K-split decode kernel (kgemm.hip): widest output it is used for, and a test override
 # (-1 = automatic, 0 = never, 1/2/4 = force that many n-tiles per workgroup).
 KGEMM_MAX_N = int(os.environ.get("LC_KGEMM_MAX_N", str(1 << 30)))
-KGEMM_MAX_N_GATED = int(os.environ.get("LC_KGEMM_MAX_N", "8192"))
 # Most rows the in-workgroup K-split kernel is used for. Measured against the panel kernel (with
 # non-temporal weight loads) on HBM-resident weights: at 1 row it wins on the narrow projections
 # (6144x4096 10.9 vs 13.0 us, 4096x4096 7.9 vs 9.3) and on wide ones that are not gated with one
-# n-tile per workgroup (128256x4096 153 vs 179, 32000x2048 21 vs 27, 16384x4096 22 vs 31; the gated
-# 28672x4096 ties); at 8 rows it still wins there, wide ones with two n-tiles (11.9 vs 13.5, 8.4 vs
-# 9.4, 167 vs 181, 22 vs 27), but loses where K is long (3584x18944: 26.5 vs 23.9); at 16 rows it
+# n-tile per workgroup (128256x4096 153 vs 179, 32000x2048 21 vs 27, 16384x4096 22 vs 31); at 8
+# rows it still wins there, wide ones with two n-tiles (11.9 vs 13.5, 8.4 vs 9.4, 167 vs 181, 22 vs
+# 27), but loses where K is long (3584x18944: 26.5 vs 23.9); at 16 rows it
 # loses (4096x14336: 28.3 vs 21.4, 3584x18944: 36.3 vs 24.2, 152064x3584: 184 vs 182) except on
 # wide outputs over a short K (128256x2048 85 vs 102, 16384x2048 13.7 vs 19.3).
 KGEMM_MAX_M = int(os.environ.get("LC_KGEMM_MAX_M", "8"))
@@ -163,14 +162,21 @@ def _kgemm_ntw(n_pad: int, M: int, swiglu: bool, K: int = 0) -> int:
     It re-reads the activations once per workgroup from L2, so it is limited to a few rows."""
     if KGEMM_FORCE_NTW >= 0:
         return KGEMM_FORCE_NTW if M <= 64 else 0
-    wide = n_pad > 8192
-    if n_pad > (KGEMM_MAX_N_GATED if swiglu else KGEMM_MAX_N) or (K > KGEMM_LONG_K and M > KGEMM_LONG_K_MAX_M):
+    wide, tiles = n_pad > 8192, n_pad // 16
+    if n_pad > KGEMM_MAX_N or (K > KGEMM_LONG_K and M > KGEMM_LONG_K_MAX_M):
         return 0
+    if swiglu:
+        # wide gated outputs: halves of two tiles, where they fill whole rounds of the CUs (28672x4096 at 1, 4, 8 rows
+        # 37.0, 37.7, 39.8 us against 45.3, 43.5, 43.2 on the panel kernel; 37888x3584, 9.25 rounds, 44.2, 46.5, 49.8
+        # against 44.6, 44.4, 44.2). Up to 8192 columns whole tiles are as fast (8192x2048 8.1 and 8.5 us).
+        if not wide:
+            return 2 if M <= KGEMM_MAX_M else 0
+        return 1 if M <= KGEMM_MAX_M and tiles >= 0.95 * 256 * ((tiles + 255) // 256) else 0
     if M > KGEMM_MAX_M and not (wide and K <= KGEMM_SHORT_K and M <= KGEMM_SHORT_K_MAX_M):
         return 0
-    if not swiglu and (M <= 4 or n_pad < 8192):
-        return 1
-    return 4 if swiglu and n_pad >= 16384 else 2
+    if 256 < tiles < 384:          # (one tile each would start a second round of the CUs: 4608x3584 at 1 row 9.2 and 8.4 us, 6144x4096 11.1 and 12.0)
+        return 2
+    return 1 if M <= 4 or n_pad < 8192 else 2
 
 
 def _choose_panel_splits(n_pad: int, K: int) -> int:

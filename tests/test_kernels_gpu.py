@@ -154,6 +154,25 @@ def test_kgemm_in_workgroup_ksplit(M, N, K, ntw):
         ops.KGEMM_FORCE_NTW = old
 
 
+@pytest.mark.parametrize("M", [1, 7, 16, 17, 64])
+@pytest.mark.parametrize("N,K", [(128, 64), (224, 192), (8192, 320), (12288, 4096)])
+def test_gated_products_from_halves_of_two_tiles(M, N, K):
+    """One n-tile per workgroup: ragged widths, depths that leave waves without work, two and four row tiles, a bias."""
+    Wg, Wu = bf(rand(N // 2, K, scale=0.3, seed=3)), bf(rand(N // 2, K, scale=0.3, seed=4))
+    X, b = bf(rand(M, K, scale=0.5)), bf(rand(N, seed=5))
+    old, ops.KGEMM_FORCE_NTW = ops.KGEMM_FORCE_NTW, 1
+    try:
+        for bias in (None, b):
+            lw = ops.LinearWeight.from_dense(ops.interleave_gate_up(Wg, Wu), bias, DEV, swiglu=True)
+            g, u = X.float() @ Wg.float().t(), X.float() @ Wu.float().t()
+            if bias is not None:
+                bi = b.float().view(N // 32, 2, 16)
+                g, u = g + bi[:, 0].reshape(-1), u + bi[:, 1].reshape(-1)
+            assert rel_err(ops.linear(X.to(DEV), lw), torch.nn.functional.silu(g) * u) < 8e-3
+    finally:
+        ops.KGEMM_FORCE_NTW = old
+
+
 @pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16, 17])
 @pytest.mark.parametrize("N,K", [(8192, 64), (8200, 2048), (8320, 2112)])
 def test_few_rows_against_outputs_around_the_rule_for_wide_ones(M, N, K):
