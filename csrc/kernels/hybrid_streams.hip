@@ -241,13 +241,14 @@ __global__ __launch_bounds__(256) void hc_step4_kernel(float* __restrict__ xs, c
 }
 
 // ---------------------------------------------------------------- rotary positions on q, k and v; cache write
-// One block per token. qkv [T, ld] fp32: q [H*D] | k [G*D] | v [G*Dv] (biases already added by the product). The
+// One block per token (of few tokens a wider one: 4 of them 10 us with 256 threads and 4.7 us with 1024). qkv [T, ld] fp32:
+// q [H*D] | k [G*D] | v [G*Dv] (biases already added by the product). The
 // first rot_dims coordinates of every query and key head turn by position * inv_freq[i] in the pair layout
 // ``pairs`` (0: i with i + rot_dims / 2; 1: neighbours); with ``inv_freq_v`` every value head turns over its whole
 // width by position * inv_freq_v[m] in the layout ``v_pairs``, and is cached so. Keys go to [blocks, G, BS, D],
 // values to [blocks, G, BS, Dv] at the token's slot; the turned queries to q_out [T, H*D].
 template <bool CF32>
-__global__ __launch_bounds__(256) void rope_qkv_write_kernel(
+__global__ __launch_bounds__(1024) void rope_qkv_write_kernel(
     const float* __restrict__ qkv, int ld, const double* __restrict__ inv_freq, const double* __restrict__ inv_freq_v,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ slot_mapping, void* __restrict__ kc,
     void* __restrict__ vc, float* __restrict__ q_out, int H, int G, int D, int Dv, int BS, int rot_dims, int pairs,
@@ -285,33 +286,56 @@ __global__ __launch_bounds__(256) void rope_qkv_write_kernel(
 }
 
 // ---------------------------------------------------------------- mixed heads' weights behind the weighted sums
-// One block per token. o [T, H, G, Dv] fp32: head g's softmax weights applied to the values of EVERY key/value head
+// o [T, H, G, Dv] fp32: head g's softmax weights applied to the values of EVERY key/value head
 // c. Mixing the weights of the heads by talk [H, H] before they meet the values is linear in them, so it is done
 // on these sums: out[t, h, :] = sum_g talk[h, g] o[t, g, kv(h), :] with kv(h) = h / (H / G). With ``inv_freq_v``
 // the result turns back by -position * inv_freq_v[m] over its whole width (values cached turned by their own
 // position leave a sum that depends on position differences only).
-template <bool AF32>
+// A block per token and up to ``heads`` heads of a key/value head: they read the same sums and share one table of angles (fp64).
+// Bound by reading o once (V = 4: 16 bytes per thread, eight rows of it in flight). A block per head, 4 bytes at a time, took
+// 73 us for 2361 tokens of 16 heads over 4 of width 128 (77 MB); this one 20 us.
+template <bool AF32, int V>
 __global__ __launch_bounds__(256) void talk_mix_kernel(const float* __restrict__ o, const float* __restrict__ talk,
                                                        const int32_t* __restrict__ positions,
                                                        const double* __restrict__ inv_freq_v, void* __restrict__ out, int H,
-                                                       int G, int Dv, int v_pairs) {
-  extern __shared__ float lds_tm[];                // mixed [Dv], then cos / sin [Dv]
-  const int t = blockIdx.x, h = blockIdx.y;        // a block per (token, head)
+                                                       int G, int Dv, int v_pairs, int heads) {
+  extern __shared__ float lds_tm[];                // mixed [heads][Dv], then cos / sin [Dv]
+  const int rep = H / G, groups = (rep + heads - 1) / heads;
+  const int t = blockIdx.x, kv = blockIdx.y / groups, first = (blockIdx.y % groups) * heads;
+  const int n = min(heads, rep - first), h0 = kv * rep + first;
   float* mixed = lds_tm;
-  float* cs = lds_tm + Dv;
+  float* cs = lds_tm + heads * Dv;
   if (inv_freq_v != nullptr) angle_table(cs, Dv >> 1, static_cast<double>(positions[t]), inv_freq_v);
-  const int kv = h / (H / G);
   const float* ot = o + (static_cast<size_t>(t) * H * G + kv) * Dv;
-  for (int c = threadIdx.x; c < Dv; c += blockDim.x) {
-    float a = 0.f;
-    for (int g = 0; g < H; ++g) a += talk[h * H + g] * ot[static_cast<size_t>(g) * G * Dv + c];
-    mixed[c] = a;
+  const int pieces = Dv / V;
+  for (int i = threadIdx.x; i < n * pieces; i += blockDim.x) {
+    const int j = i / pieces, c = (i - j * pieces) * V;
+    const float* row = talk + static_cast<size_t>(h0 + j) * H;
+    float a[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) a[e] = 0.f;
+#pragma unroll 8
+    for (int g = 0; g < H; ++g) {
+      const float* src = ot + static_cast<size_t>(g) * G * Dv + c;
+      if constexpr (V == 4) {
+        const float4 v = *reinterpret_cast<const float4*>(src);
+        a[0] += row[g] * v.x;
+        a[1] += row[g] * v.y;
+        a[2] += row[g] * v.z;
+        a[3] += row[g] * v.w;
+      } else {
+        a[0] += row[g] * src[0];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < V; ++e) mixed[j * Dv + c + e] = a[e];
   }
   __syncthreads();
   typename Act<AF32>::type* dst = static_cast<typename Act<AF32>::type*>(out);
-  for (int c = threadIdx.x; c < Dv; c += blockDim.x) {
-    const float r = inv_freq_v != nullptr ? turned(mixed, c, Dv, cs, v_pairs, -1.f) : mixed[c];
-    Act<AF32>::store(dst, (static_cast<size_t>(t) * H + h) * Dv + c, r);
+  for (int i = threadIdx.x; i < n * Dv; i += blockDim.x) {
+    const int j = i / Dv, c = i - j * Dv;
+    const float r = inv_freq_v != nullptr ? turned(mixed + j * Dv, c, Dv, cs, v_pairs, -1.f) : mixed[i];
+    Act<AF32>::store(dst, (static_cast<size_t>(t) * H + h0 + j) * Dv + c, r);
   }
 }
 
@@ -322,7 +346,7 @@ __global__ __launch_bounds__(256) void talk_mix_kernel(const float* __restrict__
 // the turned query parts go to columns R .. R + rd - 1 of each head's block of qlat [T, H * (R + rd)], whose first R
 // columns per head (the query in the compressed row's coordinates) another launch writes.
 template <bool CF32>
-__global__ __launch_bounds__(256) void latent_rope_write_kernel(
+__global__ __launch_bounds__(1024) void latent_rope_write_kernel(
     const float* __restrict__ proj, int ld, int col_c, const float* __restrict__ w, float eps,
     const double* __restrict__ inv_freq, const int32_t* __restrict__ positions, const int32_t* __restrict__ slot_mapping,
     void* __restrict__ cache, float* __restrict__ qlat, int H, int D, int R, int rd, int BS, int pairs) {
@@ -423,7 +447,7 @@ LC_EXPORT int lc_rope_qkv_write(const void* qkv, int ld, const void* inv_freq, c
   const size_t lds = static_cast<size_t>(rot_dims + Dv + 1) * sizeof(float);
   if (lds > 64 * 1024) return -1;
 #define LC_RQ(C32)                                                                                                   \
-  rope_qkv_write_kernel<C32><<<dim3(T), dim3(256), lds, st>>>(                                                       \
+  rope_qkv_write_kernel<C32><<<dim3(T), dim3(row_block_threads(T, H * D)), lds, st>>>(                                                       \
       static_cast<const float*>(qkv), ld, static_cast<const double*>(inv_freq), static_cast<const double*>(inv_freq_v), \
       static_cast<const int32_t*>(positions), static_cast<const int32_t*>(slot_mapping), kc, vc,                     \
       static_cast<float*>(q_out), H, G, D, Dv, BS, rot_dims, pairs, v_pairs)
@@ -438,15 +462,20 @@ LC_EXPORT int lc_talk_mix(const void* o, const void* talk, const void* positions
   if (T <= 0) return 0;
   if (H <= 0 || G <= 0 || H % G || Dv <= 0 || o == nullptr || talk == nullptr || out == nullptr) return -1;
   if (inv_freq_v != nullptr && ((Dv & 1) || positions == nullptr)) return -1;
-  const size_t lds = static_cast<size_t>(2 * Dv + 1) * sizeof(float);
-  if (lds > 64 * 1024 || H > 65535) return -1;
-  const int threads = Dv <= 64 ? 64 : (Dv <= 128 ? 128 : 256);
-#define LC_TM(A32)                                                                                               \
-  talk_mix_kernel<A32><<<dim3(T, H), dim3(threads), lds, st>>>(static_cast<const float*>(o), static_cast<const float*>(talk), \
-                                                        static_cast<const int32_t*>(positions),                  \
-                                                        static_cast<const double*>(inv_freq_v), out, H, G, Dv, v_pairs)
-  if (act_f32) LC_TM(true);
-  else LC_TM(false);
+  if (static_cast<size_t>(2 * Dv + 1) * sizeof(float) > 64 * 1024 || H > 65535) return -1;
+  const int rep = H / G, heads = 5 * Dv * sizeof(float) <= 64 * 1024 ? (rep < 4 ? rep : 4) : 1;
+  const size_t lds = static_cast<size_t>(heads + 1) * Dv * sizeof(float);
+  const bool vec = Dv % 4 == 0 && aligned16(o);
+  const int items = heads * (vec ? Dv / 4 : Dv), threads = items <= 64 ? 64 : items <= 128 ? 128 : 256;
+  const dim3 grid(T, G * ((rep + heads - 1) / heads));
+#define LC_TM(A32, V)                                                                                               \
+  talk_mix_kernel<A32, V><<<grid, dim3(threads), lds, st>>>(static_cast<const float*>(o), static_cast<const float*>(talk), \
+                                                            static_cast<const int32_t*>(positions),                 \
+                                                            static_cast<const double*>(inv_freq_v), out, H, G, Dv, v_pairs, heads)
+  if (act_f32 && vec) LC_TM(true, 4);
+  else if (act_f32) LC_TM(true, 1);
+  else if (vec) LC_TM(false, 4);
+  else LC_TM(false, 1);
 #undef LC_TM
   LC_RETURN_LAST_ERROR();
 }
@@ -461,7 +490,7 @@ LC_EXPORT int lc_latent_rope_write(const void* proj, int ld, int col_c, const vo
   const size_t lds = static_cast<size_t>(rd + 1) * sizeof(float);
   if (lds > 64 * 1024) return -1;
 #define LC_LR(C32)                                                                                                  \
-  latent_rope_write_kernel<C32><<<dim3(T), dim3(256), lds, st>>>(                                                   \
+  latent_rope_write_kernel<C32><<<dim3(T), dim3(row_block_threads(T, H * rd + R)), lds, st>>>(                                                   \
       static_cast<const float*>(proj), ld, col_c, static_cast<const float*>(w), eps, static_cast<const double*>(inv_freq), \
       static_cast<const int32_t*>(positions), static_cast<const int32_t*>(slot_mapping), cache,                     \
       static_cast<float*>(qlat), H, D, R, rd, BS, pairs)

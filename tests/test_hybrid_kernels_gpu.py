@@ -1203,3 +1203,16 @@ def test_split_products_of_any_shape(M, N, K, adt):
     assert isinstance(y, ops.PartialSum) and tuple(y.shape) == (M, N)
     want = (x.double() @ W.double().T).float()
     torch.testing.assert_close(y.part.sum(0).cpu(), want, atol=2e-5, rtol=1e-5)      # (fp32 sums of a few thousand terms around 1/64)
+
+
+@pytest.mark.parametrize("H,G,Dv", [(1, 1, 2), (3, 3, 70), (5, 1, 64), (8, 2, 132), (18, 2, 256), (4, 1, 4000)])
+def test_mixed_heads_in_blocks_of_up_to_four(H, G, Dv):
+    """Heads of a key head that leave a block partly empty, widths that are no multiple of four, blocks of a single head."""
+    g = torch.Generator().manual_seed(H * Dv)
+    T = 5
+    o, talk, pos = torch.randn(T, H * G * Dv, generator=g), torch.randn(H, H, generator=g) / H ** 0.5, torch.arange(T, dtype=torch.int32) * 7
+    inv = 1e4 ** (-torch.arange(Dv // 2, dtype=torch.float64) / (Dv // 2))
+    for f, pairs in ((None, False), (inv, False), (inv, True)):
+        want = ref.talk_mix(o, talk, pos, f, H, G, Dv, torch.float32, pairs)
+        got = ops.talk_mix(o.to(DEV), talk.to(DEV), pos.to(DEV), None if f is None else f.to(DEV), H, G, Dv, torch.float32, pairs)
+        torch.testing.assert_close(got.cpu(), want, atol=2e-5, rtol=1e-5)
