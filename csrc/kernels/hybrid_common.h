@@ -80,6 +80,8 @@ struct ConvIn {
   long long state_stride;
   int C;
   int vec;                       // every row of x, of the state and of the weights starts on a 16-byte border
+  int parts;                     // without taps x may be as many slabs, ``slab`` elements apart, whose sum is the input
+  size_t slab;
 };
 
 inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
@@ -139,7 +141,15 @@ LC_DEVICE void conv_token(const ConvIn& a, const RowSeq& s, const float* st, int
   } else if (a.vec && a.taps == 4) {
     conv_rows4<4, SILU>(a, s, st, r, u);
   } else if (a.vec && a.taps == 0 && !SILU) {
-    for (int c = threadIdx.x * 4; c < a.C; c += 4 * blockDim.x) *reinterpret_cast<float4*>(u + c) = *reinterpret_cast<const float4*>(row + c);
+    for (int c = threadIdx.x * 4; c < a.C; c += 4 * blockDim.x) {
+      float4 v = *reinterpret_cast<const float4*>(row + c);
+#pragma unroll 8
+      for (int p = 1; p < a.parts; ++p) {              // (several slabs in flight)
+        const float4 x = *reinterpret_cast<const float4*>(row + p * a.slab + c);
+        v = make_float4(v.x + x.x, v.y + x.y, v.z + x.z, v.w + x.w);
+      }
+      *reinterpret_cast<float4*>(u + c) = v;
+    }
   } else if (a.taps > 0) {
     for (int c = threadIdx.x; c < a.C; c += blockDim.x) {
       float y = 0.f;
@@ -153,7 +163,11 @@ LC_DEVICE void conv_token(const ConvIn& a, const RowSeq& s, const float* st, int
       u[c] = conv_act<SILU>(y);
     }
   } else {
-    for (int c = threadIdx.x; c < a.C; c += blockDim.x) u[c] = conv_act<SILU>(row[c]);
+    for (int c = threadIdx.x; c < a.C; c += blockDim.x) {
+      float v = row[c];
+      for (int p = 1; p < a.parts; ++p) v += row[p * a.slab + c];
+      u[c] = conv_act<SILU>(v);
+    }
   }
 }
 

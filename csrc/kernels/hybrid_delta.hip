@@ -614,7 +614,7 @@ LC_EXPORT int lc_delta_prep(const void* proj, int ld, const void* conv_w, int ta
                               static_cast<int>(kMaxLds));
   });
   const ConvIn in{static_cast<const float*>(proj), ld, static_cast<const float*>(conv_w), taps, static_cast<float*>(state),
-                  state_stride, C, conv_vec(proj, ld, conv_w, state, state_stride, C)};
+                  state_stride, C, conv_vec(proj, ld, conv_w, state, state_stride, C), 1, 0};
   const DeltaPrepArgs a{in, col_b, col_a, static_cast<const float*>(neg_rate), static_cast<const float*>(dt_bias),
                         static_cast<const int32_t*>(row_seq), static_cast<const int32_t*>(cu_q),
                         static_cast<const int32_t*>(positions), static_cast<const int32_t*>(slots), static_cast<float*>(qk),

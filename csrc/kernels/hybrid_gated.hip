@@ -450,7 +450,8 @@ LC_EXPORT int lc_token_shift(const void* h, const void* mu, void* state, long lo
   LC_RETURN_LAST_ERROR();
 }
 
-LC_EXPORT int lc_attn_prep(const void* qkv, int ld, const void* conv_w, int taps, void* state, long long state_stride,
+// qkv: ``parts`` slabs of [T, ld] (more than one without taps only).
+LC_EXPORT int lc_attn_prep(const void* qkv, int parts, int ld, const void* conv_w, int taps, void* state, long long state_stride,
                            int norm, const void* qn, const void* kn, float eps, const void* inv_freq, int rot_dims, int pairs,
                            float rot_mag, int maps, float t_coef, float t_every, const void* v_first, int ld_vf, float lambda, void* v_save,
                            const void* row_seq, const void* cu_q, const void* positions, const void* slots,
@@ -458,7 +459,7 @@ LC_EXPORT int lc_attn_prep(const void* qkv, int ld, const void* conv_w, int taps
                            int D, int Dv, int BS, hipStream_t st) {
   if (T <= 0) return 0;
   if (H <= 0 || G <= 0 || H % G || D <= 0 || Dv <= 0 || BS <= 0 || kc == nullptr || vc == nullptr || q_out == nullptr) return -1;
-  if (maps <= 0 || G % maps) return -1;
+  if (maps <= 0 || G % maps || parts < 1 || (parts > 1 && taps != 0)) return -1;
   const int GV = G / maps, C = (H + G) * D + GV * Dv;
   if (ld < C || taps < 0 || norm < 0 || norm > 2 || (norm != 0 && (qn == nullptr || kn == nullptr))) return -1;
   if (taps > 0 && conv_w == nullptr) return -1;
@@ -478,7 +479,7 @@ LC_EXPORT int lc_attn_prep(const void* qkv, int ld, const void* conv_w, int taps
                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kMaxLds));
   });
   const ConvIn in{static_cast<const float*>(qkv), ld, static_cast<const float*>(conv_w), taps, static_cast<float*>(state),
-                  state_stride, C, conv_vec(qkv, ld, conv_w, state, state_stride, C)};
+                  state_stride, C, conv_vec(qkv, ld, conv_w, state, state_stride, C), parts, static_cast<size_t>(T) * ld};
   const PrepArgs a{in, norm, static_cast<const float*>(qn), static_cast<const float*>(kn), eps,
                    static_cast<const double*>(inv_freq), rot_dims, pairs, rot_mag, t_coef, static_cast<double>(t_every),
                    static_cast<const float*>(v_first), ld_vf, lambda, static_cast<float*>(v_save),

@@ -1689,7 +1689,7 @@ class HybridModel:
         l = L.spec
         M, D, Dv = l.maps, l.dim, l.vdim
         kc, vc = cache.k(r), cache.v(r)
-        qkv = ops.linear(xa, L.proj, out_f32=True)
+        qkv = ops.linear(xa, L.proj, out_f32=True, defer_reduce=True)
         q, _ = ops.attn_prep(qkv, positions, slot_mapping, lay, kc, vc, l.heads * M, l.kv_heads * M, D, Dv, inv_freq=L.inv_freq,
                              rot_dims=l.rot_dims, pairs=True, rot_mag=L.rot_mag, maps=M)
         a = ops.attn_masked(q, kc, vc, lay.block_tables, lay.cu_q, lay.row_seq, positions, l.heads * M, l.kv_heads * M, D, Dv,

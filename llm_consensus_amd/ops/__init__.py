@@ -1933,8 +1933,12 @@ def attn_prep(qkv: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Te
     [T, G Dv]) by ``v_mix``. Returns (q fp32 [T, H D], the values before the mix when ``save_v``).
     ``maps`` > 1: every head has that many query and key maps over one value: q and k are laid out head by head, map by
     map, H and G count the maps of all heads, the value heads are G / maps, and the queries are returned in the order
-    (key/value head, map, head of the group): the H / G queries of a key map side by side."""
-    T = qkv.shape[0]
+    (key/value head, map, head of the group): the H / G queries of a key map side by side. qkv may be a ``PartialSum``, whose
+    slabs are summed on the way when it has neither a bias nor a convolution."""
+    if isinstance(qkv, PartialSum) and (conv_w is not None or qkv.bias is not None):
+        qkv = qkv.reduce(out_f32=True)
+    qkv, parts = (qkv.part.flatten(0, 1), qkv.part.shape[0]) if isinstance(qkv, PartialSum) else (qkv, 1)      # (slabs: one below the other)
+    T = qkv.shape[0] // parts
     if maps < 1 or G % maps:
         raise ValueError("attn_prep: every head has the same number of maps")
     GV = G // maps
@@ -1965,7 +1969,7 @@ def attn_prep(qkv: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Te
     q = torch.empty(T, H * D, dtype=torch.float32, device=qkv.device)
     vs = torch.empty(T, GV * Dv, dtype=torch.float32, device=qkv.device) if save_v else None
     p = _hip().ptr
-    _hip().call("lc_attn_prep", qkv.data_ptr(), max(qkv.stride(0), qkv.shape[1]), p(conv_w), taps,
+    _hip().call("lc_attn_prep", qkv.data_ptr(), parts, max(qkv.stride(0), qkv.shape[1]), p(conv_w), taps,
                 p(conv_state) if taps > 1 else None, max(conv_state.stride(0), conv_state.shape[1]) if taps > 1 else 0,
                 ("", "whole", "head").index(norm), p(q_norm), p(k_norm), float(eps), p(inv_freq), int(rot_dims),
                 1 if pairs else 0, float(rot_mag), int(maps), float(temperature[0]), float(temperature[1]), p(v_first),

@@ -96,7 +96,7 @@ _SIGNATURES = {
     # gated residual steps, token shifts, attention pre-processing with convolutions and mixed values (hybrid_gated.hip)
     "lc_gated_step": [_P, _P, _I, _P, _P, _I, _P, _P, _F, _P, _P, _P, _P, _I, _I, _I, _P, _P, _L, _P, _P, _P, _P, _I, _I, _P],
     "lc_token_shift": [_P, _P, _P, _L, _P, _P, _P, _P, _P, _I, _I, _I, _P],
-    "lc_attn_prep": [_P, _I, _P, _I, _P, _L, _I, _P, _P, _F, _P, _I, _I, _F, _I, _F, _F, _P, _I, _F, _P, _P, _P, _P, _P, _P, _P, _P,
+    "lc_attn_prep": [_P, _I, _I, _P, _I, _P, _L, _I, _P, _P, _F, _P, _I, _I, _F, _I, _F, _F, _P, _I, _F, _P, _P, _P, _P, _P, _P, _P, _P,
                      _I, _P, _I, _I, _I, _I, _I, _I, _P],
     "lc_softcap": [_P, _L, _F, _P],
     "lc_lightning_scan": [_P, _I, _P, _P, _L, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P],

@@ -1216,3 +1216,24 @@ def test_mixed_heads_in_blocks_of_up_to_four(H, G, Dv):
         want = ref.talk_mix(o, talk, pos, f, H, G, Dv, torch.float32, pairs)
         got = ops.talk_mix(o.to(DEV), talk.to(DEV), pos.to(DEV), None if f is None else f.to(DEV), H, G, Dv, torch.float32, pairs)
         torch.testing.assert_close(got.cpu(), want, atol=2e-5, rtol=1e-5)
+
+
+@pytest.mark.parametrize("H,G,D,Dv,rot", [(4, 2, 32, 64, 16), (5, 5, 7, 6, 2)])
+@pytest.mark.parametrize("T", [1, 33, 520])
+def test_attention_inputs_from_the_slabs_of_a_split_product(H, G, D, Dv, rot, T):
+    g = torch.Generator().manual_seed(T + D)
+    C = (H + G) * D + G * Dv
+    part = torch.randn(5, T, C, generator=g).to(DEV)
+    pos = torch.arange(T, dtype=torch.int32, device=DEV)
+    inv = torch.tensor([1e3 ** (-2.0 * j / rot) for j in range(rot // 2)], dtype=torch.float64, device=DEV)
+    lay = _Layout(torch.tensor([0, T], dtype=torch.int32), torch.zeros(T, dtype=torch.int32), torch.zeros(1, dtype=torch.int32), DEV)
+    res = []
+    forms = [part[0] + part[1] + part[2] + part[3] + part[4], ops.PartialSum(part)]
+    if C % 32 == 0:                                          # (whole groups of columns: a bias makes it a reduction of its own)
+        forms.append(ops.PartialSum(part, torch.zeros(C, dtype=torch.bfloat16, device=DEV)))
+    for qkv in forms:
+        k, v = torch.zeros(T // 16 + 1, G, 16, D, device=DEV), torch.zeros(T // 16 + 1, G, 16, Dv, device=DEV)
+        res.append((ops.attn_prep(qkv, pos, pos, lay, k, v, H, G, D, Dv, inv_freq=inv, rot_dims=rot)[0], k, v))
+    for want, *got in zip(*res):
+        for x in got:
+            torch.testing.assert_close(x, want, atol=2e-6, rtol=1e-6)      # (five fp32 numbers added in the same order)
