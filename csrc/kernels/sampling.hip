@@ -160,7 +160,7 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(
     for (int u = 0; u < kQuads; ++u)
 #pragma unroll
       for (int q = 0; q < 4; ++q) m = fmaxf(m, v[u][q] * inv_t);
-    if (m > am.v) {
+    if (m > am.v || (m == -INFINITY && am.i == 0x7fffffff)) {       // (the first -inf where there is nothing else)
       run_s = am.v > -INFINITY ? run_s * __expf(am.v - m) : 0.f;
       int at = 0x7fffffff;
 #pragma unroll
