@@ -249,6 +249,22 @@ def use_wide_panel(M: int, n_pad: int, k: int) -> bool:
             and (n_pad // 16 + 9) // 10 <= 256 and _choose_panel_splits(n_pad, k) == 1)
 
 
+def _remainder_tiles(M: int, w: LinearWeight) -> Tuple[int, int]:
+    """(columns of 256 x 256 tiles, parts of their depth) that a product of just over a whole number of rounds of the 256 CUs
+    leaves to a second launch, or (0, 1). Up to 16 tiles in parts of the depth take a fraction of the nearly empty round they
+    would hold up, the launch that sums the parts included (2811 x 6144 x 4096, 264 tiles: 161 -> 133 us, fp32 171 -> 138; 2048 x
+    8448 x 2048 90 -> 83 us, fp32 98 -> 86; 260 tiles 86 -> 74 us); with 24 (280 tiles) or behind two rounds (528) nothing is
+    gained (87 -> 89, 140 -> 139 us)."""
+    m_tiles, n_tiles = (M + 255) // 256, w.n_pad // 256
+    tiles, steps = m_tiles * n_tiles, w.k // 64
+    over = tiles - 256
+    if not 0 < over <= 16 or steps < 32:
+        return 0, 1
+    rest = (over + m_tiles - 1) // m_tiles
+    best = max(s for s in (1, 2, 4, 8, 16) if steps % s == 0 and steps // s >= 4 and (s == 1 or rest * m_tiles * s <= 256))
+    return (rest, best) if best >= 4 and rest < n_tiles and w.n > 256 * (n_tiles - rest) else (0, 1)
+
+
 def linear(x: torch.Tensor, w: LinearWeight, out_f32: bool = False, defer_reduce: bool = False):
     """y = x @ W^T (+bias). With ``w.swiglu`` returns silu(gate)*up of width N/2. With
     ``defer_reduce`` a split-K product may come back as a ``PartialSum``."""
@@ -293,8 +309,17 @@ def linear(x: torch.Tensor, w: LinearWeight, out_f32: bool = False, defer_reduce
                 h.call("lc_gemm256w", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad,
                        out_n, epi)
             else:
-                h.call("lc_gemm256", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad,
+                rest, splits = _remainder_tiles(M, w) if not w.swiglu and w.n % 32 == 0 else (0, 1)
+                n_main = w.n_pad - 256 * rest
+                h.call("lc_gemm256", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, min(w.n, n_main), w.k, n_main,
                        out_n, epi, 0.0, 0.0)
+                if rest:
+                    n = w.n - n_main
+                    part = torch.empty(splits, M, n, dtype=torch.float32, device=x.device)
+                    h.call("lc_gemm256_splitk", w.data.data_ptr() + 2 * n_main * w.k, x.data_ptr(), part.data_ptr(), M, n, w.k,
+                           256 * rest, n, splits)
+                    h.call("lc_splitk_reduce", part.data_ptr(), h.ptr(w.bias[n_main:] if w.bias is not None else None),
+                           y.data_ptr() + n_main * y.element_size(), splits, M, n, out_n, 1 if out_f32 else 0)
             return y
         h.call("lc_gemm_tile", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad,
                out_n, epi)

@@ -154,6 +154,19 @@ def test_kgemm_in_workgroup_ksplit(M, N, K, ntw):
         ops.KGEMM_FORCE_NTW = old
 
 
+@pytest.mark.parametrize("M,N,K", [(2048, 8448, 2048), (2100, 7424, 2048), (300, 33024, 2048), (1025, 13280, 2048)])
+def test_products_of_just_over_a_round_of_tiles(M, N, K):
+    """The tiles of the last, nearly empty round run with their depth split: ragged rows and columns, both types, a bias."""
+    X, W, b = bf(rand(M, K, scale=0.5)), bf(rand(N, K, scale=0.5, seed=1)), bf(rand(N, seed=2))
+    w0, w1 = ops.LinearWeight.from_dense(W, None, DEV), ops.LinearWeight.from_dense(W, b, DEV)
+    assert ops._remainder_tiles(M, w0)[0] >= 1
+    x = X.to(DEV)
+    want = torch.cat([x.float() @ W[i:i + 4096].to(DEV).float().t() for i in range(0, N, 4096)], 1)
+    for lw, ref_ in ((w0, want), (w1, want + b.to(DEV).float())):
+        assert rel_err(ops.linear(x, lw), ref_) < 6e-3
+        assert rel_err(ops.linear(x, lw, out_f32=True), ref_) < 1e-4
+
+
 @pytest.mark.parametrize("M", [1, 7, 16, 17, 64])
 @pytest.mark.parametrize("N,K", [(128, 64), (224, 192), (8192, 320), (12288, 4096)])
 def test_gated_products_from_halves_of_two_tiles(M, N, K):
