@@ -29,10 +29,10 @@ constexpr int GT_BN = 128, GT_BM = 128, GT_BK = 64;
 constexpr int GT_STAGE_BYTES = 32 * 1024;
 
 LC_DEVICE void gt_stage(char* stage, const bf16_t* __restrict__ Wp, const bf16_t* __restrict__ X,
-                        int nt0, int m0, int m_hi, const int32_t* __restrict__ row_index, int kt0, int KT,
+                        int nt0, int m0, int m_hi, int kt0, int KT,
                         int K, int wave, int lane) {
   // 32 one-KiB pieces per stage, 8 per wave: pieces [0,16) are W, [16,32) are X.
-  // X rows are clamped to m_hi-1 (tail tiles) and optionally gathered through row_index.
+  // X rows are clamped to m_hi-1 (tail tiles).
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int p = wave * 8 + i;
@@ -46,7 +46,6 @@ LC_DEVICE void gt_stage(char* stage, const bf16_t* __restrict__ Wp, const bf16_t
       const int mt = q >> 1, kt = q & 1;
       int row = m0 + mt * 16 + (lane & 15);
       row = row < m_hi ? row : m_hi - 1;
-      if (row_index) row = row_index[row];
       const bf16_t* src = X + static_cast<size_t>(row) * K + (kt0 + kt) * 32 + 8 * (lane >> 4);
       __builtin_amdgcn_global_load_lds(LC_GLOBAL_PTR(src), LC_LDS_PTR(dst), 16, 0, 0);
     }
@@ -82,13 +81,13 @@ __global__ __launch_bounds__(256) void gemm_tile_kernel(const bf16_t* __restrict
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  gt_stage(smem, Wp, X, nt0, m0, M, nullptr, 0, KT, K, wave, lane);
+  gt_stage(smem, Wp, X, nt0, m0, M, 0, KT, K, wave, lane);
   __syncthreads();  // emits s_waitcnt vmcnt(0) for the LDS-DMA before the barrier
 
   for (int t = 0; t < nk; ++t) {
     char* cur = smem + (t & 1) * GT_STAGE_BYTES;
     if (t + 1 < nk)
-      gt_stage(smem + ((t + 1) & 1) * GT_STAGE_BYTES, Wp, X, nt0, m0, M, nullptr, (t + 1) * 2, KT, K, wave, lane);
+      gt_stage(smem + ((t + 1) & 1) * GT_STAGE_BYTES, Wp, X, nt0, m0, M, (t + 1) * 2, KT, K, wave, lane);
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) {
       bf16x8 a[4], b[4];
@@ -123,88 +122,165 @@ __global__ __launch_bounds__(256) void gemm_tile_kernel(const bf16_t* __restrict
 
 
 // ---------------------------------------------------------------------------------
-// Grouped (MoE) variant of the tile kernel: rows [offsets[e], offsets[e+1]) of the
-// expert-sorted activation matrix multiply expert e's packed weights. Blocks are laid
-// out as (m-tile slot, n-tile); a block finds its expert by walking the E+1 offsets and
-// exits if its slot is past the last used tile. `row_index` (optional) gathers source
-// rows, so the permutation of tokens into expert order never materialises a copy.
+// Grouped (MoE) products: rows [offsets[e], offsets[e+1]) of the expert-sorted activation matrix multiply expert e's packed
+// weights. `row_index` (optional) gathers source rows, so the permutation of tokens into expert order never
+// materialises a copy.
+//
+// Many small experts (a hundred or two rows each against a few MB of weights) are bound by the weights' way from HBM, and
+// what has to be hidden is its latency: a tile's depth is only 8 to 32 K-tiles long. Block tile 128(n) x BM(m) x 64(k), a wave
+// per 32 columns and 64 rows; both operands go through a ring of three LDS stages filled by LDS-DMA two K-tiles ahead, one barrier
+// per K-tile, and the requests are never drained inside the loop. The two loops that were here before waited for every K-tile's
+// requests at its end and fetched the activations as half lines.
+//
+// One MI355X, 32 experts of 512 x 2048 / 2048 x 512 (67 MB each way, 11 us at 6 TB/s), before and now: 6000 routed rows up 82 -> 29 us,
+// down (fp32 out, 49 MB) 59 -> 33; 800 rows 63 -> 18 and 25 -> 15; 16384 rows 99 -> 40 and 114 -> 66.
 // ---------------------------------------------------------------------------------
-template <int EPI>
-__global__ __launch_bounds__(256) void gemm_grouped_kernel(const bf16_t* __restrict__ Wp_all,
-                                                           long long expert_stride,
-                                                           const bf16_t* __restrict__ X,
-                                                           const int32_t* __restrict__ row_index,
-                                                           const int32_t* __restrict__ offsets, int E,
-                                                           void* __restrict__ Y, int N, int K, int ldy,
-                                                           int tiles_n, GluClamp glu) {
+constexpr int GG_BN = 128, GG_BK = 64;
+
+// Rows of a block tile, and stages of its ring (two workgroups a CU either way, 72 or 64 KiB). 64 rows (four waves) while the launch
+// has a place on the CUs for every workgroup at once: the depth is a chain then, and shorter for small tiles (6000 rows up, 384
+// workgroups: 29 us against 32). 128 rows (eight waves) beyond, where experts fill them: half as many readings of the weights
+// (6000 rows down, 1536 workgroups of 64 rows: 39 us against 33; 8000 rows 51 and 36).
+static inline int gg_rows(int rows, int E, int tiles_n) {
+  const long long tiles = (static_cast<long long>(rows) + 64 * E - 1) / (64 * E) * E * tiles_n;
+  return rows > 100ll * E && tiles > 512 ? 128 : 64;
+}
+constexpr int gg_stages(int bm) { return bm == 128 ? 2 : 3; }
+constexpr int GG_W_BYTES = GG_BN * GG_BK * 2;
+
+// Whose tile a block has: the experts' row tiles are numbered through all experts, n-tiles inside a row tile, and every XCD gets a
+// contiguous run of them (blocks b and b + 8 share one), so that an expert's weights are read into one L2 and its
+// rows as well. The lanes of a wave look at 64 experts at a time: a walk over the offsets is a chain of loads that costs more than
+// the K-tiles of a small expert.
+template <int BM>
+LC_DEVICE bool gg_find(const int32_t* __restrict__ offsets, int E, int tiles_n, int lane, int& e, int& m0, int& m_hi, int& tn) {
+  int used = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int x = e0 + lane;
+    int n = x < E ? (offsets[x + 1] - offsets[x] + BM - 1) / BM : 0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+    used += n;
+  }
+  const int nwg = __builtin_amdgcn_readfirstlane(used) * tiles_n, orig = blockIdx.x;
+  if (orig >= nwg) return false;
+  const int xcd = orig & 7, q = nwg >> 3, r = nwg & 7;
+  const int tile = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (orig >> 3);
+  int slot = tile / tiles_n;
+  tn = tile % tiles_n;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int x = e0 + lane;
+    const int lo = x < E ? offsets[x] : 0, hi = x < E ? offsets[x + 1] : 0;
+    const int n = (hi - lo + BM - 1) / BM;
+    int end = n;                                    // row tiles up to and including this expert's
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int before = __shfl_up(end, off, 64);
+      if (lane >= off) end += before;
+    }
+    const uint64_t here = __ballot(end > slot);
+    if (here != 0) {
+      const int at = __builtin_ctzll(here);
+      e = e0 + at;
+      m0 = __builtin_amdgcn_readlane(lo, at) + (slot - (__builtin_amdgcn_readlane(end, at) - __builtin_amdgcn_readlane(n, at))) * BM;
+      m_hi = __builtin_amdgcn_readlane(hi, at);
+      return true;
+    }
+    slot -= __builtin_amdgcn_readlane(end, 63);
+  }
+  return false;
+}
+
+template <int EPI, int BM>
+__global__ __launch_bounds__(BM * 4, 4) void gemm_grouped_kernel(const bf16_t* __restrict__ Wp_all, long long expert_stride,
+                                                              const bf16_t* __restrict__ X, const int32_t* __restrict__ row_index,
+                                                              const int32_t* __restrict__ offsets, int E, void* __restrict__ Y, int N,
+                                                              int K, int ldy, int tiles_n, GluClamp glu) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int WAVES = BM / 16, NS = gg_stages(BM), STAGE = GG_W_BYTES + BM * 128, WPW = 16 / WAVES;       // KiB pieces of the weights per wave and K-tile
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wn = wave >> 1, wm = wave & 1;
-  const int tn = blockIdx.x % tiles_n;
-  int slot = blockIdx.x / tiles_n;
-  int e = 0, m0 = 0, m_hi = 0;
-  bool found = false;
-  for (e = 0; e < E; ++e) {
-    const int lo = offsets[e], hi = offsets[e + 1];
-    const int nt = (hi - lo + GT_BM - 1) / GT_BM;
-    if (slot < nt) {
-      m0 = lo + slot * GT_BM;
-      m_hi = hi;
-      found = true;
-      break;
-    }
-    slot -= nt;
-  }
-  if (!found) return;
-  const bf16_t* Wp = Wp_all + static_cast<size_t>(e) * expert_stride;
-  const int nt0 = tn * (GT_BN / 16);
-  const int KT = K / 32, nk = K / GT_BK;
+  const int wn = wave & 3, wm = wave >> 2;
+  int e = 0, m0 = 0, m_hi = 0, tn = 0;
+  if (!gg_find<BM>(offsets, E, tiles_n, lane, e, m0, m_hi, tn)) return;                 // block-uniform, before any barrier
+  const int KT = K / 32, nk = K / GG_BK;
 
-  f32x4 acc[4][4];
+  // What this wave stages of a K-tile: WPW pieces of the weights (fragment f of the 16: n-tile f / 2, k-step f % 2) and two pieces
+  // of eight whole 128-byte rows, swizzled on the source side as in gemm256.hip.
+  const bf16_t* wsrc[WPW];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < WPW; ++i) {
+    const int f = wave * WPW + i;
+    wsrc[i] = Wp_all + static_cast<size_t>(e) * expert_stride + (static_cast<size_t>(tn * (GG_BN / 16) + (f >> 1)) * KT + (f & 1)) * 512 + lane * 8;
+  }
+  const bf16_t* xsrc[2];
+  const int rr = lane >> 3, lc = lane & 7;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    int row = m0 + (wave * 2 + i) * 8 + rr;
+    row = row < m_hi ? row : m_hi - 1;
+    if (row_index) row = row_index[row];
+    xsrc[i] = X + static_cast<size_t>(row) * K + ((lc ^ rr) << 3);
+  }
+  auto request = [&](int kt) {                      // K-tile kt into its stage (behind the last one: the last one again)
+    char* stage = smem + (kt % NS) * STAGE;
+    const int k = kt < nk ? kt : nk - 1;
+#pragma unroll
+    for (int i = 0; i < WPW; ++i)
+      __builtin_amdgcn_global_load_lds(LC_GLOBAL_PTR(wsrc[i] + static_cast<size_t>(k) * 1024), LC_LDS_PTR(stage + (wave * WPW + i) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_global_load_lds(LC_GLOBAL_PTR(xsrc[i] + k * GG_BK), LC_LDS_PTR(stage + GG_W_BYTES + (wave * 2 + i) * 1024), 16, 0, 0);
+  };
+
+  f32x4 acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int r7 = lane & 7;
+  int xoff[2];
+#pragma unroll
+  for (int kt = 0; kt < 2; ++kt) xoff[kt] = ((lane & 15) >> 3) * 1024 + r7 * 128 + (((kt * 4 + (lane >> 4)) ^ r7) << 4);
 
-  gt_stage(smem, Wp, X, nt0, m0, m_hi, row_index, 0, KT, K, wave, lane);
-  __syncthreads();
+#pragma unroll
+  for (int t = 0; t + 1 < NS; ++t) request(t);
   for (int t = 0; t < nk; ++t) {
-    char* cur = smem + (t & 1) * GT_STAGE_BYTES;
-    if (t + 1 < nk)
-      gt_stage(smem + ((t + 1) & 1) * GT_STAGE_BYTES, Wp, X, nt0, m0, m_hi, row_index, (t + 1) * 2, KT, K, wave, lane);
+    // all but the requests of K-tile t + 1 have landed; behind the barrier everyone's have, and nobody reads K-tile t - 1 any more
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * (WPW + 2)) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    request(t + NS - 1);
+    const char* w = smem + (t % NS) * STAGE + wn * 4096 + lane * 16;
+    const char* x = smem + (t % NS) * STAGE + GG_W_BYTES + wm * 8192;
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) {
-      bf16x8 a[4], b[4];
+      bf16x8 a[2], b[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        a[i] = *reinterpret_cast<const bf16x8*>(cur + ((wn * 4 + i) * 2 + kt) * 1024 + lane * 16);
+      for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const bf16x8*>(w + (i * 2 + kt) * 1024);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        b[j] = *reinterpret_cast<const bf16x8*>(cur + 16 * 1024 + ((wm * 4 + j) * 2 + kt) * 1024 + lane * 16);
+      for (int j = 0; j < 4; ++j) b[j] = *reinterpret_cast<const bf16x8*>(x + j * 2048 + xoff[kt]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
     }
-    __syncthreads();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // this wave's reads are over before it lets the stage be written again
   }
-  const int nbase = tn * GT_BN + wn * 64, mbase = m0 + wm * 64;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // (requests behind the last K-tile)
+
+  const int nbase = tn * GG_BN + wn * 32, mbase = m0 + wm * 64;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int j = 0; j < 4; ++j) {
+    if constexpr (EPI == EPI_GLU_CLAMPED) {
+      store_tile_glu_clamped(acc[0][j], acc[1][j], Y, glu, mbase + j * 16, nbase, m_hi, N, ldy, lane);
+    } else if constexpr (EPI == EPI_SWIGLU) {
+      store_tile<EPI>(acc[0][j], &acc[1][j], Y, nullptr, mbase + j * 16, nbase, m_hi, N, ldy, lane, 0);
+    } else {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if constexpr (EPI == EPI_GLU_CLAMPED) {
-        if (i & 1) continue;
-        store_tile_glu_clamped(acc[i][j], acc[i + 1][j], Y, glu, mbase + j * 16, nbase + i * 16, m_hi, N, ldy, lane);
-      } else if constexpr (EPI == EPI_SWIGLU) {
-        if (i & 1) continue;
-        store_tile<EPI>(acc[i][j], &acc[i + 1][j], Y, nullptr, mbase + j * 16, nbase + i * 16, m_hi, N, ldy, lane, 0);
-      } else {
-        store_tile<EPI>(acc[i][j], nullptr, Y, nullptr, mbase + j * 16, nbase + i * 16, m_hi, N, ldy, lane, 0);
-      }
+      for (int i = 0; i < 2; ++i) store_tile<EPI>(acc[i][j], nullptr, Y, nullptr, mbase + j * 16, nbase + i * 16, m_hi, N, ldy, lane, 0);
     }
+  }
 }
 
 // Sums S fp32 slabs [S, M, N] (+bias) and writes bf16 (mode 0), fp32 (mode 1) or
@@ -313,16 +389,26 @@ static int launch_gemm_grouped(const void* Wp_all, long long expert_stride, cons
                                int epi, GluClamp glu, hipStream_t stream) {
   if (total_rows <= 0) return 0;
   if (K % 64 || n_pad % 128 || N > n_pad || E < 1) return -1;
-  const int tiles_n = n_pad / GT_BN;
-  const int max_tiles_m = (total_rows + GT_BM - 1) / GT_BM + E;
-  const dim3 grid(max_tiles_m * tiles_n), block(256);
-  const size_t lds = 2 * GT_STAGE_BYTES;
+  const int tiles_n = n_pad / GG_BN, bm = gg_rows(total_rows, E, tiles_n);
+  const int max_tiles_m = (total_rows + bm - 1) / bm + E;
+  const dim3 grid(max_tiles_m * tiles_n), block(bm * 4);
+  const size_t lds = gg_stages(bm) * (GG_W_BYTES + bm * 128);
   auto w = static_cast<const bf16_t*>(Wp_all);
   auto x = static_cast<const bf16_t*>(X);
   auto ri = static_cast<const int32_t*>(row_index);
   auto off = static_cast<const int32_t*>(offsets);
-#define LC_GG(EPI_) \
-  gemm_grouped_kernel<EPI_><<<grid, block, lds, stream>>>(w, expert_stride, x, ri, off, E, Y, N, K, ldy, tiles_n, glu)
+#define LC_GG(EPI_)                                                                                                                     \
+  do {                                                                                                                                  \
+    static LcDeviceOnce once;                                                                                                           \
+    once.run([&] {                                                                                                                      \
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_grouped_kernel<EPI_, 64>), hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                gg_stages(64) * (GG_W_BYTES + 64 * 128));                                                                       \
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_grouped_kernel<EPI_, 128>), hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                gg_stages(128) * (GG_W_BYTES + 128 * 128));                                                                      \
+    });                                                                                                                                 \
+    if (bm == 128) gemm_grouped_kernel<EPI_, 128><<<grid, block, lds, stream>>>(w, expert_stride, x, ri, off, E, Y, N, K, ldy, tiles_n, glu); \
+    else gemm_grouped_kernel<EPI_, 64><<<grid, block, lds, stream>>>(w, expert_stride, x, ri, off, E, Y, N, K, ldy, tiles_n, glu);      \
+  } while (0)
   if (epi == EPI_BF16) LC_GG(EPI_BF16);
   else if (epi == EPI_SWIGLU) LC_GG(EPI_SWIGLU);
   else if (epi == EPI_RELU2) LC_GG(EPI_RELU2);

@@ -771,6 +771,14 @@ def moe_permute(ids: torch.Tensor, E: int):
     return offsets, sorted_src, slot_of
 
 
+def _panel_experts(rows: int, E: int) -> bool:
+    """Whether grouped products of ``rows`` routed rows take the panel kernel, a panel of ALL rows' height per expert and column tile.
+    With up to eight experts it keeps pace with the tiles to a few hundred rows (8 of 3584 x 4096 at 128 and 256 rows: 43.6 and 43.6 us,
+    43.5 and 43.9 in tiles). With more of them an expert has a few rows, and from about a hundred on the tiles are faster
+    (32 experts of 512 x 2048 at 96, 128, 256, 384 rows: 16.7, 27.5, 51.1, 39.8 us against 16.6, 17.0, 17.4, 17.3)."""
+    return rows <= (MOE_PANEL_MAX_ROWS if E <= 8 else min(MOE_PANEL_MAX_ROWS, 96))
+
+
 def experts_on_sorted(x: torch.Tensor, row_index: Optional[torch.Tensor], offsets: torch.Tensor, expert0: int,
                       w_gate_up: "ExpertWeights", w_down: "ExpertWeights", rows_bound: int,
                       zero_unwritten: bool = False) -> torch.Tensor:
@@ -799,7 +807,7 @@ def experts_on_sorted(x: torch.Tensor, row_index: Optional[torch.Tensor], offset
         zero_(y)
     # Decode steps (a few dozen routed rows in total): every expert's weights are streamed once
     # against one small panel. Prefill-sized batches use the tiled grouped kernels.
-    gg = "lc_gemm_panel_grouped" if rows_bound <= MOE_PANEL_MAX_ROWS else "lc_gemm_grouped"
+    gg = "lc_gemm_panel_grouped" if _panel_experts(rows_bound, E_local) else "lc_gemm_grouped"
     if (gg == "lc_gemm_grouped" and rows_bound >= MOE_GEMM256_MIN_ROWS and w_gate_up.n_pad % 256 == 0
             and w_down.n_pad % 256 == 0 and w_gate_up.k % 64 == 0 and w_down.k % 64 == 0):
         # Prefill-sized batches: the 256x256 pipelined tile per expert. It reads contiguous rows,
@@ -1570,7 +1578,7 @@ def grouped_linear(x: torch.Tensor, row_index: Optional[torch.Tensor], offsets: 
     W[e] x[row_index[p]] (x[p] without an index); ``relu2_epi``: square of relu. W is either a
     row-major tensor [E, N, K] of any shape and type (fp32 matrix instructions) or
     packed ``ExpertWeights`` (bf16 activations, the grouped MFMA kernels: one panel per expert for a
-    few hundred rows, 128 x 128 tiles beyond). Positions of experts >= E are left unwritten.
+    few hundred rows or a hundred over many experts, row tiles beyond). Positions of experts >= E are left unwritten.
     ``glu_clamp`` = (row_scale fp32 [rows] or None, limit, slope, shift), packed weights marked ``swiglu``
     only (16-row tiles alternate gate / up, ``interleave_gate_up``): the clamped gated unit of the product,
     scaled per sorted row, as the epilogue; the result is bf16 [rows, N / 2]."""
@@ -1583,7 +1591,7 @@ def grouped_linear(x: torch.Tensor, row_index: Optional[torch.Tensor], offsets: 
         if scale is not None and (scale.dtype != torch.float32 or scale.numel() < rows):
             raise ValueError("grouped_linear: one fp32 scale per sorted row")
         y = torch.empty(rows, W.n // 2, dtype=torch.bfloat16, device=x.device)
-        gg = "lc_gemm_panel_grouped_glu" if rows <= MOE_PANEL_MAX_ROWS else "lc_gemm_grouped_glu"
+        gg = "lc_gemm_panel_grouped_glu" if _panel_experts(rows, W.data.shape[0]) else "lc_gemm_grouped_glu"
         _hip().call(gg, W.data.data_ptr(), W.data[0].numel(), x.data_ptr(), _hip().ptr(row_index), offsets.data_ptr(),
                     W.data.shape[0], y.data_ptr(), int(rows), W.n, W.k, W.n_pad, W.n // 2, _hip().ptr(scale), float(limit),
                     float(slope), float(shift))
@@ -1601,7 +1609,7 @@ def grouped_linear(x: torch.Tensor, row_index: Optional[torch.Tensor], offsets: 
             raise ValueError("grouped_linear: the relu^2 epilogue of the packed kernels writes bf16")
         y = torch.empty(rows, W.n, dtype=out_dtype, device=x.device)
         epi = 3 if relu2_epi else (EPI_F32 if out_dtype == torch.float32 else EPI_BF16)
-        gg = "lc_gemm_panel_grouped" if rows <= MOE_PANEL_MAX_ROWS else "lc_gemm_grouped"
+        gg = "lc_gemm_panel_grouped" if _panel_experts(rows, W.data.shape[0]) else "lc_gemm_grouped"
         _hip().call(gg, W.data.data_ptr(), W.data[0].numel(), x.data_ptr(), _hip().ptr(row_index), offsets.data_ptr(),
                     W.data.shape[0], y.data_ptr(), int(rows), W.n, W.k, W.n_pad, W.n, epi)
         return y

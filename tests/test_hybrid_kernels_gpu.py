@@ -381,6 +381,38 @@ def test_sorted_expert_products_on_the_packed_mfma_kernels(T, top, E, d, ff):
     torch.testing.assert_close(ye.cpu()[:real], ye_ref[:real], atol=3e-2, rtol=3e-2)
 
 
+@pytest.mark.parametrize("counts,n,k", [
+    ([0, 1, 63, 64, 65, 0], 96, 64),                            # tiles of 64 rows, one K-tile
+    ([129, 127, 128, 3], 300, 128),                             # two K-tiles, a ragged last column tile
+    ([0] * 3 + [1, 0, 2] * 22 + [150, 0], 128, 192),            # more experts than a wave has lanes, most of them empty
+    ([257, 0, 128, 129, 64, 255, 1, 130, 256] * 2, 2048, 320),  # tiles of 128 rows
+    ([700, 5], 130, 64),
+])
+def test_grouped_tiles_at_their_edges(counts, n, k):
+    """Row tiles of 64 and 128 rows, experts without rows, row counts around a tile, gathered and plain rows, against fp32 products. An
+    fp32 sum of k products of magnitude k^-1/2 is off by less than k 2^-24 of their absolute sum, 1e-5 at k = 320."""
+    g = torch.Generator().manual_seed(n + k)
+    E, rows = len(counts), sum(counts)
+    off = torch.tensor([0] + counts).cumsum(0).to(torch.int32)
+    x = torch.randn(rows + 7, k, generator=g).to(torch.bfloat16)
+    src = torch.randperm(rows + 7, generator=g)[:rows].to(torch.int32)
+    W = (torch.randn(E, n, k, generator=g) / k ** 0.5).to(torch.bfloat16)
+    Wd, offd, xd = ops.ExpertWeights.from_dense(W, DEV), off.to(DEV), x.to(DEV)
+    old, ops.MOE_PANEL_MAX_ROWS = ops.MOE_PANEL_MAX_ROWS, 0
+    try:
+        got = ops.grouped_linear(xd, src.to(DEV), offd, Wd, torch.float32, rows).cpu()
+        plain = ops.grouped_linear(xd, None, offd, Wd, torch.float32, rows).cpu()
+        act = ops.grouped_linear(xd, src.to(DEV), offd, Wd, torch.bfloat16, rows, relu2_epi=True).float().cpu()
+    finally:
+        ops.MOE_PANEL_MAX_ROWS = old
+    for e in range(E):
+        a, b = int(off[e]), int(off[e + 1])
+        want = x[src[a:b].long()].float() @ W[e].float().T
+        torch.testing.assert_close(got[a:b], want, atol=1e-5, rtol=1e-5)
+        torch.testing.assert_close(plain[a:b], x[a:b].float() @ W[e].float().T, atol=1e-5, rtol=1e-5)
+        torch.testing.assert_close(act[a:b], torch.relu(want) ** 2, atol=2e-4, rtol=2 ** -8)      # (rounded to bf16)
+
+
 # ---- Dynamic Tanh residual step, neighbouring rotary pairs with keys as values, clamped gated units ----
 @pytest.mark.parametrize("dt", ACTS)
 @pytest.mark.parametrize("T,d", [(3, 10), (600, 132), (1, 64)])
