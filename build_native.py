@@ -94,7 +94,7 @@ def build_selftest(sanitize: str = "address,undefined") -> Path:
 # model family on a fresh checkout builds only what that family launches (the device runtime,
 # the GEMMs, the row kernels and the sampler are common to all). Files not listed are "transformer".
 KERNEL_GROUPS = {
-    "base": ["device_runtime.hip", "elementwise.hip", "gemm.hip", "gemm256.hip", "gemm256w.hip", "gemm_panel.hip",
+    "base": ["device_runtime.hip", "elementwise.hip", "gemm.hip", "gemm256.hip", "gemm256w.hip", "gemm_panel.hip", "gemm_strip.hip",
              "kgemm.hip", "sampling.hip"],
     "hybrid": ["hybrid.hip", "hybrid_attn.hip", "hybrid_delta.hip", "hybrid_gated.hip", "hybrid_gemm.hip", "hybrid_linear.hip", "hybrid_moe.hip", "hybrid_streams.hip"],
 }

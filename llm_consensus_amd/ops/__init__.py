@@ -187,6 +187,19 @@ def _kgemm_ntw(n_pad: int, M: int, swiglu: bool, K: int = 0) -> int:
     return 1 if M <= 4 or n_pad < 8192 else 2
 
 
+STRIP_MAX_M, STRIP_MAX_K = 64, 4096
+
+
+def _strip_tiles(M: int, w: "LinearWeight") -> int:
+    """Column tiles of 16 per workgroup for the product and activation of up to 64 rows in one launch (gemm_strip.hip), or 0. It takes
+    outputs whose 128-column panels leave the depth to be split over workgroups (up to 16384 columns, 64 to a workgroup from 8192
+    on: 9728 x 896 at 32 rows 6.4 us, 8.0 with 32), and depths of up to 4096: a workgroup walks its whole depth, 0.19 us per
+    K-tile (2048 x 8192 24 us against 14 for a split product and its activation; 4096 x 4096 13 and 15)."""
+    if M > STRIP_MAX_M or w.k > STRIP_MAX_K or w.n_pad > 16384 or w.n_pad % 64:
+        return 0
+    return 4 if w.n_pad > 8192 else 2
+
+
 def _choose_panel_splits(n_pad: int, K: int) -> int:
     """K splits of the panel kernel (gemm_panel.hip). Its LDS ring admits one workgroup per CU,
     so the aim is as many workgroups as possible WITHOUT exceeding the 256 CUs (a 257th would
@@ -351,6 +364,10 @@ def linear(x: torch.Tensor, w: LinearWeight, out_f32: bool = False, defer_reduce
     kernel, splits, extra = "lc_gemm_panel", _choose_panel_splits(w.n_pad, w.k) if w.n % 32 == 0 else 1, (1 if PANEL_DEEP else 0,)
     if wide:
         extra = (2,)
+    strip = _strip_tiles(M, w) if w.swiglu and splits > 1 else 0
+    if strip:
+        h.call("lc_gemm_strip", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, out_n, epi, strip, 0.0, 0.0)
+        return y
     if splits == 1:
         h.call(kernel, w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, out_n, epi, 1,
                *extra)
@@ -1086,7 +1103,7 @@ COLUMN_ACTS = ("relu2", "xielu")
 
 def act_linear(x: torch.Tensor, w: LinearWeight, kind: str, act_dtype: torch.dtype, ap: float = 0.0, an: float = 0.0) -> torch.Tensor:
     """act(x @ W^T + bias) in ``act_dtype`` (kind: "relu2", or "xielu" with its two numbers). Packed products of bf16 activations
-    that are one launch of 256 x 256 tiles or of the split-in-the-workgroup kernel apply it to their accumulators; otherwise it
+    that are one launch of 256 x 256 tiles, of the split-in-the-workgroup kernel or of narrow strips apply it to their accumulators; otherwise it
     is a launch behind the fp32 product, which also sums the slabs of a split one."""
     if not x.is_cuda:
         return _column_act(linear(x, w, out_f32=True), kind, ap, an, act_dtype)
@@ -1098,11 +1115,12 @@ def act_linear(x: torch.Tensor, w: LinearWeight, kind: str, act_dtype: torch.dty
     if x.dtype == torch.bfloat16 and act_dtype == torch.bfloat16 and not w.swiglu and M > 0:
         h, epi = _hip(), EPI_RELU2 if kind == "relu2" else EPI_XIELU
         ntw = _kgemm_ntw(w.n_pad, M, False, w.k) if M <= WS_MAX_M else 0
-        if ntw or _whole_tiles256(M, w):
+        strip = _strip_tiles(M, w)
+        if ntw or strip or _whole_tiles256(M, w):
             x, y = x.contiguous(), torch.empty(M, w.n, dtype=act_dtype, device=x.device)
             args = (w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, w.n, epi)
-            if ntw:
-                h.call("lc_kgemm", *args, ntw, float(ap), float(an))
+            if ntw or strip:
+                h.call("lc_kgemm" if ntw else "lc_gemm_strip", *args, ntw or strip, float(ap), float(an))
             else:
                 h.call("lc_gemm256", *args, float(ap), float(an))
             return y
@@ -1486,17 +1504,19 @@ def _residual_step(x: torch.Tensor, y, w_out=None, w_in=None, w_in2=None, eps: f
 
 def glu_linear(x: torch.Tensor, w: LinearWeight, kind: str, act_dtype: torch.dtype, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """act(gate) * up of x's product with ``w`` (rows gate | up, or in alternate tiles of 16 when ``w.tiled``), [T, n] in
-    ``act_dtype``, into ``out`` (a block of a wider matrix) when given. Large bf16 products of tiled weights store the gated unit
-    from their accumulators (gelu_tanh, relu); otherwise the fp32 product is gated in a launch of its own, which also sums the slabs
+    ``act_dtype``, into ``out`` (a block of a wider matrix) when given. bf16 products of tiled weights in 256 x 256 tiles or of up to
+    64 rows store the gated unit from their accumulators (gelu_tanh, relu); otherwise the fp32 product is gated in a launch of its own, which also sums the slabs
     of a split one."""
     M, n = x.shape[0], w.n // 2
+    strip = _strip_tiles(M, w)
     if x.is_cuda and w.is_packed and w.tiled and w.bias is None and kind in GLU_EPILOGUES and act_dtype == torch.bfloat16 \
-            and _whole_tiles256(M, w):
+            and x.dtype == torch.bfloat16 and M > 0 and (strip or _whole_tiles256(M, w)):
         y = _out_block(out, M, n, act_dtype, x.device, "glu_linear")
         ldy = max(y.stride(0), n)
         if ldy % 8 == 0 and y.data_ptr() % 16 == 0:
-            _hip().call("lc_gemm256", w.data.data_ptr(), x.contiguous().data_ptr(), y.data_ptr(), None, M, w.n, w.k, w.n_pad, ldy,
-                        GLU_EPILOGUES[kind], 0.0, 0.0)
+            x = x.contiguous()
+            args = (w.data.data_ptr(), x.data_ptr(), y.data_ptr(), None, M, w.n, w.k, w.n_pad, ldy, GLU_EPILOGUES[kind])
+            _hip().call("lc_gemm_strip" if strip else "lc_gemm256", *args, *((strip,) if strip else ()), 0.0, 0.0)
             return y
     return glu(linear(x, w, out_f32=True, defer_reduce=True), act_dtype, kind, out=out, tiled=w.tiled)
 

@@ -218,6 +218,46 @@ def test_panel_gemm_with_and_without_splitk(M, N, K):
         ops.KGEMM_FORCE_NTW = old_k
 
 
+@pytest.mark.parametrize("M", [1, 32, 33, 64])
+@pytest.mark.parametrize("N,K,kind", [(96, 64, "relu2"), (300, 320, "xielu"), (1024, 4096, "relu2"), (8448, 448, "xielu"), (96, 128, "gelu_tanh"),
+                                      (8192, 384, "relu"), (16384, 512, "gelu_tanh"), (1248, 896, "swiglu"), (9728, 896, "swiglu")])
+def test_products_and_their_activations_in_strips(M, N, K, kind):
+    """Both widths of a workgroup, both panel heights, depths below and beyond the ring, ragged widths, with a bias where the epilogue
+    has one. bf16 results: half a unit of 2^-8 of the value, and of the inputs' fp32 sum below that."""
+    from llm_consensus_amd.ops import hip
+    g = torch.Generator().manual_seed(M + N + K)
+    gated = kind not in ("relu2", "xielu")
+    W = (torch.randn(N, K, generator=g) / K ** 0.5).to(torch.bfloat16)
+    b = None if gated and kind != "swiglu" else torch.randn(N, generator=g).to(torch.bfloat16)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = ops.LinearWeight.from_dense(W, b, device=DEV, swiglu=kind == "swiglu")
+    w.tiled = gated
+    assert ops._strip_tiles(M, w) == (4 if N > 8192 else 2)
+    rec, old = hip.start_recording(), ops.KGEMM_FORCE_NTW
+    ops.KGEMM_FORCE_NTW = 0                   # (a few rows take the split-in-the-workgroup kernel otherwise)
+    try:
+        if kind == "swiglu":
+            got = ops.linear(x.to(DEV), w)
+        elif gated:
+            wide = torch.full((M, N // 2 + 24), 7.0, dtype=torch.bfloat16, device=DEV)
+            got = ops.glu_linear(x.to(DEV), w, kind, torch.bfloat16, out=wide[:, 8:8 + N // 2])
+            assert (wide[:, :8] == 7).all() and (wide[:, 8 + N // 2:] == 7).all()
+        else:
+            got = ops.act_linear(x.to(DEV), w, kind, torch.bfloat16, 0.8, 0.9)
+    finally:
+        hip.stop_recording()
+        ops.KGEMM_FORCE_NTW = old
+    assert {n for _, _, n in rec} == {"lc_gemm_strip"}
+    y = x.float() @ W.float().T + (b.float() if b is not None else 0.0)
+    if gated:
+        gate, up = y.view(M, N // 32, 2, 16).transpose(1, 2).reshape(M, 2, N // 2).unbind(1)
+        act = {"swiglu": torch.nn.functional.silu, "relu": torch.relu, "gelu_tanh": lambda z: torch.nn.functional.gelu(z, approximate="tanh")}[kind]
+        want = act(gate) * up
+    else:
+        want = torch.relu(y) ** 2 if kind == "relu2" else torch.where(y > 0, 0.8 * y * y, 0.9 * (torch.expm1(y) - y)) + 0.5 * y
+    torch.testing.assert_close(got.float().cpu(), want, atol=1e-4, rtol=2 ** -8)
+
+
 @pytest.mark.parametrize("M", [5, 64, 128, 400])
 def test_fused_swiglu_epilogue(M):
     K, dff = 256, 384
