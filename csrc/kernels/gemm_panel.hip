@@ -4,16 +4,15 @@
 // At these shapes the weights dominate the traffic (a 7-8B model streams ~15 GB per decode
 // step) and the job is to keep enough loads in flight per CU to saturate HBM while the
 // MFMA work rides along. The kernel is a 128(n) x BM(m) x 64(k) tile whose K loop runs over
-// a deep ring of LDS stages filled by LDS-DMA (global_load_lds, 16 B per lane):
+// a ring of LDS stages filled by LDS-DMA (global_load_lds, 16 B per lane):
 //
-//     BM    stage (W 16 KiB + X BM*128 B)   stages   K-tiles in flight   wave grid (n x m)   frags / wave
-//     256   48 KiB                          3        2                   2 x 4               4 nt x 4 mt
-//     128   32 KiB                          4        3                   4 x 2               2 nt x 4 mt
-//      64   24 KiB                          6        5                   4 x 2               2 nt x 2 mt
-//      32   20 KiB                          7        6                   4 x 2               2 nt x 1 mt
+//     BM    stage (W 16 KiB + X BM*128 B)   stages (grouped)   wave grid (n x m)   frags / wave
+//     256   48 KiB                          3 (3)              2 x 4               4 nt x 4 mt
+//     128   32 KiB                          3 (4)              4 x 2               2 nt x 4 mt
+//      64   24 KiB                          3 (6)              4 x 2               2 nt x 2 mt
+//      32   20 KiB                          3 (7)              4 x 2               2 nt x 1 mt
 //
-// so at BM = 64 a CU has up to 5 x 24 KiB = 120 KiB of loads outstanding, without spending a
-// single VGPR on staging. One barrier per K-tile does both jobs of the ring:
+// without spending a single VGPR on staging. One barrier per K-tile does both jobs of the ring:
 //
 //     wait vmcnt(P*(D-1))   this wave's P pieces of K-tile t have landed; D-1 tiles stay in flight
 //     barrier               => K-tile t is visible to everybody, and everybody is done with t-1
@@ -37,10 +36,12 @@ constexpr int GP_BN = 128, GP_BK = 64, GP_WBYTES = 16 * 1024;
 // 28672 x 4096 matrix at 32 rows, and 4-9 % on the narrower projections.
 constexpr int GP_NT = 2;
 
-// DEEP = true: the ring takes (almost) all of a CU's LDS, one workgroup per CU, most loads in
-// flight -- best when the GEMM has the GPU to itself. DEEP = false: a ring of three stages
-// (<= 72 KiB at BM <= 64) so two workgroups fit on a CU -- for ensembles whose member engines
-// run on concurrent streams and fill each other's gaps.
+// DEEP = true: the ring takes (almost) all of a CU's LDS, most loads in flight. DEEP = false: a ring of three stages (<= 72 KiB at
+// BM <= 64), which leaves room for a second workgroup, another engine's included. The dense kernel has the short ring: filling the
+// deep one costs more than it gains (us, deep and short, at 9, 32, 64, 128 rows: 6144 x 4096 in four splits 12.9 13.3 14.2 16.5 and
+// 11.1 11.8 12.6 16.3; 2048 x 8192 in sixteen 9.8 10.5 11.3 13.7 and 8.3 9.0 9.9 13.1; 28672 x 4096 40.8 39.7 39.2 48.4 and 39.1 37.7
+// 38.4 47.7; 3584 x 18944 in eight 22.7 23.8 25.5 31.7 and 22.2 23.7 25.2 31.6). The grouped kernel keeps the deep one, experts stream
+// one after the other through it (8 of 4096 x 14336 at 96 rows 140 us, 195 with the short ring).
 template <int BM, bool DEEP>
 struct PanelShape {
   static constexpr int STAGE = GP_WBYTES + BM * 128;
@@ -61,9 +62,9 @@ struct GpCtx {
   int nt0, M, K, KT, kt_lo, nk, wave, lane;
 };
 
-template <int BM, bool DEEP, bool UNCHECKED = false>
+template <int BM, bool UNCHECKED = false>
 LC_DEVICE void gp_issue_tile(const GpCtx& c, int t) {
-  using S = PanelShape<BM, DEEP>;
+  using S = PanelShape<BM, false>;
   if (!UNCHECKED && t >= c.nk) return;
   char* stage = c.smem + (t % S::NSTAGE) * S::STAGE;
   const int k_tile = c.kt_lo + t;
@@ -109,12 +110,12 @@ LC_DEVICE void gp_wait_tiles_in_flight(int tiles) {
   }
 }
 
-template <int BM, bool DEEP, int EPI>
+template <int BM, int EPI>
 __global__ __launch_bounds__(512) void gemm_panel_kernel(const bf16_t* __restrict__ Wp,
                                                          const bf16_t* __restrict__ X, void* __restrict__ Y,
                                                          const bf16_t* __restrict__ bias, int M, int N, int K,
                                                          int ldy, int nk_per_split) {
-  using S = PanelShape<BM, DEEP>;
+  using S = PanelShape<BM, false>;
   static_assert(S::P * S::DEPTH <= 63, "vmcnt is a 6-bit counter");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
@@ -168,7 +169,7 @@ __global__ __launch_bounds__(512) void gemm_panel_kernel(const bf16_t* __restric
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       if (MAIN || after >= 0) read_frags(t + 1, set ^ 1);
-      if (MAIN || t + S::NSTAGE < c.nk) gp_issue_tile<BM, DEEP, true>(c, t + S::NSTAGE);
+      if (MAIN || t + S::NSTAGE < c.nk) gp_issue_tile<BM, true>(c, t + S::NSTAGE);
       if constexpr (!MAIN) __builtin_amdgcn_s_setprio(1);   // (a priority change would pin the schedule)
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
@@ -200,7 +201,7 @@ __global__ __launch_bounds__(512) void gemm_panel_kernel(const bf16_t* __restric
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
 #pragma unroll
-    for (int t = 0; t < S::NSTAGE; ++t) gp_issue_tile<BM, DEEP>(c, t);
+    for (int t = 0; t < S::NSTAGE; ++t) gp_issue_tile<BM>(c, t);
     gp_wait_tiles_in_flight<S::P>(c.nk - 1 < S::NSTAGE - 1 ? c.nk - 1 : S::NSTAGE - 1);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -217,7 +218,7 @@ __global__ __launch_bounds__(512) void gemm_panel_kernel(const bf16_t* __restric
     }
   } else {
 #pragma unroll
-  for (int t = 0; t < S::DEPTH; ++t) gp_issue_tile<BM, DEEP>(c, t);
+  for (int t = 0; t < S::DEPTH; ++t) gp_issue_tile<BM>(c, t);
 
   for (int t = 0; t < c.nk; ++t) {
     const int behind = c.nk - 1 - t;   // K-tiles after t that exist at all
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(512) void gemm_panel_kernel(const bf16_t* __restric
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    gp_issue_tile<BM, DEEP>(c, t + S::DEPTH);
+    gp_issue_tile<BM>(c, t + S::DEPTH);
 
     const char* stage = smem + (t % S::NSTAGE) * S::STAGE;
     const char* wimg = stage + (wn * S::NT_W * 2) * 1024 + lane * 16;
@@ -271,28 +272,28 @@ __global__ __launch_bounds__(512) void gemm_panel_kernel(const bf16_t* __restric
     }
 }
 
-template <int BM, bool DEEP>
+template <int BM>
 int launch_panel(int epi, const bf16_t* w, const bf16_t* x, void* Y, const bf16_t* b, int M, int N, int K,
                  int n_pad, int ldy, int splits, hipStream_t stream) {
-  using S = PanelShape<BM, DEEP>;
+  using S = PanelShape<BM, false>;
   const dim3 grid(n_pad / GP_BN, splits), block(512);
   const int lds = S::NSTAGE * S::STAGE;
   const int nk = (K / GP_BK) / splits;
   static LcDeviceOnce attr_once;
   attr_once.run([&] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_panel_kernel<BM, DEEP, EPI_BF16>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_panel_kernel<BM, EPI_BF16>),
                         hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_panel_kernel<BM, DEEP, EPI_F32>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_panel_kernel<BM, EPI_F32>),
                         hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_panel_kernel<BM, DEEP, EPI_SWIGLU>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_panel_kernel<BM, EPI_SWIGLU>),
                         hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   });
   if (epi == EPI_BF16)
-    gemm_panel_kernel<BM, DEEP, EPI_BF16><<<grid, block, lds, stream>>>(w, x, Y, b, M, N, K, ldy, nk);
+    gemm_panel_kernel<BM, EPI_BF16><<<grid, block, lds, stream>>>(w, x, Y, b, M, N, K, ldy, nk);
   else if (epi == EPI_F32)
-    gemm_panel_kernel<BM, DEEP, EPI_F32><<<grid, block, lds, stream>>>(w, x, Y, b, M, N, K, ldy, nk);
+    gemm_panel_kernel<BM, EPI_F32><<<grid, block, lds, stream>>>(w, x, Y, b, M, N, K, ldy, nk);
   else if (epi == EPI_SWIGLU)
-    gemm_panel_kernel<BM, DEEP, EPI_SWIGLU><<<grid, block, lds, stream>>>(w, x, Y, b, M, N, K, ldy, nk);
+    gemm_panel_kernel<BM, EPI_SWIGLU><<<grid, block, lds, stream>>>(w, x, Y, b, M, N, K, ldy, nk);
   else
     return -2;
   return static_cast<int>(hipGetLastError());
@@ -311,7 +312,7 @@ int launch_panel(int epi, const bf16_t* w, const bf16_t* x, void* Y, const bf16_
 template <int BM>
 struct Panel5Shape {
   static constexpr int NT = 10, WBYTES = NT * 2048, STAGE = WBYTES + BM * 128;
-  static constexpr int NSTAGE = BM >= 256 ? 3 : (BM >= 128 ? 4 : (BM >= 64 ? 5 : 6));   // 156 / 144 / 140 / 144 KiB
+  static constexpr int NSTAGE = BM >= 256 || BM < 64 ? 3 : 4;    // 156 / 144 / 112 / 72 KiB (37888 x 3584 at 16 rows 42.6 us, 43.0 with six)
   static constexpr int DEPTH = NSTAGE - 1;
   static constexpr int MT_W = BM / 16;
   static constexpr int XP = BM >= 64 ? BM / 64 : 1;         // X pieces a wave stages per K-tile
@@ -608,24 +609,21 @@ int launch_panel_grouped(int epi, const bf16_t* w, long long stride, const bf16_
 }  // namespace
 
 // Y[M<=256, N] = X * W^T. Requirements: K % 64 == 0, (K/64) % splits == 0, n_pad % 128 == 0.
-// splits > 1 requires epi == EPI_F32 and Y = fp32 workspace [splits, M, ldy]. deep = 0 selects the
-// three-stage ring (two workgroups per CU) for M <= 128; deep = 2 the 160-column workgroups
+// splits > 1 requires epi == EPI_F32 and Y = fp32 workspace [splits, M, ldy]. shape = 2 selects the 160-column workgroups
 // (splits == 1, bf16 or SwiGLU epilogue; n_pad need not be a multiple of 160).
 LC_EXPORT int lc_gemm_panel(const void* Wp, const void* X, void* Y, const void* bias, int M, int N, int K,
-                            int n_pad, int ldy, int epi, int splits, int deep, hipStream_t stream) {
+                            int n_pad, int ldy, int epi, int splits, int shape, hipStream_t stream) {
   if (M <= 0) return 0;
   if (M > 256 || K % 64 || n_pad % GP_BN || N > n_pad || splits < 1 || (K / GP_BK) % splits) return -1;
   if (splits > 1 && epi != EPI_F32) return -1;
   auto w = static_cast<const bf16_t*>(Wp);
   auto x = static_cast<const bf16_t*>(X);
   auto b = static_cast<const bf16_t*>(bias);
-#define LC_PANEL(BM_)                                                                            \
-  return deep ? launch_panel<BM_, true>(epi, w, x, Y, b, M, N, K, n_pad, ldy, splits, stream)    \
-              : launch_panel<BM_, false>(epi, w, x, Y, b, M, N, K, n_pad, ldy, splits, stream)
+#define LC_PANEL(BM_) return launch_panel<BM_>(epi, w, x, Y, b, M, N, K, n_pad, ldy, splits, stream)
   // Wide outputs whose 128-column tiles need a second, mostly empty round on the 256 CUs take
-  // 160-column workgroups instead when that saves the round (deep = 2 asks for it; the caller
+  // 160-column workgroups instead when that saves the round (shape = 2 asks for it; the caller
   // knows whether the GEMM has the GPU to itself).
-  if (deep == 2) {
+  if (shape == 2) {
     if (splits != 1 || epi == EPI_F32) return -1;
     if (M <= 32) return launch_panel5<32>(epi, w, x, Y, b, M, N, K, n_pad, ldy, stream);
     if (M <= 64) return launch_panel5<64>(epi, w, x, Y, b, M, N, K, n_pad, ldy, stream);
@@ -635,7 +633,7 @@ LC_EXPORT int lc_gemm_panel(const void* Wp, const void* X, void* Y, const void* 
   if (M <= 32) LC_PANEL(32);
   if (M <= 64) LC_PANEL(64);
   if (M <= 128) LC_PANEL(128);
-  return launch_panel<256, true>(epi, w, x, Y, b, M, N, K, n_pad, ldy, splits, stream);
+  LC_PANEL(256);
 #undef LC_PANEL
 }
 

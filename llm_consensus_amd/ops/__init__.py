@@ -27,13 +27,9 @@ GEMM256_MIN_TILES = int(os.environ.get("LC_GEMM256_MIN_TILES", "1"))
 # Reduction depth from which prefill-sized GEMMs take the four-wave 256 x 256 kernel (gemm256w.hip):
 # its longer prologue pays off only over many K-tiles (0 = never).
 GEMM256W_MIN_K = int(os.environ.get("LC_GEMM256W_MIN_K", "8192")) or (1 << 30)
-# Decode GEMM for 9..256 rows: the panel kernel (gemm_panel.hip, deep LDS-DMA ring) and its split-K policy.
+# Decode GEMM for 9..256 rows: the panel kernel (gemm_panel.hip, an LDS-DMA ring) and its split-K policy.
 PANEL_MAX_BLOCKS = int(os.environ.get("LC_PANEL_MAX_BLOCKS", "256"))
 PANEL_MIN_KTILES = int(os.environ.get("LC_PANEL_MIN_KTILES", "4"))
-# Ring depth of the panel kernel for M <= 128: deep (all of a CU's LDS, one workgroup per CU, fastest
-# alone) or three stages (two workgroups per CU, for member engines that share the GPU on
-# concurrent streams). Chosen when a decode graph is captured; see set_concurrent_engines().
-PANEL_DEEP = os.environ.get("LC_PANEL_DEEP", "1") == "1"
 PANEL_WIDE = os.environ.get("LC_PANEL_WIDE", "1") == "1"   # 160-column workgroups where they save a round (see linear())
 PANEL_WIDE_MAX_M = int(os.environ.get("LC_PANEL_WIDE_MAX_M", "256"))
 
@@ -41,12 +37,6 @@ PANEL_WIDE_MAX_M = int(os.environ.get("LC_PANEL_WIDE_MAX_M", "256"))
 # Decode attention: how many of the KV splits the waves of one workgroup may take (1, 2 or 4).
 ATTN_DECODE_MAX_WAVES = int(os.environ.get("LC_ATTN_WAVES", "4"))
 
-
-def set_concurrent_engines(n: int) -> None:
-    """Tells the op layer how many engines will issue decode steps on concurrent streams."""
-    global PANEL_DEEP
-    if "LC_PANEL_DEEP" not in os.environ:
-        PANEL_DEEP = n <= 1
 # In-workgroup K-split decode kernel (kgemm.hip): widest output it is used for, and a test override
 # (-1 = automatic, 0 = never, 1/2/4 = force that many n-tiles per workgroup).
 KGEMM_MAX_N = int(os.environ.get("LC_KGEMM_MAX_N", str(1 << 30)))
@@ -201,10 +191,9 @@ def _strip_tiles(M: int, w: "LinearWeight") -> int:
 
 
 def _choose_panel_splits(n_pad: int, K: int) -> int:
-    """K splits of the panel kernel (gemm_panel.hip). Its LDS ring admits one workgroup per CU,
-    so the aim is as many workgroups as possible WITHOUT exceeding the 256 CUs (a 257th would
-    run alone in a second round); every split is a whole number of 64-deep K-tiles and at
-    least PANEL_MIN_KTILES of them."""
+    """K splits of the panel kernel (gemm_panel.hip): as many workgroups as possible WITHOUT
+    exceeding the 256 CUs (more would share some CUs and their way to memory, and bring slabs);
+    every split is a whole number of 64-deep K-tiles and at least PANEL_MIN_KTILES of them."""
     blocks = n_pad // 128
     nk = K // 64
     best = 1
@@ -361,20 +350,20 @@ def linear(x: torch.Tensor, w: LinearWeight, out_f32: bool = False, defer_reduce
         h.call("lc_gemm256", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad,
                out_n, epi, 0.0, 0.0)
         return y
-    kernel, splits, extra = "lc_gemm_panel", _choose_panel_splits(w.n_pad, w.k) if w.n % 32 == 0 else 1, (1 if PANEL_DEEP else 0,)
+    kernel, splits, shape = "lc_gemm_panel", _choose_panel_splits(w.n_pad, w.k) if w.n % 32 == 0 else 1, 0
     if wide:
-        extra = (2,)
+        shape = 2
     strip = _strip_tiles(M, w) if w.swiglu and splits > 1 else 0
     if strip:
         h.call("lc_gemm_strip", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, out_n, epi, strip, 0.0, 0.0)
         return y
     if splits == 1:
         h.call(kernel, w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, out_n, epi, 1,
-               *extra)
+               shape)
         return y
     part = torch.empty(splits, M, w.n, dtype=torch.float32, device=x.device)
     h.call(kernel, w.data.data_ptr(), x.data_ptr(), part.data_ptr(), None, M, w.n, w.k, w.n_pad, w.n, EPI_F32, splits,
-           *extra)
+           shape)
     if defer_reduce and not w.swiglu:
         return PartialSum(part, w.bias)
     mode = 2 if w.swiglu else (1 if out_f32 else 0)
