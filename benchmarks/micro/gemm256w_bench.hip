@@ -18,7 +18,7 @@
 extern "C" int lc_gemm256w(const void* Wp, const void* X, void* Y, const void* bias, int M, int N, int K, int n_pad,
                            int ldy, int epi, hipStream_t stream);
 extern "C" int lc_gemm256(const void* Wp, const void* X, void* Y, const void* bias, int M, int N, int K, int n_pad,
-                          int ldy, int epi, hipStream_t stream);
+                          int ldy, int epi, float ap, float an, int mf, hipStream_t stream);
 
 static float bf2f(uint16_t h) {
   uint32_t u = static_cast<uint32_t>(h) << 16;
@@ -66,7 +66,7 @@ int main(int argc, char** argv) {
   const double flop = 2.0 * M * N * K;
   for (int which = 0; which < 2; ++which) {
     auto run = [&]() {
-      return which == 0 ? lc_gemm256(dw, dx, dy0, nullptr, M, N, K, N, ldy, epi, nullptr)
+      return which == 0 ? lc_gemm256(dw, dx, dy0, nullptr, M, N, K, N, ldy, epi, 0.f, 0.f, 8, nullptr)
                         : lc_gemm256w(dw, dx, dy1, nullptr, M, N, K, N, ldy, epi, nullptr);
     };
     for (int i = 0; i < 10; ++i)

@@ -9,6 +9,7 @@ from __future__ import annotations
 import math
 import os
 from dataclasses import dataclass
+from functools import lru_cache
 from typing import Optional, Tuple
 
 import torch
@@ -205,20 +206,53 @@ def _choose_panel_splits(n_pad: int, K: int) -> int:
     return best
 
 
-def _choose_gemm256_splits(tiles: int, K: int) -> int:
-    """K splits for the 256x256 kernel when its tiles alone cover less than half of the CUs:
-    the most splits that keep tiles * splits within the 256 CUs, in whole 64-deep K-tiles, at
-    least 8 of them each (below that the pipeline's fill and the slab traffic dominate)."""
-    if tiles * 2 > 256 or GEMM256_MAX_SPLITS <= 1:
-        return 1
-    nk = K // 64
-    best = 1
-    for s in (2, 3, 4, 6, 7, 8):
-        if tiles * s > 256 or s > GEMM256_MAX_SPLITS:
-            break
-        if nk % s == 0 and nk // s >= 8:
-            best = s
+# Tiles of 256 columns and 32 f rows (gemm256.hip; 0: the four-wave kernel, 256 rows): us per 64-deep K-tile with a tile on every CU, operands
+# not in the caches. A tile fetches its 256 weight columns whatever its height, so that the low ones cost more per row: at depth 8192 with
+# operands in the caches 1147 TFLOP/s at 128 rows, 1250, 1360, 1450 and 1465 at 256.
+GEMM256_KTILE_US = {8: 1.48, 7: 1.34, 6: 1.235, 5: 1.155, 4: 1.005, 0: 1.49}
+# What is taken off the estimate of the 256-row tiles and of the four-wave kernel: long launches run at the card's power, which the K-tile
+# times above do not show (1752 x 28672 x 4096 in 784 tiles of 256 rows 341 us, in 896 of 224 372).
+GEMM256_BIAS = {8: 0.95, 0: 0.89}
+GEMM256_REST_US = 28.0       # a product in a round of whole tiles and a split rest (_remainder_tiles), beside its round's K-tiles and its stores
+
+
+@lru_cache(maxsize=4096)
+def _gemm256_plan(M: int, n_pad: int, K: int, out_bytes: int, deferred: bool, max_splits: int, four_wave: bool, full_height: bool) -> Tuple[int, int, float]:
+    """(height f, depth splits, us) of a product of M rows in 256-column tiles of 32 f rows, the least of an estimate: the K-tiles of the
+    rounds that the tiles take on 256 CUs (the last round runs faster the fewer tiles it holds, by up to 40 %), a start and an end
+    per round, the stores, and for a split depth the fp32 slabs read again. Splits are whole numbers of at least 8 K-tiles, within one
+    round. The numbers are a fit to 3900 measured launches (257 to 7072 rows, 1024 to 28672 columns, depths 1024 to 14336; the choice
+    is within 1 % of the best one in the mean). Against 256 rows whatever the size (and the most splits that fit a round): 12 % less in
+    the mean, at most 1.05 x; 2361 x 8192 x 2048 106 -> 95 us, 3360 x 28672 x 4096 618 -> 585, 3360 x 6144 x 4096 160 -> 139."""
+    nk, nt, numbers = K // 64, n_pad // 256, M * n_pad * 1e-6
+    best = (8, 1, float("inf"))
+    for f in ((8,) if full_height else (8, 7, 6, 5, 4)) + ((0,) if four_wave else ()):
+        for s in (1, 2, 3, 4, 6, 7, 8) if f else (1,):
+            tiles = s * nt * -(-M // (32 * f or 256))
+            if s > max_splits or (s > 1 and (tiles > 256 or nk % s or nk // s < 8)):
+                continue
+            full, last = divmod(tiles, 256)
+            least = 0.57 if full else 0.64
+            rounds = full + (least + (1 - least) * (last / 256) ** 0.79 if last else 0.0)
+            us = rounds * (nk // s) * GEMM256_KTILE_US[f] + 4.0 + 2.07 * (full + (last > 0))
+            if s == 1:
+                us += 0.177 * numbers * out_bytes
+            else:
+                us += 0.177 * numbers * 4 * s + (0.117 * numbers * 4 * (s - 1) if deferred else 4.3 + 0.117 * numbers * 4 * s)
+            us *= GEMM256_BIAS.get(f, 1.0)
+            if us < best[2]:
+                best = (f, s, us)
     return best
+
+
+def gemm256_plan(M: int, w: "LinearWeight", out_bytes: int, deferred: bool = False, split: bool = True, four_wave: bool = False) -> Tuple[int, int, float]:
+    """_gemm256_plan under the module's settings: GEMM256_MIN_TILES = 0 keeps every tile at 256 rows and the four-wave kernel wherever
+    its depth allows it."""
+    full = GEMM256_MIN_TILES == 0
+    max_splits = max(1, GEMM256_MAX_SPLITS) if split else 1
+    if full and four_wave and max_splits == 1:
+        return 0, 1, 0.0
+    return _gemm256_plan(M, w.n_pad, w.k, out_bytes, deferred, max_splits, four_wave, full)
 
 
 @dataclass
@@ -300,34 +334,35 @@ def linear(x: torch.Tensor, w: LinearWeight, out_f32: bool = False, defer_reduce
     if M == 0:
         return y
     if M > WS_MAX_M:
-        tiles256 = ((M + 255) // 256) * (w.n_pad // 256)
-        # (the reduction of the split-K slabs works on whole groups of 32 columns)
-        splits = _choose_gemm256_splits(tiles256, w.k) if (w.n_pad % 256 == 0 and not w.swiglu and w.n % 32 == 0) else 1
-        if splits > 1 and GEMM256_MIN_TILES >= 0:
-            # Too few 256x256 tiles to fill the chip (a few hundred rows, narrow output): split K.
-            part = torch.empty(splits, M, w.n, dtype=torch.float32, device=x.device)
-            h.call("lc_gemm256_splitk", w.data.data_ptr(), x.data_ptr(), part.data_ptr(), M, w.n, w.k, w.n_pad, w.n,
-                   splits)
-            if defer_reduce:
-                return PartialSum(part, w.bias)
-            h.call("lc_splitk_reduce", part.data_ptr(), h.ptr(w.bias), y.data_ptr(), splits, M, w.n, out_n,
-                   1 if out_f32 else 0)
-            return y
-        if GEMM256_MIN_TILES >= 0 and w.n_pad % 256 == 0 and tiles256 >= GEMM256_MIN_TILES:
-            # long K (down projections): four waves of 128 x 128 with the accumulators in AGPRs
-            if use_four_wave_gemm(w.k, epi == EPI_F32):
+        if GEMM256_MIN_TILES >= 0 and w.n_pad % 256 == 0 and ((M + 255) // 256) * (w.n_pad // 256) >= GEMM256_MIN_TILES:
+            # (the reduction of the split-K slabs works on whole groups of 32 columns)
+            split = not w.swiglu and w.n % 32 == 0
+            f, splits, us = gemm256_plan(M, w, y.element_size() if not w.swiglu else 1, defer_reduce, split,
+                                         use_four_wave_gemm(w.k, epi == EPI_F32))
+            if splits > 1:
+                # Too few tiles to fill the chip (a few hundred rows, narrow output): split K.
+                part = torch.empty(splits, M, w.n, dtype=torch.float32, device=x.device)
+                h.call("lc_gemm256_splitk", w.data.data_ptr(), x.data_ptr(), part.data_ptr(), M, w.n, w.k, w.n_pad, w.n,
+                       splits, f)
+                if defer_reduce:
+                    return PartialSum(part, w.bias)
+                h.call("lc_splitk_reduce", part.data_ptr(), h.ptr(w.bias), y.data_ptr(), splits, M, w.n, out_n,
+                       1 if out_f32 else 0)
+            elif f == 0:   # long K (down projections): four waves of 128 x 128 with the accumulators in AGPRs
                 h.call("lc_gemm256w", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad,
                        out_n, epi)
             else:
-                rest, splits = _remainder_tiles(M, w) if not w.swiglu and w.n % 32 == 0 else (0, 1)
+                rest, splits = _remainder_tiles(M, w) if split else (0, 1)
+                if rest and w.k // 64 * GEMM256_KTILE_US[8] + GEMM256_REST_US + 0.177e-6 * y.numel() * y.element_size() > us:
+                    rest = 0
                 n_main = w.n_pad - 256 * rest
                 h.call("lc_gemm256", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, min(w.n, n_main), w.k, n_main,
-                       out_n, epi, 0.0, 0.0)
+                       out_n, epi, 0.0, 0.0, 8 if rest else f)
                 if rest:
                     n = w.n - n_main
                     part = torch.empty(splits, M, n, dtype=torch.float32, device=x.device)
                     h.call("lc_gemm256_splitk", w.data.data_ptr() + 2 * n_main * w.k, x.data_ptr(), part.data_ptr(), M, n, w.k,
-                           256 * rest, n, splits)
+                           256 * rest, n, splits, 8)
                     h.call("lc_splitk_reduce", part.data_ptr(), h.ptr(w.bias[n_main:] if w.bias is not None else None),
                            y.data_ptr() + n_main * y.element_size(), splits, M, n, out_n, 1 if out_f32 else 0)
             return y
@@ -348,7 +383,7 @@ def linear(x: torch.Tensor, w: LinearWeight, out_f32: bool = False, defer_reduce
     # a second round of 128-column tiles would start; 256x256 tiles (half as many) do better.
     if M > 128 and not wide and w.n_pad // 128 > 256 and w.n_pad % 256 == 0 and GEMM256_MIN_TILES >= 0:
         h.call("lc_gemm256", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad,
-               out_n, epi, 0.0, 0.0)
+               out_n, epi, 0.0, 0.0, gemm256_plan(M, w, y.element_size(), split=False)[0])
         return y
     kernel, splits, shape = "lc_gemm_panel", _choose_panel_splits(w.n_pad, w.k) if w.n % 32 == 0 else 1, 0
     if wide:
@@ -821,9 +856,9 @@ def experts_on_sorted(x: torch.Tensor, row_index: Optional[torch.Tensor], offset
         # of a percent of the GEMMs' time).
         xs = embed(row_index, x) if row_index is not None else x
         h.call("lc_gemm256_grouped", w_gate_up.data.data_ptr(), w_gate_up.data[0].numel(), xs.data_ptr(), off_ptr,
-               E_local, act.data_ptr(), rows_bound, w_gate_up.n, w_gate_up.k, w_gate_up.n_pad, dff, EPI_SWIGLU)
+               E_local, act.data_ptr(), rows_bound, w_gate_up.n, w_gate_up.k, w_gate_up.n_pad, dff, EPI_SWIGLU, 8)
         h.call("lc_gemm256_grouped", w_down.data.data_ptr(), w_down.data[0].numel(), act.data_ptr(), off_ptr,
-               E_local, y.data_ptr(), rows_bound, w_down.n, w_down.k, w_down.n_pad, d, EPI_BF16)
+               E_local, y.data_ptr(), rows_bound, w_down.n, w_down.k, w_down.n_pad, d, EPI_BF16, 8)
         return y
     h.call(gg, w_gate_up.data.data_ptr(), w_gate_up.data[0].numel(), x.data_ptr(), h.ptr(row_index), off_ptr, E_local,
            act.data_ptr(), rows_bound, w_gate_up.n, w_gate_up.k, w_gate_up.n_pad, dff, EPI_SWIGLU)
@@ -1105,23 +1140,24 @@ def act_linear(x: torch.Tensor, w: LinearWeight, kind: str, act_dtype: torch.dty
         h, epi = _hip(), EPI_RELU2 if kind == "relu2" else EPI_XIELU
         ntw = _kgemm_ntw(w.n_pad, M, False, w.k) if M <= WS_MAX_M else 0
         strip = _strip_tiles(M, w)
-        if ntw or strip or _whole_tiles256(M, w):
+        rows = _whole_tiles256(M, w, 2)
+        if ntw or strip or rows:
             x, y = x.contiguous(), torch.empty(M, w.n, dtype=act_dtype, device=x.device)
             args = (w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, w.n, epi)
             if ntw or strip:
                 h.call("lc_kgemm" if ntw else "lc_gemm_strip", *args, ntw or strip, float(ap), float(an))
             else:
-                h.call("lc_gemm256", *args, float(ap), float(an))
+                h.call("lc_gemm256", *args, float(ap), float(an), rows)
             return y
     return _column_act(linear(x, w, out_f32=True, defer_reduce=True), kind, ap, an, act_dtype)
 
 
-def _whole_tiles256(M: int, w: LinearWeight) -> bool:
-    """Whether a product of M rows is one launch of 256 x 256 tiles whose depth is not split."""
-    if M <= WS_MAX_M or w.n_pad % 256 or GEMM256_MIN_TILES < 0:
-        return False
-    tiles = ((M + 255) // 256) * (w.n_pad // 256)
-    return tiles >= max(GEMM256_MIN_TILES, 1) and _choose_gemm256_splits(tiles, w.k) == 1
+def _whole_tiles256(M: int, w: LinearWeight, out_bytes: int) -> int:
+    """The height (in 32 rows) of the 256-column tiles of a product of M rows that is one launch whose depth is not split, or 0."""
+    if M <= WS_MAX_M or w.n_pad % 256 or GEMM256_MIN_TILES < 0 or ((M + 255) // 256) * (w.n_pad // 256) < max(GEMM256_MIN_TILES, 1):
+        return 0
+    f, splits, _ = gemm256_plan(M, w, out_bytes)
+    return f if splits == 1 else 0
 
 
 def _scan_scratch(B: int, max_len: int, state_floats: int, decay_floats: int, device) -> Optional[torch.Tensor]:
@@ -1497,15 +1533,15 @@ def glu_linear(x: torch.Tensor, w: LinearWeight, kind: str, act_dtype: torch.dty
     64 rows store the gated unit from their accumulators (gelu_tanh, relu); otherwise the fp32 product is gated in a launch of its own, which also sums the slabs
     of a split one."""
     M, n = x.shape[0], w.n // 2
-    strip = _strip_tiles(M, w)
+    strip, rows = _strip_tiles(M, w), _whole_tiles256(M, w, 1)
     if x.is_cuda and w.is_packed and w.tiled and w.bias is None and kind in GLU_EPILOGUES and act_dtype == torch.bfloat16 \
-            and x.dtype == torch.bfloat16 and M > 0 and (strip or _whole_tiles256(M, w)):
+            and x.dtype == torch.bfloat16 and M > 0 and (strip or rows):
         y = _out_block(out, M, n, act_dtype, x.device, "glu_linear")
         ldy = max(y.stride(0), n)
         if ldy % 8 == 0 and y.data_ptr() % 16 == 0:
             x = x.contiguous()
             args = (w.data.data_ptr(), x.data_ptr(), y.data_ptr(), None, M, w.n, w.k, w.n_pad, ldy, GLU_EPILOGUES[kind])
-            _hip().call("lc_gemm_strip" if strip else "lc_gemm256", *args, *((strip,) if strip else ()), 0.0, 0.0)
+            _hip().call(*(("lc_gemm_strip", *args, strip, 0.0, 0.0) if strip else ("lc_gemm256", *args, 0.0, 0.0, rows)))
             return y
     return glu(linear(x, w, out_f32=True, defer_reduce=True), act_dtype, kind, out=out, tiled=w.tiled)
 

@@ -25,15 +25,15 @@ _SIGNATURES = {
     "lc_embed_pool": [_P, _P, _P, _P, _I, _I, _I, _P],
     "lc_l2_normalize": [_P, _P, _I, _I, _P],
     "lc_gemm_tile": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
-    "lc_gemm256": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _P],
+    "lc_gemm256": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _I, _P],
     "lc_gemm256w": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "lc_gemm_panel": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P],
     "lc_gemm_strip": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _P],
     "lc_kgemm": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _F, _P],
     "lc_splitk_reduce": [_P, _P, _P, _I, _I, _I, _I, _I, _P],
     "lc_gemm_grouped": [_P, _L, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P],
-    "lc_gemm256_splitk": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
-    "lc_gemm256_grouped": [_P, _L, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P],
+    "lc_gemm256_splitk": [_P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
+    "lc_gemm256_grouped": [_P, _L, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "lc_gemm_panel_grouped": [_P, _L, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P],
     "lc_gemm_grouped_glu": [_P, _L, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _P, _F, _F, _F, _P],
     "lc_gemm_panel_grouped_glu": [_P, _L, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _P, _F, _F, _F, _P],

@@ -167,6 +167,36 @@ def test_products_of_just_over_a_round_of_tiles(M, N, K):
         assert rel_err(ops.linear(x, lw, out_f32=True), ref_) < 1e-4
 
 
+@pytest.mark.parametrize("f", [8, 7, 6, 5, 4])
+@pytest.mark.parametrize("N,K", [(256, 64), (512, 128), (480, 320), (768, 1088)])
+def test_gemm256_tile_heights(f, N, K):
+    """Tiles of 128 to 256 rows: one to 17 K-tiles, rows that end before, at and behind a tile's edge and its halves, an N that ends
+    inside the last tile, every kind of epilogue, a split depth. An accumulator meets the same products in the same order
+    whatever the height: bit for bit the 256-row tile's, which is checked against the fp32 reference."""
+    from llm_consensus_amd.ops import hip as h
+
+    W, b = bf(rand(N, K, scale=0.5, seed=1) + torch.arange(N)[:, None] * 1e-3), bf(rand(N, seed=2)).to(DEV)
+    lw = ops.LinearWeight.from_dense(W, None, DEV)
+    for M in (1, 16 * f - 1, 16 * f + 1, 32 * f, 32 * f + 1, 64 * f + 3):
+        X = bf(rand(M, K, scale=0.5) + torch.arange(M)[:, None] * 1e-3)
+        want = X.float() @ W.float().t()
+        x = X.to(DEV)
+        for epi, dtype in ((0, torch.bfloat16), (1, torch.float32), (2, torch.bfloat16), (3, torch.bfloat16), (5, torch.bfloat16), (7, torch.bfloat16)):
+            n = N // 2 if epi in (2, 5) else N
+            out = [torch.full((M + 1, n), 7.0, dtype=dtype, device=DEV) for _ in range(2)]
+            for y, height in zip(out, (8, f)):
+                h.call("lc_gemm256", lw.data.data_ptr(), x.data_ptr(), y.data_ptr(), b.data_ptr(), M, N, K, lw.n_pad, n, epi, 0.7, 0.3, height)
+            assert torch.equal(out[0], out[1]), (M, epi)
+            assert torch.equal(out[1][M], torch.full_like(out[1][M], 7.0)), (M, epi)
+            if epi == 1:
+                assert rel_err(out[1][:M], want + b.float().cpu()) < 1e-4
+        if K % 128 == 0:
+            part = torch.full((2 * M + 1, N), 7.0, device=DEV)
+            h.call("lc_gemm256_splitk", lw.data.data_ptr(), x.data_ptr(), part.data_ptr(), M, N, K, lw.n_pad, N, 2, f)
+            assert rel_err(part[:M] + part[M:2 * M], want) < 1e-4
+            assert torch.equal(part[2 * M], torch.full_like(part[2 * M], 7.0))
+
+
 @pytest.mark.parametrize("M", [1, 7, 16, 17, 64])
 @pytest.mark.parametrize("N,K", [(128, 64), (224, 192), (8192, 320), (12288, 4096)])
 def test_gated_products_from_halves_of_two_tiles(M, N, K):

@@ -54,3 +54,20 @@ def test_wide_outputs_of_few_rows_go_by_their_depth():
     assert [ops._kgemm_ntw(28672, 1, True, k) > 0 for k in (64, 256, 512, 4096)] == [False, False, True, True]
     assert [ops._kgemm_ntw(9216, rows, False, 8192) > 0 for rows in (1, 4, 5, 8)] == [True, True, False, False]
     assert all(ops._kgemm_ntw(8192, 8, False, k) > 0 for k in (64, 2048, 8192))
+
+
+def test_gemm256_plan_stays_within_its_kernels():
+    """Every height is one that the kernel has, splits are whole numbers of at least eight K-tiles within one round, and the four-wave
+    kernel comes up only where its depth allows it."""
+    for M in (1, 129, 257, 300, 513, 1500, 2048, 2361, 3001, 7072, 8192, 40000):
+        for n_pad in (256, 512, 2048, 2304, 8448, 28672, 152064):
+            for K in (64, 192, 512, 2048, 3584, 8192, 14336):
+                for four in (False, True):
+                    f, s, us = ops._gemm256_plan(M, n_pad, K, 2, False, 8, four, False)
+                    tiles = (n_pad // 256) * -(-M // (32 * f or 256))
+                    assert f in (4, 5, 6, 7, 8) or (f == 0 and four and s == 1)
+                    assert s == 1 or (tiles * s <= 256 and (K // 64) % s == 0 and K // 64 // s >= 8)
+                    assert us > 0
+    assert ops._gemm256_plan(3001, 2048, 8192, 4, True, 8, False, True)[0] == 8
+    # 320 tiles of 256 rows are a round and a quarter; lower tiles fill two rounds that are shorter
+    assert ops._gemm256_plan(2361, 8192, 2048, 2, False, 8, False, False)[0] < 8
