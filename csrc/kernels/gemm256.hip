@@ -19,10 +19,10 @@ namespace {
 constexpr int G2_BN = 256, G2_BK = 64;
 constexpr int G2_BAND = 4;
 
-// Rows of a tile, and its LDS: three activation stages of 128 bytes a row; the epilogue stages the output
-// tile (256 columns, two bytes each) through the same memory.
+// Rows of a tile, and its LDS: three activation stages of 128 bytes a row; the epilogue stages the output tile through the same
+// memory, all of its 256 columns in bf16 or half of its rows in fp32.
 constexpr int g2_rows(int mf) { return 32 * mf; }
-constexpr int g2_lds(int mf) { return g2_rows(mf) * 512; }
+constexpr int g2_lds(int mf) { return (mf + 1) / 2 * 32 * 1024; }
 
 struct G2Ctx {
   const bf16_t* __restrict__ Wp;
@@ -240,7 +240,41 @@ __global__ __launch_bounds__(512) void gemm256_kernel(const bf16_t* __restrict__
   // as ten K-tiles of math. Instead every wave transposes its sub-tile through a private LDS
   // region (the ring is idle by now) and writes whole rows of it: 16 bytes per lane, 8 (plain)
   // or 16 (SwiGLU) rows of 128 or 64 contiguous bytes per instruction.
-  if constexpr (EPI != EPI_F32) {
+  if constexpr (EPI == EPI_F32) {
+    if ((ldy & 3) == 0 && (tn + 1) * G2_BN <= N) {   // uniform, as below
+      G2_BARRIER();                                    // every wave is past its last ring read
+      // A wave's 64 columns are 256 bytes a row, half of its rows at a time: four whole rows per store instruction. Stored
+      // from the accumulator layout (16 rows of 64 bytes) 2048 x 6144 x 2048 took 61.3 us instead of 57.6, 2361 x 6720 x 2048
+      // 90.4 instead of 83.3, 2048 x 2048 x 8192 in four parts 72.1 instead of 67.7.
+      constexpr int JH = (MF + 1) / 2;
+      char* mine = smem + wave * (JH * 16 * 256);
+      const int g = lane >> 4, r16 = lane & 15;
+      const bf16_t* add = gridDim.y > 1 ? nullptr : bias;
+      float* out = static_cast<float*>(Y) + (static_cast<size_t>(blockIdx.y) * M + mbase) * ldy + nbase + r16 * 4;
+#pragma unroll
+      for (int j0 = 0; j0 < MF; j0 += JH) {
+#pragma unroll
+        for (int j = j0; j < (j0 + JH < MF ? j0 + JH : MF); ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            f32x4 v = acc[i][j];
+            if (add != nullptr) {
+#pragma unroll
+              for (int r = 0; r < 4; ++r) v[r] += bf16_to_f32(add[nbase + i * 16 + 4 * g + r]);
+            }
+            // chunk c of row m lives at position c ^ (m mod 16)
+            *reinterpret_cast<f32x4*>(mine + ((j - j0) * 16 + r16) * 256 + (((i * 4 + g) ^ r16) << 4)) = v;
+          }
+#pragma unroll
+        for (int p = 0; p < (j0 + JH < MF ? JH : MF - j0) * 4; ++p) {
+          const int row = p * 4 + g, m = j0 * 16 + row;
+          const f32x4 v = *reinterpret_cast<const f32x4*>(mine + row * 256 + ((r16 ^ (row & 15)) << 4));
+          if (mbase + m < M) *reinterpret_cast<f32x4*>(out + static_cast<size_t>(m) * ldy) = v;
+        }
+      }
+      return;
+    }
+  } else {
     if ((ldy & 7) == 0 && (tn + 1) * G2_BN <= N) {   // uniform: the whole block tile is inside Y
       G2_BARRIER();                                    // every wave is past its last ring read
       // Staged rows are 128 bytes: a wave's 64 columns, or with SwiGLU the 32 + 32 output
