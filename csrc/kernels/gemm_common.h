@@ -36,11 +36,27 @@ LC_DEVICE float gelu_tanh(float x) { return x / (1.f + __expf(-1.595769121605730
 template <int EPI>
 LC_DEVICE float gate_act(float x) { return EPI == EPI_GEGLU ? gelu_tanh(x) : EPI == EPI_REGLU ? fmaxf(x, 0.f) : silu(x); }
 
+// xielu (common.h) for results that are rounded to bf16, without expm1f's two paths: e^x - 1 - x is x^2 times a polynomial down to
+// -1 (degree 6, fitted at the Chebyshev points of [-1, 0], 1e-8 of the value in exact numbers), the difference itself
+// below. Rounded to bf16 it equals the form with expm1f on 3M normal values. A
+// tile's epilogue holds 128 values a lane: 2361 x 8192 x 2048 115.6 -> 109.2 us (relu^2 98.9), 40 x 8192 x 2048 10.7 -> 10.2.
+LC_DEVICE float xielu_bf16(float x, float ap, float an) {
+  float p = 1.6928126569837332e-05f;
+  p = fmaf(p, x, 1.8832476052921265e-04f);
+  p = fmaf(p, x, 1.3822416076436639e-03f);
+  p = fmaf(p, x, 8.3310501649975780e-03f);
+  p = fmaf(p, x, 4.1666291654109955e-02f);
+  p = fmaf(p, x, 1.6666664183139801e-01f);
+  p = fmaf(p, x, 0.5f);
+  const float near_ = x * x * p, far_ = __expf(x) - 1.f - x;
+  return (x > 0.f ? ap * x * x : an * (x > -1.f ? near_ : far_)) + 0.5f * x;
+}
+
 // The activation of an EPI_RELU2 or EPI_XIELU epilogue (ap, an: the two numbers of xIELU), v itself in the others.
 template <int EPI>
 LC_DEVICE float column_act(float v, float ap, float an) {
   if constexpr (EPI == EPI_RELU2) return relu2(v);
-  if constexpr (EPI == EPI_XIELU) return xielu(v, ap, an);
+  if constexpr (EPI == EPI_XIELU) return xielu_bf16(v, ap, an);
   return v;
 }
 
