@@ -81,7 +81,7 @@ def build_selftest(sanitize: str = "address,undefined") -> Path:
     sanitizer: ``address,undefined`` or ``thread``. Host code only; GPU code is never
     built with sanitizers."""
     src_dir = ROOT / "csrc" / "core"
-    srcs = [s for s in sorted(src_dir.glob("*.cpp")) if s.name != "bindings.cpp"]
+    srcs = [s for s in sorted(src_dir.glob("*.cpp")) if s.name not in ("bindings.cpp", "native_call.cpp")]
     out = BUILD_DIR / ("selftest_" + sanitize.replace(",", "_"))
     BUILD_DIR.mkdir(parents=True, exist_ok=True)
     static = "-static-libtsan" if sanitize == "thread" else "-static-libasan"

@@ -5,6 +5,7 @@
 
 #include "kv_manager.hpp"
 #include "metrics.hpp"
+#include "native_call.hpp"
 #include "placement.hpp"
 #include "prompts.hpp"
 #include "reducers.hpp"
@@ -413,4 +414,10 @@ PYBIND11_MODULE(_core, m) {
       .def("count", &Metrics::count)
       .def("snapshot", &Metrics::snapshot)
       .def("reset", &Metrics::reset);
+
+  m.def("native_call", [](uint64_t address, const std::string& kinds, const std::string& name) {
+    PyObject* f = make_native_call(address, kinds, name);
+    if (f == nullptr) throw py::error_already_set();
+    return py::reinterpret_steal<py::object>(f);
+  });
 }

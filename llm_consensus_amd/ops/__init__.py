@@ -9,7 +9,7 @@ from __future__ import annotations
 import math
 import os
 from dataclasses import dataclass
-from functools import lru_cache
+from functools import cached_property, lru_cache
 from typing import Optional, Tuple
 
 import torch
@@ -117,7 +117,7 @@ class LinearWeight:
     swiglu: bool = False
     tiled: bool = False
 
-    @property
+    @cached_property
     def n_pad(self) -> int:
         return padded_rows(self.n)
 
@@ -1353,13 +1353,13 @@ def attn_masked(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, b
             return [(-1, 1, 0)] if Dv <= cap else []
         n = cap // Dv
         return [(v0, min(n, G - v0), v0 * Dv) for v0 in range(0, G, n)] if n else []
+    h = _hip()
+
     def opts(first: int):
         g = gate[first:] if gate is not None else None
-        return (float(softcap), 1 if (sink or sinks is not None) else 0, _hip().ptr(sinks), _hip().ptr(slopes), int(keep),
-                _hip().ptr(g), max(gate.stride(0), H) if gate is not None else 0, float(out_scale), o_row, int(value_share))
+        return (float(softcap), 1 if (sink or sinks is not None) else 0, h.ptr(sinks), h.ptr(slopes), int(keep),
+                h.ptr(g), max(gate.stride(0), H) if gate is not None else 0, float(out_scale), o_row, int(value_share))
     first = 0
-    # value heads side by side in one tile: equal groups whose width the tiles take (whole MFMA steps of 16 columns)
-    tile_cols = max([n * Dv for n in range(1, nv + 1) if nv % n == 0 and Dv % 8 == 0 and attn_tile_ok(D, n * Dv)] or [0])
     portions = n_portions > 0 and portion_rows > 0 and max_len >= ATTN_TILE_MIN_ROWS
     if portions and not cf and slopes is None and keep == 0 and k_ld % 8 == 0 and v_ld % 8 == 0 and o_row % 4 == 0 and Dv % 8 == 0 and \
             all(t.data_ptr() % 16 == 0 for t in (q, k_cache, v_cache, out)):
@@ -1373,7 +1373,9 @@ def attn_masked(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, b
                         o_row, int(value_share), vh0, nvh, o_ld, col0)
             first, portions = portion_rows, False
     aligned = k_ld % 8 == 0 and v_ld % 8 == 0 and k_cache.data_ptr() % 16 == 0 and v_cache.data_ptr() % 16 == 0
-    if portions and tile_cols and aligned:
+    # value heads side by side in one tile: equal groups whose width the tiles take (whole MFMA steps of 16 columns)
+    tile_cols = max([n * Dv for n in range(1, nv + 1) if nv % n == 0 and Dv % 8 == 0 and attn_tile_ok(D, n * Dv)] or [0]) if portions else 0
+    if tile_cols and aligned:
         for vh0, nvh, col0 in value_groups(tile_cols):
             _hip().call("lc_attn_tile", q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), cf, block_tables.data_ptr(),
                         MB, cu_q.data_ptr(), positions.data_ptr(), out.data_ptr(), af, int(n_portions), int(max_len), H, G,
@@ -1383,17 +1385,19 @@ def attn_masked(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, b
         if Dv > 512:
             raise ValueError("attn_masked: the row kernel takes value widths up to 512")
         line = 4 if cf else 8
-        if k_ld % line == 0 and v_ld % line == 0 and o_row % 4 == 0 and _hip().lib().lc_attn_rows_ok(D, Dv, BS) and \
-                all(t.data_ptr() % 16 == 0 for t in (q[first:], k_cache, v_cache, out[first:])):
-            _hip().call("lc_attn_rows", q[first:].data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), cf, block_tables.data_ptr(), MB,
-                        row_seq[first:].data_ptr(), positions[first:].data_ptr(), out[first:].data_ptr(), af, T - first, H, G, D, Dv,
-                        BS, float(scale), int(chunk), int(window), k_ld, v_ld, *opts(first), 1 if all_value_heads else 0, o_ld)
+        rows, qp, op = T - first, q.data_ptr() + 4 * first * q.stride(0), out.data_ptr() + out.element_size() * first * out.stride(0)
+        seqs, pos = (row_seq, positions) if first == 0 else (row_seq[first:], positions[first:])
+        if k_ld % line == 0 and v_ld % line == 0 and o_row % 4 == 0 and h.lib().lc_attn_rows_ok(D, Dv, BS) and \
+                qp % 16 == 0 and op % 16 == 0 and k_cache.data_ptr() % 16 == 0 and v_cache.data_ptr() % 16 == 0:
+            h.call("lc_attn_rows", qp, k_cache.data_ptr(), v_cache.data_ptr(), cf, block_tables.data_ptr(), MB,
+                   seqs.data_ptr(), pos.data_ptr(), op, af, rows, H, G, D, Dv,
+                   BS, float(scale), int(chunk), int(window), k_ld, v_ld, *opts(first), 1 if all_value_heads else 0, o_ld)
             return out
         # (value heads side by side: a block along z per value head; the short rows' scores are formed again there)
-        _hip().call("lc_attn_masked", q[first:].data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), cf,
-                    block_tables.data_ptr(), MB, row_seq[first:].data_ptr(), positions[first:].data_ptr(),
-                    out[first:].data_ptr(), af, T - first, H, G, D, Dv, BS, float(scale), int(chunk), int(window),
-                    k_ld, v_ld, *opts(first), 0 if all_value_heads else -1, 1, o_ld, 0, nv)
+        h.call("lc_attn_masked", qp, k_cache.data_ptr(), v_cache.data_ptr(), cf,
+               block_tables.data_ptr(), MB, seqs.data_ptr(), pos.data_ptr(),
+               op, af, rows, H, G, D, Dv, BS, float(scale), int(chunk), int(window),
+               k_ld, v_ld, *opts(first), 0 if all_value_heads else -1, 1, o_ld, 0, nv)
     return out
 
 
@@ -1790,7 +1794,7 @@ def hc_step(xs: torch.Tensor, y: Optional[torch.Tensor], mix: Optional[torch.Ten
     T, S, d = xs.shape
     if xs.dtype != torch.float32 or not xs.is_contiguous() or S > MAX_STREAMS:
         raise ValueError(f"hc_step: the streams are a contiguous fp32 [T, S, d] tensor, S <= {MAX_STREAMS}")
-    if y is not None and (not _is_result(y, xs[:, 0]) or mix is None or out_w is None
+    if y is not None and (tuple(y.shape) != (T, d) or not (isinstance(y, PartialSum) or y.dtype == torch.float32) or mix is None or out_w is None
                           or mix.numel() != S * S or out_w.numel() != S):
         raise ValueError("hc_step: an fp32 [T, d] result with mix [S, S] and out [S]")
     if (in_w is not None and in_w.numel() != S) or (norm_w is not None and (in_w is None or norm_w.numel() != d)):
@@ -1805,9 +1809,10 @@ def hc_step(xs: torch.Tensor, y: Optional[torch.Tensor], mix: Optional[torch.Ten
     u = torch.empty(T, d, dtype=torch.float32, device=xs.device) if in_w is not None and norm_w is None else None
     xa = torch.empty(T, d, dtype=act_dtype, device=xs.device) if norm_w is not None else None
     part, parts, bias = _slabs(y, "hc_step", bias=True) if y is not None else (None, 1, None)
-    _hip().call("lc_hc_step", xs.data_ptr(), _hip().ptr(part), parts, _hip().ptr(bias), _hip().ptr(mix),
-                _hip().ptr(out_w), _hip().ptr(in_w), _hip().ptr(norm_w), float(eps), _hip().ptr(u), _hip().ptr(xa),
-                _f32flag(act_dtype) if xa is not None else 0, T, S, d)
+    h = _hip()
+    p = h.ptr
+    h.call("lc_hc_step", xs.data_ptr(), p(part), parts, p(bias), p(mix), p(out_w), p(in_w), p(norm_w), float(eps), p(u), p(xa),
+           _f32flag(act_dtype) if xa is not None else 0, T, S, d)
     return xa if xa is not None else u
 
 

@@ -14,7 +14,7 @@ from typing import Optional
 
 import torch
 
-from .._native import kernels
+from .._native import core, kernels
 
 _P, _I, _F, _L = c_void_p, c_int, c_float, c_longlong
 
@@ -145,9 +145,12 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return t.data_ptr()
 
 
+_raw_stream, _device = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
+
+
 def stream() -> int:
     # the current stream's handle without a Stream object around it: torch.cuda.current_stream() costs 4 us of a launch's 13
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return _raw_stream(_device())
 
 
 # While a list is installed here, every launch is also appended to it as (function, args with
@@ -173,20 +176,37 @@ def stop_recording() -> None:
 _TRACE = os.environ.get("LC_TRACE_LAUNCHES", "0") == "1"
 
 
+# Launchers by name: (callable that takes ints, floats and None without ctypes, the ctypes function for anything else).
+_KINDS = {_P: "P", _I: "I", _L: "L", _F: "F"}
+_launchers: dict = {}
+
+
+def _launcher(name: str):
+    fn = getattr(lib(), name)
+    try:
+        fast = core.native_call(ctypes.cast(fn, c_void_p).value, "".join(_KINDS[t] for t in _SIGNATURES[name]), name)
+    except (KeyError, ValueError):      # argument kinds that the fast way does not take
+        fast = fn
+    _launchers[name] = fast, fn
+    return fast, fn
+
+
 def call(name: str, *args) -> None:
-    fn = getattr(_lib or lib(), name)
+    fast, fn = _launchers.get(name) or _launcher(name)
     st = stream()
     if _TRACE:
         sys.stderr.write(f"[launch] {name} {[a for a in args if isinstance(a, (int, float))][-10:]}\n")
         sys.stderr.flush()
-    rc = fn(*args, st)
+    rc = fast(*args, st)
+    if rc is NotImplemented:
+        fast, rc = fn, fn(*args, st)
     if _TRACE and not torch.cuda.is_current_stream_capturing():
         torch.cuda.synchronize()
     if rc != 0:
         what = "invalid arguments for this kernel" if rc < 0 else f"HIP error {rc}"
         raise KernelLaunchError(f"{name} failed: {what}")
     if _recording is not None:
-        _recording.append((fn, args + (st,), name))
+        _recording.append((fast, args + (st,), name))
 
 
 def replay(cmds: list) -> None:
