@@ -22,6 +22,7 @@ struct AnyGemm {
   int epi;                       // 1: square of relu
   int a_hs, c_hs;                // first column of head h in A and in C
   int ld_gate, gate_full;
+  int c_vec;                     // C's rows and heads start on 16 bytes
   int splits;                    // > 1: part s of the depth leaves its sums in slab s of C (fp32, [M, ldc] each; no bias, epi or gate)
 };
 
@@ -214,6 +215,140 @@ __global__ __launch_bounds__(256 * KG) void gemm_any_tile_kernel(AnyGemm g, cons
         finish_any(g, h, m0 + 32 * wm + 16 * i + 4 * lq + r, n0 + 32 * wn + 16 * j + lr, acc[i][j][r], split);
 }
 
+// ---------------------------------------------------------------- more rows, fp32 throughout
+// The same tiles for fp32 activations and weights whose depth is in whole lines: slabs of 32 depths go
+// from memory to LDS as whole 128-byte rows (LDS-DMA, no registers in between, two stages, one barrier per slab), in an
+// XOR-swizzled image (chunk c of row r lies at c ^ (r mod 8): the source addresses are permuted, the 16-byte reads of eight rows hit
+// all banks). W's rows are the first operand, so that a lane holds four neighbouring outputs of a row. Four sums of every fourth depth
+// keep the rounding of a sum at what up to four depth groups had above.
+// 801 rows: 4096 x 1024 92 -> 82 us (82 TFLOP/s), 32000 x 1024 524 -> 471 (111; registers alone reach 154), 1024 x 4096 in eight parts 78 -> 67;
+// 151 rows, 1024 x 1024 in eight parts 10.5 -> 8.0. The matrix units are busy 77 % of the time, whatever the waves per SIMD (three
+// stages 1 - 3 % either way). Every wave with the whole tile for a quarter of the depth, operands straight into registers: 98 us
+// for the first (256 registers do not hold the sums and two steps).
+constexpr int kLineSlab = 32, kLineStage = 2 * 64 * 128;      // bytes of a stage: A | W, 64 rows of a line each
+
+template <int KG, bool GROUPED>
+__global__ __launch_bounds__(256 * KG) void gemm_f32_tile_kernel(AnyGemm g, const int32_t* __restrict__ row_index,
+                                                                 const int32_t* __restrict__ offsets, int E) {
+  extern __shared__ __attribute__((aligned(16))) char lines[];          // [KG][2][A | W][64][128]
+  const int tid = threadIdx.x & 255, lane = tid & 63;
+  const int kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lq = lane >> 4, wm = wave >> 1, wn = wave & 1;
+  const int n0 = blockIdx.x * 64;
+  const int split = g.splits > 1 ? blockIdx.z : 0;     // (products per head are not split)
+  int m0 = blockIdx.y * 64, h = g.splits > 1 ? 0 : blockIdx.z;
+  size_t w_first = static_cast<size_t>(h) * g.N * g.K;
+  if constexpr (GROUPED) {
+    int e = 0, tile = blockIdx.y, lo = 0, hi = 0;
+    for (; e < E; ++e) {
+      lo = offsets[e];
+      hi = offsets[e + 1];
+      const int nt = (hi - lo + 63) >> 6;
+      if (tile < nt) break;
+      tile -= nt;
+    }
+    if (e >= E) return;                                // the same for the whole block
+    m0 = lo + tile * 64;
+    g.M = hi;
+    w_first = static_cast<size_t>(e) * g.N * g.K;
+  }
+  // this wave's pieces of a slab: rows 8 wave .. + 7 and 32 + 8 wave .. of either operand
+  const int rr = lane >> 3, chunk = ((lane & 7) ^ rr) * 4;
+  const float *asrc[2], *wsrc[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int row = (4 * p + wave) * 8 + rr;
+    int a_at = min(m0 + row, g.M - 1);
+    if (GROUPED && row_index != nullptr) a_at = row_index[a_at];
+    asrc[p] = static_cast<const float*>(g.A) + static_cast<size_t>(a_at) * g.lda + static_cast<size_t>(h) * g.a_hs + chunk;
+    wsrc[p] = static_cast<const float*>(g.W) + w_first + static_cast<size_t>(min(n0 + row, g.N - 1)) * g.K + chunk;
+  }
+  const int groups = KG * g.splits, all = g.K / kLineSlab, per = (all + groups - 1) / groups;
+  const int first = min((split * KG + kg) * per, all), mine = min(per, all - first);
+  char* const stages = lines + kg * 2 * kLineStage;
+  auto issue = [&](int s) {
+    char* dst = stages + (s & 1) * kLineStage;
+    const int k = (first + s) * kLineSlab;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      __builtin_amdgcn_global_load_lds(LC_GLOBAL_PTR(asrc[p] + k), LC_LDS_PTR(dst + (4 * p + wave) * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(LC_GLOBAL_PTR(wsrc[p] + k), LC_LDS_PTR(dst + 64 * 128 + (4 * p + wave) * 1024), 16, 0, 0);
+    }
+  };
+  f32x4 part[4][2][2], acc[2][2];                       // [16 columns][16 rows]; a part sums every fourth depth
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) part[k][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (mine > 0) issue(0);
+  for (int s = 0; s < mine; ++s) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();                       // slab s has landed; whoever is past this has read slab s - 1
+    asm volatile("" ::: "memory");
+    if (s + 1 < mine) issue(s + 1);
+    const char* as = stages + (s & 1) * kLineStage + (32 * wm + lr) * 128;
+    const char* ws = stages + (s & 1) * kLineStage + 64 * 128 + (32 * wn + lr) * 128;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int at = ((4 * t + lq) ^ (lr & 7)) << 4;
+      f32x4 af[2], wf[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        af[i] = *reinterpret_cast<const f32x4*>(as + i * 2048 + at);
+        wf[i] = *reinterpret_cast<const f32x4*>(ws + i * 2048 + at);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) part[k][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][k], af[j][k], part[k][i][j], 0, 0, 0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's reads are over before the stage may be written again
+  }
+  for (int s = max(mine, 0); s < per; ++s) __builtin_amdgcn_s_barrier();   // (every depth group takes every barrier)
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = (part[0][i][j] + part[1][i][j]) + (part[2][i][j] + part[3][i][j]);
+  if constexpr (KG > 1) {
+    __syncthreads();
+    f32x4* red = reinterpret_cast<f32x4*>(lines);       // [KG - 1][4][256]
+    if (kg > 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[((kg - 1) * 4 + i) * 256 + tid] = acc[i >> 1][i & 1];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int q = 0; q < KG - 1; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i >> 1][i & 1] += red[(q * 4 + i) * 256 + tid];
+  }
+  const bool plain = g.bias == nullptr && g.gate == nullptr && g.c_f32 && g.c_vec;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int row = m0 + 32 * wm + 16 * j + lr, col = n0 + 32 * wn + 16 * i + 4 * lq;
+      if (plain && col + 3 < g.N) {
+        if (row >= g.M) continue;
+        f32x4 v = acc[i][j];
+        if (g.epi == 1) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = relu2(v[r]);
+        }
+        const size_t at = (static_cast<size_t>(split) * g.M + row) * g.ldc + static_cast<size_t>(h) * g.c_hs + col;
+        *reinterpret_cast<f32x4*>(static_cast<float*>(g.C) + at) = v;
+        continue;
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) finish_any(g, h, row, col + r, acc[i][j][r], split);
+    }
+}
+
 template <int KG, bool GROUPED>
 int launch_tiles(const AnyGemm& g, const dim3& grid, const int32_t* row_index, const int32_t* offsets, int E, hipStream_t st) {
   constexpr size_t lds = 2 * KG * 2 * 64 * kSlabLd * sizeof(float);
@@ -228,11 +363,24 @@ int launch_tiles(const AnyGemm& g, const dim3& grid, const int32_t* row_index, c
   LC_RETURN_LAST_ERROR();
 }
 
-// Depth groups: enough waves for four on each of the 1024 SIMDs, none shorter than four slabs.
+template <int KG, bool GROUPED>
+int launch_f32_tiles(const AnyGemm& g, const dim3& grid, const int32_t* row_index, const int32_t* offsets, int E, hipStream_t st) {
+  gemm_f32_tile_kernel<KG, GROUPED><<<grid, dim3(256 * KG), 2 * KG * kLineStage, st>>>(g, row_index, offsets, E);
+  LC_RETURN_LAST_ERROR();
+}
+
+// Depth groups: enough waves for four on each of the 1024 SIMDs, none shorter than four slabs. Whole lines of fp32: two groups where they
+// leave no CU a second block (151 rows, 4096 x 1024, 192 blocks, 22.2 -> 20.8 us; 312 blocks 37.1 -> 39.8) or where there are more
+// than two and a depth to share (832 blocks of depth 1024 83.5 -> 82, of 128 10.7 -> 13.9).
 template <bool GROUPED>
 int tiles_any(const AnyGemm& g, int m_tiles, int heads, const int32_t* row_index, const int32_t* offsets, int E, hipStream_t st) {
   const dim3 grid((g.N + 63) / 64, m_tiles, g.splits > 1 ? g.splits : heads);
   const long long blocks = static_cast<long long>(grid.x) * grid.y * grid.z;
+  if (g.a_f32 && g.w_f32 && g.a_vec && g.w_vec && g.K % kLineSlab == 0) {
+    if (blocks <= 256 ? g.K / g.splits >= 256 : blocks > 512 && g.K / g.splits >= 512)
+      return launch_f32_tiles<2, GROUPED>(g, grid, row_index, offsets, E, st);
+    return launch_f32_tiles<1, GROUPED>(g, grid, row_index, offsets, E, st);
+  }
   if (blocks <= 512 && g.K >= 256) return launch_tiles<4, GROUPED>(g, grid, row_index, offsets, E, st);
   if (blocks <= 1024 && g.K >= 128) return launch_tiles<2, GROUPED>(g, grid, row_index, offsets, E, st);
   return launch_tiles<1, GROUPED>(g, grid, row_index, offsets, E, st);
@@ -274,7 +422,7 @@ LC_EXPORT int lc_gemm_any(const void* A, int a_f32, int lda, const void* W, int 
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || lda < K || splits < 1 || splits > 64 || (splits > 1 && (bias != nullptr || epi != 0 || !c_f32))) return -1;
   const AnyGemm g{A, W, bias, C, nullptr, a_f32, w_f32, c_f32, K % 4 == 0 && lda % 4 == 0 && four_border(A, a_f32),
-                  K % 4 == 0 && four_border(W, w_f32), lda, N, M, N, K, epi, 0, 0, 0, 0, splits};
+                  K % 4 == 0 && four_border(W, w_f32), lda, N, M, N, K, epi, 0, 0, 0, 0, N % 4 == 0 && four_border(C, 1), splits};
   return any_product(g, 1, st);
 }
 
@@ -290,7 +438,7 @@ LC_EXPORT int lc_head_linear(const void* A, int a_f32, int lda, const void* W, i
   if (gate == nullptr && gate_full) return -1;
   const AnyGemm g{A, W, nullptr, C, static_cast<const float*>(gate), a_f32, w_f32, c_f32,
                   K % 4 == 0 && lda % 4 == 0 && a_hs % 4 == 0 && four_border(A, a_f32), K % 4 == 0 && four_border(W, w_f32),
-                  lda, c_ld, M, N, K, 0, a_hs, c_hs, ld_gate, gate_full, 1};
+                  lda, c_ld, M, N, K, 0, a_hs, c_hs, ld_gate, gate_full, c_ld % 4 == 0 && c_hs % 4 == 0 && four_border(C, 1), 1};
   return any_product(g, H, st);
 }
 
@@ -303,6 +451,6 @@ LC_EXPORT int lc_gemm_any_grouped(const void* A, int a_f32, int lda, const void*
   const int tiles = (rows + 63) / 64 + E;
   if (tiles > 65535) return -1;
   const AnyGemm g{A, W, nullptr, C, nullptr, a_f32, w_f32, c_f32, K % 4 == 0 && lda % 4 == 0 && four_border(A, a_f32),
-                  K % 4 == 0 && four_border(W, w_f32), lda, N, rows, N, K, epi, 0, 0, 0, 0, 1};
+                  K % 4 == 0 && four_border(W, w_f32), lda, N, rows, N, K, epi, 0, 0, 0, 0, N % 4 == 0 && four_border(C, 1), 1};
   return tiles_any<true>(g, tiles, 1, static_cast<const int32_t*>(row_index), static_cast<const int32_t*>(offsets), E, st);
 }

@@ -1386,6 +1386,46 @@ def test_relu_gated_unit_of_a_product_with_tiled_weights(M, N, K):
     torch.testing.assert_close(ops.glu_linear(x.to(DEV), w, "relu", torch.bfloat16).float().cpu(), want, **_tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 64, 32), (66, 65, 64), (127, 6, 96), (129, 4096, 224), (131, 70, 288), (200, 1000, 1056), (801, 3000, 544)])
+def test_products_of_whole_lines_in_fp32(M, N, K):
+    """Activations and weights in fp32 whose depth is in lines of 128 bytes (LDS-DMA tiles): one to 33 slabs in one and two depth groups, some
+    without a slab, ragged rows and widths, a bias, relu^2, a column slice whose neighbours are no numbers, slabs of a split
+    depth, heads with gates, sorted rows of experts."""
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    tol = dict(atol=1e-5, rtol=1e-5)        # (sums of up to 1056 products around 1 / sqrt(K): a few 1e-7 each side)
+    wide = torch.full((M, K + 8), float("nan"), device=DEV)
+    wide[:, 4:4 + K] = rnd(M, K)
+    x, W, b = wide[:, 4:4 + K], rnd(N, K) / K ** 0.5, rnd(N)
+    want = x.double() @ W.double().T
+    for bias in (None, b):
+        w = ops.LinearWeight.from_dense(W, bias, DEV, dtype=torch.float32, plain=True)
+        full = want if bias is None else want + b.double()
+        torch.testing.assert_close(ops.linear_any(x, w).double(), full, **tol)
+        torch.testing.assert_close(ops.linear_any(x, w, epi_relu2=True).double(), full.clamp(min=0) ** 2, atol=1e-4, rtol=1e-5)
+    from llm_consensus_amd.ops import hip as h
+
+    for splits in (2, 5):
+        part = torch.full((splits * M + 1, N), 7.0, device=DEV)
+        h.call("lc_gemm_any", x.data_ptr(), 1, x.stride(0), W.data_ptr(), 1, None, part.data_ptr(), 1, M, N, K, 0, splits)
+        torch.testing.assert_close(part[:-1].view(splits, M, N).double().sum(0), want, **tol)
+        assert torch.equal(part[-1], torch.full_like(part[-1], 7.0))
+    H = 3
+    xh, Wh, gate = rnd(M, H * K), rnd(H, N, K) / K ** 0.5, rnd(M, H)
+    got = ops.head_linear(xh, Wh, torch.float32, gate)
+    wh = torch.stack([xh[:, i * K:(i + 1) * K].double() @ Wh[i].double().T * torch.sigmoid(gate[:, i:i + 1].double()) for i in range(H)], 1)
+    torch.testing.assert_close(got.double().view(M, H, N), wh, **tol)
+    lens = [0, M // 3, 0, M - M // 3]
+    off = torch.tensor([0, *lens], device=DEV).cumsum(0).to(torch.int32)
+    src = torch.randperm(M, generator=g, device=DEV).to(torch.int32)
+    We = rnd(4, N, K) / K ** 0.5
+    y = ops.grouped_linear(x.contiguous(), src, off, We, torch.float32, M)
+    lo = 0
+    for e, n in enumerate(lens):
+        torch.testing.assert_close(y[lo:lo + n].double(), x[src[lo:lo + n].long()].double() @ We[e].double().T, **tol)
+        lo += n
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 1024, 4096), (3, 100, 3000), (64, 48, 2050), (65, 64, 512), (65, 70, 1030), (130, 1024, 4096), (800, 1000, 2050)])
 @pytest.mark.parametrize("adt", [torch.float32, torch.bfloat16])
 def test_split_products_of_any_shape(M, N, K, adt):
