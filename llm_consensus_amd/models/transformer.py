@@ -265,6 +265,12 @@ class TransformerModel:
             delta = self.comm.all_reduce(delta)
         return ops.rmsnorm(h, w, eps, delta)
 
+    def _norm_linear(self, h: torch.Tensor, delta, w: torch.Tensor, lw, defer_reduce: bool = False):
+        """(the stream with ``delta`` added, the product of its norm with ``lw``)."""
+        if self.tp_size > 1:
+            return h, ops.linear(self._reduce_norm(h, delta, w), lw, defer_reduce=defer_reduce)
+        return ops.norm_linear(h, delta, w, self.cfg.rms_eps, lw, defer_reduce)
+
     def forward(self, token_ids: torch.Tensor, positions: torch.Tensor, slot_mapping: torch.Tensor,
                 meta: AttnMeta, kv: KVCache) -> torch.Tensor:
         """Returns the final-norm hidden states [T, d] for the step's tokens."""
@@ -272,8 +278,7 @@ class TransformerModel:
         h = ops.embed(token_ids, self.embed, meta.token_feed)
         delta = None
         for i, L in enumerate(self.layers):
-            x = self._reduce_norm(h, delta, L.ln1)
-            qkv = ops.linear(x, L.qkv, defer_reduce=True)
+            h, qkv = self._norm_linear(h, delta, L.ln1, L.qkv, defer_reduce=True)
             kc, vc = kv.k(i), kv.vt(i)
             qkv = ops.rope_kv_write(qkv, positions, slot_mapping, self.cos_t, self.sin_t, kc, vc, self.hq, self.hkv,
                                     c.head_dim)
@@ -293,14 +298,17 @@ class TransformerModel:
                 a = ops.attn_decode(qkv, kc, vc, meta.block_tables, meta.ctx_lens, self.hq, self.hkv, c.head_dim,
                                     self.scale, c.sliding_window, meta.nsplit, meta.groups, meta.kv_begin,
                                     meta.max_group_rows, meta.prefix_splits)
-            x2 = self._reduce_norm(h, ops.linear(a, L.o, defer_reduce=True), L.ln2)
-            if c.is_moe and self.ep_size > 1:
+            o = ops.linear(a, L.o, defer_reduce=True)
+            if not c.is_moe:
+                h, g = self._norm_linear(h, o, L.ln2, L.gate_up)
+                delta = ops.linear(g, L.down, defer_reduce=True)
+                continue
+            x2 = self._reduce_norm(h, o, L.ln2)
+            if self.ep_size > 1:
                 delta = moe_ffn_ep(x2, L.router, L.experts_gate_up, L.experts_down, c.experts_per_tok, self.comm,
                                    self.expert_lo, self.ep_mode)
-            elif c.is_moe:
-                delta = ops.moe_ffn(x2, L.router, L.experts_gate_up, L.experts_down, c.experts_per_tok)
             else:
-                delta = ops.linear(ops.linear(x2, L.gate_up), L.down, defer_reduce=True)
+                delta = ops.moe_ffn(x2, L.router, L.experts_gate_up, L.experts_down, c.experts_per_tok)
         return self._reduce_norm(h, delta, self.final_norm)
 
     def logits(self, hidden_rows: torch.Tensor) -> torch.Tensor:

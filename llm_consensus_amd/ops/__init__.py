@@ -442,6 +442,39 @@ def rmsnorm(hstate: torch.Tensor, w: torch.Tensor, eps: float, delta=None) -> to
     return y
 
 
+NORM_LINEAR_MAX_M = 4
+
+
+def _norm_linear_ntw(M: int, w: LinearWeight) -> int:
+    """n-tiles per workgroup for a norm and the product of its rows in one launch (kgemm.hip), or 0 for two launches. Plain products of up
+    to four rows that the split-in-the-workgroup kernel takes anyway (one row 1.1 - 2 us less than in two launches, four rows 0.4 - 1.1), and
+    gated ones of rows below 4096 (2 - 5.5 us less; 28672 x 4096 the same, 57344 x 8192 9 more), where below 1024 two rows are the most
+    (9728 x 896 8.0 -> 7.4 at one, 8.1 -> 8.5 at four)."""
+    if not 0 < M <= NORM_LINEAR_MAX_M or w.k > 8192 or M * w.k > 24576:
+        return 0
+    if KGEMM_FORCE_NTW >= 0 or not w.swiglu:
+        ntw = _kgemm_ntw(w.n_pad, M, w.swiglu, w.k)
+        return ntw if ntw in (1, 2) else 0
+    return 2 if w.k < 4096 and (w.k >= 1024 or M <= 2) else 0
+
+
+def norm_linear(hstate: torch.Tensor, delta, gain: torch.Tensor, eps: float, w: LinearWeight, defer_reduce: bool = False):
+    """(the residual stream with ``delta`` added, linear(RMSNorm(stream) * gain, w)). The stream comes back as a tensor that may or may not
+    be ``hstate`` updated in place. A few rows are one launch (every workgroup forms the norm while its first weights are on
+    their way); otherwise ``rmsnorm`` and ``linear``."""
+    M, d = hstate.shape
+    ntw = _norm_linear_ntw(M, w) if hstate.is_cuda and w.is_packed and w.k == d else 0
+    if ntw and hstate.dtype == gain.dtype == torch.bfloat16 and hstate.is_contiguous() and \
+            (delta is None or (isinstance(delta, torch.Tensor) and delta.dtype == torch.bfloat16 and delta.shape == hstate.shape and delta.is_contiguous())):
+        h, out_n = _hip(), w.n // 2 if w.swiglu else w.n
+        y = torch.empty(M, out_n, dtype=torch.bfloat16, device=hstate.device)
+        x = torch.empty_like(hstate) if delta is not None else hstate
+        h.call("lc_kgemm_norm", w.data.data_ptr(), hstate.data_ptr(), h.ptr(delta), gain.data_ptr(), x.data_ptr(), float(eps), y.data_ptr(),
+               h.ptr(w.bias), M, w.n, w.k, w.n_pad, out_n, EPI_SWIGLU if w.swiglu else EPI_BF16, ntw)
+        return x, y
+    return hstate, linear(rmsnorm(hstate, gain, eps, delta), w, defer_reduce=defer_reduce)
+
+
 def embed_pool(hidden: torch.Tensor, cu: torch.Tensor, mode: int = 0) -> torch.Tensor:
     """Pooled, L2-normalised embeddings of the sequences whose rows are [cu[s], cu[s+1])
     (mode 0: mean, 1: last row)."""

@@ -25,6 +25,7 @@ _SIGNATURES = {
     "lc_embed_pool": [_P, _P, _P, _P, _I, _I, _I, _P],
     "lc_l2_normalize": [_P, _P, _I, _I, _P],
     "lc_gemm_tile": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
+    "lc_kgemm_norm": [_P, _P, _P, _P, _P, _F, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P],
     "lc_gemm256": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _I, _P],
     "lc_gemm256w": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
     "lc_gemm_panel": [_P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P],

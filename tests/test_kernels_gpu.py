@@ -197,6 +197,42 @@ def test_gemm256_tile_heights(f, N, K):
             assert torch.equal(part[2 * M], torch.full_like(part[2 * M], 7.0))
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("N,K,gated", [(128, 64, False), (224, 192, True), (1152, 896, False), (8192, 2048, False), (18464, 1088, True), (33000, 128, False),
+                                       (640, 2112, True), (96, 4160, False), (64, 6144, True)])
+def test_norm_and_product_in_one_launch(M, N, K, gated):
+    """One and two n-tiles per workgroup, tiles in turn (more than 512), waves without a k-tile, rows of one, two and four chunks per
+    thread, with and without an addend and a bias: the stream and the normed rows are rmsnorm's bit for bit, the product its
+    split-in-the-workgroup one's where the same number of tiles a workgroup is forced."""
+    W, b = bf(rand(N, K, scale=K ** -0.5, seed=1)), bf(rand(N, seed=2))
+    hs, d, gain = bf(rand(M, K, seed=3)).to(DEV), bf(rand(M, K, seed=4)).to(DEV), bf(1.0 + 0.1 * rand(K, seed=5)).to(DEV)
+    old = ops.KGEMM_FORCE_NTW
+    from llm_consensus_amd.ops import hip
+
+    try:
+        for bias in (None, b):
+            lw = ops.LinearWeight.from_dense(W, bias, DEV, swiglu=gated)
+            for ntw in (1, 2):
+                ops.KGEMM_FORCE_NTW = ntw
+                for delta in (None, d):
+                    h0, h1 = hs.clone(), hs.clone()
+                    rec = hip.start_recording()
+                    x, y = ops.norm_linear(h0, delta, gain, 1e-5, lw)
+                    hip.stop_recording()
+                    assert [n for _, _, n in rec] == ["lc_kgemm_norm"]
+                    want = ops.linear(ops.rmsnorm(h1, gain, 1e-5, delta), lw)
+                    assert torch.equal(x, h1) and torch.equal(h0, hs)
+                    assert torch.equal(y, want)
+            ops.KGEMM_FORCE_NTW = -1
+            h1 = hs.clone()
+            x, y = ops.norm_linear(hs.clone(), d, gain, 1e-5, lw)
+            ref_ = ops.linear(ops.rmsnorm(h1, gain, 1e-5, d), lw)
+            assert torch.equal(x, h1) and rel_err(y, ref_.reduce() if isinstance(ref_, ops.PartialSum) else ref_) < 6e-3
+    finally:
+        hip.stop_recording()
+        ops.KGEMM_FORCE_NTW = old
+
+
 @pytest.mark.parametrize("M", [1, 7, 16, 17, 64])
 @pytest.mark.parametrize("N,K", [(128, 64), (224, 192), (8192, 320), (12288, 4096)])
 def test_gated_products_from_halves_of_two_tiles(M, N, K):
