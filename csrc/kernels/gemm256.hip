@@ -365,10 +365,10 @@ static int g2_launch(const void* Wp, const void* X, void* Y, const void* bias, i
   LC_RETURN_LAST_ERROR();
 }
 
-template <int EPI, bool GROUPED = false>
+template <int EPI>
 static int g2_rows_launch(int mf, const void* Wp, const void* X, void* Y, const void* bias, int M, int N, int K, int n_pad, int ldy,
-                          int splits, long long expert_stride, const void* offsets, int E, float ap, float an, hipStream_t stream) {
-#define G2_MF(F) g2_launch<EPI, GROUPED, F>(Wp, X, Y, bias, M, N, K, n_pad, ldy, splits, expert_stride, offsets, E, ap, an, stream)
+                          int splits, float ap, float an, hipStream_t stream) {
+#define G2_MF(F) g2_launch<EPI, false, F>(Wp, X, Y, bias, M, N, K, n_pad, ldy, splits, 0, nullptr, 0, ap, an, stream)
   switch (mf) {
     case 8: return G2_MF(8);
     case 7: return G2_MF(7);
@@ -386,7 +386,7 @@ LC_EXPORT int lc_gemm256(const void* Wp, const void* X, void* Y, const void* bia
   if (M <= 0) return 0;
   if (K % 64 || n_pad % 256 || N > n_pad) return -1;
 #define G2_EPI(E) \
-  case E: return g2_rows_launch<E>(mf, Wp, X, Y, bias, M, N, K, n_pad, ldy, 1, 0, nullptr, 0, ap, an, stream)
+  case E: return g2_rows_launch<E>(mf, Wp, X, Y, bias, M, N, K, n_pad, ldy, 1, ap, an, stream)
   switch (epi) {
     G2_EPI(EPI_BF16);
     G2_EPI(EPI_F32);
@@ -401,18 +401,17 @@ LC_EXPORT int lc_gemm256(const void* Wp, const void* X, void* Y, const void* bia
 }
 
 // Grouped form over E experts for prefill-sized MoE batches: X [total_rows, K] and Y are in
-// expert-sorted row order, offsets [E+1] delimit the experts' rows. Requirements as lc_gemm256.
+// expert-sorted row order, offsets [E+1] delimit the experts' rows. Requirements as lc_gemm256. Tiles of 256 rows whatever the experts
+// get: lower ones pad less, and lose all the same (8 experts of 28672 x 4096, 4316 routed rows 1018 us, 1055 with 224 rows, 1241 with 160).
 LC_EXPORT int lc_gemm256_grouped(const void* Wp_all, long long expert_stride, const void* X, const void* offsets,
-                                 int E, void* Y, int total_rows, int N, int K, int n_pad, int ldy, int epi, int mf,
+                                 int E, void* Y, int total_rows, int N, int K, int n_pad, int ldy, int epi,
                                  hipStream_t stream) {
   if (total_rows <= 0) return 0;
   if (K % 64 || n_pad % 256 || N > n_pad || E < 1) return -1;
   if (epi == EPI_BF16)
-    return g2_rows_launch<EPI_BF16, true>(mf, Wp_all, X, Y, nullptr, total_rows, N, K, n_pad, ldy, 1, expert_stride, offsets, E, 0.f,
-                                          0.f, stream);
+    return g2_launch<EPI_BF16, true, 8>(Wp_all, X, Y, nullptr, total_rows, N, K, n_pad, ldy, 1, expert_stride, offsets, E, 0.f, 0.f, stream);
   if (epi == EPI_SWIGLU)
-    return g2_rows_launch<EPI_SWIGLU, true>(mf, Wp_all, X, Y, nullptr, total_rows, N, K, n_pad, ldy, 1, expert_stride, offsets, E, 0.f,
-                                            0.f, stream);
+    return g2_launch<EPI_SWIGLU, true, 8>(Wp_all, X, Y, nullptr, total_rows, N, K, n_pad, ldy, 1, expert_stride, offsets, E, 0.f, 0.f, stream);
   return -2;
 }
 
@@ -422,5 +421,5 @@ LC_EXPORT int lc_gemm256_splitk(const void* Wp, const void* X, void* Y, int M, i
                                 int splits, int mf, hipStream_t stream) {
   if (M <= 0) return 0;
   if (K % 64 || n_pad % 256 || N > n_pad || splits < 1 || (K / G2_BK) % splits) return -1;
-  return g2_rows_launch<EPI_F32>(mf, Wp, X, Y, nullptr, M, N, K, n_pad, ldy, splits, 0, nullptr, 0, 0.f, 0.f, stream);
+  return g2_rows_launch<EPI_F32>(mf, Wp, X, Y, nullptr, M, N, K, n_pad, ldy, splits, 0.f, 0.f, stream);
 }
