@@ -1,7 +1,7 @@
-// Products of up to 64 rows whose result passes through an activation: Y[M, .] = act(X[M, K] * W[N, K]^T), in one launch.
+// Products of up to 64 rows in one launch, whose result may pass through an activation: Y[M, .] = act(X[M, K] * W[N, K]^T).
 //
-// The panel kernel (gemm_panel.hip) gives a workgroup 128 columns. An output of 4096 to 16384 columns then fills the CUs only with
-// its depth split over workgroups, and the activation needs another launch that adds up the fp32 slabs. Here a workgroup has
+// The panel kernel (gemm_panel.hip) gives a workgroup 128 columns. An output of up to 16384 columns then fills the CUs only with
+// its depth split over workgroups, and the activation (or a plain result) needs another launch that adds up the fp32 slabs. Here a workgroup has
 // 32 or 64 columns over the whole depth (as many as it takes for 128 to 256 workgroups), so that the activation of a
 // column, or of the gate and up tiles next to each other, is applied to the accumulators.
 //
@@ -165,6 +165,8 @@ int launch_strip(int epi, const bf16_t* w, const bf16_t* x, void* Y, const bf16_
     break;                                                                                                                             \
   }
   switch (epi) {
+    GS_CASE(EPI_BF16)
+    GS_CASE(EPI_F32)
     GS_CASE(EPI_SWIGLU)
     GS_CASE(EPI_GEGLU)
     GS_CASE(EPI_REGLU)
@@ -178,7 +180,7 @@ int launch_strip(int epi, const bf16_t* w, const bf16_t* x, void* Y, const bf16_
 
 }  // namespace
 
-// Y = act(X * W^T + bias) of 1 to 64 rows (the gated epilogues without a bias read n-tiles that alternate gate / up). ``tiles``: column
+// Y = act(X * W^T + bias) of 1 to 64 rows, in bf16, or plain in fp32 (the gated epilogues without a bias read n-tiles that alternate gate / up). ``tiles``: column
 // tiles of 16 per workgroup, 2 or 4. Requirements: K % 64 == 0, n_pad % 64 == 0.
 LC_EXPORT int lc_gemm_strip(const void* Wp, const void* X, void* Y, const void* bias, int M, int N, int K, int n_pad, int ldy, int epi, int tiles,
                             float ap, float an, hipStream_t stream) {

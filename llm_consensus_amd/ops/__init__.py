@@ -388,7 +388,10 @@ def linear(x: torch.Tensor, w: LinearWeight, out_f32: bool = False, defer_reduce
     kernel, splits, shape = "lc_gemm_panel", _choose_panel_splits(w.n_pad, w.k) if w.n % 32 == 0 else 1, 0
     if wide:
         shape = 2
-    strip = _strip_tiles(M, w) if w.swiglu and splits > 1 else 0
+    # A product whose slabs nobody sums on the way would need a launch that does. 32 rows in fp32, weights from HBM: 1024 x 1024 7.1 -> 5.2
+    # us, 5376 x 2048 10.7 -> 8.3, 12288 x 2048 16.8 -> 12.1, 8192 x 4096 19.2 -> 15.7 (4096 x 4096 13.7 and 13.3, 6144 x 4096 15.3 and 14.7 at
+    # 32 rows, 12.6 and 13.2 at 16: too few workgroups for so long a depth)
+    strip = _strip_tiles(M, w) if splits > 1 and (w.swiglu or (not defer_reduce and (w.k <= 2048 or w.n_pad >= 8192))) else 0
     if strip:
         h.call("lc_gemm_strip", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, out_n, epi, strip, 0.0, 0.0)
         return y
@@ -889,9 +892,9 @@ def experts_on_sorted(x: torch.Tensor, row_index: Optional[torch.Tensor], offset
         # of a percent of the GEMMs' time).
         xs = embed(row_index, x) if row_index is not None else x
         h.call("lc_gemm256_grouped", w_gate_up.data.data_ptr(), w_gate_up.data[0].numel(), xs.data_ptr(), off_ptr,
-               E_local, act.data_ptr(), rows_bound, w_gate_up.n, w_gate_up.k, w_gate_up.n_pad, dff, EPI_SWIGLU, 8)
+               E_local, act.data_ptr(), rows_bound, w_gate_up.n, w_gate_up.k, w_gate_up.n_pad, dff, EPI_SWIGLU)
         h.call("lc_gemm256_grouped", w_down.data.data_ptr(), w_down.data[0].numel(), act.data_ptr(), off_ptr,
-               E_local, y.data_ptr(), rows_bound, w_down.n, w_down.k, w_down.n_pad, d, EPI_BF16, 8)
+               E_local, y.data_ptr(), rows_bound, w_down.n, w_down.k, w_down.n_pad, d, EPI_BF16)
         return y
     h.call(gg, w_gate_up.data.data_ptr(), w_gate_up.data[0].numel(), x.data_ptr(), h.ptr(row_index), off_ptr, E_local,
            act.data_ptr(), rows_bound, w_gate_up.n, w_gate_up.k, w_gate_up.n_pad, dff, EPI_SWIGLU)

@@ -233,6 +233,28 @@ def test_norm_and_product_in_one_launch(M, N, K, gated):
         ops.KGEMM_FORCE_NTW = old
 
 
+@pytest.mark.parametrize("M", [9, 31, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(96, 512), (1120, 896), (5344, 2048), (8224, 512), (8192, 4096)])
+def test_whole_products_of_strips(M, N, K):
+    """Results of a split depth that nobody sums on the way: ragged rows and columns, both types, a bias, both widths of a strip."""
+    from llm_consensus_amd.ops import hip
+
+    X, W, b = bf(rand(M, K, scale=0.5)), bf(rand(N, K, scale=0.5, seed=1)), bf(rand(N, seed=2))
+    want = ref.linear(X, W, None, torch.float32)
+    x = X.to(DEV)
+    for bias in (None, b):
+        lw = ops.LinearWeight.from_dense(W, bias, DEV)
+        full = want if bias is None else want + b.float()
+        rec = hip.start_recording()
+        try:
+            y, y32 = ops.linear(x, lw), ops.linear(x, lw, out_f32=True)
+        finally:
+            hip.stop_recording()
+        few_wide = M <= ops.KGEMM_SHORT_K_MAX_M and N > 8192
+        assert {n for _, _, n in rec} == {"lc_kgemm" if few_wide else "lc_gemm_strip"}
+        assert rel_err(y, full) < 6e-3 and rel_err(y32, full) < 1e-4
+
+
 @pytest.mark.parametrize("M", [1, 7, 16, 17, 64])
 @pytest.mark.parametrize("N,K", [(128, 64), (224, 192), (8192, 320), (12288, 4096)])
 def test_gated_products_from_halves_of_two_tiles(M, N, K):
