@@ -19,6 +19,9 @@
 // columns half the rows and one of the two k-steps of every K-tile; the two halves of the sum meet in the LDS at the end.
 // Operand conventions as in gemm_panel.hip.
 //
+// A plain fp32 product may come in parts of the depth (blockIdx.y), one slab each: with a quarter of a panel's columns and four times its
+// depth a workgroup reads as many weights and leaves a quarter of the slabs (ops._strip_splits).
+//
 // One MI355X, weights from HBM (16384 x 2048: 10.3 us at 6.5 TB/s), split product and activation before, and now: gated 16384 x 2048 at
 // 8, 32, 64 rows 15.6, 20.1, 21.4 us -> 13.3, 13.4, 14.3; relu^2 8192 x 2048 at 32 rows 13.6 -> 8.7.
 #include "gemm_common.h"
@@ -56,14 +59,15 @@ __global__ __launch_bounds__(256) void gemm_strip_kernel(const bf16_t* __restric
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int nt0 = static_cast<int>(blockIdx.x) * NTB, KT = K / 32, nk = K / GS_BK;
+  const int nt0 = static_cast<int>(blockIdx.x) * NTB, KT = K / 32;
+  const int nk = K / GS_BK / static_cast<int>(gridDim.y), kt0 = static_cast<int>(blockIdx.y) * nk;   // this workgroup's K-tiles
 
   // KiB piece q * 4 + wave of a stage: the weights' fragments (n-tile, k-step), then eight rows of 128 bytes each, swizzled on the source side
   const bf16_t* wsrc[S::WP];
 #pragma unroll
   for (int q = 0; q < S::WP; ++q) {
     const int f = q * 4 + wave;
-    wsrc[q] = Wp + (static_cast<size_t>(nt0 + (f >> 1)) * KT + (f & 1)) * 512 + lane * 8;
+    wsrc[q] = Wp + (static_cast<size_t>(nt0 + (f >> 1)) * KT + 2 * kt0 + (f & 1)) * 512 + lane * 8;
   }
   const bf16_t* xsrc[S::XP];
   const int rr = lane >> 3, lc = lane & 7;
@@ -71,7 +75,7 @@ __global__ __launch_bounds__(256) void gemm_strip_kernel(const bf16_t* __restric
   for (int q = 0; q < S::XP; ++q) {
     int row = (q * 4 + wave) * 8 + rr;
     row = row < M ? row : M - 1;
-    xsrc[q] = X + static_cast<size_t>(row) * K + ((lc ^ rr) << 3);
+    xsrc[q] = X + static_cast<size_t>(row) * K + kt0 * GS_BK + ((lc ^ rr) << 3);
   }
   auto issue = [&](int t) {
     if (t >= nk) return;
@@ -143,17 +147,17 @@ __global__ __launch_bounds__(256) void gemm_strip_kernel(const bf16_t* __restric
       store_tile<EPI>(acc[0][j], &acc[1][j], Y, bias, m0, nbase, M, N, ldy, lane, 0);
     } else {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) store_tile<EPI>(acc[i][j], nullptr, Y, bias, m0, nbase + i * 16, M, N, ldy, lane, 0, ap, an);
+      for (int i = 0; i < 2; ++i) store_tile<EPI>(acc[i][j], nullptr, Y, bias, m0, nbase + i * 16, M, N, ldy, lane, EPI == EPI_F32 ? static_cast<size_t>(blockIdx.y) * M * ldy : 0, ap, an);
     }
   }
 }
 
 template <int NTB, int BM>
 int launch_strip(int epi, const bf16_t* w, const bf16_t* x, void* Y, const bf16_t* b, int M, int N, int K, int n_pad, int ldy, float ap, float an,
-                 hipStream_t stream) {
+                 int splits, hipStream_t stream) {
   using S = StripShape<NTB, BM>;
   constexpr int lds = S::NSTAGE * S::STAGE;
-  const dim3 grid(n_pad / (16 * NTB)), block(256);
+  const dim3 grid(n_pad / (16 * NTB), splits), block(256);
 #define GS_CASE(E)                                                                                                                     \
   case E: {                                                                                                                            \
     static LcDeviceOnce once;                                                                                                          \
@@ -181,16 +185,17 @@ int launch_strip(int epi, const bf16_t* w, const bf16_t* x, void* Y, const bf16_
 }  // namespace
 
 // Y = act(X * W^T + bias) of 1 to 64 rows, in bf16, or plain in fp32 (the gated epilogues without a bias read n-tiles that alternate gate / up). ``tiles``: column
-// tiles of 16 per workgroup, 2 or 4. Requirements: K % 64 == 0, n_pad % 64 == 0.
+// tiles of 16 per workgroup, 2 or 4. ``splits`` > 1 (fp32, no bias): Y is [splits, M, ldy], the sums of as many parts of the depth. Requirements: K % 64 == 0, n_pad % 64 == 0.
 LC_EXPORT int lc_gemm_strip(const void* Wp, const void* X, void* Y, const void* bias, int M, int N, int K, int n_pad, int ldy, int epi, int tiles,
-                            float ap, float an, hipStream_t stream) {
+                            float ap, float an, int splits, hipStream_t stream) {
   if (M <= 0) return 0;
   if (M > 64 || K <= 0 || K % 64 || n_pad % 64 || N > n_pad || N <= 0 || (tiles != 2 && tiles != 4)) return -1;
   if (epi_gated(epi) && N % 32) return -1;
+  if (splits < 1 || (K / GS_BK) % splits || (splits > 1 && (epi != EPI_F32 || bias != nullptr))) return -1;
   auto w = static_cast<const bf16_t*>(Wp);
   auto x = static_cast<const bf16_t*>(X);
   auto b = static_cast<const bf16_t*>(bias);
-#define GS_GO(T, B) launch_strip<T, B>(epi, w, x, Y, b, M, N, K, n_pad, ldy, ap, an, stream)
+#define GS_GO(T, B) launch_strip<T, B>(epi, w, x, Y, b, M, N, K, n_pad, ldy, ap, an, splits, stream)
   if (tiles == 4) return M <= 32 ? GS_GO(4, 32) : GS_GO(4, 64);
   return M <= 32 ? GS_GO(2, 32) : GS_GO(2, 64);
 #undef GS_GO

@@ -191,6 +191,22 @@ def _strip_tiles(M: int, w: "LinearWeight") -> int:
     return 4 if w.n_pad > 8192 else 2
 
 
+STRIP_SPLIT_MAX_M = 32
+
+
+def _strip_splits(n_pad: int, K: int) -> Tuple[int, int]:
+    """(column tiles of 16 per workgroup, parts of the depth) of a plain product of 9 to 32 rows whose 128-column panels would be split: strips
+    leave half and fewer of the panels' slabs to the consumer for the same number of workgroups. Two tiles (32 columns) up to 2048 columns,
+    up to 4096 at depths of 8192, four beyond; as many parts of at least four K-tiles as one round of the CUs holds. 32 rows, weights
+    from HBM, a norm that sums the slabs included: 2048 x 8192 14.0 us in 16 panels' slabs, 12.1 in 4 strips'; 2048 x 2048 9.0 -> 7.5; 4096 x
+    4096 14.9 -> 12.9 (14.3 with four tiles), 3584 x 18944 30.7 -> 27.9 (31.3 with two), 4096 x 14336 27.4 -> 24.3, 6144 x 4096 18.9 -> 18.2
+    (18.8). With 33 to 64 rows, stages of twice the activations, 6144 x 4096 20.8 -> 20.0 and 3584 x 18944 32.7 -> 32.8: a Mixtral step of 48 rows
+    gained nothing. 4608 x 3584 at 16 rows takes 8.5 us in 7 panels' slabs, 10.5 in 144 strips, 8.1 in 504; a step of sixteen 7B chats is fastest with 144."""
+    t = 2 if n_pad <= 2048 or (n_pad <= 4096 and K <= 8192) else 4
+    blocks, nk = n_pad // (16 * t), K // 64
+    return t, max(s for s in (1, 2, 3, 4, 5, 6, 7, 8, 12, 14, 16) if s == 1 or (blocks * s <= PANEL_MAX_BLOCKS and nk % s == 0 and nk // s >= PANEL_MIN_KTILES))
+
+
 def _choose_panel_splits(n_pad: int, K: int) -> int:
     """K splits of the panel kernel (gemm_panel.hip): as many workgroups as possible WITHOUT
     exceeding the 256 CUs (more would share some CUs and their way to memory, and bring slabs);
@@ -393,15 +409,23 @@ def linear(x: torch.Tensor, w: LinearWeight, out_f32: bool = False, defer_reduce
     # 32 rows, 12.6 and 13.2 at 16: too few workgroups for so long a depth)
     strip = _strip_tiles(M, w) if splits > 1 and (w.swiglu or (not defer_reduce and (w.k <= 2048 or w.n_pad >= 8192))) else 0
     if strip:
-        h.call("lc_gemm_strip", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, out_n, epi, strip, 0.0, 0.0)
+        h.call("lc_gemm_strip", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, out_n, epi, strip, 0.0, 0.0, 1)
         return y
     if splits == 1:
         h.call(kernel, w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, out_n, epi, 1,
                shape)
         return y
-    part = torch.empty(splits, M, w.n, dtype=torch.float32, device=x.device)
-    h.call(kernel, w.data.data_ptr(), x.data_ptr(), part.data_ptr(), None, M, w.n, w.k, w.n_pad, w.n, EPI_F32, splits,
-           shape)
+    if M <= STRIP_SPLIT_MAX_M and not w.swiglu:
+        tiles, splits = _strip_splits(w.n_pad, w.k)
+        if splits == 1:
+            h.call("lc_gemm_strip", w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, out_n, epi, tiles, 0.0, 0.0, 1)
+            return y
+        part = torch.empty(splits, M, w.n, dtype=torch.float32, device=x.device)
+        h.call("lc_gemm_strip", w.data.data_ptr(), x.data_ptr(), part.data_ptr(), None, M, w.n, w.k, w.n_pad, w.n, EPI_F32, tiles, 0.0, 0.0, splits)
+    else:
+        part = torch.empty(splits, M, w.n, dtype=torch.float32, device=x.device)
+        h.call(kernel, w.data.data_ptr(), x.data_ptr(), part.data_ptr(), None, M, w.n, w.k, w.n_pad, w.n, EPI_F32, splits,
+               shape)
     if defer_reduce and not w.swiglu:
         return PartialSum(part, w.bias)
     mode = 2 if w.swiglu else (1 if out_f32 else 0)
@@ -1181,7 +1205,7 @@ def act_linear(x: torch.Tensor, w: LinearWeight, kind: str, act_dtype: torch.dty
             x, y = x.contiguous(), torch.empty(M, w.n, dtype=act_dtype, device=x.device)
             args = (w.data.data_ptr(), x.data_ptr(), y.data_ptr(), h.ptr(w.bias), M, w.n, w.k, w.n_pad, w.n, epi)
             if ntw or strip:
-                h.call("lc_kgemm" if ntw else "lc_gemm_strip", *args, ntw or strip, float(ap), float(an))
+                h.call(*(("lc_kgemm", *args, ntw, float(ap), float(an)) if ntw else ("lc_gemm_strip", *args, strip, float(ap), float(an), 1)))
             else:
                 h.call("lc_gemm256", *args, float(ap), float(an), rows)
             return y
@@ -1581,7 +1605,7 @@ def glu_linear(x: torch.Tensor, w: LinearWeight, kind: str, act_dtype: torch.dty
         if ldy % 8 == 0 and y.data_ptr() % 16 == 0:
             x = x.contiguous()
             args = (w.data.data_ptr(), x.data_ptr(), y.data_ptr(), None, M, w.n, w.k, w.n_pad, ldy, GLU_EPILOGUES[kind])
-            _hip().call(*(("lc_gemm_strip", *args, strip, 0.0, 0.0) if strip else ("lc_gemm256", *args, 0.0, 0.0, rows)))
+            _hip().call(*(("lc_gemm_strip", *args, strip, 0.0, 0.0, 1) if strip else ("lc_gemm256", *args, 0.0, 0.0, rows)))
             return y
     return glu(linear(x, w, out_f32=True, defer_reduce=True), act_dtype, kind, out=out, tiled=w.tiled)
 

@@ -233,6 +233,27 @@ def test_norm_and_product_in_one_launch(M, N, K, gated):
         ops.KGEMM_FORCE_NTW = old
 
 
+@pytest.mark.parametrize("M", [1, 31, 33, 64])
+@pytest.mark.parametrize("N,K,tiles,splits", [(96, 256, 2, 4), (1000, 512, 2, 1), (2048, 8192, 2, 4), (480, 1024, 4, 4), (3584, 1792, 4, 7), (128, 4096, 2, 16)])
+def test_strips_in_parts_of_the_depth(M, N, K, tiles, splits):
+    """Slabs of one K-tile and more, ragged rows and columns; nothing behind the last slab is written; a bias or another type is refused."""
+    from llm_consensus_amd.ops import hip as h
+
+    X, W = bf(rand(M, K, scale=0.5)), bf(rand(N, K, scale=0.5, seed=1))
+    lw, x = ops.LinearWeight.from_dense(W, None, DEV), X.to(DEV)
+    part = torch.full((splits * M + 1, N), 7.0, device=DEV)
+    args = (M, N, K, lw.n_pad, N)
+    h.call("lc_gemm_strip", lw.data.data_ptr(), x.data_ptr(), part.data_ptr(), None, *args, ops.EPI_F32, tiles, 0.0, 0.0, splits)
+    assert rel_err(part[:-1].view(splits, M, N).sum(0), ref.linear(X, W, None, torch.float32)) < 1e-4
+    k = K // splits
+    assert rel_err(part[(splits - 1) * M:-1], ref.linear(X[:, K - k:], W[:, K - k:], None, torch.float32)) < 1e-4
+    assert torch.equal(part[-1], torch.full_like(part[-1], 7.0))
+    if splits > 1:
+        for epi, bias in ((ops.EPI_BF16, None), (ops.EPI_F32, x.data_ptr())):
+            with pytest.raises(h.KernelLaunchError):
+                h.call("lc_gemm_strip", lw.data.data_ptr(), x.data_ptr(), part.data_ptr(), bias, *args, epi, tiles, 0.0, 0.0, splits)
+
+
 @pytest.mark.parametrize("M", [9, 31, 32, 33, 64])
 @pytest.mark.parametrize("N,K", [(96, 512), (1120, 896), (5344, 2048), (8224, 512), (8192, 4096)])
 def test_whole_products_of_strips(M, N, K):

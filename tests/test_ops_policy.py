@@ -71,3 +71,11 @@ def test_gemm256_plan_stays_within_its_kernels():
     assert ops._gemm256_plan(3001, 2048, 8192, 4, True, 8, False, True)[0] == 8
     # 320 tiles of 256 rows are a round and a quarter; lower tiles fill two rounds that are shorter
     assert ops._gemm256_plan(2361, 8192, 2048, 2, False, 8, False, False)[0] < 8
+
+
+def test_strip_splits_stay_within_a_round():
+    for n_pad in (128, 1024, 2048, 3584, 4096, 4608, 6144, 8192, 12288, 16384, 28672):
+        for K in (64, 512, 896, 2048, 3584, 8192, 14336, 18944):
+            tiles, s = ops._strip_splits(n_pad, K)
+            assert tiles in (2, 4) and n_pad % (16 * tiles) == 0
+            assert s == 1 or ((n_pad // (16 * tiles)) * s <= 256 and (K // 64) % s == 0 and K // 64 // s >= 4)
