@@ -27,7 +27,7 @@
 // (benchmarks/micro/gemm256w_bench.hip, 8192 rows, random data, results bit-identical):
 // K = 14336 (down projection) 645 vs 666 us (1.49 vs 1.44 PFLOP/s); at K = 4096 the longer
 // prologue (four activation stages, two weight sets) costs more than the loop gains: gate/up 1360 vs
-// 1311 us, QKV 293 vs 290, O 194 vs 198. ops.linear therefore takes this kernel for K >= 8192 only.
+// 1311 us, QKV 293 vs 290, O 194 vs 198. ops.linear therefore considers this kernel for K >= 8192 only (gemm256_plan).
 //
 // Operand conventions as in gemm256.hip: packed weights (1-KiB MFMA fragments) are the A operand and
 // never pass through LDS, activations are the B operand, staged as whole 128-byte rows into an

@@ -23,7 +23,7 @@ WS_MAX_M = int(os.environ.get("LC_WS_MAX_M", "256"))
 # Fewest 256x256 tiles for which the 256x256 pipelined kernel is used. It beats the 128x128 kernel
 # even when its tiles cover a third of the CUs (160 tiles: 171 vs 308 us, 80 tiles: 145 vs 155 us at
 # K = 8192), and below half coverage its split-K form takes over, so the default is "always".
-# -1 disables the kernel (128x128 tiles everywhere).
+# 0 keeps every tile at 256 rows (gemm256_plan), -1 disables the kernel (128x128 tiles everywhere).
 GEMM256_MIN_TILES = int(os.environ.get("LC_GEMM256_MIN_TILES", "1"))
 # Reduction depth from which prefill-sized GEMMs take the four-wave 256 x 256 kernel (gemm256w.hip):
 # its longer prologue pays off only over many K-tiles (0 = never).
@@ -294,8 +294,8 @@ class PartialSum:
 
 
 def use_four_wave_gemm(k: int, out_f32: bool = False) -> bool:
-    """Whether a prefill-sized GEMM (256 x 256 tiles) of reduction depth ``k`` takes the four-wave
-    kernel (gemm256w.hip) instead of the eight-wave one: from GEMM256W_MIN_K on (the down
+    """Whether a prefill-sized GEMM of reduction depth ``k`` may take the four-wave
+    kernel (gemm256w.hip) instead of the eight-wave one (gemm256_plan decides): from GEMM256W_MIN_K on (the down
     projections of the served models: K = 14336 / 18944 / 28672; QKV, O and gate/up have K = d_model).
     The four-wave kernel has bf16 and SwiGLU epilogues only and needs at least four K-tiles."""
     return not out_f32 and k >= max(GEMM256W_MIN_K, 256)
